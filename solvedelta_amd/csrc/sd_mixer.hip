@@ -23,6 +23,33 @@ __device__ __forceinline__ float softplus20(float x) {
   return x > 20.f ? x : log1pf(__expf(x));
 }
 
+// VEC (1 or 2) neighbouring bf16 channels of one token, kept packed until used:
+// two channels are one 4-byte access.
+template <int VEC> struct BfV;
+template <> struct BfV<1> {
+  __bf16 v;
+  __device__ __forceinline__ void get(float (&x)[1]) const { x[0] = bf2f(v); }
+};
+template <> struct BfV<2> {
+  unsigned v;
+  __device__ __forceinline__ void get(float (&x)[2]) const {
+    x[0] = __uint_as_float(v << 16);
+    x[1] = __uint_as_float(v & 0xffff0000u);
+  }
+};
+template <int VEC>
+__device__ __forceinline__ BfV<VEC> ldv(const __bf16* p) {
+  return *reinterpret_cast<const BfV<VEC>*>(p);
+}
+template <int VEC>
+__device__ __forceinline__ void stv(__bf16* p, const float (&x)[VEC]) {
+  typedef __bf16 V __attribute__((ext_vector_type(VEC)));
+  V v;
+#pragma unroll
+  for (int c = 0; c < VEC; ++c) v[c] = f2bf(x[c]);
+  *reinterpret_cast<V*>(p) = v;
+}
+
 // ---------------------------------------------------------------------------
 // conv4 + SiLU.  One thread per (channel, batch row, CONV_TC-token chunk): the
 // chunk's inputs (plus the 3-token halo) are loaded into registers up front so
@@ -371,145 +398,321 @@ static inline int cdiv(long long a, int b) { return (int)((a + b - 1) / b); }
 // conv4 + SiLU under valid / reset masks, the CPU loop's semantics
 // (model.py:146-164): a reset on a valid token zeroes the 3-token state first;
 // an invalid token emits 0 and leaves the state; a valid token emits
-// silu(w . [state, x_t]) and shifts x_t into the state.  One thread per
-// (channel, batch row) walks the row, 8 tokens' loads issued at a time: the
-// masks make each window depend on the row's whole history, so the row is not
-// cut into chunks.
+// silu(w . [state, x_t]) and shifts x_t into the state.
+//
+// A chunk's window depends on the row's history only through the last three
+// valid tokens since the last reset, so each workgroup finds those by scanning
+// the masks backwards from its chunk, 64 tokens per ballot (the result is wave
+// uniform, held in scalar registers), and chunks run in parallel.  The scan ends
+// within its first ballot unless the row holds long invalid stretches.  HBM
+// bound: 33 us forward (3.1 TB/s of x and y) and 55 us backward (2.8 TB/s of x,
+// dy and dx) at B4 T2048 D3072, where one thread walking a whole row serially
+// (a load latency per 8 tokens, 48 workgroups in all) took 1374 and 1588 us.
 // ---------------------------------------------------------------------------
 struct ConvMask {
   const uint8_t* __restrict__ valid;  // [B,T] at b*sb + t*st, nullable (all valid)
   const uint8_t* __restrict__ reset;  // nullable (no reset)
   long long sb, st;
 };
-constexpr int MCONV_U = 8;
+// Backward workgroups (and dw partial rows) per batch row: with more chunks than
+// this a workgroup takes every MCONV_PARTS-th, which bounds the workspace
+// whatever the row length.
+constexpr int MCONV_PARTS = 64;
+constexpr int MCONV_TC = 32;   // tokens per chunk (16 in the backward measured the same, 56 us)
+constexpr int kNoSlot = -4;    // a window slot cleared by a reset
 
-__device__ __forceinline__ void conv_mask_at(const ConvMask& m, int b, int t, bool& v, bool& r) {
-  const long long o = (long long)b * m.sb + (long long)t * m.st;
-  v = m.valid ? m.valid[o] != 0 : true;
-  r = v && m.reset && m.reset[o] != 0;
+// Valid bits and reset-on-valid bits of tokens base .. base + 63 (0 outside [0, T)).
+__device__ __forceinline__ void conv_mask_bits(const ConvMask& m, int b, int base, int T,
+                                               unsigned long long& V, unsigned long long& R) {
+  const int t = base + lane_id();
+  const bool in = t >= 0 && t < T;
+  const long long o = (long long)b * m.sb + (long long)(in ? t : 0) * m.st;
+  const bool v = in && (m.valid ? m.valid[o] != 0 : true);
+  const bool r = v && m.reset && m.reset[o] != 0;
+  V = __ballot(v);
+  R = __ballot(r);
 }
 
-__global__ __launch_bounds__(NTHREADS) void k_conv_masked_fwd(ConvArgs a, ConvMask m,
-                                                              __bf16* __restrict__ y,
-                                                              __bf16* __restrict__ fin) {
-  const int d = blockIdx.x * NTHREADS + threadIdx.x, b = blockIdx.y;
-  if (d >= a.D) return;
-  const int T = a.T;
-  const float w0 = a.w[d * 4], w1 = a.w[d * 4 + 1], w2 = a.w[d * 4 + 2], w3 = a.w[d * 4 + 3];
-  float s0 = conv_x(a, b, -3, d), s1 = conv_x(a, b, -2, d), s2 = conv_x(a, b, -1, d);
-  for (int t0 = 0; t0 < T; t0 += MCONV_U) {
-    float xv[MCONV_U];
-    bool vv[MCONV_U], rr[MCONV_U];
-#pragma unroll
-    for (int j = 0; j < MCONV_U; ++j) {
-      const int t = t0 + j < T ? t0 + j : T - 1;
-      xv[j] = bf2f(a.x[(long long)b * a.sb + (long long)t * a.st + d]);
-      conv_mask_at(m, b, t, vv[j], rr[j]);
+// The window before token t0: p[0] the newest slot .. p[2] the oldest, each a
+// token (>= 0), an initial-state slot (-1 newest .. -3) or kNoSlot.
+__device__ __forceinline__ void conv_lookback(const ConvMask& m, int b, int t0, int T, int (&p)[3]) {
+  int n = 0;
+  bool closed = false;
+  p[0] = p[1] = p[2] = kNoSlot;
+  for (int base = t0 - 64; n < 3 && !closed && base > -64; base -= 64) {
+    unsigned long long V, R;
+    conv_mask_bits(m, b, base, T, V, R);
+    while (V && n < 3 && !closed) {
+      const int i = 63 - __clzll((long long)V);
+      if (n == 0) p[0] = base + i;
+      else if (n == 1) p[1] = base + i;
+      else p[2] = base + i;
+      ++n;
+      closed = (R >> i) & 1;
+      V &= ~(1ull << i);
     }
-#pragma unroll
-    for (int j = 0; j < MCONV_U; ++j) {
-      const int t = t0 + j;
-      if (t < T) {
-        if (rr[j]) s0 = s1 = s2 = 0.f;
-        const float acc = w0 * s0 + w1 * s1 + w2 * s2 + w3 * xv[j];
-        y[((long long)b * T + t) * a.D + d] = f2bf(vv[j] ? silu(acc) : 0.f);
-        if (vv[j]) {
-          s0 = s1;
-          s1 = s2;
-          s2 = xv[j];
-        }
+  }
+  if (!closed) {  // the row's start: the initial state's newest slots follow
+    if (n == 0) { p[0] = -1; p[1] = -2; p[2] = -3; }
+    else if (n == 1) { p[1] = -1; p[2] = -2; }
+    else if (n == 2) p[2] = -1;
+  }
+}
+
+// Up to three valid tokens from t1 on, up to the first reset (which sees
+// nothing earlier); returns their count.  closed: a reset ended the scan.
+__device__ __forceinline__ int conv_lookahead(const ConvMask& m, int b, int t1, int T, int (&p)[3],
+                                              bool& closed) {
+  int n = 0;
+  closed = false;
+  p[0] = p[1] = p[2] = T - 1;
+  for (int base = t1; n < 3 && !closed && base < T; base += 64) {
+    unsigned long long V, R;
+    conv_mask_bits(m, b, base, T, V, R);
+    while (V && n < 3 && !closed) {
+      const int i = __ffsll((unsigned long long)V) - 1;
+      if ((R >> i) & 1) {
+        closed = true;
+      } else {
+        if (n == 0) p[0] = base + i;
+        else if (n == 1) p[1] = base + i;
+        else p[2] = base + i;
+        ++n;
+        V &= ~(1ull << i);
       }
     }
   }
-  if (fin) {
-    __bf16* f = fin + ((long long)b * a.D + d) * 3;
-    f[0] = f2bf(s0);
-    f[1] = f2bf(s1);
-    f[2] = f2bf(s2);
+  return n;
+}
+
+// One window slot's values for this thread's channels.
+template <int VEC>
+__device__ __forceinline__ void conv_slot(const ConvArgs& a, int b, int p, unsigned d, float (&v)[VEC]) {
+  ldv<VEC>(a.x + (long long)b * a.sb + (long long)(p >= 0 ? p : 0) * a.st + d).get(v);
+#pragma unroll
+  for (int c = 0; c < VEC; ++c) {
+    if (p < 0) v[c] = 0.f;
+    if (p < 0 && p > kNoSlot && a.init) v[c] = bf2f(a.init[((long long)b * a.D + d + c) * 3 + p + 3]);
   }
 }
 
-// Backward in one forward walk.  Each window slot carries its owner (a token
-// t >= 0, an initial-state slot -1..-3, or kNoOwner after a reset) and the
-// cotangent gathered for it so far; a slot's cotangent is complete when its
-// value leaves the window (shift, reset, or the end of the row, where the
-// final-state cotangent joins it) and is written to dx / dinit then.  Invalid
-// tokens get dx = 0.  dw partials per (row, channel) go to the workspace.
-constexpr int kNoOwner = -1000;
-
-__device__ __forceinline__ void conv_flush(int owner, float g, __bf16* __restrict__ dx,
-                                           float* __restrict__ dinit, int b, int T, int D, int d) {
-  if (owner >= 0) dx[((long long)b * T + owner) * D + d] = f2bf(g);
-  else if (owner > kNoOwner && dinit) dinit[((long long)b * D + d) * 3 + (-owner - 1)] = g;
+template <int VEC>
+__global__ __launch_bounds__(NTHREADS) void k_conv_masked_fwd(ConvArgs a, ConvMask m,
+                                                              __bf16* __restrict__ y,
+                                                              __bf16* __restrict__ fin) {
+  constexpr int TC = MCONV_TC;
+  const int d0 = (blockIdx.x * NTHREADS + threadIdx.x) * VEC, b = blockIdx.z;
+  const int T = a.T, D = a.D;
+  const bool live = d0 < D;  // (whole waves take part in the ballots)
+  const unsigned d = live ? d0 : 0;  // 32-bit lane offset from a wave-uniform row
+  float w[VEC][4];
+#pragma unroll
+  for (int c = 0; c < VEC; ++c)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[c][k] = a.w[(d + c) * 4 + k];
+  for (int t0 = blockIdx.y * TC; t0 < T; t0 += gridDim.y * TC) {
+    unsigned long long V, R;
+    conv_mask_bits(m, b, t0, T, V, R);
+    const bool last = t0 + TC >= T;
+    __bf16* yr = y + ((long long)b * T + t0) * D;
+    if ((unsigned)V == 0 && !(last && fin)) {  // no valid token in the chunk
+      if (live)
+#pragma unroll
+        for (int j = 0; j < TC; ++j)
+          if (t0 + j < T) stv<VEC>(yr + (long long)j * D + d, {});
+      continue;
+    }
+    BfV<VEC> xv[TC];
+#pragma unroll
+    for (int j = 0; j < TC; ++j)
+      xv[j] = ldv<VEC>(a.x + (long long)b * a.sb + (long long)min(t0 + j, T - 1) * a.st + d);
+    int p[3];
+    conv_lookback(m, b, t0, T, p);
+    float s0[VEC], s1[VEC], s2[VEC];
+    conv_slot<VEC>(a, b, p[2], d, s0);
+    conv_slot<VEC>(a, b, p[1], d, s1);
+    conv_slot<VEC>(a, b, p[0], d, s2);
+    if (!live) continue;
+#pragma unroll
+    for (int j = 0; j < TC; ++j) {
+      const bool v = (V >> j) & 1, r = (R >> j) & 1;
+      float x[VEC], o[VEC];
+      xv[j].get(x);
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) {
+        if (r) s0[c] = s1[c] = s2[c] = 0.f;
+        const float acc = w[c][0] * s0[c] + w[c][1] * s1[c] + w[c][2] * s2[c] + w[c][3] * x[c];
+        o[c] = v ? silu(acc) : 0.f;
+        s0[c] = v ? s1[c] : s0[c];
+        s1[c] = v ? s2[c] : s1[c];
+        s2[c] = v ? x[c] : s2[c];
+      }
+      if (t0 + j < T) stv<VEC>(yr + (long long)j * D + d, o);
+    }
+    if (fin && last) {
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) {
+        __bf16* f = fin + ((long long)b * D + d + c) * 3;
+        f[0] = f2bf(s0[c]);
+        f[1] = f2bf(s1[c]);
+        f[2] = f2bf(s2[c]);
+      }
+    }
+  }
 }
 
+// Backward.  A forward sweep over the chunk's tokens and the next three valid
+// ones forms da_t = dy_t silu'(a_t) and the dw partials; a reverse sweep then
+// gathers dx_s = w3 da_s + w2 da_n1 + w1 da_n2 + w0 da_n3 over the next valid
+// tokens n1, n2, n3 of s's segment, plus the final state's cotangent where s is
+// one of the row's last three.  Chunk 0 holds (through its look-ahead) the
+// row's first three valid tokens and forms dinit.
+template <int VEC>
 __global__ __launch_bounds__(NTHREADS) void k_conv_masked_bwd(ConvArgs a, ConvMask m,
                                                               const __bf16* __restrict__ dy,
                                                               const __bf16* __restrict__ dfin,
                                                               __bf16* __restrict__ dx,
                                                               float* __restrict__ dinit,
                                                               float* __restrict__ dw_part) {
-  const int d = blockIdx.x * NTHREADS + threadIdx.x, b = blockIdx.y;
-  if (d >= a.D) return;
+  constexpr int TC = MCONV_TC;
+  const int d0 = (blockIdx.x * NTHREADS + threadIdx.x) * VEC, b = blockIdx.z;
   const int T = a.T, D = a.D;
-  const float w0 = a.w[d * 4], w1 = a.w[d * 4 + 1], w2 = a.w[d * 4 + 2], w3 = a.w[d * 4 + 3];
-  float s0 = conv_x(a, b, -3, d), s1 = conv_x(a, b, -2, d), s2 = conv_x(a, b, -1, d);
-  int o0 = a.init ? -1 : kNoOwner, o1 = a.init ? -2 : kNoOwner, o2 = a.init ? -3 : kNoOwner;
-  float p0 = 0.f, p1 = 0.f, p2 = 0.f;
-  float g0 = 0.f, g1 = 0.f, g2 = 0.f, g3 = 0.f;
-  for (int t0 = 0; t0 < T; t0 += MCONV_U) {
-    float xv[MCONV_U], gv[MCONV_U];
-    bool vv[MCONV_U], rr[MCONV_U];
+  const bool live = d0 < D;  // (whole waves take part in the ballots)
+  const unsigned d = live ? d0 : 0;  // 32-bit lane offset from a wave-uniform row
+  float w[VEC][4], gw[VEC][4];
 #pragma unroll
-    for (int j = 0; j < MCONV_U; ++j) {
-      const int t = t0 + j < T ? t0 + j : T - 1;
-      xv[j] = bf2f(a.x[(long long)b * a.sb + (long long)t * a.st + d]);
-      gv[j] = bf2f(dy[((long long)b * T + t) * D + d]);
-      conv_mask_at(m, b, t, vv[j], rr[j]);
+  for (int c = 0; c < VEC; ++c)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      w[c][k] = a.w[(d + c) * 4 + k];
+      gw[c][k] = 0.f;
     }
+  for (int t0 = blockIdx.y * TC; t0 < T; t0 += gridDim.y * TC) {
+    unsigned long long V, R;
+    conv_mask_bits(m, b, t0, T, V, R);
+    __bf16* dxr = dx + ((long long)b * T + t0) * D;
+    if ((unsigned)V == 0 && !(t0 == 0 && dinit && a.init)) {
+      if (live)
 #pragma unroll
-    for (int j = 0; j < MCONV_U; ++j) {
-      const int t = t0 + j;
-      if (t >= T) continue;
-      if (!vv[j]) {
-        dx[((long long)b * T + t) * D + d] = f2bf(0.f);
-        continue;
+        for (int j = 0; j < TC; ++j)
+          if (t0 + j < T) stv<VEC>(dxr + (long long)j * D + d, {});
+      continue;
+    }
+    BfV<VEC> xv[TC], gv[TC], xh[3], gh[3];
+#pragma unroll
+    for (int j = 0; j < TC; ++j) {
+      const int t = min(t0 + j, T - 1);
+      xv[j] = ldv<VEC>(a.x + (long long)b * a.sb + (long long)t * a.st + d);
+      gv[j] = ldv<VEC>(dy + ((long long)b * T + t) * D + d);
+    }
+    int p[3], q[3];
+    bool closed;
+    conv_lookback(m, b, t0, T, p);
+    const int nh = conv_lookahead(m, b, t0 + TC, T, q, closed);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      xh[i] = ldv<VEC>(a.x + (long long)b * a.sb + (long long)q[i] * a.st + d);
+      gh[i] = ldv<VEC>(dy + ((long long)b * T + q[i]) * D + d);
+    }
+    float s0[VEC], s1[VEC], s2[VEC];
+    conv_slot<VEC>(a, b, p[2], d, s0);
+    conv_slot<VEC>(a, b, p[1], d, s1);
+    conv_slot<VEC>(a, b, p[0], d, s2);
+    if (!live) continue;
+    // (V and R are wave uniform: scalar branches, with no memory operation inside)
+    float da[TC + 3][VEC];
+#pragma unroll
+    for (int j = 0; j < TC + 3; ++j) {
+      const bool v = j < TC ? (V >> j) & 1 : j - TC < nh, r = j < TC ? (R >> j) & 1 : false;
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) da[j][c] = 0.f;
+      if (!v) continue;  // an invalid token's values may be anything
+      float x[VEC], g[VEC];
+      (j < TC ? xv[j < TC ? j : 0] : xh[j < TC ? 0 : j - TC]).get(x);
+      (j < TC ? gv[j < TC ? j : 0] : gh[j < TC ? 0 : j - TC]).get(g);
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) {
+        if (r) s0[c] = s1[c] = s2[c] = 0.f;
+        const float acc = w[c][0] * s0[c] + w[c][1] * s1[c] + w[c][2] * s2[c] + w[c][3] * x[c];
+        const float sg = sigm(acc);
+        da[j][c] = g[c] * sg * (1.f + acc * (1.f - sg));
+        if (j < TC) {
+          gw[c][0] += da[j][c] * s0[c];
+          gw[c][1] += da[j][c] * s1[c];
+          gw[c][2] += da[j][c] * s2[c];
+          gw[c][3] += da[j][c] * x[c];
+        }
+        s0[c] = s1[c];
+        s1[c] = s2[c];
+        s2[c] = x[c];
       }
-      if (rr[j]) {
-        conv_flush(o0, p0, dx, dinit, b, T, D, d);
-        conv_flush(o1, p1, dx, dinit, b, T, D, d);
-        conv_flush(o2, p2, dx, dinit, b, T, D, d);
-        s0 = s1 = s2 = 0.f;
-        p0 = p1 = p2 = 0.f;
-        o0 = o1 = o2 = kNoOwner;
+    }
+    // the final state's cotangent: the token with `rank` valid ones after it, and
+    // no reset in between, is slot 2 - rank of the final window
+    float df[VEC][3], e1[VEC], e2[VEC], e3[VEC];
+    int rank = nh;
+    bool alive = dfin && !closed && nh < 3;
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) df[c][k] = alive ? bf2f(dfin[((long long)b * D + d + c) * 3 + k]) : 0.f;
+      e1[c] = da[TC][c];
+      e2[c] = da[TC + 1][c];
+      e3[c] = da[TC + 2][c];
+    }
+    auto dfin_at = [&](int c, int slot) {
+      return !alive || slot < 0 ? 0.f : slot == 2 ? df[c][2] : slot == 1 ? df[c][1] : df[c][0];
+    };
+#pragma unroll
+    for (int j = TC - 1; j >= 0; --j) {
+      float o[VEC] = {};
+      if ((V >> j) & 1) {
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) {
+          o[c] = w[c][3] * da[j][c] + w[c][2] * e1[c] + w[c][1] * e2[c] + w[c][0] * e3[c] +
+                 dfin_at(c, 2 - rank);
+          e3[c] = e2[c];
+          e2[c] = e1[c];
+          e1[c] = da[j][c];
+        }
+        ++rank;
+        if ((R >> j) & 1) {
+          alive = false;
+#pragma unroll
+          for (int c = 0; c < VEC; ++c) e1[c] = e2[c] = e3[c] = 0.f;
+        }
       }
-      const float acc = w0 * s0 + w1 * s1 + w2 * s2 + w3 * xv[j];
-      const float sg = sigm(acc);
-      const float da = gv[j] * sg * (1.f + acc * (1.f - sg));
-      g0 += da * s0; g1 += da * s1; g2 += da * s2; g3 += da * xv[j];
-      p0 += da * w0; p1 += da * w1; p2 += da * w2;
-      conv_flush(o0, p0, dx, dinit, b, T, D, d);  // slot 0 leaves the window
-      s0 = s1; o0 = o1; p0 = p1;
-      s1 = s2; o1 = o2; p1 = p2;
-      s2 = xv[j]; o2 = t; p2 = da * w3;
+      if (t0 + j < T) stv<VEC>(dxr + (long long)j * D + d, o);
+    }
+    if (t0 == 0 && dinit && a.init) {  // e1, e2, e3: the row's first valid tokens, up to a reset
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) {
+        float* di = dinit + ((long long)b * D + d + c) * 3;
+        di[0] = w[c][0] * e1[c] + dfin_at(c, 0 - rank);
+        di[1] = w[c][1] * e1[c] + w[c][0] * e2[c] + dfin_at(c, 1 - rank);
+        di[2] = w[c][2] * e1[c] + w[c][1] * e2[c] + w[c][0] * e3[c] + dfin_at(c, 2 - rank);
+      }
     }
   }
-  if (dfin) {
-    const __bf16* f = dfin + ((long long)b * D + d) * 3;
-    p0 += bf2f(f[0]);
-    p1 += bf2f(f[1]);
-    p2 += bf2f(f[2]);
+  if (!live) return;
+#pragma unroll
+  for (int c = 0; c < VEC; ++c) {
+    float* wp = dw_part + (((long long)b * gridDim.y + blockIdx.y) * D + d + c) * 4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) wp[k] = gw[c][k];
   }
-  conv_flush(o0, p0, dx, dinit, b, T, D, d);
-  conv_flush(o1, p1, dx, dinit, b, T, D, d);
-  conv_flush(o2, p2, dx, dinit, b, T, D, d);
-  float* wp = dw_part + ((long long)b * D + d) * 4;
-  wp[0] = g0; wp[1] = g1; wp[2] = g2; wp[3] = g3;
 }
 
 }  // namespace sd
 
 using namespace sd;
+
+// Two channels per thread where every row of the three [.., D] operands starts
+// on a 4-byte boundary (an even channel count and even strides).
+static bool conv_pairs(const ConvArgs& a, const void* p, const void* q) {
+  const uintptr_t bits = (uintptr_t)a.x | (uintptr_t)p | (uintptr_t)q;
+  return a.D % 2 == 0 && a.sb % 2 == 0 && a.st % 2 == 0 && bits % 4 == 0;
+}
 
 extern "C" {
 
@@ -548,7 +751,7 @@ int sd_conv4_silu_bwd(int B, int T, int D, const void* x, int64_t x_sb, int64_t 
 
 size_t sd_conv4_masked_workspace_bytes(int B, int D) {
   if (B <= 0 || D <= 0) return 0;
-  return (size_t)B * D * 4 * sizeof(float);
+  return (size_t)B * MCONV_PARTS * D * 4 * sizeof(float);
 }
 
 int sd_conv4_silu_masked_fwd(int B, int T, int D, const void* x, int64_t x_sb, int64_t x_st,
@@ -559,8 +762,15 @@ int sd_conv4_silu_masked_fwd(int B, int T, int D, const void* x, int64_t x_sb, i
   if (!x || !w || !y) return SD_ERR_ARG;
   ConvArgs a{B, T, D, (const __bf16*)x, x_sb, x_st, w, (const __bf16*)init};
   ConvMask m{valid, reset, m_sb, m_st};
-  SD_LAUNCH("k_conv_masked_fwd", k_conv_masked_fwd, dim3(cdiv(D, NTHREADS), B), dim3(NTHREADS), 0,
-            (hipStream_t)stream, a, m, (__bf16*)y, (__bf16*)final_state);
+  const bool v2 = conv_pairs(a, y, y);
+  const int nch = cdiv(T, MCONV_TC);
+  const dim3 grid(cdiv(D, NTHREADS * (v2 ? 2 : 1)), nch < 32768 ? nch : 32768, B);
+  if (v2)
+    SD_LAUNCH("k_conv_masked_fwd", k_conv_masked_fwd<2>, grid, dim3(NTHREADS), 0,
+              (hipStream_t)stream, a, m, (__bf16*)y, (__bf16*)final_state);
+  else
+    SD_LAUNCH("k_conv_masked_fwd", k_conv_masked_fwd<1>, grid, dim3(NTHREADS), 0,
+              (hipStream_t)stream, a, m, (__bf16*)y, (__bf16*)final_state);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 
@@ -575,11 +785,17 @@ int sd_conv4_silu_masked_bwd(int B, int T, int D, const void* x, int64_t x_sb, i
   ConvArgs a{B, T, D, (const __bf16*)x, x_sb, x_st, w, (const __bf16*)init};
   ConvMask m{valid, reset, m_sb, m_st};
   hipStream_t st = (hipStream_t)stream;
-  SD_LAUNCH("k_conv_masked_bwd", k_conv_masked_bwd, dim3(cdiv(D, NTHREADS), B), dim3(NTHREADS), 0,
-            st, a, m, (const __bf16*)dy, (const __bf16*)dfinal, (__bf16*)dx, dinit,
-            (float*)workspace);
+  const bool v2 = conv_pairs(a, dy, dx);
+  const int nch = cdiv(T, MCONV_TC), parts = nch < MCONV_PARTS ? nch : MCONV_PARTS;
+  const dim3 grid(cdiv(D, NTHREADS * (v2 ? 2 : 1)), parts, B);
+  if (v2)
+    SD_LAUNCH("k_conv_masked_bwd", k_conv_masked_bwd<2>, grid, dim3(NTHREADS), 0, st, a, m,
+              (const __bf16*)dy, (const __bf16*)dfinal, (__bf16*)dx, dinit, (float*)workspace);
+  else
+    SD_LAUNCH("k_conv_masked_bwd", k_conv_masked_bwd<1>, grid, dim3(NTHREADS), 0, st, a, m,
+              (const __bf16*)dy, (const __bf16*)dfinal, (__bf16*)dx, dinit, (float*)workspace);
   SD_LAUNCH("k_sum_parts", k_sum_parts, dim3(cdiv(4LL * D, 32)), dim3(NTHREADS), 0, st,
-            (const float*)workspace, B, 4 * D, dw);
+            (const float*)workspace, B * parts, 4 * D, dw);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 

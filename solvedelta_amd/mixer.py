@@ -157,8 +157,12 @@ class _Conv4SiluMaskedFn(torch.autograd.Function):
             if init.shape != (B, D, 3):
                 raise ValueError("conv initial state must have shape [B,D,3]")
             init = init.to(torch.bfloat16).contiguous()
-        valid = valid.to(torch.uint8).contiguous()
-        reset = reset.to(torch.uint8).contiguous()
+        if valid.dtype == reset.dtype == torch.bool and valid.shape == reset.shape:
+            # the copies the backward reads, in one launch (a bool is 0 or 1)
+            valid, reset = torch.stack((valid, reset)).view(torch.uint8)
+        else:
+            valid = valid.to(torch.uint8).contiguous()
+            reset = reset.to(torch.uint8).contiguous()
         y = torch.empty(B, T, D, dtype=torch.bfloat16, device=x.device)
         fin = torch.empty(B, D, 3, dtype=torch.bfloat16, device=x.device) if want_final else None
         rc = lib.sd_conv4_silu_masked_fwd(B, T, D, x.data_ptr(), x.stride(0), x.stride(1),

@@ -250,6 +250,49 @@ def test_conv4_masked_matches_oracle_loop_with_grads(with_init):
     assert torch.all(grads[0][~valid.cuda()] == 0)
 
 
+@pytest.mark.parametrize("T,D,pad", [(32, 6, 2), (33, 5, 0), (64, 6, 1), (97, 64, 0), (260, 5, 3),
+                                     (2300, 4, 0)])
+def test_conv4_masked_chunk_edges(T, D, pad):
+    """The chunk-parallel masked conv4 where a window spans chunks: resets and
+    single valid tokens at chunk edges, invalid stretches longer than one and
+    several mask scans, more chunks than dw partial rows, and odd channel counts
+    and strides (one channel per thread); invalid tokens hold NaN."""
+    mx = _mx()
+    g = torch.Generator().manual_seed(T + D)
+    B = 4
+    wide = torch.randn(B, T, D + pad, generator=g).to(torch.bfloat16)
+    valid = torch.rand(B, T, generator=g) > 0.3
+    reset = torch.rand(B, T, generator=g) > 0.95
+    valid[0, 5:max(6, T - 3)] = False       # the window reaches back over the whole row
+    valid[1] = torch.arange(T) % 31 == 0    # about one valid token per chunk
+    reset[1] = False
+    valid[2, 31::32] = True
+    reset[2, 31::32] = True                 # a reset on every chunk's last token
+    valid[3, :T // 2] = False               # the first valid token far into the row
+    reset[3] = False
+    x = wide[..., :D].clone()
+    x[~valid] = 0.0
+    w = 0.5 * torch.randn(D, 4, generator=g)
+    init = torch.randn(B, D, 3, generator=g).to(torch.bfloat16)
+    cy = torch.randn(B, T, D, generator=g).to(torch.bfloat16)
+    cf = torch.randn(B, D, 3, generator=g).to(torch.bfloat16)
+    wide[~valid] = float("nan")
+    xc = wide.cuda()[..., :D].requires_grad_()
+    wc, ic = w.cuda().requires_grad_(), init.cuda().requires_grad_()
+    y, fin = mx.conv4_silu_masked(xc, wc, valid.cuda(), reset.cuda(), ic, True)
+    grads = torch.autograd.grad((y, fin), (xc, wc, ic), (cy.cuda(), cf.cuda()))
+    leaves = [t.double().requires_grad_() for t in (x, w, init)]
+    yo, fo = conv4_loop(*leaves, valid_mask=valid, reset_mask=reset)
+    rg = torch.autograd.grad((yo, fo), leaves, (cy.double(), cf.double()))
+    assert torch.equal(fin.double().cpu(), fo.detach())
+    # bf16 results round at 2^-9 of each value; dw and dinit (bf16) sum in FP32
+    for name, a, b in zip(("y", "dx", "dw", "dinit"), (y, *grads), (yo, *rg)):
+        e = rel(a.float(), b)
+        print(f"[conv masked T{T} D{D}] {name} {e:.1e}", flush=True)
+        assert e < (1e-5 if name == "dw" else 4e-3), name
+    assert torch.all(grads[0][~valid.cuda()] == 0) and torch.all(y[~valid.cuda()] == 0)
+
+
 def test_mixer_masks_backward_matches_oracle():
     """The masked mixer (masked conv4 + masked operator, no repacking) forward and
     every parameter / input gradient against the FP64 mixer oracle."""
