@@ -315,133 +315,266 @@ __device__ __forceinline__ void stage_panels(const float* const (&src)[NA], floa
   }
 }
 
-__global__ __launch_bounds__(WT) void k_w_prep(OpParams p) {
-  extern __shared__ __align__(16) float sm[];
-  const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, vw = p.vw, ld = kw + 1;
-  float* xs = sm;                 // x  [32][kw+1]
-  float* ks = xs + WBT * ld;      // k
-  float* Gs = ks + WBT * ld;      // G
-  float* qs = Gs + WBT * ld;      // q (column output)
-  float* Ls = qs + WBT * ld;      // L, then A  [32][33]
-  float* Ps = Ls + WBT * MS;      // P
-  const long long tb = (long long)s * p.Tp + ch * WBT;
-  if (p.colout) {
-    const float* const src[4] = {p.x, p.k, p.G, p.q};
-    float* const dst[4] = {xs, ks, Gs, qs};
-    stage_panels<4>(src, dst, tb, kw, ld);
-  } else {
-    const float* const src[3] = {p.x, p.k, p.G};
-    float* const dst[3] = {xs, ks, Gs};
-    stage_panels<3>(src, dst, tb, kw, ld);
-  }
-  // this lane's values for U = A v (the MFMA B operand: tokens kb * 16 + 4 g + e
-  // of column block w + 4 j), loaded before any store of the kernel (a load
-  // issued after a store waits for it: one counter retires both)
-  const int c = threadIdx.x;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15;
-  constexpr int NJ = WMAX / 16 / 4;
-  float vb[NJ][2][4];
+// The prep and backward-prep kernels: PW waves, wave w owning the 16-coordinate
+// blocks w, w + 8 of the key axis.  Lane (g, m) holds coordinates 4 g .. 4 g + 3
+// of tokens m and 16 + m: a 16-byte load per panel and token, and the operand
+// layout of v_mfma_f32_16x16x4f32 with the sum index k = 4 g + e, so the decayed
+// Grams run from registers, each operand element formed once.
+constexpr int PW = 8;
+constexpr int PT = PW * 64;
+constexpr int PNB = WMAX / 16 / PW;  // 16-wide blocks per wave
+constexpr int XTS = WMAX + 4;        // row stride (FP32) of a staged [32][kw] panel
+constexpr int KHS = WMAX + 8;        // row stride (16-bit) of a staged [32][kw] panel
+constexpr int AS = WBT + 4;          // row stride of the staged 32 x 32 matrices
+
+struct Quad { float v[4]; };
+__device__ __forceinline__ Quad ldq(const float* p) { return *reinterpret_cast<const Quad*>(p); }
+
+// The three lower 16 x 16 blocks (0,0), (1,0), (1,1) of a 32 x 32 token Gram,
+// summed over one 16-coordinate block from factored operands a (rows) and b
+// (columns).
+__device__ __forceinline__ void gram3(const Quad (&a)[2], const Quad (&b)[2], f4 (&acc)[3]) {
 #pragma unroll
-  for (int j = 0; j < NJ; ++j)
+  for (int e = 0; e < 4; ++e) {
+    acc[0] = mfma4(a[0].v[e], b[0].v[e], acc[0]);
+    acc[1] = mfma4(a[1].v[e], b[0].v[e], acc[1]);
+    acc[2] = mfma4(a[1].v[e], b[1].v[e], acc[2]);
+  }
+}
+
+// Adds the exact terms of the block's wild coordinates (wild[e]: this lane
+// group's coordinate 4 g + e is wild) to the lane's Gram entries; fx(i, j, c) is
+// the term of tokens i, j at coordinate c, strict keeps j < i, else j <= i.
+template <class FX>
+__device__ __forceinline__ void gram3_wild(const bool (&wild)[4], int c0, bool strict, FX fx, f4 (&acc)[3]) {
+  const int l = threadIdx.x & 63, g = l >> 4, m = l & 15;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const unsigned long long mask = __ballot(wild[e]);
+    if (mask == 0) continue;
+    for (int gg = 0; gg < 4; ++gg) {
+      if (!((mask >> (gg * 16)) & 1)) continue;
+      const int c = c0 + 4 * gg + e;
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int e2 = 0; e2 < 4; ++e2) {
+          const int i = (q > 0 ? 16 : 0) + 4 * g + e2, j = (q > 1 ? 16 : 0) + m;
+          if (strict ? j < i : j <= i) acc[q][e2] += fx(i, j, c);
+        }
+    }
+  }
+}
+
+// A wave's partial Gram blocks to LDS: [slot][3][64 lanes] x 4, and the sum of
+// one block entry group over np slots from slot s0 on.
+__device__ __forceinline__ void gram3_put(float* part, int slot, const f4 (&acc)[3]) {
+  const int l = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) *reinterpret_cast<f4*>(part + ((slot * 3 + q) * 64 + l) * 4) = acc[q];
+}
+template <int NP>
+__device__ __forceinline__ f4 gram3_sum(const float* part, int s0, int q, int l) {
+  f4 a = zero4();
+#pragma unroll
+  for (int s = 0; s < NP; ++s) a += *reinterpret_cast<const f4*>(part + (((s0 + s) * 3 + q) * 64 + l) * 4);
+  return a;
+}
+
+// (I + L)^-1 of a strictly lower 32 x 32 L in LDS (row stride AS), in place, by
+// one wave: the two 16 x 16 diagonal blocks by forward substitution (one lane
+// per column), then the off-diagonal block -D1 (L10 D0) on the matrix cores.
+// Two 16-step chains side by side instead of one 32-step chain per column
+// (32 lanes each walking a whole column took 10052 clocks of the kernel).
+__device__ __forceinline__ void inverse32(float* L) {
+  const int l = threadIdx.x & 63, g = l >> 4, m = l & 15;
+  const int B0 = (g & 1) * 16;
+  float col[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    float a = (i == m) ? 1.f : 0.f;
+#pragma unroll
+    for (int q = 0; q < i; ++q) a -= L[(B0 + i) * AS + B0 + q] * col[q];
+    col[i] = (i < m) ? 0.f : a;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (g < 2) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) L[(B0 + i) * AS + B0 + m] = col[i];
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  f4 t = zero4(), a = zero4();
+#pragma unroll
+  for (int e = 0; e < 4; ++e) t = mfma4(L[(16 + m) * AS + 4 * g + e], L[(4 * g + e) * AS + m], t);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) a = mfma4(L[(16 + m) * AS + 16 + 4 * g + e], t[e], a);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int e = 0; e < 4; ++e) L[(16 + 4 * g + e) * AS + m] = -a[e];
+}
+
+// Chunk-transposed 16-bit panel dst[kw][32 tokens] from its staged rows
+// src[32][KHS]: a thread's piece is 8 tokens of one coordinate (16 bytes), a
+// wave's pieces contiguous.
+template <class E>
+__device__ __forceinline__ void store_transposed(E* dst, const E* src, int kw) {
+  typedef E V8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+  for (int q = 0; q < WMAX * 4 / PT; ++q) {
+    const int pc = threadIdx.x + PT * q, c = pc >> 2, t8 = (pc & 3) * 8;
+    if (c < kw) {
+      V8 v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = src[(t8 + e) * KHS + c];
+      *reinterpret_cast<V8*>(dst + (long long)c * WBT + t8) = v;
+    }
+  }
+}
+
+// What bounds it: at r = V = 256 a chunk moves 192 KiB (C) / 256 KiB (S) through
+// one or two workgroups per CU, so the phases between its loads and stores must
+// be short: two workgroups fit a CU (79 KB of LDS, 128 VGPRs) and overlap.  110 us
+// (C, 3.7 TB/s) and 123 us (S, 4.4 TB/s) at B4 T2048 H8 r = V = 256; one
+// four-wave workgroup per CU with every operand panel staged in LDS (110-140 KB,
+// each Gram element formed once per 16 x 16 block) took 226 us per op.
+template <bool COL>
+__global__ __launch_bounds__(PT, 4) void k_w_prep(OpParams p) {
+  extern __shared__ __align__(16) float sm[];
+  const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, vw = p.vw, nkb = kw / 16, nvb = vw / 16;
+  float* xt = sm;                                               // x~ = x e^{Gx} [32][XTS]
+  _Float16* kh = reinterpret_cast<_Float16*>(xt + WBT * XTS);   // K^ [32][KHS]
+  float* part = reinterpret_cast<float*>(kh + WBT * KHS);       // partial Grams [8][3][64][4]
+  float* Ls = part + PW * 3 * 256;                              // L, then A [32][AS]
+  const long long tb = (long long)s * p.Tp + ch * WBT;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15;
+  const long long cbase = (long long)s * p.NT + ch;
+  // this lane's values for U = A v (the MFMA B operand: tokens kb * 16 + 4 g + e
+  // of column block w + 8 j), loaded before any store of the kernel (a load
+  // issued after a store waits for it: one counter retires both)
+  float vb[PNB][2][4];
+#pragma unroll
+  for (int j = 0; j < PNB; ++j)
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        vb[j][kb][e] = p.v[(tb + kb * 16 + 4 * g + e) * vw + min(w + PW * j, nvb - 1) * 16 + m];
+  // L_ij = sum_c x_ic k_jc e^{Gx_ic - G_jc} (j < i), and for the column output
+  // P_ij = sum_c q_ic k_jc e^{G_ic - G_jc} (j <= i): the waves split the key
+  // axis; with both Grams waves 0-3 form L's and waves 4-7 P's partials
+  const bool second = COL && w >= PW / 2;
+  constexpr int STEP = COL ? PW / 2 : PW;
+  f4 acc[3] = {zero4(), zero4(), zero4()};
+#pragma unroll 1
+  for (int kb = w % STEP; kb < nkb; kb += STEP) {
+    const int c0 = kb * 16 + 4 * g;
+    const float* lp = second ? p.q : p.x;
+    const Quad gl = ldq(p.G + (tb + WBT - 1) * kw + c0);
+    Quad a[2], b[2], G[2], Gx[2];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const long long o = (tb + t2 * 16 + m) * kw + c0;
+      a[t2] = ldq(lp + o);
+      b[t2] = ldq(p.k + o);
+      G[t2] = ldq(p.G + o);
+      if constexpr (!COL) Gx[t2] = ldq(p.G + (t2 == 0 && m == 0 ? o : o - kw));  // prefix before the token
+    }
+    bool wild[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wild[e] = -gl.v[e] > WILD;
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      f16x4 k4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float gx = G[t2].v[e];
+        if constexpr (!COL) gx = t2 == 0 && m == 0 ? 0.f : Gx[t2].v[e];
+        a[t2].v[e] *= __expf(gx);
+        k4[e] = (_Float16)(b[t2].v[e] * __expf(gl.v[e] - G[t2].v[e]));
+        b[t2].v[e] = keep_exp(!wild[e], b[t2].v[e], -G[t2].v[e]);
+      }
+      const int i = t2 * 16 + m;
+      if (second) {
+        *reinterpret_cast<Quad*>(p.Qt + (tb + i) * kw + c0) = a[t2];
+      } else {
+        *reinterpret_cast<Quad*>(xt + i * XTS + c0) = a[t2];
+        *reinterpret_cast<f16x4*>(kh + i * KHS + c0) = k4;
+      }
+    }
+    if (!second && m == 0) {
+      Quad ge;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ge.v[e] = __expf(gl.v[e]);
+      *reinterpret_cast<Quad*>(p.Gam + cbase * kw + c0) = ge;
+    }
+    gram3(a, b, acc);
+    gram3_wild(wild, kb * 16, !second, [&](int i, int j, int c) {
+      const float gx = COL ? p.G[(tb + i) * kw + c] : i > 0 ? p.G[(tb + i - 1) * kw + c] : 0.f;
+      return lp[(tb + i) * kw + c] * p.k[(tb + j) * kw + c] * __expf(gx - p.G[(tb + j) * kw + c]);
+    }, acc);
+  }
+  gram3_put(part, w, acc);
+  __syncthreads();
+  if (threadIdx.x < (COL ? 2 : 1) * 192) {
+    const int half = threadIdx.x / 192, q = (threadIdx.x % 192) >> 6;
+    const f4 v = gram3_sum<STEP>(part, half * STEP, q, l);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = (q > 0 ? 16 : 0) + 4 * g + e, j = (q > 1 ? 16 : 0) + m;
+      if (half == 0) Ls[i * AS + j] = j < i ? v[e] : 0.f;
+      else p.P[cbase * WBT * WBT + i * WBT + j] = j <= i ? v[e] : 0.f;
+    }
+  } else if (threadIdx.x >= 448) {  // the zero upper blocks
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      Ls[(4 * g + e) * AS + 16 + m] = 0.f;
+      if constexpr (COL) p.P[cbase * WBT * WBT + (4 * g + e) * WBT + 16 + m] = 0.f;
+    }
+  }
+  __syncthreads();
+  if (w == 0) inverse32(Ls);  // A = (I + L)^-1
+  __syncthreads();
+  if (threadIdx.x < WBT * WBT / 4) {
+    const int i = threadIdx.x >> 3, j = (threadIdx.x & 7) * 4;
+    *reinterpret_cast<Quad*>(p.A + cbase * WBT * WBT + i * WBT + j) = *reinterpret_cast<const Quad*>(Ls + i * AS + j);
+  }
+  // W = A x~ and U = A v on FP32 matrix cores over A's lower blocks.  W is
+  // formed transposed (a lane holds four neighbouring columns of one token: one
+  // 8-byte store), -W fp16 for the state pass; U in accumulator order.
+#pragma unroll
+  for (int j = 0; j < PNB; ++j) {
+    const int nb = w + PW * j;
+    f4 aw[2] = {zero4(), zero4()}, au[2] = {zero4(), zero4()};
+    const int nk = min(nb, nkb - 1);
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int nb = w + 4 * j;
-        vb[j][kb][e] = nb * 16 < vw ? p.v[(tb + kb * 16 + 4 * g + e) * vw + nb * 16 + m] : 0.f;
+        const int k = kb * 16 + 4 * g + e;
+        const float xv = xt[k * XTS + nk * 16 + m];
+#pragma unroll
+        for (int t2 = kb; t2 < 2; ++t2) {
+          const float av = Ls[(t2 * 16 + m) * AS + k];
+          aw[t2] = mfma4(xv, av, aw[t2]);
+          au[t2] = mfma4(av, vb[j][kb][e], au[t2]);
+        }
       }
-  __syncthreads();
-  // L_ij = sum_c x_ic k_jc e^{Gx_ic - G_jc} (j < i); P_ij = sum_c q_ic k_jc e^{G_ic - G_jc} (j <= i)
-  int* wl = reinterpret_cast<int*>(Ps + WBT * MS);
-  const int nw = wild_list(Gs, ld, kw, wl, wl + WMAX);
-  auto wild = [&](int c) { return -Gs[(WBT - 1) * ld + c] > WILD; };
-  auto kb = [&](int j, int c) { return keep_exp(!wild(c), ks[j * ld + c], -Gs[j * ld + c]); };
-  gram_mfma(
-      kw, wl, nw,
-      [&](int i, int c) { return xs[i * ld + c] * __expf(gx_at(Gs, ld, i, c, p.excl)); }, kb,
-      [&](int i, int j, int c) {
-        return xs[i * ld + c] * ks[j * ld + c] * __expf(gx_at(Gs, ld, i, c, p.excl) - Gs[j * ld + c]);
-      },
-      [](int i, int j) { return j < i; }, Ls);
-  if (p.colout)
-    gram_mfma(
-        kw, wl, nw, [&](int i, int c) { return qs[i * ld + c] * __expf(Gs[i * ld + c]); }, kb,
-        [&](int i, int j, int c) {
-          return qs[i * ld + c] * ks[j * ld + c] * __expf(Gs[i * ld + c] - Gs[j * ld + c]);
-        },
-        [](int i, int j) { return j <= i; }, Ps);
-  __syncthreads();
-  // A = (I + L)^-1, one column per thread: a_i = [i == j] - sum_{m < i} L_im a_m
-  float acol[WBT];
-  if (threadIdx.x < WBT) {
-    const int j = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < WBT; ++i) {
-      float a = (i == j) ? 1.f : 0.f;
-#pragma unroll
-      for (int m = 0; m < i; ++m) a -= Ls[i * MS + m] * acol[m];
-      acol[i] = (i < j) ? 0.f : a;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x < WBT) {
-#pragma unroll
-    for (int i = 0; i < WBT; ++i) Ls[i * MS + threadIdx.x] = acol[i];
-  }
-  __syncthreads();
-  const long long mb = ((long long)s * p.NT + ch) * WBT * WBT;
-  for (int idx = threadIdx.x; idx < WBT * WBT; idx += WT) {
-    p.A[mb + idx] = Ls[(idx >> 5) * MS + (idx & 31)];
-    if (p.colout) p.P[mb + idx] = Ps[(idx >> 5) * MS + (idx & 31)];
-  }
-  // W = A x~ and U = A v on FP32 matrix cores (the sum index k = 4 g + e carried
-  // by MFMA e and lane group g); -W stored fp16 for the state pass
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int nb = w + 4 * j;
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      if (nb * 16 < kw) {
-        f4 a = zero4();
+      if (nb < nkb) {
+        f16x4 h;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int k = kb * 16 + 4 * g + e, cc = nb * 16 + m;
-            a = mfma4(Ls[(t2 * 16 + m) * MS + k], xs[k * ld + cc] * __expf(gx_at(Gs, ld, k, cc, p.excl)), a);
-          }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) p.Wneg[tb * kw + frag_off(t2 * 16 + 4 * g + e, nb * 16 + m, kw)] = (_Float16)(-a[e]);
+        for (int e = 0; e < 4; ++e) h[e] = (_Float16)(-aw[t2][e]);
+        *reinterpret_cast<f16x4*>(p.Wneg + tb * kw + frag_off(t2 * 16 + m, nb * 16 + 4 * g, kw)) = h;
       }
-      if (nb * 16 < vw) {
-        f4 a = zero4();
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a = mfma4(Ls[(t2 * 16 + m) * MS + kb * 16 + 4 * g + e], vb[j][kb][e], a);
-        *reinterpret_cast<f4*>(p.U + tb * vw + acc_off(t2, nb, l, vw)) = a;
-      }
+      if (nb < nvb) *reinterpret_cast<f4*>(p.U + tb * vw + acc_off(t2, nb, l, vw)) = au[t2];
     }
   }
-  // K^, Qt, Gam: one key coordinate per thread (K^ in fp16 for the state pass,
-  // transposed per chunk: this thread's 32 tokens contiguous)
-  if (c < kw) {
-    _Float16* const kt = p.Kt + (((long long)s * p.NT + ch) * kw + c) * WBT;
-    f16x8 kv;
-    const float gl = Gs[(WBT - 1) * ld + c];
-#pragma unroll
-    for (int i = 0; i < WBT; ++i) {
-      const long long o = (tb + i) * kw + c;
-      kv[i & 7] = (_Float16)(ks[i * ld + c] * __expf(gl - Gs[i * ld + c]));
-      if ((i & 7) == 7) *reinterpret_cast<f16x8*>(kt + i - 7) = kv;
-      if (p.colout) p.Qt[o] = qs[i * ld + c] * __expf(Gs[i * ld + c]);
-    }
-    p.Gam[((long long)s * p.NT + ch) * kw + c] = __expf(gl);
-  }
+  store_transposed(p.Kt + cbase * kw * WBT, kh, kw);
 }
 
-constexpr size_t prep_smem(int kw) {
-  return (size_t)(4 * WBT * (kw + 1) + 2 * WBT * MS + WMAX + 4) * sizeof(float);  // + wild list
+constexpr size_t prep_smem() {
+  return (size_t)(WBT * XTS + PW * 3 * 256 + WBT * AS) * sizeof(float) + (size_t)WBT * KHS * 2;
 }
 
 // ---------------------------------------------------------------------------
@@ -1955,15 +2088,19 @@ WideBwd carve_wide_bwd(void* base, const WideDims& d, size_t* total) {
 }
 
 constexpr size_t kMaxLds = 160 * 1024;  // LDS of one gfx950 CU
-static_assert(prep_smem(WMAX) <= kMaxLds && state_smem() <= kMaxLds && out_smem(WMAX, WMAX, 0) <= kMaxLds &&
+static_assert(prep_smem() <= kMaxLds / 2 && state_smem() <= kMaxLds && out_smem(WMAX, WMAX, 0) <= kMaxLds &&
                   out_smem(WMAX, WMAX, 1) <= kMaxLds && bprep_smem(WMAX) <= kMaxLds &&
                   grad_smem(WMAX) <= kMaxLds,
               "a wide kernel's LDS exceeds the CU");
 
 void launch_wprep(const OpParams& op, int n, hipStream_t st) {
-  const size_t sm = prep_smem(op.kw);
-  SD_SMEM_ONCE(k_w_prep, (int)prep_smem(WMAX));
-  SD_LAUNCH("k_w_prep", k_w_prep, dim3(op.NT, n), dim3(WT), sm, st, op);
+  if (op.colout) {
+    SD_SMEM_ONCE(k_w_prep<true>, (int)prep_smem());
+    SD_LAUNCH("k_w_prep", k_w_prep<true>, dim3(op.NT, n), dim3(PT), prep_smem(), st, op);
+  } else {
+    SD_SMEM_ONCE(k_w_prep<false>, (int)prep_smem());
+    SD_LAUNCH("k_w_prep", k_w_prep<false>, dim3(op.NT, n), dim3(PT), prep_smem(), st, op);
+  }
 }
 
 void launch_wstate(const char* name, const WStateParams& sp, int n, hipStream_t st) {
