@@ -197,15 +197,6 @@ struct OpParams {
   float *U, *Qt, *Gam;             // Qt [Tp][kw]; U [Tp][vw] (accumulator order); Gam [NT][kw]
 };
 
-// G of the erase read for token i at coordinate c: the prefix before token i
-// (predictor) or through it (memory).
-__device__ __forceinline__ float gx_at(const float* Gs, int ld, int i, int c, int excl) {
-  // branch-free: the read is unconditional (a branch around it would serialise
-  // every operand behind its own LDS wait), the first token's value selected away
-  const float v = Gs[(excl && i > 0 ? i - 1 : i) * ld + c];
-  return excl && i == 0 ? 0.f : v;
-}
-
 // Decay factors of the matrix-core Grams and applies are factored per
 // coordinate c as exp(Ga_i) * exp(-Gb_j), both prefixes inside the chunk.  That
 // is exact up to rounding while the coordinate's decay over the chunk,
@@ -239,81 +230,6 @@ __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-
-// The chunk's wild coordinates in increasing order (deterministic: wave
-// ballots and a prefix over the four waves), from the last row of the in-chunk
-// prefix G (row stride ld).  Every thread must call it; returns the count.
-__device__ __forceinline__ int wild_list(const float* Gs, int ld, int kw, int* wl, int* cnt) {
-  const int c = threadIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const bool f = c < kw && -Gs[(WBT - 1) * ld + c] > WILD;
-  const unsigned long long mask = __ballot(f);
-  if (l == 0) cnt[w] = __popcll(mask);
-  __syncthreads();
-  int off = 0;
-  for (int v = 0; v < w; ++v) off += cnt[v];
-  if (f) wl[off + __popcll(mask & ((1ull << l) - 1ull))] = c;
-  const int total = cnt[0] + cnt[1] + cnt[2] + cnt[3];
-  __syncthreads();
-  return total;
-}
-
-// M[i][j] = sum_c A(i, c) B(j, c) exp(Ga(i, c) - Gb(j, c)) for i, j < 32, kept
-// where keep(i, j), on FP32 matrix cores: wave w forms the 16 x 16 block
-// (w >> 1, w & 1) from fa(i, c) = A e^{Ga} and fb(j, c) = B e^{-Gb} (zero on
-// wild coordinates), then adds the wild coordinates' exact terms fx(i, j, c).
-template <class FA, class FB, class FX, class KEEP>
-__device__ __forceinline__ void gram_mfma(int kw, const int* wl, int nw, FA fa, FB fb, FX fx,
-                                          KEEP keep, float* M) {
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15;
-  const int bi = w >> 1, bj = w & 1;
-  f4 acc = zero4();
-#pragma unroll 4
-  for (int kb = 0; kb < kw; kb += 16) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int c = kb + 4 * g + e;
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fa(bi * 16 + m, c), fb(bj * 16 + m, c), acc, 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int i = bi * 16 + 4 * g + e, j = bj * 16 + m;
-    float v = acc[e];
-    for (int t = 0; t < nw; ++t) v += fx(i, j, wl[t]);
-    M[i * MS + j] = keep(i, j) ? v : 0.f;
-  }
-}
-
-// Stages NA [32][kw] FP32 token panels (rows from token tb) into LDS panels of
-// row stride ld.  Every thread's 16-byte loads of all of them are issued before
-// its first LDS write, so the staging costs one memory latency, not one per row.
-template <int NA>
-__device__ __forceinline__ void stage_panels(const float* const (&src)[NA], float* const (&dst)[NA],
-                                             long long tb, int kw, int ld) {
-  constexpr int PQ = WBT * WMAX / 4 / WT;  // 16-byte pieces per thread and panel at kw = 256
-  const int npc = WBT * kw / 4;
-  float4 v[NA][PQ];
-#pragma unroll
-  for (int q = 0; q < PQ; ++q) {
-    const int idx = threadIdx.x + WT * q, i = (idx * 4) / kw, c = (idx * 4) % kw;
-    if (idx < npc)
-#pragma unroll
-      for (int a = 0; a < NA; ++a) v[a][q] = *reinterpret_cast<const float4*>(src[a] + (tb + i) * kw + c);
-  }
-#pragma unroll
-  for (int q = 0; q < PQ; ++q) {
-    const int idx = threadIdx.x + WT * q, i = (idx * 4) / kw, c = (idx * 4) % kw;
-    if (idx < npc)
-#pragma unroll
-      for (int a = 0; a < NA; ++a) {
-        float* d = dst[a] + i * ld + c;
-        d[0] = v[a][q].x;
-        d[1] = v[a][q].y;
-        d[2] = v[a][q].z;
-        d[3] = v[a][q].w;
-      }
-  }
-}
 
 // The prep and backward-prep kernels: PW waves, wave w owning the 16-coordinate
 // blocks w, w + 8 of the key axis.  Lane (g, m) holds coordinates 4 g .. 4 g + 3
@@ -1260,146 +1176,185 @@ struct BprepParams {
   __bf16 *Wneg, *Kt, *At;  // reverse-pass panels: -Wn [Tp][kw] (fragment order); Kn, Ia transposed per chunk [NT][kw][32]
 };
 
-__global__ __launch_bounds__(WT) void k_w_bprep(BprepParams p) {
+// Same organisation as k_w_prep: a lane's four coordinates of a token are loaded
+// once and give the Pp Gram's operands, K^, Kn and Ia; the value side runs
+// straight from registers.  Two workgroups per CU (76 KB of LDS, 128 VGPRs):
+// 91 us (S, 4.6 TB/s) and 127 us (C, 4.2 TB/s) at B4 T2048 H8 r = V = 256, where
+// one four-wave workgroup per CU (LDS copies of every operand, 4-byte loads of
+// each panel's columns) took 174 us per op.
+template <bool COL>
+__global__ __launch_bounds__(PT, 4) void k_w_bprep(BprepParams p) {
   extern __shared__ __align__(16) float sm[];
-  const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, vw = p.vw, ld = kw + 1;
+  const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, vw = p.vw, nkb = kw / 16, nvb = vw / 16;
   const long long tb = (long long)s * p.Tp + ch * WBT;
-  const long long mb = ((long long)s * p.NT + ch) * WBT * WBT;
-  float* Al = sm;              // A [32][33]
-  float* Pl = Al + WBT * MS;   // P or Pp [32][33]
-  float* dOl = Pl + WBT * MS;  // row output: dO, k, G [32][kw+1]
-  float* kl = dOl + WBT * ld;
-  float* Gl = kl + WBT * ld;
-  // column vectors [32][256] (element i of column t at i*256+t), over the
-  // row-output panels once the Pp Gram is done with them
-  float* cv = dOl;
-  const int tid = threadIdx.x;
-  for (int idx = threadIdx.x; idx < WBT * WBT; idx += WT) {
-    Al[(idx >> 5) * MS + (idx & 31)] = p.A[mb + idx];
-    if (p.colout) Pl[(idx >> 5) * MS + (idx & 31)] = p.P[mb + idx];
-  }
-  if (!p.colout) {
-    {
-      const float* const src[3] = {p.dO, p.k, p.G};
-      float* const dst[3] = {dOl, kl, Gl};
-      stage_panels<3>(src, dst, tb, kw, ld);
-    }
-    __syncthreads();
-    int* wl = reinterpret_cast<int*>(Gl + WBT * ld);
-    const int nw = wild_list(Gl, ld, kw, wl, wl + WMAX);
-    gram_mfma(
-        kw, wl, nw, [&](int i, int c) { return dOl[i * ld + c] * __expf(Gl[i * ld + c]); },
-        [&](int j, int c) {
-          return keep_exp(-Gl[(WBT - 1) * ld + c] <= WILD, kl[j * ld + c], -Gl[j * ld + c]);
-        },
-        [&](int i, int j, int c) {
-          return dOl[i * ld + c] * kl[j * ld + c] * __expf(Gl[i * ld + c] - Gl[j * ld + c]);
-        },
-        [](int i, int j) { return j <= i; }, Pl);
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < WBT * WBT; idx += WT)
-      p.Pp[mb + idx] = Pl[(idx >> 5) * MS + (idx & 31)];
-  }
-  __syncthreads();
-  // The key side's inputs are loaded first, before any store of the value
-  // side: a load issued after a store waits for it (one counter retires both).
-  const int c = threadIdx.x;
-  float kg[WBT], kk[WBT], kx[WBT], ks2[WBT];
-  if (c < kw)
-#pragma unroll
-    for (int i = 0; i < WBT; ++i) {
-      const long long o = (tb + i) * kw + c;
-      kg[i] = p.G[o];
-      kk[i] = p.k[o];
-      kx[i] = p.x[o];
-      ks2[i] = p.colout ? p.q[o] : p.dO[o];
-    }
-  // value side: rhs = dW + P^T Y and dU = A^T rhs on FP32 matrix cores (the sum
-  // index k = 4 g + e carried by MFMA e and lane group g, so the rhs
-  // accumulators are the B operands of the dU product as they stand); Y's
-  // columns are staged in LDS by one thread per value column
+  const long long cbase = (long long)s * p.NT + ch;
+  const float* Y = COL ? p.dO : p.q;   // [Tp][vw]
+  const float* Yk = COL ? p.q : p.dO;  // [Tp][kw]
+  float* kh = sm;               // K^ [32][XTS]
+  float* Al = kh + WBT * XTS;   // A [32][AS]
+  float* Pl = Al + WBT * AS;    // P or Pp [32][AS]
+  // Kn and Ia rows [32][KHS]; their storage first holds the partial Pp Grams
+  __bf16* kn = reinterpret_cast<__bf16*>(Pl + WBT * AS);
+  __bf16* ia = kn + WBT * KHS;
+  float* part = reinterpret_cast<float*>(kn);
+  static_assert(PW * 3 * 256 * sizeof(float) <= 2 * WBT * KHS * 2, "partial Grams fit");
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15;
-  constexpr int NJ = WMAX / 16 / 4;  // column blocks per wave
-  if (c < vw)
-    for (int i = 0; i < WBT; ++i)
-      cv[i * WT + tid] = p.colout ? p.dO[(tb + i) * vw + c] : p.q[(tb + i) * vw + c];
-  f4 rhs[2][NJ];
+  if (threadIdx.x < WBT * WBT / 4) {
+    const int i = threadIdx.x >> 3, j = (threadIdx.x & 7) * 4;
+    const long long o = cbase * WBT * WBT + i * WBT + j;
+    const Quad av = ldq(p.A + o);
+    if constexpr (COL) *reinterpret_cast<Quad*>(Pl + i * AS + j) = ldq(p.P + o);
+    *reinterpret_cast<Quad*>(Al + i * AS + j) = av;
+  }
+  // key side: this lane's coordinates; row output: also the Gram
+  // Pp_ij = sum_c dO_ic k_jc e^{G_ic - G_jc} (j <= i)
+  f4 acc[3] = {zero4(), zero4(), zero4()};
+  bf16x4 kn4[PNB][2], ia4[PNB][2];
 #pragma unroll
-  for (int j = 0; j < NJ; ++j)
+  for (int j = 0; j < PNB; ++j) {
+    const int kb = w + PW * j;
+    if (kb >= nkb) continue;
+    const int c0 = kb * 16 + 4 * g;
+    const Quad gl = ldq(p.G + (tb + WBT - 1) * kw + c0);
+    Quad x[2], k[2], y[2], G[2], Gx[2];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const long long o = (tb + t2 * 16 + m) * kw + c0;
+      x[t2] = ldq(p.x + o);
+      k[t2] = ldq(p.k + o);
+      y[t2] = ldq(Yk + o);
+      G[t2] = ldq(p.G + o);
+      if constexpr (!COL) Gx[t2] = ldq(p.G + (t2 == 0 && m == 0 ? o : o - kw));  // prefix before the token
+    }
+    bool wild[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wild[e] = -gl.v[e] > WILD;
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      Quad kd;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float gx = G[t2].v[e];
+        if constexpr (!COL) gx = t2 == 0 && m == 0 ? 0.f : Gx[t2].v[e];
+        kd.v[e] = k[t2].v[e] * __expf(gl.v[e] - G[t2].v[e]);
+        kn4[j][t2][e] = (__bf16)(-x[t2].v[e] * __expf(gx));
+        y[t2].v[e] *= __expf(G[t2].v[e]);
+        ia4[j][t2][e] = (__bf16)y[t2].v[e];
+        if constexpr (!COL) k[t2].v[e] = keep_exp(!wild[e], k[t2].v[e], -G[t2].v[e]);
+      }
+      *reinterpret_cast<Quad*>(kh + (t2 * 16 + m) * XTS + c0) = kd;
+    }
+    if constexpr (!COL) {
+      gram3(y, k, acc);
+      gram3_wild(wild, kb * 16, false, [&](int i, int jj, int c) {
+        return Yk[(tb + i) * kw + c] * p.k[(tb + jj) * kw + c] *
+               __expf(p.G[(tb + i) * kw + c] - p.G[(tb + jj) * kw + c]);
+      }, acc);
+    }
+  }
+  // the value side's rows, issued before any store of the kernel
+  float yv[PNB][2][4];
+  f4 rhs[PNB][2];
+#pragma unroll
+  for (int j = 0; j < PNB; ++j) {
+    const int nb = min(w + PW * j, nvb - 1);
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int nb = w + 4 * j;
-        rhs[t2][j][e] = (p.dW && nb * 16 < vw) ? p.dW[(tb + t2 * 16 + 4 * g + e) * vw + nb * 16 + m] : 0.f;
+        const long long o = (tb + t2 * 16 + 4 * g + e) * vw + nb * 16 + m;
+        yv[j][t2][e] = Y[o];
+        rhs[j][t2][e] = COL ? 0.f : p.dW[o];
       }
-  __syncthreads();
+  }
+  if constexpr (!COL) {
+    gram3_put(part, w, acc);
+    __syncthreads();
+    if (threadIdx.x < 192) {
+      const int q = threadIdx.x >> 6;
+      const f4 v = gram3_sum<PW>(part, 0, q, l);
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int nb = w + 4 * j;
-    if (nb * 16 >= vw) continue;
+      for (int e = 0; e < 4; ++e) {
+        const int i = (q > 0 ? 16 : 0) + 4 * g + e, j = (q > 1 ? 16 : 0) + m;
+        Pl[i * AS + j] = j <= i ? v[e] : 0.f;
+      }
+    } else if (threadIdx.x < 256) {
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          rhs[t2][j] = mfma4(Pl[(kb * 16 + 4 * g + e) * MS + t2 * 16 + m],
-                             cv[(kb * 16 + 4 * g + e) * WT + nb * 16 + m], rhs[t2][j]);
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      f4 du = zero4();
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          du = mfma4(Al[(kb * 16 + 4 * g + e) * MS + t2 * 16 + m], rhs[kb][j][e], du);
-      *reinterpret_cast<f4*>(p.dU + tb * vw + acc_off(t2, nb, l, vw)) = du;
+      for (int e = 0; e < 4; ++e) Pl[(4 * g + e) * AS + 16 + m] = 0.f;
+    }
+    __syncthreads();
+    if (threadIdx.x < WBT * WBT / 4) {
+      const int i = threadIdx.x >> 3, j = (threadIdx.x & 7) * 4;
+      *reinterpret_cast<Quad*>(p.Pp + cbase * WBT * WBT + i * WBT + j) =
+          *reinterpret_cast<const Quad*>(Pl + i * AS + j);
     }
   }
-  __syncthreads();  // cv is reused for the decayed keys
-  // key side: Kn, Ia (transposed per chunk, one key coordinate per thread) and
-  // the decayed keys' columns for Wn = -A^T K^ (matrix cores, as dU)
-  if (c < kw) {
-    const float gl = kg[WBT - 1];
-    const long long cb = (((long long)s * p.NT + ch) * kw + c) * WBT;
-    bf16x8 kv, av;
 #pragma unroll
-    for (int i = 0; i < WBT; ++i) {
-      const float gi = kg[i];
-      cv[i * WT + tid] = kk[i] * __expf(gl - gi);
-      const float gx = p.excl ? (i > 0 ? kg[i - 1] : 0.f) : gi;
-      kv[i & 7] = (__bf16)(-kx[i] * __expf(gx));
-      av[i & 7] = (__bf16)(ks2[i] * __expf(gi));
-      if ((i & 7) == 7) {
-        *reinterpret_cast<bf16x8*>(p.Kt + cb + i - 7) = kv;
-        *reinterpret_cast<bf16x8*>(p.At + cb + i - 7) = av;
-      }
+  for (int j = 0; j < PNB; ++j) {
+    const int kb = w + PW * j;
+    if (kb >= nkb) continue;
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const int o = (t2 * 16 + m) * KHS + kb * 16 + 4 * g;
+      *reinterpret_cast<bf16x4*>(kn + o) = kn4[j][t2];
+      *reinterpret_cast<bf16x4*>(ia + o) = ia4[j][t2];
     }
   }
   __syncthreads();
+  // value side: rhs = dW + P^T Y and dU = A^T rhs on FP32 matrix cores over the
+  // lower blocks of P and A (the rhs accumulators are the B operands of the dU
+  // product as they stand)
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int nb = w + 4 * j;
-    if (nb * 16 >= kw) continue;
+  for (int j = 0; j < PNB; ++j) {
+    const int nb = w + PW * j;
+    f4 du[2] = {zero4(), zero4()};
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      f4 a = zero4();
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          a = mfma4(Al[(kb * 16 + 4 * g + e) * MS + t2 * 16 + m],
-                    cv[(kb * 16 + 4 * g + e) * WT + nb * 16 + m], a);
+        for (int t2 = 0; t2 <= kb; ++t2)
+          rhs[j][t2] = mfma4(Pl[(kb * 16 + 4 * g + e) * AS + t2 * 16 + m], yv[j][kb][e], rhs[j][t2]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) p.Wneg[tb * kw + frag_off(t2 * 16 + 4 * g + e, nb * 16 + m, kw)] = (__bf16)a[e];
-    }
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t2 = 0; t2 <= kb; ++t2)
+          du[t2] = mfma4(Al[(kb * 16 + 4 * g + e) * AS + t2 * 16 + m], rhs[j][kb][e], du[t2]);
+    if (nb < nvb)
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) *reinterpret_cast<f4*>(p.dU + tb * vw + acc_off(t2, nb, l, vw)) = du[t2];
   }
+  // key side: Wn = -A^T K^ (stored negated), transposed as k_w_prep's W
+#pragma unroll
+  for (int j = 0; j < PNB; ++j) {
+    const int nb = w + PW * j, nk = min(nb, nkb - 1);
+    f4 aw[2] = {zero4(), zero4()};
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = kb * 16 + 4 * g + e;
+        const float kv = kh[k * XTS + nk * 16 + m];
+#pragma unroll
+        for (int t2 = 0; t2 <= kb; ++t2) aw[t2] = mfma4(kv, Al[k * AS + t2 * 16 + m], aw[t2]);
+      }
+    if (nb < nkb)
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        bf16x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = (__bf16)aw[t2][e];
+        *reinterpret_cast<bf16x4*>(p.Wneg + tb * kw + frag_off(t2 * 16 + m, nb * 16 + 4 * g, kw)) = h;
+      }
+  }
+  store_transposed(p.Kt + cbase * kw * WBT, kn, kw);
+  store_transposed(p.At + cbase * kw * WBT, ia, kw);
 }
 
-constexpr size_t bprep_smem(int kw) {
-  const size_t panels = 3 * WBT * (size_t)(kw + 1) + WMAX + 4, cols = (size_t)WBT * WT;
-  return (2 * WBT * MS + (panels > cols ? panels : cols)) * sizeof(float);
+constexpr size_t bprep_smem() {
+  return (size_t)(WBT * XTS + 2 * WBT * AS) * sizeof(float) + (size_t)2 * WBT * KHS * 2;
 }
 
 // ---------------------------------------------------------------------------
@@ -1635,7 +1590,7 @@ __global__ __launch_bounds__(GT) void k_w_grad(GradParams p) {
   //   dk = e^{-G} (e^{G_C} wL + M2^T Y~ - M1^T x~),  Y~ = Yk e^{G}, x~ = x e^{Gx}
   //   dq = e^{G} (dOX + M2 k~)                   (column output)
   const float* Yk = p.colout ? p.q : p.dO;  // [Tp][kw]
-  auto gx_g = [&](int i, int rr) {  // branch-free, as gx_at
+  auto gx_g = [&](int i, int rr) {  // branch-free
     const float v = p.G[(tb + (p.excl && i > 0 ? i - 1 : i)) * kw + rr];
     return p.excl && i == 0 ? 0.f : v;
   };
@@ -2089,7 +2044,7 @@ WideBwd carve_wide_bwd(void* base, const WideDims& d, size_t* total) {
 
 constexpr size_t kMaxLds = 160 * 1024;  // LDS of one gfx950 CU
 static_assert(prep_smem() <= kMaxLds / 2 && state_smem() <= kMaxLds && out_smem(WMAX, WMAX, 0) <= kMaxLds &&
-                  out_smem(WMAX, WMAX, 1) <= kMaxLds && bprep_smem(WMAX) <= kMaxLds &&
+                  out_smem(WMAX, WMAX, 1) <= kMaxLds && bprep_smem() <= kMaxLds / 2 &&
                   grad_smem(WMAX) <= kMaxLds,
               "a wide kernel's LDS exceeds the CU");
 
@@ -2194,7 +2149,6 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   dp.dout = (const __bf16*)dout; dp.dO = w.dO;
   SD_LAUNCH("k_w_dout", k_w_dout, dim3(64, d.n), dim3(WT), 0, st, dp);
 
-  SD_SMEM_ONCE(k_w_bprep, (int)bprep_smem(WMAX));
   SD_SMEM_ONCE(k_w_grad, (int)grad_smem(WMAX));
 
   // ---- memory S op ----
@@ -2203,7 +2157,8 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   bs.k = f.d; bs.x = f.e; bs.q = f.chi; bs.G = f.G; bs.A = f.AS; bs.P = f.PS;
   bs.dO = w.dO; bs.dW = nullptr;
   bs.dU = w.dU; bs.Wneg = w.Wneg; bs.Kt = w.Kt; bs.At = w.At; bs.Pp = w.Pp;
-  SD_LAUNCH("k_w_bprep_s", k_w_bprep, dim3(d.NT, d.n), dim3(WT), bprep_smem(d.KP), st, bs);
+  SD_SMEM_ONCE(k_w_bprep<true>, (int)bprep_smem());
+  SD_LAUNCH("k_w_bprep_s", k_w_bprep<true>, dim3(d.NT, d.n), dim3(PT), bprep_smem(), st, bs);
   WStateParams rs{};
   rs.NT = d.NT; rs.Tp = d.Tp; rs.kw = d.KP; rs.vw = d.VP; rs.rows = in->r; rs.cols = in->V; rs.rev = 1;
   rs.Wneg = w.Wneg; rs.U = w.dU; rs.Kt = w.Kt; rs.Gam = f.Gam; rs.At = w.At; rs.Ib = w.dO;
@@ -2231,7 +2186,8 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   bc.k = f.uh; bc.x = f.xC; bc.q = f.kh; bc.G = f.G; bc.A = f.AC; bc.P = nullptr;
   bc.dO = w.dd; bc.dW = w.ddelta;
   bc.dU = w.dU; bc.Wneg = w.Wneg; bc.Kt = w.Kt; bc.At = w.At; bc.Pp = w.Pp;
-  SD_LAUNCH("k_w_bprep_c", k_w_bprep, dim3(d.NT, d.n), dim3(WT), bprep_smem(d.KP), st, bc);
+  SD_SMEM_ONCE(k_w_bprep<false>, (int)bprep_smem());
+  SD_LAUNCH("k_w_bprep_c", k_w_bprep<false>, dim3(d.NT, d.n), dim3(PT), bprep_smem(), st, bc);
   WStateParams rc{};
   rc.NT = d.NT; rc.Tp = d.Tp; rc.kw = d.KP; rc.vw = d.KP; rc.rows = in->r; rc.cols = in->r; rc.rev = 1;
   rc.Wneg = w.Wneg; rc.U = w.dU; rc.Kt = w.Kt; rc.Gam = f.Gam; rc.At = w.At; rc.Ib = f.kh;
