@@ -1382,34 +1382,101 @@ struct GradParams {
 constexpr int GW = 8;
 constexpr int GT = GW * 64;
 constexpr int GRB = WMAX / 16 / GW;
+constexpr int GS16 = 20;  // row stride (FP32) of a wave's staged [32 tokens][16 coordinates] panel
 
-__global__ __launch_bounds__(GT) void k_w_grad(GradParams p) {
+// Lane i of a 16-lane row takes lane i + N's value, 0 past the row's end.
+template <int N>
+__device__ __forceinline__ float row_next(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 + N, 0xF, 0xF, true));
+}
+// Sum over this and the following lanes of a 16-lane row.
+__device__ __forceinline__ float row_suffix(float v) {
+  v += row_next<1>(v);
+  v += row_next<2>(v);
+  v += row_next<4>(v);
+  return v + row_next<8>(v);
+}
+
+__device__ __forceinline__ f4 mma_bf(bf16x8 a, bf16x8 b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+template <class V8>
+__device__ __forceinline__ void split8(const V8& v, bf16x8& hi, bf16x8& lo) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float x = (float)v[j];
+    const __bf16 h = (__bf16)x;
+    hi[j] = h;
+    lo[j] = (__bf16)(x - (float)h);
+  }
+}
+__device__ __forceinline__ void split4_to(__bf16* hi, __bf16* lo, const Quad& q) {
+  bf16x4 h, o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    h[e] = (__bf16)q.v[e];
+    o[e] = (__bf16)(q.v[e] - (float)h[e]);
+  }
+  *reinterpret_cast<bf16x4*>(hi) = h;
+  *reinterpret_cast<bf16x4*>(lo) = o;
+}
+
+// What bounds it: the state slots (X0 and lambda, 256 KiB of a chunk's 608 KiB
+// at r = V = 256) stream through phase 1; every product's output is formed
+// transposed, so a lane holds four neighbouring coordinates of one token and
+// reads and writes the token panels 16 bytes at a time, and the rows shared by
+// all waves are split into bf16 halves once, in LDS.  301 us (S, 4.2 TB/s) and
+// 386 us (C) per launch at B4 T2048 H8 r = V = 256; with 4-byte panel accesses
+// in the MFMA layout, the rows split by every wave and dO e^G X0 on FP32 MFMAs
+// over 2-byte gathers of the slot, 360 and 500 us.
+template <bool COL>
+__global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   extern __shared__ __align__(16) float sm[];
   int ch, s;
   xcd_map(blockIdx.x, p.NT, gridDim.x / p.NT, ch, s);
-  const int kw = p.kw, vw = p.vw;
+  const int kw = p.kw, vw = p.vw, nrb = kw / 16, nvb = vw / 16;
   const long long tb = (long long)s * p.Tp + ch * WBT;
   const long long slot = (long long)s * (p.NT + 1) + ch;
   const xs_t* X0 = p.Xslots + slot * kw * vw;
   const xs_t* XC = X0 + (long long)kw * vw;
   const ls_t* Lm = p.Lslots + slot * kw * vw;
-  // LDS: the token Grams M1, M2 [32][33]; the rows dw, w, Y [3][32][vw+4]
-  // (first pass), then for the row output dO e^G [32][kw+4]
-  float* M1 = sm;
-  float* M2 = M1 + WBT * MS;
-  float* TR = M2 + WBT * MS;
-  float* DG = TR;
-  const int r = threadIdx.x;
-  const int wv_ = r >> 6, l = r & 63, g = l >> 4, m = l & 15;
-  const int nrb = kw / 16, nvb = vw / 16;
-  const float* Y = p.colout ? p.dO : p.q;  // [Tp][vw]
-  // phase 1 on matrix cores: the row products dwX = dw X0^T, wL = w lam^T, dOX = dO X0^T
-  // (column output) over this wave's 16-row blocks of the state, kept in
-  // accumulators (lane (g, n): tokens 4g..4g+3 of state row 16 rb + n) for
-  // phase 3, and the token Grams M1 = dw w^T, M2 = Y w^T (one 16 x 16 block of
-  // each per wave of the first four); the rows from LDS, the state slots by
-  // 16-byte global loads.
-  f4 aX[GRB][2], aL[GRB][2], aO[GRB][2];
+  float* M1 = sm;              // token Grams [32][AS]
+  float* M2 = M1 + WBT * AS;
+  // phase 1: dw, w, Y rows split [32][KHS]; phase 2 (row output): dO e^G split
+  // and two X0 row blocks; phase 3: per wave k~, Y~, x~ [32][GS16]
+  __bf16* TR = reinterpret_cast<__bf16*>(M2 + WBT * AS);
+  constexpr int RP = WBT * KHS;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15, kq = g * 8;
+  const float* Y = COL ? p.dO : p.q;   // [Tp][vw]
+  const float* Yk = COL ? p.q : p.dO;  // [Tp][kw]
+  {
+    constexpr int PQ = WBT * WMAX / 4 / GT;
+    Quad v[PQ][3];
+#pragma unroll
+    for (int q = 0; q < PQ; ++q) {
+      const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 4 - 1);
+      const long long o = tb * vw + idx * 4;
+      v[q][0] = ldq(p.dw + o);
+      v[q][1] = ldq(p.w + o);
+      v[q][2] = ldq(Y + o);
+    }
+#pragma unroll
+    for (int q = 0; q < PQ; ++q) {
+      const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 4 - 1);
+      const int i = (idx * 4) / vw, c = (idx * 4) % vw;
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        split4_to(TR + 2 * a * RP + i * KHS + c, TR + (2 * a + 1) * RP + i * KHS + c, v[q][a]);
+    }
+  }
+  __syncthreads();
+  // phase 1 on bf16 matrix cores (the cotangents may take any scale), K = 32
+  // value columns per step: this wave's rows of dwX = dw X0^T, wL = w lam^T and
+  // (column output) dOX = dO X0^T, transposed (lane (g, m): rows 4 g .. + 3 of
+  // token m), and one lower 16 x 16 block of M1 = dw w^T or M2 = Y w^T per wave
+  // of the first six.  The rows and the fp16 state X0 enter split into bf16
+  // high and low halves (three MFMAs per product); lambda is exact in its slot.
+  f4 aX[GRB][2], aL[GRB][2], aO[GRB][2], am = zero4();
   float rs[GRB];  // partial rowsum(X_C (.) lam) of state row 16 rb + m over this lane's columns
 #pragma unroll
   for (int q = 0; q < GRB; ++q) {
@@ -1417,325 +1484,352 @@ __global__ __launch_bounds__(GT) void k_w_grad(GradParams p) {
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) aX[q][t2] = aL[q][t2] = aO[q][t2] = zero4();
   }
-  // the chunk's dw, w, Y rows staged once into LDS (every wave reads all of them)
-  const int lt = vw + 4;
-#pragma unroll
-  for (int q = 0; q < WBT * WMAX / 4 / GT; ++q) {
-    const int idx = threadIdx.x + GT * q, i = (idx * 4) / vw, c = (idx * 4) % vw;
-    if (idx < WBT * vw / 4) {
-      const long long o = (tb + i) * vw + c;
-      const float4 a0 = *reinterpret_cast<const float4*>(p.dw + o);
-      const float4 a1 = *reinterpret_cast<const float4*>(p.w + o);
-      const float4 a2 = *reinterpret_cast<const float4*>(Y + o);
-      *reinterpret_cast<float4*>(TR + i * lt + c) = a0;
-      *reinterpret_cast<float4*>(TR + (WBT + i) * lt + c) = a1;
-      *reinterpret_cast<float4*>(TR + (2 * WBT + i) * lt + c) = a2;
-    }
-  }
-  __syncthreads();
+  const int gq = w % 3, bi = gq > 0, bj = gq > 1, gm = w < 3 ? 0 : 2;  // Gram block, left rows
   {
-    f4 m1a = zero4(), m2a = zero4();
-    const int bi = (wv_ >> 1) & 1, bj = wv_ & 1;
-    const bool gram = wv_ < 4;  // one 16 x 16 block of M1 and M2 per wave of the first four
-    const int kq = g * 8;
-    // 16-bit matrix cores over K = 32 columns per step (bf16: the cotangents
-    // may take any scale).  The FP32 rows dw, w, Y and the fp16 state X0 enter
-    // split into bf16 high and low halves (three MFMAs per product: hi.hi,
-    // hi.lo, lo.hi); lambda is exact in its bf16 slot (two MFMAs).
-    auto split8 = [](const float* v, bf16x8& hi, bf16x8& lo) {
+    unsigned ro[GRB];  // row offsets of this wave's blocks (clamped: loads stay unconditional)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const __bf16 h = (__bf16)v[j];
-        hi[j] = h;
-        lo[j] = (__bf16)(v[j] - (float)h);
-      }
-    };
-    auto mma = [](bf16x8 a, bf16x8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); };
-#pragma unroll 2
-    for (int cb = 0; cb < vw; cb += 32) {
-      bf16x8 dwh[2], dwl[2], wh[2], wl[2], yh[2], yl[2];
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
-        const int o = (t2 * 16 + m) * lt + cb + kq;
-        float v[8];
-        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(TR + o);
-        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(TR + o + 4);
-        split8(v, dwh[t2], dwl[t2]);
-        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(TR + WBT * lt + o);
-        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(TR + WBT * lt + o + 4);
-        split8(v, wh[t2], wl[t2]);
-        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(TR + 2 * WBT * lt + o);
-        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(TR + 2 * WBT * lt + o + 4);
-        split8(v, yh[t2], yl[t2]);
-      }
+    for (int q = 0; q < GRB; ++q) ro[q] = (unsigned)((min(w + GW * q, nrb - 1) * 16 + m) * vw + kq);
+    f16x8 x8[2][GRB], c8[2][GRB];
+    bf16x8 l8[2][GRB];
+    auto fetch = [&](int cb, int f) {
 #pragma unroll
       for (int q = 0; q < GRB; ++q) {
-        const int rb = wv_ + GW * q;
-        if (rb < nrb) {
-          const long long o = (long long)(rb * 16 + m) * vw + cb + kq;
-          const f16x8 x8 = *reinterpret_cast<const f16x8*>(X0 + o);
-          const f16x8 c8 = *reinterpret_cast<const f16x8*>(XC + o);
-          const bf16x8 lb = *reinterpret_cast<const bf16x8*>(Lm + o);
-          float xv[8];
+        x8[f][q] = *reinterpret_cast<const f16x8*>(X0 + cb + ro[q]);
+        l8[f][q] = *reinterpret_cast<const bf16x8*>(Lm + cb + ro[q]);
+        c8[f][q] = *reinterpret_cast<const f16x8*>(XC + cb + ro[q]);
+      }
+    };
+    auto step = [&](int cb, int f) {
+      auto row = [&](int a, int t2) { return *reinterpret_cast<const bf16x8*>(TR + a * RP + (t2 * 16 + m) * KHS + cb + kq); };
+      bf16x8 xh[GRB], xl[GRB];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            xv[j] = (float)x8[j];
-            rs[q] += (float)c8[j] * (float)lb[j];
-          }
-          bf16x8 xh, xl;
-          split8(xv, xh, xl);
+      for (int q = 0; q < GRB; ++q) {
+        split8(x8[f][q], xh[q], xl[q]);
 #pragma unroll
-          for (int t2 = 0; t2 < 2; ++t2) {
-            aX[q][t2] = mma(dwl[t2], xh, aX[q][t2]);
-            aX[q][t2] = mma(dwh[t2], xl, aX[q][t2]);
-            aX[q][t2] = mma(dwh[t2], xh, aX[q][t2]);
-            aL[q][t2] = mma(wl[t2], lb, aL[q][t2]);
-            aL[q][t2] = mma(wh[t2], lb, aL[q][t2]);
-            if (p.colout) {
-              aO[q][t2] = mma(yl[t2], xh, aO[q][t2]);
-              aO[q][t2] = mma(yh[t2], xl, aO[q][t2]);
-              aO[q][t2] = mma(yh[t2], xh, aO[q][t2]);
-            }
+        for (int j = 0; j < 8; ++j) rs[q] += (float)c8[f][q][j] * (float)l8[f][q][j];
+      }
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        const bf16x8 dh = row(0, t2), dl = row(1, t2), wh = row(2, t2), wl = row(3, t2);
+#pragma unroll
+        for (int q = 0; q < GRB; ++q) {
+          aX[q][t2] = mma_bf(xh[q], dl, aX[q][t2]);
+          aL[q][t2] = mma_bf(l8[f][q], wl, aL[q][t2]);
+          aX[q][t2] = mma_bf(xl[q], dh, aX[q][t2]);
+          aL[q][t2] = mma_bf(l8[f][q], wh, aL[q][t2]);
+          aX[q][t2] = mma_bf(xh[q], dh, aX[q][t2]);
+        }
+        if constexpr (COL) {
+          const bf16x8 yh = row(4, t2), yl = row(5, t2);
+#pragma unroll
+          for (int q = 0; q < GRB; ++q) {
+            aO[q][t2] = mma_bf(xh[q], yl, aO[q][t2]);
+            aO[q][t2] = mma_bf(xl[q], yh, aO[q][t2]);
+            aO[q][t2] = mma_bf(xh[q], yh, aO[q][t2]);
           }
         }
       }
-      if (gram) {  // selects, not indexing: a runtime index would put the arrays in scratch
-        const bf16x8 dah = bi ? dwh[1] : dwh[0], dal = bi ? dwl[1] : dwl[0];
-        const bf16x8 yah = bi ? yh[1] : yh[0], yal = bi ? yl[1] : yl[0];
-        const bf16x8 wbh = bj ? wh[1] : wh[0], wbl = bj ? wl[1] : wl[0];
-        m1a = mma(dal, wbh, m1a);
-        m1a = mma(dah, wbl, m1a);
-        m1a = mma(dah, wbh, m1a);
-        m2a = mma(yal, wbh, m2a);
-        m2a = mma(yah, wbl, m2a);
-        m2a = mma(yah, wbh, m2a);
+      if (w < 6) {
+        const bf16x8 ah = row(gm * 2, bi), al = row(gm * 2 + 1, bi), bh = row(2, bj), bl = row(3, bj);
+        am = mma_bf(al, bh, am);
+        am = mma_bf(ah, bl, am);
+        am = mma_bf(ah, bh, am);
+      }
+    };
+    fetch(0, 0);
+    int cb = 0;
+    for (; cb + 32 < vw; cb += 64) {  // (the last fetch past an odd count rereads the first columns)
+      fetch(cb + 32, 1);
+      step(cb, 0);
+      fetch(cb + 64 < vw ? cb + 64 : 0, 0);
+      step(cb + 32, 1);
+    }
+    if (cb < vw) step(cb, 0);
+  }
+  if (w < 6) {
+    float* M = w < 3 ? M1 : M2;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = bi * 16 + 4 * g + e, j = bj * 16 + m;
+      M[i * AS + j] = (w < 3 ? j < i : j <= i) ? am[e] : 0.f;
+    }
+  }
+  // this lane's elements of the key-side panels (tokens m and 16 + m), loaded
+  // before any store of the kernel
+  Quad kr[GRB][2], yr[GRB][2], xr[GRB][2], G[GRB][2], Gp[GRB][2], orw[GRB][2], gl[GRB];
+  int c0[GRB];
+#pragma unroll
+  for (int q = 0; q < GRB; ++q) {
+    c0[q] = min(w + GW * q, nrb - 1) * 16 + 4 * g;
+    gl[q] = ldq(p.G + (tb + WBT - 1) * kw + c0[q]);
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const long long o = (tb + t2 * 16 + m) * kw + c0[q];
+      kr[q][t2] = ldq(p.k + o);
+      yr[q][t2] = ldq(Yk + o);
+      xr[q][t2] = ldq(p.x + o);
+      G[q][t2] = ldq(p.G + o);
+      if constexpr (!COL) {
+        Gp[q][t2] = ldq(p.G + (t2 == 0 && m == 0 ? o : o - kw));
+        orw[q][t2] = ldq(p.o + o);
       }
     }
-    if (gram)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = bi * 16 + 4 * g + e, j = bj * 16 + m;
-        M1[i * MS + j] = j < i ? m1a[e] : 0.f;
-        M2[i * MS + j] = j <= i ? m2a[e] : 0.f;
-      }
   }
   // rowsum(X_C (.) lam): the four lane groups' partials of each state row
-  // (every lane of the row ends with the total)
 #pragma unroll
   for (int q = 0; q < GRB; ++q) {
     rs[q] += __shfl_xor(rs[q], 16);
     rs[q] += __shfl_xor(rs[q], 32);
   }
-  // phase 2 (row output): dq = (dO e^G) X0 + Pp w on matrix cores, this wave's
-  // 16-column blocks of the value axis; dO e^G is formed once into LDS
-  if (!p.colout) {
-    const long long mb = ((long long)s * p.NT + ch) * WBT * WBT;
-    const int la = kw + 4;
-    __syncthreads();  // every wave is done reading the rows DG overwrites
+  __syncthreads();  // M1, M2 complete; the split rows are dead
+  // phase 2 (row output): dq = (dO e^G) X0 + Pp w, this wave's 16-column blocks
+  // of the value axis, transposed.  The contraction runs along the slot's rows,
+  // so 32-row blocks pass through LDS (double buffered, one barrier each) and
+  // are read down their columns; bf16 halves as in phase 1, Pp w in FP32.
+  if constexpr (!COL) {
+    __bf16 *Dh = TR, *Dl = TR + RP;
+    _Float16* Xt = reinterpret_cast<_Float16*>(TR + 2 * RP);  // [2][32][KHS]
+    constexpr int XQ = WBT * WMAX / 8 / GT;
+    f16x8 xb[XQ];
+    auto fetch = [&](int rb) {
 #pragma unroll
-    for (int q = 0; q < WBT * WMAX / 4 / GT; ++q) {
-      const int idx = threadIdx.x + GT * q, i = (idx * 4) / kw, c = (idx * 4) % kw;
-      if (idx < WBT * kw / 4) {
-        const float4 d4 = *reinterpret_cast<const float4*>(p.dO + (tb + i) * kw + c);
-        const float4 g4 = *reinterpret_cast<const float4*>(p.G + (tb + i) * kw + c);
-        *reinterpret_cast<float4*>(DG + i * la + c) =
-            make_float4(d4.x * __expf(g4.x), d4.y * __expf(g4.y), d4.z * __expf(g4.z), d4.w * __expf(g4.w));
+      for (int q = 0; q < XQ; ++q) {
+        const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 8 - 1);
+        xb[q] = *reinterpret_cast<const f16x8*>(X0 + (long long)rb * vw + idx * 8);
       }
-    }
-    __syncthreads();
+    };
+    auto put = [&](int f) {
+#pragma unroll
+      for (int q = 0; q < XQ; ++q) {
+        const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 8 - 1);
+        *reinterpret_cast<f16x8*>(Xt + f * RP + (idx * 8) / vw * KHS + (idx * 8) % vw) = xb[q];
+      }
+    };
+    fetch(0);
+    float wv[GRB][2][4];
+    int nb[GRB];
 #pragma unroll
     for (int q = 0; q < GRB; ++q) {
-      const int nb = wv_ + GW * q;
-      if (nb >= nvb) continue;
-      f4 acc[2] = {zero4(), zero4()};
-#pragma unroll 4
-      for (int rb = 0; rb < nrb; ++rb) {
-        float bx[4];
+      nb[q] = min(w + GW * q, nvb - 1) * 16;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) bx[e] = (float)X0[(long long)(rb * 16 + 4 * g + e) * vw + nb * 16 + m];
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
-          const float4 a4 = *reinterpret_cast<const float4*>(DG + (t2 * 16 + m) * la + rb * 16 + 4 * g);
-          acc[t2] = mfma4(a4.x, bx[0], acc[t2]);
-          acc[t2] = mfma4(a4.y, bx[1], acc[t2]);
-          acc[t2] = mfma4(a4.z, bx[2], acc[t2]);
-          acc[t2] = mfma4(a4.w, bx[3], acc[t2]);
-        }
-      }
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        float bw[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bw[e] = p.w[(tb + kb * 16 + 4 * g + e) * vw + nb * 16 + m];
-#pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
-          const float4 a4 = *reinterpret_cast<const float4*>(p.Pp + mb + (t2 * 16 + m) * WBT + kb * 16 + 4 * g);
-          acc[t2] = mfma4(a4.x, bw[0], acc[t2]);
-          acc[t2] = mfma4(a4.y, bw[1], acc[t2]);
-          acc[t2] = mfma4(a4.z, bw[2], acc[t2]);
-          acc[t2] = mfma4(a4.w, bw[3], acc[t2]);
-        }
-      }
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) p.dq[(tb + t2 * 16 + 4 * g + e) * vw + nb * 16 + m] = acc[t2][e];
+        for (int e = 0; e < 4; ++e) wv[q][kb][e] = p.w[(tb + kb * 16 + 4 * g + e) * vw + nb[q] + m];
     }
+    Quad pp[2][2];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        pp[t2][kb] = ldq(p.Pp + ((long long)s * p.NT + ch) * WBT * WBT + (t2 * 16 + m) * WBT + kb * 16 + 4 * g);
+#pragma unroll
+    for (int q = 0; q < GRB; ++q)
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        Quad d;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d.v[e] = yr[q][t2].v[e] * __expf(G[q][t2].v[e]);
+        const int o = (t2 * 16 + m) * KHS + c0[q];
+        split4_to(Dh + o, Dl + o, d);
+      }
+    put(0);
+    __syncthreads();
+    f4 aq[GRB][2];
+#pragma unroll
+    for (int q = 0; q < GRB; ++q) aq[q][0] = aq[q][1] = zero4();
+    for (int rb = 0; rb < kw; rb += 32) {
+      const int f = (rb >> 5) & 1;
+      if (rb + 32 < kw) fetch(rb + 32);
+      bf16x8 dh[2], dl[2];
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        dh[t2] = *reinterpret_cast<const bf16x8*>(Dh + (t2 * 16 + m) * KHS + rb + kq);
+        dl[t2] = *reinterpret_cast<const bf16x8*>(Dl + (t2 * 16 + m) * KHS + rb + kq);
+      }
+#pragma unroll
+      for (int q = 0; q < GRB; ++q) {
+        f16x8 xc;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) xc[j] = Xt[f * RP + (kq + j) * KHS + nb[q] + m];
+        bf16x8 xh, xl;
+        split8(xc, xh, xl);
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2) {
+          aq[q][t2] = mma_bf(xh, dl[t2], aq[q][t2]);
+          aq[q][t2] = mma_bf(xl, dh[t2], aq[q][t2]);
+          aq[q][t2] = mma_bf(xh, dh[t2], aq[q][t2]);
+        }
+      }
+      if (rb + 32 < kw) put(f ^ 1);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < GRB; ++q)
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+#pragma unroll
+        for (int kb = 0; kb <= t2; ++kb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) aq[q][t2] = mfma4(wv[q][kb][e], pp[t2][kb].v[e], aq[q][t2]);
+        if (w + GW * q < nvb)
+          *reinterpret_cast<f4*>(p.dq + (tb + t2 * 16 + m) * vw + nb[q] + 4 * g) = aq[q][t2];
+      }
   }
-  __syncthreads();  // M1, M2 complete
-  // phase 3: the in-chunk applies on matrix cores, decay factored per state
-  // row r as e^{Ga_i} e^{-Gb_j} (exact while r's decay over the chunk is at
-  // most WILD; wild rows take the exact per-term sums):
+  // phase 3: the in-chunk applies on FP32 matrix cores over the Grams' lower
+  // blocks, decay factored per state row r as e^{Ga_i} e^{-Gb_j} (exact while r's
+  // decay over the chunk is at most WILD; wild rows take the exact per-term sums):
   //   dx = -e^{Gx} (dwX + M1 k~),               k~_jr = k_jr e^{-G_jr}
   //   dk = e^{-G} (e^{G_C} wL + M2^T Y~ - M1^T x~),  Y~ = Yk e^{G}, x~ = x e^{Gx}
   //   dq = e^{G} (dOX + M2 k~)                   (column output)
-  const float* Yk = p.colout ? p.q : p.dO;  // [Tp][kw]
-  auto gx_g = [&](int i, int rr) {  // branch-free
-    const float v = p.G[(tb + (p.excl && i > 0 ? i - 1 : i)) * kw + rr];
-    return p.excl && i == 0 ? 0.f : v;
-  };
-  float rdx[GRB][2][4], rdk[GRB][2][4], rdq[GRB][2][4], rdg[GRB][2][4];
+  // k~, Y~, x~ of a wave's 16 coordinates pass through its own LDS panels.
+  float* kt = reinterpret_cast<float*>(TR) + w * 3 * WBT * GS16;
+  float *yt = kt + WBT * GS16, *xt = yt + WBT * GS16;
+  f4 m1[2][2], m2[2][2], m1t[2][2], m2t[2][2];  // [i block][j block] of M and, for the transposes, M^T
+#pragma unroll
+  for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+    for (int jb = 0; jb <= ib; ++jb) {
+      m1[ib][jb] = *reinterpret_cast<const f4*>(M1 + (ib * 16 + m) * AS + jb * 16 + 4 * g);
+      m2[ib][jb] = *reinterpret_cast<const f4*>(M2 + (ib * 16 + m) * AS + jb * 16 + 4 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        m1t[ib][jb][e] = -M1[(ib * 16 + 4 * g + e) * AS + jb * 16 + m];
+        m2t[ib][jb][e] = M2[(ib * 16 + 4 * g + e) * AS + jb * 16 + m];
+      }
+    }
 #pragma unroll
   for (int q = 0; q < GRB; ++q) {
-    const int rb = wv_ + GW * q;
-    if (rb >= nrb) continue;
-    const int rr = rb * 16 + m;  // this lane's state row (output column)
-    const float gl = p.G[(tb + WBT - 1) * kw + rr];
-    const bool wild = -gl > WILD;
-    // the lane's operands at tokens jb * 16 + 4 g + e of row rr: the same
-    // tokens its outputs (t2 = jb) cover, so the decay closure below needs no
-    // further loads
-    float kt[2][4], yt[2][4], xt[2][4], kr[2][4], yr[2][4], xr[2][4], orw[2][4];
+    if (w + GW * q >= nrb) continue;
+    bool wild[4];
+    float gx[2][4];
+    bool any = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      wild[e] = -gl[q].v[e] > WILD;
+      any |= wild[e];
+    }
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      Quad a, b, c;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        gx[t2][e] = COL ? G[q][t2].v[e] : t2 == 0 && m == 0 ? 0.f : Gp[q][t2].v[e];
+        a.v[e] = keep_exp(!wild[e], kr[q][t2].v[e], -G[q][t2].v[e]);
+        b.v[e] = keep_exp(!wild[e], yr[q][t2].v[e], G[q][t2].v[e]);
+        c.v[e] = keep_exp(!wild[e], xr[q][t2].v[e], gx[t2][e]);
+      }
+      const int o = (t2 * 16 + m) * GS16 + 4 * g;
+      *reinterpret_cast<Quad*>(kt + o) = a;
+      *reinterpret_cast<Quad*>(yt + o) = b;
+      *reinterpret_cast<Quad*>(xt + o) = c;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own panels
+    f4 ax[2], ak[2], aq[2];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      ax[t2] = aX[q][t2];
+      aq[t2] = aO[q][t2];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ak[t2][e] = __expf(gl[q].v[e]) * aL[q][t2][e];
+    }
 #pragma unroll
     for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int j = jb * 16 + 4 * g + e;
-        const long long o = (tb + j) * kw + rr;
-        const float gj = p.G[o];
-        kr[jb][e] = p.k[o];
-        yr[jb][e] = Yk[o];
-        xr[jb][e] = p.x[o];
-        orw[jb][e] = p.colout ? 0.f : p.o[o];
-        kt[jb][e] = keep_exp(!wild, kr[jb][e], -gj);
-        yt[jb][e] = keep_exp(!wild, yr[jb][e], gj);
-        xt[jb][e] = keep_exp(!wild, xr[jb][e], gx_g(j, rr));
+        const int o = (jb * 16 + 4 * g + e) * GS16 + m;
+        const float kv = kt[o], yv = yt[o], xv = xt[o];
+#pragma unroll
+        for (int t2 = jb; t2 < 2; ++t2) {
+          ax[t2] = mfma4(kv, m1[t2][jb][e], ax[t2]);
+          if constexpr (COL) aq[t2] = mfma4(kv, m2[t2][jb][e], aq[t2]);
+        }
+#pragma unroll
+        for (int t2 = 0; t2 <= jb; ++t2) {
+          ak[t2] = mfma4(yv, m2t[jb][t2][e], ak[t2]);
+          ak[t2] = mfma4(xv, m1t[jb][t2][e], ak[t2]);
+        }
       }
-    const float egl = __expf(gl);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block overwrites them
+    Quad rdx[2], rdk[2], rdq[2];
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      f4 ax = aX[q][t2], aq = aO[q][t2], ak;
+    for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ak[e] = egl * aL[q][t2][e];
+      for (int e = 0; e < 4; ++e) {
+        rdx[t2].v[e] = -__expf(gx[t2][e]) * ax[t2][e];
+        rdk[t2].v[e] = __expf(fminf(-G[q][t2].v[e], 80.f)) * ak[t2][e];
+        rdq[t2].v[e] = __expf(G[q][t2].v[e]) * aq[t2][e];
+      }
+    if (__any(any)) {  // exact sums of the wild rows
 #pragma unroll
-      for (int jb = 0; jb < 2; ++jb)
+      for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int jj = jb * 16 + 4 * g + e, ii = t2 * 16 + m;
-          ax = mfma4(M1[ii * MS + jj], kt[jb][e], ax);
-          ak = mfma4(M2[jj * MS + ii], yt[jb][e], ak);
-          ak = mfma4(-M1[jj * MS + ii], xt[jb][e], ak);
-          if (p.colout) aq = mfma4(M2[ii * MS + jj], kt[jb][e], aq);
-        }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = t2 * 16 + 4 * g + e;
-        const long long o = (tb + i) * kw + rr;
-        const float gi = p.G[o], gxi = gx_g(i, rr);
-        float dx, dk, dq = 0.f;
-        if (!wild) {
-          dx = -__expf(gxi) * ax[e];
-          dk = __expf(-gi) * ak[e];
-          dq = __expf(gi) * aq[e];
-        } else {
+          if (!wild[e]) continue;
+          const int i = t2 * 16 + m;
+          const float* gc = p.G + tb * kw + c0[q] + e;
+          const float *kc = p.k + tb * kw + c0[q] + e, *yc = Yk + tb * kw + c0[q] + e,
+                      *xc = p.x + tb * kw + c0[q] + e;
+          const float gi = G[q][t2].v[e], gxi = gx[t2][e];
+          auto gxa = [&](int j) { return COL ? gc[(long long)j * kw] : j > 0 ? gc[(long long)(j - 1) * kw] : 0.f; };
           float a = __expf(gxi) * aX[q][t2][e];
           for (int j = 0; j < i; ++j)
-            a += M1[i * MS + j] * p.k[(tb + j) * kw + rr] * __expf(gxi - p.G[(tb + j) * kw + rr]);
-          dx = -a;
-          float b = __expf(gl - gi) * aL[q][t2][e];
+            a += M1[i * AS + j] * kc[(long long)j * kw] * __expf(gxi - gc[(long long)j * kw]);
+          rdx[t2].v[e] = -a;
+          float b = __expf(gl[q].v[e] - gi) * aL[q][t2][e];
           for (int j = i; j < WBT; ++j)
-            b += M2[j * MS + i] * Yk[(tb + j) * kw + rr] * __expf(p.G[(tb + j) * kw + rr] - gi);
+            b += M2[j * AS + i] * yc[(long long)j * kw] * __expf(gc[(long long)j * kw] - gi);
           for (int j = i + 1; j < WBT; ++j)
-            b -= M1[j * MS + i] * p.x[(tb + j) * kw + rr] * __expf(gx_g(j, rr) - gi);
-          dk = b;
-          if (p.colout) {
+            b -= M1[j * AS + i] * xc[(long long)j * kw] * __expf(gxa(j) - gi);
+          rdk[t2].v[e] = b;
+          if constexpr (COL) {
             float c2 = __expf(gi) * aO[q][t2][e];
             for (int j = 0; j <= i; ++j)
-              c2 += M2[i * MS + j] * p.k[(tb + j) * kw + rr] * __expf(gi - p.G[(tb + j) * kw + rr]);
-            dq = c2;
+              c2 += M2[i * AS + j] * kc[(long long)j * kw] * __expf(gi - gc[(long long)j * kw]);
+            rdq[t2].v[e] = c2;
           }
         }
-        rdx[q][t2][e] = dx;
-        rdk[q][t2][e] = dk;
-        rdq[q][t2][e] = dq;
-      }
     }
-    // decay closure of row rr: dG = q dq - k dk (column) / o dO - k dk (row)
-    // + x dx (of the next token when the erase reads before the decay), and
-    // dg = rowsum(X_C lam) + the in-chunk reverse cumulative sum of dG.  The
-    // lane holds tokens t2 * 16 + 4 g + e; the next token of e = 3 sits in lane
-    // group g + 1 (g = 3, t2 = 0: group 0 of t2 = 1).
-    float dG[2][4], xd[2][4];
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        dG[t2][e] = -kr[t2][e] * rdk[q][t2][e] +
-                    (p.colout ? yr[t2][e] * rdq[q][t2][e] : orw[t2][e] * yr[t2][e]);
-        xd[t2][e] = xr[t2][e] * rdx[q][t2][e];
-      }
-    if (p.excl) {
-      const int src = g < 3 ? l + 16 : l - 48;
-      const float n0 = __shfl(xd[0][0], src), n1 = __shfl(xd[1][0], src);
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-        for (int e = 0; e < 3; ++e) dG[t2][e] += xd[t2][e + 1];
-      dG[0][3] += g < 3 ? n0 : n1;
-      dG[1][3] += g < 3 ? n1 : 0.f;
-    } else {
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dG[t2][e] += xd[t2][e];
-    }
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-      for (int e = 2; e >= 0; --e) dG[t2][e] += dG[t2][e + 1];  // suffix within the lane
-    float later[2], total1 = 0.f;  // sums of the later lane groups' tokens, per t2
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      const float s1 = __shfl(dG[t2][0], (l + 16) & 63), s2 = __shfl(dG[t2][0], (l + 32) & 63),
-                  s3 = __shfl(dG[t2][0], (l + 48) & 63);
-      later[t2] = (g < 3 ? s1 : 0.f) + (g < 2 ? s2 : 0.f) + (g < 1 ? s3 : 0.f);
-      if (t2 == 1) total1 = dG[1][0] + s1 + s2 + s3;
-    }
+    // decay closure: dG = q dq - k dk (column) / o dO - k dk (row) + x dx (of the
+    // next token when the erase reads before the decay), and
+    // dg = rowsum(X_C lam) + the in-chunk reverse cumulative sum of dG: a
+    // suffix scan over the row's 16 lanes (tokens), block 1's total added to block 0
+    Quad rdg[2];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      rdg[q][1][e] = rs[q] + dG[1][e] + later[1];
-      rdg[q][0][e] = rs[q] + dG[0][e] + later[0] + total1;
-    }
-  }
-  // stores after every row block's loads (a load issued after a store waits for it)
+      float dG[2], xd[2];
 #pragma unroll
-  for (int q = 0; q < GRB; ++q) {
-    const int rb = wv_ + GW * q;
-    if (rb >= nrb) continue;
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const long long o = (tb + t2 * 16 + 4 * g + e) * kw + rb * 16 + m;
-        p.dx[o] = rdx[q][t2][e];
-        p.dk[o] = rdk[q][t2][e];
-        if (p.colout) p.dq[o] = rdq[q][t2][e];
-        p.dg[o] = rdg[q][t2][e];
+      for (int t2 = 0; t2 < 2; ++t2) {
+        dG[t2] = -kr[q][t2].v[e] * rdk[t2].v[e] +
+                 (COL ? yr[q][t2].v[e] * rdq[t2].v[e] : orw[q][t2].v[e] * yr[q][t2].v[e]);
+        xd[t2] = xr[q][t2].v[e] * rdx[t2].v[e];
       }
+      if constexpr (COL) {
+        dG[0] += xd[0];
+        dG[1] += xd[1];
+      } else {
+        // (every lane takes part: a lane read across lanes must not be switched off)
+        const float n1 = __shfl(xd[1], l & 48), n0 = row_next<1>(xd[0]);
+        dG[0] += m == 15 ? n1 : n0;
+        dG[1] += row_next<1>(xd[1]);
+      }
+      const float rsum = __shfl(rs[q], 4 * g + e);
+      const float s1 = row_suffix(dG[1]), s0 = row_suffix(dG[0]);
+      rdg[1].v[e] = rsum + s1;
+      rdg[0].v[e] = rsum + s0 + __shfl(s1, l & 48);
+    }
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const long long o = (tb + t2 * 16 + m) * kw + c0[q];
+      *reinterpret_cast<Quad*>(p.dx + o) = rdx[t2];
+      *reinterpret_cast<Quad*>(p.dk + o) = rdk[t2];
+      if constexpr (COL) *reinterpret_cast<Quad*>(p.dq + o) = rdq[t2];
+      *reinterpret_cast<Quad*>(p.dg + o) = rdg[t2];
+    }
   }
 }
 
-constexpr size_t grad_smem(int w) { return (2 * WBT * MS + 3 * WBT * (w + 4)) * sizeof(float); }
+constexpr size_t grad_smem() { return (size_t)2 * WBT * AS * sizeof(float) + (size_t)6 * WBT * KHS * 2; }
+static_assert(6 * WBT * KHS * 2 >= GW * 3 * WBT * GS16 * 4, "phase 3's panels fit the split rows' storage");
 
 // ---------------------------------------------------------------------------
 // Source closure (per token): cotangents of e, chi, z back to u^, delta, k^, q^,
@@ -2045,7 +2139,7 @@ WideBwd carve_wide_bwd(void* base, const WideDims& d, size_t* total) {
 constexpr size_t kMaxLds = 160 * 1024;  // LDS of one gfx950 CU
 static_assert(prep_smem() <= kMaxLds / 2 && state_smem() <= kMaxLds && out_smem(WMAX, WMAX, 0) <= kMaxLds &&
                   out_smem(WMAX, WMAX, 1) <= kMaxLds && bprep_smem() <= kMaxLds / 2 &&
-                  grad_smem(WMAX) <= kMaxLds,
+                  grad_smem() <= kMaxLds,
               "a wide kernel's LDS exceeds the CU");
 
 void launch_wprep(const OpParams& op, int n, hipStream_t st) {
@@ -2149,8 +2243,6 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   dp.dout = (const __bf16*)dout; dp.dO = w.dO;
   SD_LAUNCH("k_w_dout", k_w_dout, dim3(64, d.n), dim3(WT), 0, st, dp);
 
-  SD_SMEM_ONCE(k_w_grad, (int)grad_smem(WMAX));
-
   // ---- memory S op ----
   BprepParams bs{};
   bs.NT = d.NT; bs.Tp = d.Tp; bs.kw = d.KP; bs.vw = d.VP; bs.excl = 0; bs.colout = 1;
@@ -2170,7 +2262,8 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   gs.k = f.d; gs.x = f.e; gs.q = f.chi; gs.G = f.G; gs.dO = w.dO; gs.o = nullptr;
   gs.w = f.wS; gs.dw = w.dwS; gs.Xslots = f.XS; gs.Lslots = w.LS; gs.Pp = nullptr;
   gs.dk = w.dd; gs.dx = w.de; gs.dq = w.dchi; gs.dg = w.dgS;
-  SD_LAUNCH("k_w_grad_s", k_w_grad, dim3(d.NT * d.n), dim3(GT), grad_smem(d.KP > d.VP ? d.KP : d.VP), st, gs);
+  SD_SMEM_ONCE(k_w_grad<true>, (int)grad_smem());
+  SD_LAUNCH("k_w_grad_s", k_w_grad<true>, dim3(d.NT * d.n), dim3(GT), grad_smem(), st, gs);
 
   SrcBwdParams sb{};
   sb.in = *in; sb.Tp = d.Tp; sb.KP = d.KP; sb.VP = d.VP;
@@ -2199,7 +2292,8 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   gc.k = f.uh; gc.x = f.xC; gc.q = f.kh; gc.G = f.G; gc.dO = w.dd; gc.o = f.oC;
   gc.w = f.delta; gc.dw = w.dwC; gc.Xslots = f.XC; gc.Lslots = w.LC; gc.Pp = w.Pp;
   gc.dk = w.dkC; gc.dx = w.dxC; gc.dq = w.dqC; gc.dg = w.dgC;
-  SD_LAUNCH("k_w_grad_c", k_w_grad, dim3(d.NT * d.n), dim3(GT), grad_smem(d.KP > d.VP ? d.KP : d.VP), st, gc);
+  SD_SMEM_ONCE(k_w_grad<false>, (int)grad_smem());
+  SD_LAUNCH("k_w_grad_c", k_w_grad<false>, dim3(d.NT * d.n), dim3(GT), grad_smem(), st, gc);
 
   FinalParams fp{};
   fp.in = *in; fp.Tp = d.Tp; fp.KP = d.KP;
