@@ -20,8 +20,9 @@
 // and backward, per op in reverse order:
 //     k_w_bprep   dU = A^T (dW + pair^T dO), W' = -A^T K^, K' = -x~, injection;
 //     k_w_state   reverse cotangent pass (lambda, dw);
-//     k_w_grad    closed-form chunk gradients dk, dx, dq and the decay closure;
-//   k_w_src_bwd, k_w_final (per token)  source and norm closures.
+//     k_w_grad    closed-form chunk gradients dk, dx, dq and the decay closure
+//                 (the predictor's ends with the closures of u, k, h and gamma);
+//   k_w_src_bwd (per token, between the ops)  source and q closures.
 //
 // Every decay factor is exp(a - b) with a <= b prefix sums inside one chunk (no
 // reciprocal decays), formed per element; padding tokens and coordinates are
@@ -1370,12 +1371,45 @@ constexpr size_t bprep_smem() {
 //   dg = in-chunk reverse cumulative sum of dG.
 // ---------------------------------------------------------------------------
 struct GradParams {
-  int NT, Tp, kw, vw, excl, colout;
+  int NT, Tp, kw, vw;
   const float *k, *x, *q, *G, *dO, *o, *w, *dw, *Pp;
   const xs_t* Xslots;
   const ls_t* Lslots;
+  // column output (S): the panels dk, dx, dq, dg
   float *dk, *dx, *dq, *dg;
+  // row output (C): the layer's closure of u, h, k, gamma and the log-decay
+  sd_inputs in;
+  const float *gam, *rs, *duh, *dkh, *dgS;
+  __bf16 *du, *dh, *dkey;
+  float *dlog_decay, *dgamma;
+  int vec;  // the gradients' rows take 4-element stores
 };
+
+// Four elements of a gradient row at column c of r (a padded column is dropped).
+__device__ __forceinline__ void store_row4(__bf16* row, int c, int r, int vec, bf16x4 h) {
+  if (vec) {
+    if (c < r) *reinterpret_cast<bf16x4*>(row + c) = h;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < r) row[c + e] = h[e];
+  }
+}
+__device__ __forceinline__ void store_row4(__bf16* row, int c, int r, int vec, const Quad& q) {
+  bf16x4 h;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) h[e] = f2bf(q.v[e]);
+  store_row4(row, c, r, vec, h);
+}
+__device__ __forceinline__ void store_row4(float* row, int c, int r, int vec, const Quad& q) {
+  if (vec) {
+    if (c < r) *reinterpret_cast<Quad*>(row + c) = q;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < r) row[c + e] = q.v[e];
+  }
+}
 
 // Eight waves (two per SIMD, so one wave's loads overlap another's matrix
 // work), each owning the 16-row blocks rb = wave + 8 q of the state.
@@ -1388,6 +1422,10 @@ constexpr int GS16 = 20;  // row stride (FP32) of a wave's staged [32 tokens][16
 template <int N>
 __device__ __forceinline__ float row_next(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 + N, 0xF, 0xF, true));
+}
+// Lane i takes lane i - 1's value, 0 at the row's start.
+__device__ __forceinline__ float row_prev(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xF, 0xF, true));
 }
 // Sum over this and the following lanes of a 16-lane row.
 __device__ __forceinline__ float row_suffix(float v) {
@@ -1426,9 +1464,10 @@ __device__ __forceinline__ void split4_to(__bf16* hi, __bf16* lo, const Quad& q)
 // transposed, so a lane holds four neighbouring coordinates of one token and
 // reads and writes the token panels 16 bytes at a time, and the rows shared by
 // all waves are split into bf16 halves once, in LDS.  301 us (S, 4.2 TB/s) and
-// 386 us (C) per launch at B4 T2048 H8 r = V = 256; with 4-byte panel accesses
-// in the MFMA layout, the rows split by every wave and dO e^G X0 on FP32 MFMAs
-// over 2-byte gathers of the slot, 360 and 500 us.
+// 468 us (C, with the layer's closure) per launch at B4 T2048 H8 r = V = 256; with
+// 4-byte panel accesses in the MFMA layout, the rows split by every wave and
+// dO e^G X0 on FP32 MFMAs over 2-byte gathers of the slot, 360 us and, with the
+// closure as a kernel of its own, 500 + 217 us.
 template <bool COL>
 __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   extern __shared__ __align__(16) float sm[];
@@ -1556,7 +1595,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   }
   // this lane's elements of the key-side panels (tokens m and 16 + m), loaded
   // before any store of the kernel
-  Quad kr[GRB][2], yr[GRB][2], xr[GRB][2], G[GRB][2], Gp[GRB][2], orw[GRB][2], gl[GRB];
+  Quad kr[GRB][2], yr[GRB][2], xr[GRB][2], G[GRB][2], orw[GRB][2], gl[GRB];
   int c0[GRB];
 #pragma unroll
   for (int q = 0; q < GRB; ++q) {
@@ -1569,10 +1608,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
       yr[q][t2] = ldq(Yk + o);
       xr[q][t2] = ldq(p.x + o);
       G[q][t2] = ldq(p.G + o);
-      if constexpr (!COL) {
-        Gp[q][t2] = ldq(p.G + (t2 == 0 && m == 0 ? o : o - kw));
-        orw[q][t2] = ldq(p.o + o);
-      }
+      if constexpr (!COL) orw[q][t2] = ldq(p.o + o);
     }
   }
   // rowsum(X_C (.) lam): the four lane groups' partials of each state row
@@ -1586,6 +1622,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   // of the value axis, transposed.  The contraction runs along the slot's rows,
   // so 32-row blocks pass through LDS (double buffered, one barrier each) and
   // are read down their columns; bf16 halves as in phase 1, Pp w in FP32.
+  [[maybe_unused]] f4 dqc[GRB][2];
   if constexpr (!COL) {
     __bf16 *Dh = TR, *Dl = TR + RP;
     _Float16* Xt = reinterpret_cast<_Float16*>(TR + 2 * RP);  // [2][32][KHS]
@@ -1671,8 +1708,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
         for (int kb = 0; kb <= t2; ++kb)
 #pragma unroll
           for (int e = 0; e < 4; ++e) aq[q][t2] = mfma4(wv[q][kb][e], pp[t2][kb].v[e], aq[q][t2]);
-        if (w + GW * q < nvb)
-          *reinterpret_cast<f4*>(p.dq + (tb + t2 * 16 + m) * vw + nb[q] + 4 * g) = aq[q][t2];
+        dqc[q][t2] = aq[q][t2];  // vw = kw: the same coordinates as the key side's
       }
   }
   // phase 3: the in-chunk applies on FP32 matrix cores over the Grams' lower
@@ -1684,22 +1720,40 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   // k~, Y~, x~ of a wave's 16 coordinates pass through its own LDS panels.
   float* kt = reinterpret_cast<float*>(TR) + w * 3 * WBT * GS16;
   float *yt = kt + WBT * GS16, *xt = yt + WBT * GS16;
-  f4 m1[2][2], m2[2][2], m1t[2][2], m2t[2][2];  // [i block][j block] of M and, for the transposes, M^T
+  // Row output: the closure of u, k, h, gamma follows from registers (the
+  // workgroup holds its 32 tokens' whole rows): with du' = duh + dk + gamma dx,
+  // dk' = dkh + dd + dq and the row sums su = du'.u, sk = dk'.k, sg = u.dx + h.dw
+  // over all waves, du = (du' - su u) / |u|, dk = (dk' - sk k) / |k|, dh = gamma dw.
+  // As a kernel of its own it read ten panels back (217 us at B4 T2048 H8 r = V = 256).
+  [[maybe_unused]] Quad gu[GRB][2], gk[GRB][2], dgo[GRB][2];
+  [[maybe_unused]] bf16x4 dh4[GRB][2];
+  [[maybe_unused]] float su[2] = {0.f, 0.f}, sk[2] = {0.f, 0.f}, sg[2] = {0.f, 0.f}, gmv[2], xk[2];
+  [[maybe_unused]] const int T = p.in.T, H = p.in.H, r = p.in.r, hb = s / H, hh = s % H;
+  if constexpr (!COL) {
 #pragma unroll
-  for (int ib = 0; ib < 2; ++ib)
-#pragma unroll
-    for (int jb = 0; jb <= ib; ++jb) {
-      m1[ib][jb] = *reinterpret_cast<const f4*>(M1 + (ib * 16 + m) * AS + jb * 16 + 4 * g);
-      m2[ib][jb] = *reinterpret_cast<const f4*>(M2 + (ib * 16 + m) * AS + jb * 16 + 4 * g);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        m1t[ib][jb][e] = -M1[(ib * 16 + 4 * g + e) * AS + jb * 16 + m];
-        m2t[ib][jb][e] = M2[(ib * 16 + 4 * g + e) * AS + jb * 16 + m];
-      }
+    for (int t2 = 0; t2 < 2; ++t2) {
+      gmv[t2] = p.gam[tb + t2 * 16 + m];
+      xk[t2] = erase_keep(p.in, hb, min(ch * WBT + t2 * 16 + m, T - 1));  // fresh: dx reaches neither u nor gamma
     }
+  }
 #pragma unroll
   for (int q = 0; q < GRB; ++q) {
     if (w + GW * q >= nrb) continue;
+    [[maybe_unused]] Quad hv[2], kn[2], dv[2];
+    if constexpr (!COL) {
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        const long long o = (tb + t2 * 16 + m) * kw + c0[q];
+        gu[q][t2] = ldq(p.duh + o);
+        gk[q][t2] = ldq(p.dkh + o);
+        kn[t2] = ldq(p.q + o);
+        dv[t2] = ldq(p.dw + o);
+        dgo[q][t2] = ldq(p.dgS + o);
+        const __bf16* hr = wrow(p.in.h, hb, min(ch * WBT + t2 * 16 + m, T - 1), hh);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hv[t2].v[e] = bf2f(hr[min(c0[q] + e, r - 1)]);
+      }
+    }
     bool wild[4];
     float gx[2][4];
     bool any = false;
@@ -1713,7 +1767,12 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
       Quad a, b, c;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        gx[t2][e] = COL ? G[q][t2].v[e] : t2 == 0 && m == 0 ? 0.f : Gp[q][t2].v[e];
+        if constexpr (COL) {
+          gx[t2][e] = G[q][t2].v[e];
+        } else {  // the prefix before the token: the previous lane's, across the blocks lane 15's
+          const float prev = row_prev(G[q][t2].v[e]), edge = __shfl(G[q][0].v[e], l | 15);
+          gx[t2][e] = m > 0 ? prev : t2 ? edge : 0.f;
+        }
         a.v[e] = keep_exp(!wild[e], kr[q][t2].v[e], -G[q][t2].v[e]);
         b.v[e] = keep_exp(!wild[e], yr[q][t2].v[e], G[q][t2].v[e]);
         c.v[e] = keep_exp(!wild[e], xr[q][t2].v[e], gx[t2][e]);
@@ -1724,6 +1783,21 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
       *reinterpret_cast<Quad*>(xt + o) = c;
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own panels
+    // M's blocks [i block][j block] and, for the transposed applies, -M1^T's and
+    // M2^T's (read again per row block: held over both they spill)
+    f4 m1[2][2], m2[2][2], m1t[2][2], m2t[2][2];
+#pragma unroll
+    for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+      for (int jb = 0; jb <= ib; ++jb) {
+        m1[ib][jb] = *reinterpret_cast<const f4*>(M1 + (ib * 16 + m) * AS + jb * 16 + 4 * g);
+        m2[ib][jb] = *reinterpret_cast<const f4*>(M2 + (ib * 16 + m) * AS + jb * 16 + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          m1t[ib][jb][e] = -M1[(ib * 16 + 4 * g + e) * AS + jb * 16 + m];
+          m2t[ib][jb][e] = M2[(ib * 16 + 4 * g + e) * AS + jb * 16 + m];
+        }
+      }
     f4 ax[2], ak[2], aq[2];
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
@@ -1817,19 +1891,85 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
       rdg[1].v[e] = rsum + s1;
       rdg[0].v[e] = rsum + s0 + __shfl(s1, l & 48);
     }
+    if constexpr (COL) {
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        const long long o = (tb + t2 * 16 + m) * kw + c0[q];
+        *reinterpret_cast<Quad*>(p.dx + o) = rdx[t2];
+        *reinterpret_cast<Quad*>(p.dk + o) = rdk[t2];
+        *reinterpret_cast<Quad*>(p.dq + o) = rdq[t2];
+        *reinterpret_cast<Quad*>(p.dg + o) = rdg[t2];
+      }
+    } else {
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float u = kr[q][t2].v[e], dxc = xk[t2] * rdx[t2].v[e];
+          gu[q][t2].v[e] += rdk[t2].v[e] + gmv[t2] * dxc;
+          gk[q][t2].v[e] += yr[q][t2].v[e] + dqc[q][t2][e];
+          su[t2] += gu[q][t2].v[e] * u;
+          sk[t2] += gk[q][t2].v[e] * kn[t2].v[e];
+          sg[t2] += u * dxc + (c0[q] + e < r ? hv[t2].v[e] : 0.f) * dv[t2].v[e];
+          dh4[q][t2][e] = f2bf(gmv[t2] * dv[t2].v[e]);
+          dgo[q][t2].v[e] += rdg[t2].v[e];
+        }
+    }
+  }
+  if constexpr (!COL) {
+    // row sums over the lane groups, then over the waves: red[sum][token][wave]
+    float* red = reinterpret_cast<float*>(TR) + GW * 3 * WBT * GS16;
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      const long long o = (tb + t2 * 16 + m) * kw + c0[q];
-      *reinterpret_cast<Quad*>(p.dx + o) = rdx[t2];
-      *reinterpret_cast<Quad*>(p.dk + o) = rdk[t2];
-      if constexpr (COL) *reinterpret_cast<Quad*>(p.dq + o) = rdq[t2];
-      *reinterpret_cast<Quad*>(p.dg + o) = rdg[t2];
+      float v[3] = {su[t2], sk[t2], sg[t2]};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        v[a] += __shfl_xor(v[a], 16);
+        v[a] += __shfl_xor(v[a], 32);
+        if (g == 0) red[(a * WBT + t2 * 16 + m) * GW + w] = v[a];
+      }
+    }
+    Quad kn[GRB][2];  // (read again: held through the loop above they spill)
+#pragma unroll
+    for (int q = 0; q < GRB; ++q)
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) kn[q][t2] = ldq(p.q + (tb + t2 * 16 + m) * kw + c0[q]);
+    __syncthreads();
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const int t = ch * WBT + t2 * 16 + m;
+      float v[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const float* rr = red + (a * WBT + t2 * 16 + m) * GW;
+        const Quad r0 = ldq(rr), r1 = ldq(rr + 4);
+        v[a] = ((r0.v[0] + r0.v[1]) + (r0.v[2] + r0.v[3])) + ((r1.v[0] + r1.v[1]) + (r1.v[2] + r1.v[3]));
+      }
+      if (t >= T) continue;
+      const float ru = p.rs[(tb + t2 * 16 + m) * 3], rk = p.rs[(tb + t2 * 16 + m) * 3 + 1];
+      const long long ob = ((long long)hb * T + t) * H + hh, o = ob * r;
+#pragma unroll
+      for (int q = 0; q < GRB; ++q) {
+        if (w + GW * q >= nrb) continue;
+        Quad a, b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          a.v[e] = (gu[q][t2].v[e] - v[0] * kr[q][t2].v[e]) * ru;
+          b.v[e] = (gk[q][t2].v[e] - v[1] * kn[q][t2].v[e]) * rk;
+        }
+        store_row4(p.du + o, c0[q], r, p.vec, a);
+        store_row4(p.dkey + o, c0[q], r, p.vec, b);
+        store_row4(p.dh + o, c0[q], r, p.vec, dh4[q][t2]);
+        store_row4(p.dlog_decay + o, c0[q], r, p.vec, dgo[q][t2]);
+      }
+      if (w == 0 && g == 0) p.dgamma[ob] = v[2];
     }
   }
 }
 
 constexpr size_t grad_smem() { return (size_t)2 * WBT * AS * sizeof(float) + (size_t)6 * WBT * KHS * 2; }
-static_assert(6 * WBT * KHS * 2 >= GW * 3 * WBT * GS16 * 4, "phase 3's panels fit the split rows' storage");
+static_assert(6 * WBT * KHS * 2 >= (GW * 3 * WBT * GS16 + 3 * WBT * GW) * 4,
+              "phase 3's panels and row sums fit the split rows' storage");
 
 // ---------------------------------------------------------------------------
 // Source closure (per token): cotangents of e, chi, z back to u^, delta, k^, q^,
@@ -1838,9 +1978,9 @@ static_assert(6 * WBT * KHS * 2 >= GW * 3 * WBT * GS16 * 4, "phase 3's panels fi
 struct SrcBwdParams {
   sd_inputs in;
   int Tp, KP, VP;
-  const float *uh, *delta, *kh, *qh, *de, *dchi, *dz;
-  float *duh, *ddelta, *dkh, *dqh;
-  __bf16 *derase, *dwrite, *dv;
+  const float *uh, *delta, *kh, *qh, *rs, *de, *dchi, *dz;
+  float *duh, *ddelta, *dkh;
+  __bf16 *dq, *derase, *dwrite, *dv;
 };
 
 __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
@@ -1917,6 +2057,11 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
     ds += dphi[j] * dl[j];
   }
   ds = wave_sum(ds);
+  float sqq = 0.f;  // the q norm's closure: dq = (dq^ - (dq^ . q^) q^) / |q|
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sqq += dqh[j] * q[j];
+  sqq = wave_sum(sqq);
+  const float rq = p.rs[((long long)s * p.Tp + t) * 3 + 2];
   const float dN2 = (-RHO * ds / (N * N)) / (2.f * N);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -1925,9 +2070,9 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
       p.duh[row + c] = duh[j] + 2.f * dN2 * dsq * u[j];
       p.ddelta[row + c] = sc * dphi[j] + 2.f * dN2 * usq * dl[j];
       p.dkh[row + c] = db[j] * se[j];
-      p.dqh[row + c] = dqh[j];
     }
     const long long obase = ((long long)b * T + t) * H + h;
+    if (tv && c < r) p.dq[obase * r + c] = f2bf((dqh[j] - sqq * q[j]) * rq);
     if (tv && c < r) p.derase[obase * r + c] = f2bf(db[j] * k[j] * se[j] * (1.f - se[j]));
     if (tv && c < V) {
       const float sw = 1.f / (1.f + __expf(-wr[j]));
@@ -1935,91 +2080,6 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
       p.dwrite[obase * V + c] = f2bf(dzv[j] * vv[j] * sw * (1.f - sw));
     }
   }
-}
-
-// ---------------------------------------------------------------------------
-// Final closure (per token): norms, gamma, and the two ops' decay gradients.
-// ---------------------------------------------------------------------------
-struct FinalParams {
-  sd_inputs in;
-  int Tp, KP;
-  const float *uh, *kh, *qh, *gam, *rs;
-  const float *duh, *dkh, *dqh, *dd, *dkC, *dxC, *dvC, *dqC, *dgS, *dgC;
-  __bf16 *du, *dh, *dq, *dk;
-  float *dlog_decay, *dgamma;
-};
-
-__global__ __launch_bounds__(WT) void k_w_final(FinalParams p) {
-  const int s = blockIdx.y, H = p.in.H, T = p.in.T, r = p.in.r;
-  const int b = s / H, h = s % H;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int t = blockIdx.x * (WT / 64) + w;
-  if (t >= T) return;
-  const long long tok = (long long)s * p.Tp + t, row = tok * p.KP;
-  const float gm = p.gam[tok];
-  const float xk = erase_keep(p.in, b, t);  // fresh tokens: dx reaches neither u nor gamma
-  // every load first, at clamped indices (masked below): no load under a branch,
-  // and none issued after a store
-  const __bf16* hr = wrow(p.in.h, b, t, h);
-  const float ru = p.rs[tok * 3], rk = p.rs[tok * 3 + 1], rq = p.rs[tok * 3 + 2];
-  float u[4], k[4], q[4], dxc[4], dvc[4], gu[4], gk[4], gq[4], hv[4], dgl[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = l + 64 * j, ck = min(c, p.KP - 1);
-    u[j] = p.uh[row + ck];
-    k[j] = p.kh[row + ck];
-    q[j] = p.qh[row + ck];
-    dxc[j] = p.dxC[row + ck];
-    dvc[j] = p.dvC[row + ck];
-    gu[j] = p.duh[row + ck] + p.dkC[row + ck];
-    gk[j] = p.dkh[row + ck] + p.dd[row + ck] + p.dqC[row + ck];
-    gq[j] = p.dqh[row + ck];
-    hv[j] = bf2f(hr[min(c, r - 1)]);
-    dgl[j] = p.dgS[row + ck] + p.dgC[row + ck];
-  }
-  float su = 0.f, sk = 0.f, sq = 0.f, sg = 0.f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = l + 64 * j;
-    const bool in = c < p.KP;
-    u[j] = in ? u[j] : 0.f;
-    k[j] = in ? k[j] : 0.f;
-    q[j] = in ? q[j] : 0.f;
-    dxc[j] = in ? xk * dxc[j] : 0.f;
-    dvc[j] = in ? dvc[j] : 0.f;
-    gu[j] = in ? gu[j] + gm * dxc[j] : 0.f;
-    gk[j] = in ? gk[j] : 0.f;
-    gq[j] = in ? gq[j] : 0.f;
-    hv[j] = c < r ? hv[j] : 0.f;
-    su += gu[j] * u[j];
-    sk += gk[j] * k[j];
-    sq += gq[j] * q[j];
-    sg += u[j] * dxc[j] + hv[j] * dvc[j];
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = l + 64 * j;
-    if (c < r) {
-      const long long o = (((long long)b * T + t) * H + h) * r + c;
-      p.dh[o] = f2bf(gm * dvc[j]);
-      p.dlog_decay[o] = dgl[j];
-    }
-  }
-  su = wave_sum(su);
-  sk = wave_sum(sk);
-  sq = wave_sum(sq);
-  sg = wave_sum(sg);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = l + 64 * j;
-    if (c < r) {
-      const long long o = (((long long)b * T + t) * H + h) * r + c;
-      p.du[o] = f2bf((gu[j] - su * u[j]) * ru);
-      p.dk[o] = f2bf((gk[j] - sk * k[j]) * rk);
-      p.dq[o] = f2bf((gq[j] - sq * q[j]) * rq);
-    }
-  }
-  if (l == 0) p.dgamma[((long long)b * T + t) * H + h] = sg;
 }
 
 // Output cotangent as an FP32 panel (zero when absent and on padded entries).
@@ -2115,7 +2175,7 @@ struct WideBwd {
   float *dU, *Pp;
   __bf16 *Wneg, *Kt, *At;
   float *dwS, *dwC, *dd, *de, *dchi, *dgS;
-  float *duh, *ddelta, *dkh, *dqh, *dkC, *dxC, *dqC, *dgC;
+  float *duh, *ddelta, *dkh;
 };
 
 WideBwd carve_wide_bwd(void* base, const WideDims& d, size_t* total) {
@@ -2130,8 +2190,7 @@ WideBwd carve_wide_bwd(void* base, const WideDims& d, size_t* total) {
   w.Pp = c.take((size_t)d.n * d.NT * WBT * WBT);
   w.dwS = c.take(pv); w.dwC = c.take(pk);
   w.dd = c.take(pk); w.de = c.take(pk); w.dchi = c.take(pk); w.dgS = c.take(pk);
-  w.duh = c.take(pk); w.ddelta = c.take(pk); w.dkh = c.take(pk); w.dqh = c.take(pk);
-  w.dkC = c.take(pk); w.dxC = c.take(pk); w.dqC = c.take(pk); w.dgC = c.take(pk);
+  w.duh = c.take(pk); w.ddelta = c.take(pk); w.dkh = c.take(pk);
   if (total) *total = c.off + 256;
   return w;
 }
@@ -2258,7 +2317,7 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   rs.init = dS_T; rs.init_t = 0; rs.fin = dS0; rs.fin_t = 0;
   launch_wstate("w_state_s_bwd", rs, d.n, st);
   GradParams gs{};
-  gs.NT = d.NT; gs.Tp = d.Tp; gs.kw = d.KP; gs.vw = d.VP; gs.excl = 0; gs.colout = 1;
+  gs.NT = d.NT; gs.Tp = d.Tp; gs.kw = d.KP; gs.vw = d.VP;
   gs.k = f.d; gs.x = f.e; gs.q = f.chi; gs.G = f.G; gs.dO = w.dO; gs.o = nullptr;
   gs.w = f.wS; gs.dw = w.dwS; gs.Xslots = f.XS; gs.Lslots = w.LS; gs.Pp = nullptr;
   gs.dk = w.dd; gs.dx = w.de; gs.dq = w.dchi; gs.dg = w.dgS;
@@ -2269,7 +2328,8 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   sb.in = *in; sb.Tp = d.Tp; sb.KP = d.KP; sb.VP = d.VP;
   sb.uh = f.uh; sb.delta = f.delta; sb.kh = f.kh; sb.qh = f.qh;
   sb.de = w.de; sb.dchi = w.dchi; sb.dz = w.dwS;
-  sb.duh = w.duh; sb.ddelta = w.ddelta; sb.dkh = w.dkh; sb.dqh = w.dqh;
+  sb.rs = f.rs;
+  sb.duh = w.duh; sb.ddelta = w.ddelta; sb.dkh = w.dkh; sb.dq = (__bf16*)dq;
   sb.derase = (__bf16*)derase; sb.dwrite = (__bf16*)dwrite; sb.dv = (__bf16*)dv;
   SD_LAUNCH("k_w_src_bwd", k_w_src_bwd, dim3(d.Tp / (WT / 64), d.n), dim3(WT), 0, st, sb);
 
@@ -2288,21 +2348,17 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   rc.init = dC_T; rc.init_t = 1; rc.fin = dC0; rc.fin_t = 1;
   launch_wstate("w_state_c_bwd", rc, d.n, st);
   GradParams gc{};
-  gc.NT = d.NT; gc.Tp = d.Tp; gc.kw = d.KP; gc.vw = d.KP; gc.excl = 1; gc.colout = 0;
+  gc.NT = d.NT; gc.Tp = d.Tp; gc.kw = d.KP; gc.vw = d.KP;
   gc.k = f.uh; gc.x = f.xC; gc.q = f.kh; gc.G = f.G; gc.dO = w.dd; gc.o = f.oC;
   gc.w = f.delta; gc.dw = w.dwC; gc.Xslots = f.XC; gc.Lslots = w.LC; gc.Pp = w.Pp;
-  gc.dk = w.dkC; gc.dx = w.dxC; gc.dq = w.dqC; gc.dg = w.dgC;
+  gc.in = *in; gc.gam = f.gam; gc.rs = f.rs; gc.duh = w.duh; gc.dkh = w.dkh; gc.dgS = w.dgS;
+  gc.du = (__bf16*)du; gc.dh = (__bf16*)dh; gc.dkey = (__bf16*)dk;
+  gc.dlog_decay = dlog_decay; gc.dgamma = dgamma;
+  gc.vec = in->r % 4 == 0 && (((uintptr_t)du | (uintptr_t)dh | (uintptr_t)dk) & 7) == 0 &&
+           ((uintptr_t)dlog_decay & 15) == 0;
   SD_SMEM_ONCE(k_w_grad<false>, (int)grad_smem());
   SD_LAUNCH("k_w_grad_c", k_w_grad<false>, dim3(d.NT * d.n), dim3(GT), grad_smem(), st, gc);
 
-  FinalParams fp{};
-  fp.in = *in; fp.Tp = d.Tp; fp.KP = d.KP;
-  fp.uh = f.uh; fp.kh = f.kh; fp.qh = f.qh; fp.gam = f.gam; fp.rs = f.rs;
-  fp.duh = w.duh; fp.dkh = w.dkh; fp.dqh = w.dqh; fp.dd = w.dd;
-  fp.dkC = w.dkC; fp.dxC = w.dxC; fp.dvC = w.dwC; fp.dqC = w.dqC; fp.dgS = w.dgS; fp.dgC = w.dgC;
-  fp.du = (__bf16*)du; fp.dh = (__bf16*)dh; fp.dq = (__bf16*)dq; fp.dk = (__bf16*)dk;
-  fp.dlog_decay = dlog_decay; fp.dgamma = dgamma;
-  SD_LAUNCH("k_w_final", k_w_final, dim3(d.Tp / (WT / 64), d.n), dim3(WT), 0, st, fp);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 

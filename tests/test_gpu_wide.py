@@ -60,6 +60,17 @@ def _check_fb(B, T, H, r, V, seed, decay="softplus", with_state=True, cot="all",
 
 
 @pytest.mark.parametrize("B,T,H,r,V,seed,decay", [
+    (2, 33, 2, 141, 131, 71, "softplus"),  # gradient rows not a multiple of 4 wide
+    (1, 31, 1, 129, 255, 72, "mixed"),     # one ragged chunk; wild coordinates; an odd value width
+    (1, 65, 1, 255, 33, 73, "mixed"),      # a value width below a wave's blocks
+    (1, 96, 1, 100, 200, 74, "softplus"),  # narrow keys, wide values: key blocks for half the waves
+])
+def test_wide_odd_widths(B, T, H, r, V, seed, decay):
+    """Widths off every block, store and tile size of the wide kernels."""
+    _check_fb(B, T, H, r, V, seed, decay)
+
+
+@pytest.mark.parametrize("B,T,H,r,V,seed,decay", [
     (1, 70, 2, 256, 256, 51, "softplus"),   # three 32-token chunks, ragged tail
     (2, 33, 1, 200, 136, 53, "softplus"),   # widths not a multiple of 32
     (1, 100, 2, 160, 64, 55, "mixed"),      # wide keys, narrow values; strongly decaying coordinates
