@@ -83,10 +83,19 @@ __device__ __forceinline__ float wgamma(const sd_view& g, int b, int t, int h) {
 // ---------------------------------------------------------------------------
 // Token preparation: G prefix, norms, gamma-scaled predictor operands.
 // ---------------------------------------------------------------------------
+// Per-token scalars: the inverse norms 1/|u|, 1/|k|, 1/|q| (u^ = ru u and so on
+// are formed from the packed bf16 rows where they are read: half the bytes of
+// FP32 panels and the same values), gamma, the erase read's gamma (0 on fresh
+// tokens), and 1/|k| again with 0 for a zero row, where it multiplies a
+// cotangent of any scale.
+struct Tok { float ru, rk, rq, gam, gx, rks, pad[2]; };
+
 struct TokParams {
   sd_inputs in;
   int NT, Tp, KP;
-  float *G, *uh, *kh, *qh, *xC, *vC, *gam, *rs;
+  float *G;
+  __bf16 *ub, *kb, *qb, *hb;  // packed raw rows [Tp][KP], zero past the widths and on invalid tokens (k, q)
+  Tok* tok;
 };
 
 // Loads here are unconditional (indices clamped into the row, invalid values
@@ -163,26 +172,22 @@ __global__ __launch_bounds__(WT) void k_w_tokens(TokParams p) {
         sq += qq[u][j] * qq[u][j];
       }
       const float ru = rsqrtf(wave_sum(su) + 1e-24f);
-      const float rk = rsqrtf(wave_sum(sk) + 1e-24f);
+      sk = wave_sum(sk);
+      const bool sk0 = sk == 0.f;
+      const float rk = rsqrtf(sk + 1e-24f);
       const float rq = rsqrtf(wave_sum(sq) + 1e-24f);
       const long long row = (pb + t) * KP;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int cc = l + 64 * j;
-        if (cc < KP) {
-          p.uh[row + cc] = uu[u][j] * ru;
-          p.kh[row + cc] = kk[u][j] * rk;
-          p.qh[row + cc] = qq[u][j] * rq;
-          p.xC[row + cc] = gx * uu[u][j] * ru;
-          p.vC[row + cc] = g1 * hv[u][j];
+        if (cc < KP) {  // (bf16 values and zeros: exact)
+          p.ub[row + cc] = f2bf(uu[u][j]);
+          p.kb[row + cc] = f2bf(kk[u][j]);
+          p.qb[row + cc] = f2bf(qq[u][j]);
+          p.hb[row + cc] = f2bf(hv[u][j]);
         }
       }
-      if (l == 0) {
-        p.gam[pb + t] = g1;
-        p.rs[(pb + t) * 3 + 0] = ru;
-        p.rs[(pb + t) * 3 + 1] = rk;
-        p.rs[(pb + t) * 3 + 2] = rq;
-      }
+      if (l == 0) p.tok[pb + t] = {ru, rk, rq, g1, gx, sk0 ? 0.f : rk, {0.f, 0.f}};
     }
   }
 }
@@ -191,8 +196,11 @@ __global__ __launch_bounds__(WT) void k_w_tokens(TokParams p) {
 // One op (state X [kw x vw]) of the chunked recurrence.
 // ---------------------------------------------------------------------------
 struct OpParams {
-  int NT, Tp, kw, vw, excl, colout;
-  const float *k, *x, *v, *q, *G;  // k, x, G [Tp][kw]; v [Tp][vw]; q [Tp][kw] (col) / [Tp][vw] (row)
+  int NT, Tp, kw, vw, colout;
+  const float *k, *x, *q, *G;  // [Tp][kw] (k, x, q: column output)
+  const __bf16 *ub, *hb;       // row output: k = u^, x = gx u^, v = gamma h
+  const Tok* tok;
+  sd_inputs in;                // column output: v = sigmoid(write_raw) v from the raw inputs
   float *A, *P;                    // [NT][32][32]
   _Float16 *Wneg, *Kt;             // state-pass panels: -W [Tp][kw] (fragment order), K^ transposed per chunk [NT][kw][32]
   float *U, *Qt, *Gam;             // Qt [Tp][kw]; U [Tp][vw] (accumulator order); Gam [NT][kw]
@@ -245,6 +253,13 @@ constexpr int KHS = WMAX + 8;        // row stride (16-bit) of a staged [32][kw]
 constexpr int AS = WBT + 4;          // row stride of the staged 32 x 32 matrices
 
 struct Quad { float v[4]; };
+__device__ __forceinline__ Quad ldq(const __bf16* p) {
+  const bf16x4 h = *reinterpret_cast<const bf16x4*>(p);
+  return {{bf2f(h[0]), bf2f(h[1]), bf2f(h[2]), bf2f(h[3])}};
+}
+__device__ __forceinline__ Quad scaled(const Quad& a, float f) {
+  return {{a.v[0] * f, a.v[1] * f, a.v[2] * f, a.v[3] * f}};
+}
 __device__ __forceinline__ Quad ldq(const float* p) { return *reinterpret_cast<const Quad*>(p); }
 
 // The three lower 16 x 16 blocks (0,0), (1,0), (1,1) of a 32 x 32 token Gram,
@@ -260,26 +275,41 @@ __device__ __forceinline__ void gram3(const Quad (&a)[2], const Quad (&b)[2], f4
 }
 
 // Adds the exact terms of the block's wild coordinates (wild[e]: this lane
-// group's coordinate 4 g + e is wild) to the lane's Gram entries; fx(i, j, c) is
-// the term of tokens i, j at coordinate c, strict keeps j < i, else j <= i.
-template <class FX>
-__device__ __forceinline__ void gram3_wild(const bool (&wild)[4], int c0, bool strict, FX fx, f4 (&acc)[3]) {
-  const int l = threadIdx.x & 63, g = l >> 4, m = l & 15;
+// group's coordinate 4 g + e is wild) to the lane's Gram entries.  left(i, c) /
+// right(j, c) give a row's / column's {value, G} at coordinate c; strict keeps
+// j < i, else j <= i.
+template <class FL, class FR>
+__device__ __forceinline__ void gram3_wild(const bool (&wild)[4], int c0, bool strict, FL left, FR right,
+                                           f4 (&acc)[3]) {
+  unsigned mask = 0;  // bit 4 g + e
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const unsigned long long mask = __ballot(wild[e]);
-    if (mask == 0) continue;
-    for (int gg = 0; gg < 4; ++gg) {
-      if (!((mask >> (gg * 16)) & 1)) continue;
-      const int c = c0 + 4 * gg + e;
+    const unsigned long long b = __ballot(wild[e]);
 #pragma unroll
-      for (int q = 0; q < 3; ++q)
+    for (int gg = 0; gg < 4; ++gg) mask |= (unsigned)((b >> (gg * 16)) & 1) << (4 * gg + e);
+  }
+  while (mask) {
+    const int c = c0 + __ffs(mask) - 1;
+    mask &= mask - 1;
+    // (opaque lane indices: hoisted out of this rare loop, its addresses would
+    // stay in registers through the common path)
+    int g = (threadIdx.x & 63) >> 4, m = threadIdx.x & 15;
+    asm volatile("" : "+v"(g), "+v"(m));
+    float2 lv[2][4], rv[2];
 #pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2) {
-          const int i = (q > 0 ? 16 : 0) + 4 * g + e2, j = (q > 1 ? 16 : 0) + m;
-          if (strict ? j < i : j <= i) acc[q][e2] += fx(i, j, c);
-        }
+    for (int h = 0; h < 2; ++h) {
+      rv[h] = right(h * 16 + m, c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) lv[h][e] = left(h * 16 + 4 * g + e, c);
     }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int bi = q > 0, bj = q > 1, i = bi * 16 + 4 * g + e, j = bj * 16 + m;
+        const float v = lv[bi][e].x * rv[bj].x * __expf(fminf(lv[bi][e].y - rv[bj].y, 0.f));
+        acc[q][e] += (strict ? j < i : j <= i) ? v : 0.f;
+      }
   }
 }
 
@@ -365,36 +395,67 @@ __global__ __launch_bounds__(PT, 4) void k_w_prep(OpParams p) {
   const long long tb = (long long)s * p.Tp + ch * WBT;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15;
   const long long cbase = (long long)s * p.NT + ch;
+  // chunk-uniform bases, 32-bit lane offsets (64-bit lane addresses spill)
+  const float* Gc = p.G + tb * kw;
+  const float *kc = COL ? p.k + tb * kw : nullptr, *xc = COL ? p.x + tb * kw : nullptr,
+              *qc = COL ? p.q + tb * kw : nullptr;
+  const __bf16 *ubc = COL ? nullptr : p.ub + tb * kw, *hbc = COL ? nullptr : p.hb + tb * kw;
+  const Tok* tokc = COL ? nullptr : p.tok + tb;
   // this lane's values for U = A v (the MFMA B operand: tokens kb * 16 + 4 g + e
   // of column block w + 8 j), loaded before any store of the kernel (a load
   // issued after a store waits for it: one counter retires both)
-  float vb[PNB][2][4];
+  __bf16 vr[PNB][2][4], wr[COL ? PNB : 1][2][4];
+  [[maybe_unused]] const int b = s / (COL ? p.in.H : 1), hh = s - b * (COL ? p.in.H : 1);
 #pragma unroll
-  for (int j = 0; j < PNB; ++j)
+  for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int e = 0; e < 4; ++e) {
+      const int i = kb * 16 + 4 * g + e;
+      if constexpr (COL) {  // clamped, masked when used
+        const int tc = min(ch * WBT + i, p.in.T - 1);
+        const __bf16 *vp = wrow(p.in.v, b, tc, hh), *wp = wrow(p.in.write_raw, b, tc, hh);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        vb[j][kb][e] = p.v[(tb + kb * 16 + 4 * g + e) * vw + min(w + PW * j, nvb - 1) * 16 + m];
+        for (int j = 0; j < PNB; ++j) {
+          const int cc = min(min(w + PW * j, nvb - 1) * 16 + m, p.in.V - 1);
+          vr[j][kb][e] = vp[cc];
+          wr[j][kb][e] = wp[cc];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < PNB; ++j) vr[j][kb][e] = hbc[(unsigned)(i * vw + min(w + PW * j, nvb - 1) * 16 + m)];
+      }
+    }
   // L_ij = sum_c x_ic k_jc e^{Gx_ic - G_jc} (j < i), and for the column output
   // P_ij = sum_c q_ic k_jc e^{G_ic - G_jc} (j <= i): the waves split the key
   // axis; with both Grams waves 0-3 form L's and waves 4-7 P's partials
   const bool second = COL && w >= PW / 2;
   constexpr int STEP = COL ? PW / 2 : PW;
   f4 acc[3] = {zero4(), zero4(), zero4()};
+  [[maybe_unused]] float tru[2], tgx[2];
+  if constexpr (!COL)
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      tru[t2] = tokc[t2 * 16 + m].ru;
+      tgx[t2] = tokc[t2 * 16 + m].gx;
+    }
 #pragma unroll 1
   for (int kb = w % STEP; kb < nkb; kb += STEP) {
     const int c0 = kb * 16 + 4 * g;
-    const float* lp = second ? p.q : p.x;
-    const Quad gl = ldq(p.G + (tb + WBT - 1) * kw + c0);
+    const float* lp = second ? qc : xc;
+    const Quad gl = ldq(Gc + (unsigned)((WBT - 1) * kw + c0));
     Quad a[2], b[2], G[2], Gx[2];
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      const long long o = (tb + t2 * 16 + m) * kw + c0;
-      a[t2] = ldq(lp + o);
-      b[t2] = ldq(p.k + o);
-      G[t2] = ldq(p.G + o);
-      if constexpr (!COL) Gx[t2] = ldq(p.G + (t2 == 0 && m == 0 ? o : o - kw));  // prefix before the token
+      const unsigned o = (t2 * 16 + m) * kw + c0;
+      if constexpr (COL) {
+        a[t2] = ldq(lp + o);
+        b[t2] = ldq(kc + o);
+      } else {
+        b[t2] = scaled(ldq(ubc + o), tru[t2]);
+        a[t2] = scaled(b[t2], tgx[t2]);
+      }
+      G[t2] = ldq(Gc + o);
+      if constexpr (!COL) Gx[t2] = ldq(Gc + (t2 == 0 && m == 0 ? o : o - kw));  // prefix before the token
     }
     bool wild[4];
 #pragma unroll
@@ -412,7 +473,7 @@ __global__ __launch_bounds__(PT, 4) void k_w_prep(OpParams p) {
       }
       const int i = t2 * 16 + m;
       if (second) {
-        *reinterpret_cast<Quad*>(p.Qt + (tb + i) * kw + c0) = a[t2];
+        *reinterpret_cast<Quad*>(p.Qt + tb * kw + (unsigned)(i * kw + c0)) = a[t2];
       } else {
         *reinterpret_cast<Quad*>(xt + i * XTS + c0) = a[t2];
         *reinterpret_cast<f16x4*>(kh + i * KHS + c0) = k4;
@@ -425,12 +486,35 @@ __global__ __launch_bounds__(PT, 4) void k_w_prep(OpParams p) {
       *reinterpret_cast<Quad*>(p.Gam + cbase * kw + c0) = ge;
     }
     gram3(a, b, acc);
-    gram3_wild(wild, kb * 16, !second, [&](int i, int j, int c) {
-      const float gx = COL ? p.G[(tb + i) * kw + c] : i > 0 ? p.G[(tb + i - 1) * kw + c] : 0.f;
-      return lp[(tb + i) * kw + c] * p.k[(tb + j) * kw + c] * __expf(gx - p.G[(tb + j) * kw + c]);
-    }, acc);
+    gram3_wild(wild, kb * 16, !second,
+               [&](int i, int c) {
+                 const float gx = COL ? Gc[i * kw + c] : i > 0 ? Gc[(i - 1) * kw + c] : 0.f;
+                 if constexpr (COL) return make_float2(lp[i * kw + c], gx);
+                 else return make_float2(tokc[i].gx * (bf2f(ubc[i * kw + c]) * tokc[i].ru), gx);
+               },
+               [&](int j, int c) {
+                 if constexpr (COL) return make_float2(kc[j * kw + c], Gc[j * kw + c]);
+                 else return make_float2(bf2f(ubc[j * kw + c]) * tokc[j].ru, Gc[j * kw + c]);
+               }, acc);
   }
   gram3_put(part, w, acc);
+  float vb[PNB][2][4];
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = kb * 16 + 4 * g + e;
+      [[maybe_unused]] const float gm = COL ? 0.f : tokc[i].gam;
+#pragma unroll
+      for (int j = 0; j < PNB; ++j) {
+        if constexpr (COL) {
+          const bool ok = ch * WBT + i < p.in.T && (w + PW * j) * 16 + m < p.in.V;
+          vb[j][kb][e] = ok ? bf2f(vr[j][kb][e]) / (1.f + __expf(-bf2f(wr[j][kb][e]))) : 0.f;
+        } else {
+          vb[j][kb][e] = gm * bf2f(vr[j][kb][e]);
+        }
+      }
+    }
   __syncthreads();
   if (threadIdx.x < (COL ? 2 : 1) * 192) {
     const int half = threadIdx.x / 192, q = (threadIdx.x % 192) >> 6;
@@ -504,7 +588,8 @@ struct WStateParams {
   const void* Wneg;  // -W [Tp][kw] in fragment order (frag_off; fp16 forward, bf16 reverse)
   const void* Kt;    // K^T per chunk [NT][kw][32] (fp16 forward, bf16 reverse)
   const __bf16* At;  // injection A^T per chunk [NT][kw][32] (reverse only; nullable)
-  const float *U, *Gam, *Ib;  // U [Tp][vw] (accumulator order), Ib [Tp][vw]; Gam [NT][kw]
+  const float *U, *Gam;  // U [Tp][vw] (accumulator order); Gam [NT][kw]
+  const __bf16* Ib;      // [Tp][vw]
   void* slots;  // xs_t (forward) or ls_t (reverse)
   float* wout;
   const float* init; int init_t;
@@ -524,11 +609,10 @@ struct WStateParams {
 // The panels Wneg, K^T and At are stored 16-bit by the prep kernels in the
 // order the MFMA operands read them, so each lane's fragment is one 16-byte
 // load; they, U, Gamma and Ib are fetched SPF - 1 chunks ahead into a ring of
-// registers (Ib as two FP32 elements per thread, staged split through LDS like
-// w).  Forward: panels fp16 (W and K are bounded by construction), X
+// registers (Ib as two bf16 elements per thread, staged through LDS).  Forward: panels fp16 (W and K are bounded by construction), X
 // and w split into fp16 halves (~22 bits).  Reverse: bf16 throughout (its
-// exponent range keeps any scale of the cotangent), lambda, dw and Ib split
-// into bf16 halves.  Two barriers per step: the next step writes the X0
+// exponent range keeps any scale of the cotangent), lambda and dw split
+// into bf16 halves (Ib, a bf16 input, enters as it is).  Two barriers per step: the next step writes the X0
 // staging only after this step's second barrier (its readers, the w tiles,
 // are done), and the w staging only after its own first barrier.
 constexpr int WRB = WMAX / 16 / 4;   // row blocks per wave (four-wave kernels)
@@ -544,7 +628,7 @@ constexpr int WLD = WBT + 8;         // row stride (16-bit) of the staged w
 constexpr int XRS = STILE + 8;       // row stride (16-bit) of the row-major slot copy
 constexpr int WFS = WBT + 4;         // row stride (FP32) of the w tile
 constexpr size_t state_smem() {
-  return (size_t)(2 * STILE * XLD + 4 * STILE * WLD + WMAX * XRS) * 2 + (size_t)STILE * WFS * 4;
+  return (size_t)(2 * STILE * XLD + 3 * STILE * WLD + WMAX * XRS) * 2 + (size_t)STILE * WFS * 4;
 }
 
 template <bool REV> struct WStateT;
@@ -571,7 +655,7 @@ struct WFrags {
   V8 W[WKS];                      // Wneg rows of token block w & 1
   V8 K[SRB];                      // K^T rows of this wave's row blocks, the chunk's 32 tokens
   bf16x8 A[REV ? SRB : 1];        // At rows (reverse)
-  float2 ib;                      // reverse: this thread's two elements of the Ib tile
+  unsigned ib;                    // reverse: this thread's two elements of the Ib tile
   f4 U;                           // U tile (C-operand layout)
   float4 G[SRB];                  // Gamma of this wave's rows 16 rb + 4 g .. + 3
 };
@@ -618,9 +702,9 @@ __device__ __forceinline__ void wstate_load(const WStateParams& p, int s, int ch
   }
   if constexpr (REV) {
     static_assert(WBT * STILE == 2 * ST, "two Ib elements per thread");
-    const float* Ip = p.At ? p.Ib : p.U;  // both [Tp][vw]
+    const __bf16* Ip = p.At ? p.Ib : reinterpret_cast<const __bf16*>(p.U);  // (U is the larger)
     const int tok = threadIdx.x / (STILE / 2), col = (threadIdx.x % (STILE / 2)) * 2;
-    f.ib = *reinterpret_cast<const float2*>(Ip + tb * vw + c0 + (unsigned)(tok * vw + col));
+    f.ib = *reinterpret_cast<const unsigned*>(Ip + tb * vw + c0 + (unsigned)(tok * vw + col));
   }
 }
 
@@ -655,8 +739,7 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
   E* wh = Xl + STILE * XLD;          // w [32 columns][WLD]
   E* wl = wh + STILE * WLD;
   E* ih = wl + STILE * WLD;          // reverse: the injection's Ib tile [32 columns][WLD]
-  E* il = ih + STILE * WLD;
-  E* Xr = il + STILE * WLD;          // X0 row-major [rows][XRS]: the slot, written back below
+  E* Xr = ih + STILE * WLD;          // X0 row-major [rows][XRS]: the slot, written back below
   float* wf = reinterpret_cast<float*>(Xr + WMAX * XRS);  // w FP32 [32 columns][WFS]
   static_assert(std::is_same<S, E>::value, "the slot holds the staged high half");
   // X0 staged split and transposed for the w product, and row-major for the slot
@@ -673,15 +756,10 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
     }
   }
   if constexpr (REV) {
-    if (p.At) {  // the Ib tile staged split and transposed ([column][token])
+    if (p.At) {  // the Ib tile (exact in bf16) staged transposed ([column][token])
       const int tok = threadIdx.x / (STILE / 2), col = (threadIdx.x % (STILE / 2)) * 2;
-      const float v2[2] = {f.ib.x, f.ib.y};
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const E hi = (E)v2[j];
-        ih[(col + j) * WLD + tok] = hi;
-        il[(col + j) * WLD + tok] = (E)(v2[j] - (float)hi);
-      }
+      ih[col * WLD + tok] = __builtin_bit_cast(E, (unsigned short)f.ib);
+      ih[(col + 1) * WLD + tok] = __builtin_bit_cast(E, (unsigned short)(f.ib >> 16));
     }
   }
   __syncthreads();
@@ -730,8 +808,6 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
       if constexpr (REV) {
         if (p.At) {
           const bf16x8 bh = *reinterpret_cast<const bf16x8*>(ih + (h * 16 + m) * WLD + kq);
-          const bf16x8 bl = *reinterpret_cast<const bf16x8*>(il + (h * 16 + m) * WLD + kq);
-          X[q][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.A[q], bl, X[q][h], 0, 0, 0);
           X[q][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.A[q], bh, X[q][h], 0, 0, 0);
         }
       }
@@ -827,7 +903,9 @@ __global__ __launch_bounds__(ST) void k_w_state(WStateParams p) {
 struct OutParams {
   int NT, Tp, kw, vw, colout, H, T, V;
   const xs_t* slots;
-  const float *w, *Qt, *P, *q, *k, *G, *base;
+  const float *w, *Qt, *P, *G;
+  const __bf16 *ub, *kb;  // row output: q = base = k^, k = u^
+  const Tok* tok;
   float *o, *d;
   __bf16* out;
 };
@@ -975,17 +1053,17 @@ __global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15, kq = g * 8;
   {
     constexpr int PQ = WBT * WMAX / 4 / WT;
-    float4 qv[PQ];
+    Quad qv[PQ];
 #pragma unroll
     for (int q = 0; q < PQ; ++q) {
       const int idx = threadIdx.x + WT * q, i = (idx * 4) / vw, c = (idx * 4) % vw;
-      if (idx < WBT * vw / 4) qv[q] = *reinterpret_cast<const float4*>(p.q + (tb + i) * vw + c);
+      if (idx < WBT * vw / 4) qv[q] = scaled(ldq(p.kb + (tb + i) * vw + c), p.tok[tb + i].rk);
     }
 #pragma unroll
     for (int q = 0; q < PQ; ++q) {
       const int idx = threadIdx.x + WT * q, i = (idx * 4) / vw, c = (idx * 4) % vw;
       if (idx < WBT * vw / 4) {
-        f4 v = {qv[q].x, qv[q].y, qv[q].z, qv[q].w};
+        f4 v = {qv[q].v[0], qv[q].v[1], qv[q].v[2], qv[q].v[3]};
         f16x4 hi, lo;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1000,13 +1078,12 @@ __global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
   {
     const int bi = w >> 1, bj = w & 1;
     f4 acc = zero4();
+    const float rk = p.tok[tb + bi * 16 + m].rk;
     for (int cb = 0; cb < vw; cb += 16) {
-      const float4 a4 = *reinterpret_cast<const float4*>(p.q + (tb + bi * 16 + m) * vw + cb + 4 * g);
-      const float4 b4 = *reinterpret_cast<const float4*>(p.w + (tb + bj * 16 + m) * vw + cb + 4 * g);
-      acc = mfma4(a4.x, b4.x, acc);
-      acc = mfma4(a4.y, b4.y, acc);
-      acc = mfma4(a4.z, b4.z, acc);
-      acc = mfma4(a4.w, b4.w, acc);
+      const Quad a4 = scaled(ldq(p.kb + (tb + bi * 16 + m) * vw + cb + 4 * g), rk);
+      const Quad b4 = ldq(p.w + (tb + bj * 16 + m) * vw + cb + 4 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = mfma4(a4.v[e], b4.v[e], acc);
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -1017,6 +1094,14 @@ __global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
   __syncthreads();
   const int nrb = kw / 16;
   float ro[WRB][2][4], rbase[WRB][2][4];
+  float tru[2][4], trk[2][4];
+#pragma unroll
+  for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      tru[jb][e] = p.tok[tb + jb * 16 + 4 * g + e].ru;
+      trk[jb][e] = p.tok[tb + jb * 16 + 4 * g + e].rk;
+    }
 #pragma unroll
   for (int q = 0; q < WRB; ++q) {
     const int rb = w + 4 * q;
@@ -1041,7 +1126,7 @@ __global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const long long o = (tb + jb * 16 + 4 * g + e) * kw + rr;
-        kt[jb][e] = keep_exp(!wild, p.k[o], -p.G[o]);
+        kt[jb][e] = keep_exp(!wild, bf2f(p.ub[o]) * tru[jb][e], -p.G[o]);
       }
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
@@ -1058,9 +1143,10 @@ __global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
         float v = __expf(gi) * a[e];
         if (wild)
           for (int j = 0; j <= i; ++j)
-            v += Ml[i * MS + j] * p.k[(tb + j) * kw + rr] * __expf(gi - p.G[(tb + j) * kw + rr]);
+            v += Ml[i * MS + j] * (bf2f(p.ub[(tb + j) * kw + rr]) * p.tok[tb + j].ru) *
+                 __expf(gi - p.G[(tb + j) * kw + rr]);
         ro[q][t2][e] = v;
-        rbase[q][t2][e] = p.base[o];
+        rbase[q][t2][e] = bf2f(p.kb[o]) * trk[t2][e];
       }
     }
   }
@@ -1087,48 +1173,48 @@ constexpr size_t out_smem(int kw, int vw, int colout) {
 }
 
 // ---------------------------------------------------------------------------
-// Dual sources (per token): phi, den, e, chi, z.
+// Dual sources (per token): phi, den, e, chi.
 // ---------------------------------------------------------------------------
 struct SrcParams {
   sd_inputs in;
   int Tp, KP, VP;
-  const float *uh, *delta, *kh, *qh;
-  float *e, *chi, *z;
+  const __bf16 *ub, *kb, *qb;
+  const Tok* tok;
+  const float* delta;
+  float *e, *chi;
 };
 
 __global__ __launch_bounds__(WT) void k_w_sources(SrcParams p) {
-  const int s = blockIdx.y, H = p.in.H, T = p.in.T, r = p.in.r, V = p.in.V;
+  const int s = blockIdx.y, H = p.in.H, T = p.in.T, r = p.in.r;
   const int b = s / H, h = s % H;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int t = blockIdx.x * (WT / 64) + w;
   if (t >= p.Tp) return;
   const bool tv = t < T;
-  const long long row = ((long long)s * p.Tp + t) * p.KP, vrow_ = ((long long)s * p.Tp + t) * p.VP;
+  const long long row = ((long long)s * p.Tp + t) * p.KP;
   // every load first, at clamped indices (masked below): no load under a branch
   const int tc = min(t, T - 1);
-  const __bf16 *err = wrow(p.in.erase_raw, b, tc, h), *vr = wrow(p.in.v, b, tc, h),
-               *wrr = wrow(p.in.write_raw, b, tc, h);
-  float u[4], dl[4], k[4], q[4], er[4], vv[4], wr[4];
+  const __bf16* err = wrow(p.in.erase_raw, b, tc, h);
+  const Tok tk = p.tok[(long long)s * p.Tp + t];
+  float u[4], dl[4], k[4], q[4], er[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int c = l + 64 * j, ck = min(c, p.KP - 1);
-    u[j] = p.uh[row + ck];
+    u[j] = bf2f(p.ub[row + ck]);
     dl[j] = p.delta[row + ck];
-    k[j] = p.kh[row + ck];
-    q[j] = p.qh[row + ck];
+    k[j] = bf2f(p.kb[row + ck]);
+    q[j] = bf2f(p.qb[row + ck]);
     er[j] = bf2f(err[min(c, r - 1)]);
-    vv[j] = bf2f(vr[min(c, V - 1)]);
-    wr[j] = bf2f(wrr[min(c, V - 1)]);
   }
   float usq = 0.f, dsq = 0.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int c = l + 64 * j;
     const bool in = c < p.KP;
-    u[j] = in ? u[j] : 0.f;
+    u[j] = in ? u[j] * tk.ru : 0.f;
     dl[j] = in ? dl[j] : 0.f;
-    k[j] = in ? k[j] : 0.f;
-    q[j] = in ? q[j] : 0.f;
+    k[j] = in ? k[j] * tk.rk : 0.f;
+    q[j] = in ? q[j] * tk.rq : 0.f;
     er[j] = (tv && c < r) ? er[j] : 0.f;
     usq += u[j] * u[j];
     dsq += dl[j] * dl[j];
@@ -1155,10 +1241,6 @@ __global__ __launch_bounds__(WT) void k_w_sources(SrcParams p) {
       p.e[row + c] = bb[j] - phi[j] * sb;
       p.chi[row + c] = q[j] - phi[j] * sq;
     }
-    if (c < p.VP) {
-      const bool ok = tv && c < V;
-      p.z[vrow_ + c] = ok ? vv[j] / (1.f + __expf(-wr[j])) : 0.f;
-    }
   }
 }
 
@@ -1166,13 +1248,15 @@ __global__ __launch_bounds__(WT) void k_w_sources(SrcParams p) {
 // Backward preparation of one op's reverse pass.
 //   column output: rhs = dW + P^T dO, injection Ia = q e^G, Ib = dO
 //   row output:    Pp_ij = sum_r dO_ir k_jr e^{G_ir - G_jr} (j <= i), rhs = dW + Pp^T q,
-//                  Ia = dO e^G, Ib = q
+//                  Ia = dO e^G / |k|, Ib = the raw k (q = k / |k|)
 //   dU = A^T rhs,  Wn = -A^T Kh,  Kn = -x~  (Wn, Kn, Ia stored bf16 for the
 //   reverse pass: -Wn token-major, Kn and Ia transposed per chunk)
 // ---------------------------------------------------------------------------
 struct BprepParams {
-  int NT, Tp, kw, vw, excl, colout;
-  const float *k, *x, *q, *G, *A, *P, *dO, *dW;
+  int NT, Tp, kw, vw;
+  const float *k, *x, *q, *G, *A, *P, *dO, *dW;  // k, x, q: column output; dO, dW: row output
+  const __bf16 *dOb, *ub, *kb;  // column output: dO; row output: u, k (k = u^, x = gx u^, q = k^)
+  const Tok* tok;
   float *dU, *Pp;  // dU [Tp][vw] in accumulator order (acc_off)
   __bf16 *Wneg, *Kt, *At;  // reverse-pass panels: -Wn [Tp][kw] (fragment order); Kn, Ia transposed per chunk [NT][kw][32]
 };
@@ -1189,8 +1273,13 @@ __global__ __launch_bounds__(PT, 4) void k_w_bprep(BprepParams p) {
   const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, vw = p.vw, nkb = kw / 16, nvb = vw / 16;
   const long long tb = (long long)s * p.Tp + ch * WBT;
   const long long cbase = (long long)s * p.NT + ch;
-  const float* Y = COL ? p.dO : p.q;   // [Tp][vw]
-  const float* Yk = COL ? p.q : p.dO;  // [Tp][kw]
+  // chunk-uniform bases, 32-bit lane offsets
+  const __bf16* Y = (COL ? p.dOb : p.kb) + tb * vw;  // [32][vw] (row output: times 1/|k|)
+  const float *Yk = (COL ? p.q : p.dO) + tb * kw, *Gc = p.G + tb * kw;  // [32][kw]
+  const float *kc = COL ? p.k + tb * kw : nullptr, *xc = COL ? p.x + tb * kw : nullptr;
+  const __bf16* ubc = COL ? nullptr : p.ub + tb * kw;
+  const float* dWc = COL ? nullptr : p.dW + tb * vw;
+  const Tok* tokc = COL ? nullptr : p.tok + tb;
   float* kh = sm;               // K^ [32][XTS]
   float* Al = kh + WBT * XTS;   // A [32][AS]
   float* Pl = Al + WBT * AS;    // P or Pp [32][AS]
@@ -1211,21 +1300,35 @@ __global__ __launch_bounds__(PT, 4) void k_w_bprep(BprepParams p) {
   // Pp_ij = sum_c dO_ic k_jc e^{G_ic - G_jc} (j <= i)
   f4 acc[3] = {zero4(), zero4(), zero4()};
   bf16x4 kn4[PNB][2], ia4[PNB][2];
+  [[maybe_unused]] float tru[2], tgx[2], trk[2];
+  if constexpr (!COL)
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const Tok* tk = tokc + t2 * 16 + m;
+      tru[t2] = tk->ru;
+      tgx[t2] = tk->gx;
+      trk[t2] = tk->rks;  // the injection's Ib is the raw bf16 k: its norm goes into Ia
+    }
 #pragma unroll
   for (int j = 0; j < PNB; ++j) {
     const int kb = w + PW * j;
     if (kb >= nkb) continue;
     const int c0 = kb * 16 + 4 * g;
-    const Quad gl = ldq(p.G + (tb + WBT - 1) * kw + c0);
+    const Quad gl = ldq(Gc + (unsigned)((WBT - 1) * kw + c0));
     Quad x[2], k[2], y[2], G[2], Gx[2];
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      const long long o = (tb + t2 * 16 + m) * kw + c0;
-      x[t2] = ldq(p.x + o);
-      k[t2] = ldq(p.k + o);
+      const unsigned o = (t2 * 16 + m) * kw + c0;
+      if constexpr (COL) {
+        x[t2] = ldq(xc + o);
+        k[t2] = ldq(kc + o);
+      } else {
+        k[t2] = scaled(ldq(ubc + o), tru[t2]);
+        x[t2] = scaled(k[t2], tgx[t2]);
+      }
       y[t2] = ldq(Yk + o);
-      G[t2] = ldq(p.G + o);
-      if constexpr (!COL) Gx[t2] = ldq(p.G + (t2 == 0 && m == 0 ? o : o - kw));  // prefix before the token
+      G[t2] = ldq(Gc + o);
+      if constexpr (!COL) Gx[t2] = ldq(Gc + (t2 == 0 && m == 0 ? o : o - kw));  // prefix before the token
     }
     bool wild[4];
 #pragma unroll
@@ -1240,17 +1343,18 @@ __global__ __launch_bounds__(PT, 4) void k_w_bprep(BprepParams p) {
         kd.v[e] = k[t2].v[e] * __expf(gl.v[e] - G[t2].v[e]);
         kn4[j][t2][e] = (__bf16)(-x[t2].v[e] * __expf(gx));
         y[t2].v[e] *= __expf(G[t2].v[e]);
-        ia4[j][t2][e] = (__bf16)y[t2].v[e];
+        ia4[j][t2][e] = (__bf16)(COL ? y[t2].v[e] : y[t2].v[e] * trk[t2]);
         if constexpr (!COL) k[t2].v[e] = keep_exp(!wild[e], k[t2].v[e], -G[t2].v[e]);
       }
       *reinterpret_cast<Quad*>(kh + (t2 * 16 + m) * XTS + c0) = kd;
     }
     if constexpr (!COL) {
       gram3(y, k, acc);
-      gram3_wild(wild, kb * 16, false, [&](int i, int jj, int c) {
-        return Yk[(tb + i) * kw + c] * p.k[(tb + jj) * kw + c] *
-               __expf(p.G[(tb + i) * kw + c] - p.G[(tb + jj) * kw + c]);
-      }, acc);
+      gram3_wild(wild, kb * 16, false,
+                 [&](int i, int c) { return make_float2(Yk[i * kw + c], Gc[i * kw + c]); },
+                 [&](int jj, int c) {
+                   return make_float2(bf2f(ubc[jj * kw + c]) * tokc[jj].ru, Gc[jj * kw + c]);
+                 }, acc);
     }
   }
   // the value side's rows, issued before any store of the kernel
@@ -1263,9 +1367,10 @@ __global__ __launch_bounds__(PT, 4) void k_w_bprep(BprepParams p) {
     for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const long long o = (tb + t2 * 16 + 4 * g + e) * vw + nb * 16 + m;
-        yv[j][t2][e] = Y[o];
-        rhs[j][t2][e] = COL ? 0.f : p.dW[o];
+        const unsigned o = (t2 * 16 + 4 * g + e) * vw + nb * 16 + m;
+        yv[j][t2][e] = bf2f(Y[o]);
+        if constexpr (!COL) yv[j][t2][e] *= tokc[t2 * 16 + 4 * g + e].rk;
+        rhs[j][t2][e] = COL ? 0.f : dWc[o];
       }
   }
   if constexpr (!COL) {
@@ -1372,14 +1477,16 @@ constexpr size_t bprep_smem() {
 // ---------------------------------------------------------------------------
 struct GradParams {
   int NT, Tp, kw, vw;
-  const float *k, *x, *q, *G, *dO, *o, *w, *dw, *Pp;
+  const float *k, *x, *q, *G, *dO, *o, *w, *dw, *Pp;  // k, x, q: column output; dO, o, Pp: row output
+  const __bf16 *dOb, *ub, *kb;  // column output: dO; row output: u, k (k = u^, x = gx u^, q = k^)
+  const Tok* tok;
   const xs_t* Xslots;
   const ls_t* Lslots;
   // column output (S): the panels dk, dx, dq, dg
   float *dk, *dx, *dq, *dg;
   // row output (C): the layer's closure of u, h, k, gamma and the log-decay
   sd_inputs in;
-  const float *gam, *rs, *duh, *dkh, *dgS;
+  const float *duh, *dkh, *dgS;
   __bf16 *du, *dh, *dkey;
   float *dlog_decay, *dgamma;
   int vec;  // the gradients' rows take 4-element stores
@@ -1486,26 +1593,34 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   __bf16* TR = reinterpret_cast<__bf16*>(M2 + WBT * AS);
   constexpr int RP = WBT * KHS;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15, kq = g * 8;
-  const float* Y = COL ? p.dO : p.q;   // [Tp][vw]
-  const float* Yk = COL ? p.q : p.dO;  // [Tp][kw]
+  // chunk-uniform bases, 32-bit lane offsets
+  const __bf16* Y = (COL ? p.dOb : p.kb) + tb * vw;  // [32][vw]: exact in bf16 (row output: M2's rows take 1/|k| at the end)
+  const float *Yk = (COL ? p.q : p.dO) + tb * kw, *Gc = p.G + tb * kw;  // [32][kw]
+  const float *dwc = p.dw + tb * vw, *wc = p.w + tb * vw;
+  const float *kpc = COL ? p.k + tb * kw : nullptr, *xpc = COL ? p.x + tb * kw : nullptr,
+              *opc = COL ? nullptr : p.o + tb * kw;
+  const __bf16 *ubc = COL ? nullptr : p.ub + tb * kw, *kbc = COL ? nullptr : p.kb + tb * kw;
+  const Tok* tokc = COL ? nullptr : p.tok + tb;
   {
     constexpr int PQ = WBT * WMAX / 4 / GT;
-    Quad v[PQ][3];
+    Quad v[PQ][2];
+    bf16x4 y[PQ];
 #pragma unroll
     for (int q = 0; q < PQ; ++q) {
       const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 4 - 1);
-      const long long o = tb * vw + idx * 4;
-      v[q][0] = ldq(p.dw + o);
-      v[q][1] = ldq(p.w + o);
-      v[q][2] = ldq(Y + o);
+      const unsigned o = idx * 4;
+      v[q][0] = ldq(dwc + o);
+      v[q][1] = ldq(wc + o);
+      y[q] = *reinterpret_cast<const bf16x4*>(Y + o);
     }
 #pragma unroll
     for (int q = 0; q < PQ; ++q) {
       const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 4 - 1);
       const int i = (idx * 4) / vw, c = (idx * 4) % vw;
 #pragma unroll
-      for (int a = 0; a < 3; ++a)
+      for (int a = 0; a < 2; ++a)
         split4_to(TR + 2 * a * RP + i * KHS + c, TR + (2 * a + 1) * RP + i * KHS + c, v[q][a]);
+      *reinterpret_cast<bf16x4*>(TR + 4 * RP + i * KHS + c) = y[q];
     }
   }
   __syncthreads();
@@ -1559,18 +1674,17 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
           aX[q][t2] = mma_bf(xh[q], dh, aX[q][t2]);
         }
         if constexpr (COL) {
-          const bf16x8 yh = row(4, t2), yl = row(5, t2);
+          const bf16x8 yh = row(4, t2);
 #pragma unroll
           for (int q = 0; q < GRB; ++q) {
-            aO[q][t2] = mma_bf(xh[q], yl, aO[q][t2]);
             aO[q][t2] = mma_bf(xl[q], yh, aO[q][t2]);
             aO[q][t2] = mma_bf(xh[q], yh, aO[q][t2]);
           }
         }
       }
       if (w < 6) {
-        const bf16x8 ah = row(gm * 2, bi), al = row(gm * 2 + 1, bi), bh = row(2, bj), bl = row(3, bj);
-        am = mma_bf(al, bh, am);
+        const bf16x8 ah = row(gm * 2, bi), bh = row(2, bj), bl = row(3, bj);
+        if (w < 3) am = mma_bf(row(1, bi), bh, am);
         am = mma_bf(ah, bl, am);
         am = mma_bf(ah, bh, am);
       }
@@ -1590,25 +1704,36 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = bi * 16 + 4 * g + e, j = bj * 16 + m;
-      M[i * AS + j] = (w < 3 ? j < i : j <= i) ? am[e] : 0.f;
+      float v = am[e];
+      if (!COL && w >= 3) v *= tokc[i].rk;
+      M[i * AS + j] = (w < 3 ? j < i : j <= i) ? v : 0.f;
     }
   }
   // this lane's elements of the key-side panels (tokens m and 16 + m), loaded
   // before any store of the kernel
   Quad kr[GRB][2], yr[GRB][2], xr[GRB][2], G[GRB][2], orw[GRB][2], gl[GRB];
   int c0[GRB];
+  Tok tk[2];
+#pragma unroll
+  for (int t2 = 0; t2 < 2; ++t2)
+    if constexpr (!COL) tk[t2] = tokc[t2 * 16 + m];
 #pragma unroll
   for (int q = 0; q < GRB; ++q) {
     c0[q] = min(w + GW * q, nrb - 1) * 16 + 4 * g;
-    gl[q] = ldq(p.G + (tb + WBT - 1) * kw + c0[q]);
+    gl[q] = ldq(Gc + (unsigned)((WBT - 1) * kw + c0[q]));
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      const long long o = (tb + t2 * 16 + m) * kw + c0[q];
-      kr[q][t2] = ldq(p.k + o);
+      const unsigned o = (t2 * 16 + m) * kw + c0[q];
+      if constexpr (COL) {
+        kr[q][t2] = ldq(kpc + o);
+        xr[q][t2] = ldq(xpc + o);
+      } else {
+        kr[q][t2] = scaled(ldq(ubc + o), tk[t2].ru);
+        xr[q][t2] = scaled(kr[q][t2], tk[t2].gx);
+      }
       yr[q][t2] = ldq(Yk + o);
-      xr[q][t2] = ldq(p.x + o);
-      G[q][t2] = ldq(p.G + o);
-      if constexpr (!COL) orw[q][t2] = ldq(p.o + o);
+      G[q][t2] = ldq(Gc + o);
+      if constexpr (!COL) orw[q][t2] = ldq(opc + o);
     }
   }
   // rowsum(X_C (.) lam): the four lane groups' partials of each state row
@@ -1651,7 +1776,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) wv[q][kb][e] = p.w[(tb + kb * 16 + 4 * g + e) * vw + nb[q] + m];
+        for (int e = 0; e < 4; ++e) wv[q][kb][e] = wc[(unsigned)((kb * 16 + 4 * g + e) * vw + nb[q] + m)];
     }
     Quad pp[2][2];
 #pragma unroll
@@ -1732,7 +1857,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   if constexpr (!COL) {
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      gmv[t2] = p.gam[tb + t2 * 16 + m];
+      gmv[t2] = tk[t2].gam;
       xk[t2] = erase_keep(p.in, hb, min(ch * WBT + t2 * 16 + m, T - 1));  // fresh: dx reaches neither u nor gamma
     }
   }
@@ -1743,12 +1868,12 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
     if constexpr (!COL) {
 #pragma unroll
       for (int t2 = 0; t2 < 2; ++t2) {
-        const long long o = (tb + t2 * 16 + m) * kw + c0[q];
-        gu[q][t2] = ldq(p.duh + o);
-        gk[q][t2] = ldq(p.dkh + o);
-        kn[t2] = ldq(p.q + o);
-        dv[t2] = ldq(p.dw + o);
-        dgo[q][t2] = ldq(p.dgS + o);
+        const unsigned o = (t2 * 16 + m) * kw + c0[q];
+        gu[q][t2] = ldq(p.duh + tb * kw + o);
+        gk[q][t2] = ldq(p.dkh + tb * kw + o);
+        kn[t2] = scaled(ldq(kbc + o), tk[t2].rk);
+        dv[t2] = ldq(dwc + o);
+        dgo[q][t2] = ldq(p.dgS + tb * kw + o);
         const __bf16* hr = wrow(p.in.h, hb, min(ch * WBT + t2 * 16 + m, T - 1), hh);
 #pragma unroll
         for (int e = 0; e < 4; ++e) hv[t2].v[e] = bf2f(hr[min(c0[q] + e, r - 1)]);
@@ -1840,25 +1965,29 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
         for (int e = 0; e < 4; ++e) {
           if (!wild[e]) continue;
           const int i = t2 * 16 + m;
-          const float* gc = p.G + tb * kw + c0[q] + e;
-          const float *kc = p.k + tb * kw + c0[q] + e, *yc = Yk + tb * kw + c0[q] + e,
-                      *xc = p.x + tb * kw + c0[q] + e;
+          const float* gc = Gc + c0[q] + e;
+          const float* yc = Yk + c0[q] + e;
+          auto kc = [&](int j) {
+            const unsigned o = (j) * kw + c0[q] + e;
+            return COL ? kpc[o] : bf2f(ubc[o]) * tokc[j].ru;
+          };
+          auto xc = [&](int j) { return COL ? xpc[j * kw + c0[q] + e] : kc(j) * tokc[j].gx; };
           const float gi = G[q][t2].v[e], gxi = gx[t2][e];
           auto gxa = [&](int j) { return COL ? gc[(long long)j * kw] : j > 0 ? gc[(long long)(j - 1) * kw] : 0.f; };
           float a = __expf(gxi) * aX[q][t2][e];
           for (int j = 0; j < i; ++j)
-            a += M1[i * AS + j] * kc[(long long)j * kw] * __expf(gxi - gc[(long long)j * kw]);
+            a += M1[i * AS + j] * kc(j) * __expf(gxi - gc[(long long)j * kw]);
           rdx[t2].v[e] = -a;
           float b = __expf(gl[q].v[e] - gi) * aL[q][t2][e];
           for (int j = i; j < WBT; ++j)
             b += M2[j * AS + i] * yc[(long long)j * kw] * __expf(gc[(long long)j * kw] - gi);
           for (int j = i + 1; j < WBT; ++j)
-            b -= M1[j * AS + i] * xc[(long long)j * kw] * __expf(gxa(j) - gi);
+            b -= M1[j * AS + i] * xc(j) * __expf(gxa(j) - gi);
           rdk[t2].v[e] = b;
           if constexpr (COL) {
             float c2 = __expf(gi) * aO[q][t2][e];
             for (int j = 0; j <= i; ++j)
-              c2 += M2[i * AS + j] * kc[(long long)j * kw] * __expf(gi - gc[(long long)j * kw]);
+              c2 += M2[i * AS + j] * kc(j) * __expf(gi - gc[(long long)j * kw]);
             rdq[t2].v[e] = c2;
           }
         }
@@ -1894,11 +2023,11 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
     if constexpr (COL) {
 #pragma unroll
       for (int t2 = 0; t2 < 2; ++t2) {
-        const long long o = (tb + t2 * 16 + m) * kw + c0[q];
-        *reinterpret_cast<Quad*>(p.dx + o) = rdx[t2];
-        *reinterpret_cast<Quad*>(p.dk + o) = rdk[t2];
-        *reinterpret_cast<Quad*>(p.dq + o) = rdq[t2];
-        *reinterpret_cast<Quad*>(p.dg + o) = rdg[t2];
+        const unsigned o = (t2 * 16 + m) * kw + c0[q];
+        *reinterpret_cast<Quad*>(p.dx + tb * kw + o) = rdx[t2];
+        *reinterpret_cast<Quad*>(p.dk + tb * kw + o) = rdk[t2];
+        *reinterpret_cast<Quad*>(p.dq + tb * kw + o) = rdq[t2];
+        *reinterpret_cast<Quad*>(p.dg + tb * kw + o) = rdg[t2];
       }
     } else {
 #pragma unroll
@@ -1933,7 +2062,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
 #pragma unroll
     for (int q = 0; q < GRB; ++q)
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) kn[q][t2] = ldq(p.q + (tb + t2 * 16 + m) * kw + c0[q]);
+      for (int t2 = 0; t2 < 2; ++t2) kn[q][t2] = scaled(ldq(kbc + (unsigned)((t2 * 16 + m) * kw + c0[q])), tk[t2].rk);
     __syncthreads();
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
@@ -1946,7 +2075,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
         v[a] = ((r0.v[0] + r0.v[1]) + (r0.v[2] + r0.v[3])) + ((r1.v[0] + r1.v[1]) + (r1.v[2] + r1.v[3]));
       }
       if (t >= T) continue;
-      const float ru = p.rs[(tb + t2 * 16 + m) * 3], rk = p.rs[(tb + t2 * 16 + m) * 3 + 1];
+      const float ru = tk[t2].ru, rk = tk[t2].rk;
       const long long ob = ((long long)hb * T + t) * H + hh, o = ob * r;
 #pragma unroll
       for (int q = 0; q < GRB; ++q) {
@@ -1967,8 +2096,8 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   }
 }
 
-constexpr size_t grad_smem() { return (size_t)2 * WBT * AS * sizeof(float) + (size_t)6 * WBT * KHS * 2; }
-static_assert(6 * WBT * KHS * 2 >= (GW * 3 * WBT * GS16 + 3 * WBT * GW) * 4,
+constexpr size_t grad_smem() { return (size_t)2 * WBT * AS * sizeof(float) + (size_t)5 * WBT * KHS * 2; }
+static_assert(5 * WBT * KHS * 2 >= (GW * 3 * WBT * GS16 + 3 * WBT * GW) * 4,
               "phase 3's panels and row sums fit the split rows' storage");
 
 // ---------------------------------------------------------------------------
@@ -1978,7 +2107,9 @@ static_assert(6 * WBT * KHS * 2 >= (GW * 3 * WBT * GS16 + 3 * WBT * GW) * 4,
 struct SrcBwdParams {
   sd_inputs in;
   int Tp, KP, VP;
-  const float *uh, *delta, *kh, *qh, *rs, *de, *dchi, *dz;
+  const __bf16 *ub, *kb, *qb;
+  const Tok* tok;
+  const float *delta, *de, *dchi, *dz;
   float *duh, *ddelta, *dkh;
   __bf16 *dq, *derase, *dwrite, *dv;
 };
@@ -1995,14 +2126,15 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
   const int tc = min(t, T - 1);
   const __bf16 *err = wrow(p.in.erase_raw, b, tc, h), *vrow = wrow(p.in.v, b, tc, h),
                *wrr = wrow(p.in.write_raw, b, tc, h);
+  const Tok tk = p.tok[(long long)s * p.Tp + t];
   float u[4], dl[4], k[4], q[4], er[4], de[4], dc[4], vv[4], wr[4], dzv[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int c = l + 64 * j, ck = min(c, p.KP - 1), cv = min(c, V - 1);
-    u[j] = p.uh[row + ck];
+    u[j] = bf2f(p.ub[row + ck]);
     dl[j] = p.delta[row + ck];
-    k[j] = p.kh[row + ck];
-    q[j] = p.qh[row + ck];
+    k[j] = bf2f(p.kb[row + ck]);
+    q[j] = bf2f(p.qb[row + ck]);
     de[j] = p.de[row + ck];
     dc[j] = p.dchi[row + ck];
     er[j] = bf2f(err[min(c, r - 1)]);
@@ -2015,10 +2147,10 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
   for (int j = 0; j < 4; ++j) {
     const int c = l + 64 * j;
     const bool in = c < p.KP;
-    u[j] = in ? u[j] : 0.f;
+    u[j] = in ? u[j] * tk.ru : 0.f;
     dl[j] = in ? dl[j] : 0.f;
-    k[j] = in ? k[j] : 0.f;
-    q[j] = in ? q[j] : 0.f;
+    k[j] = in ? k[j] * tk.rk : 0.f;
+    q[j] = in ? q[j] * tk.rq : 0.f;
     de[j] = in ? de[j] : 0.f;
     dc[j] = in ? dc[j] : 0.f;
     er[j] = (tv && c < r) ? er[j] : 0.f;
@@ -2061,7 +2193,6 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) sqq += dqh[j] * q[j];
   sqq = wave_sum(sqq);
-  const float rq = p.rs[((long long)s * p.Tp + t) * 3 + 2];
   const float dN2 = (-RHO * ds / (N * N)) / (2.f * N);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -2072,7 +2203,7 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
       p.dkh[row + c] = db[j] * se[j];
     }
     const long long obase = ((long long)b * T + t) * H + h;
-    if (tv && c < r) p.dq[obase * r + c] = f2bf((dqh[j] - sqq * q[j]) * rq);
+    if (tv && c < r) p.dq[obase * r + c] = f2bf((dqh[j] - sqq * q[j]) * tk.rq);
     if (tv && c < r) p.derase[obase * r + c] = f2bf(db[j] * k[j] * se[j] * (1.f - se[j]));
     if (tv && c < V) {
       const float sw = 1.f / (1.f + __expf(-wr[j]));
@@ -2082,19 +2213,19 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
   }
 }
 
-// Output cotangent as an FP32 panel (zero when absent and on padded entries).
+// Output cotangent as a padded bf16 panel (zero when absent and on padded entries).
 struct DoutParams {
   int H, T, V, Tp, VP;
   const __bf16* dout;
-  float* dO;
+  __bf16* dO;
 };
 __global__ __launch_bounds__(WT) void k_w_dout(DoutParams p) {
   const int s = blockIdx.y, b = s / p.H, h = s % p.H;
   const long long n = (long long)p.Tp * p.VP;
   for (long long idx = (long long)blockIdx.x * WT + threadIdx.x; idx < n; idx += (long long)gridDim.x * WT) {
     const int t = (int)(idx / p.VP), c = (int)(idx % p.VP);
-    float v = 0.f;
-    if (p.dout && t < p.T && c < p.V) v = bf2f(p.dout[(((long long)b * p.T + t) * p.H + h) * p.V + c]);
+    __bf16 v = f2bf(0.f);
+    if (p.dout && t < p.T && c < p.V) v = p.dout[(((long long)b * p.T + t) * p.H + h) * p.V + c];
     p.dO[(long long)s * n + idx] = v;
   }
 }
@@ -2136,24 +2267,27 @@ struct WCarver {
 };
 
 struct WideFwd {
-  float *G, *uh, *kh, *qh, *xC, *vC, *gam, *rs;
-  float *delta, *oC, *d, *e, *chi, *z, *wS;
+  float* G;
+  __bf16 *ub, *kb, *qb, *hb;
+  Tok* tok;
+  float *delta, *oC, *d, *e, *chi, *wS;
   float *AC, *AS, *PS;
   xs_t *XC, *XS;
   _Float16 *Wneg, *Kt;
   float *U, *Qt, *Gam;
 };
 
-// saved: what the backward reads; scratch: the forward-only panels (the C op's
-// gamma h, the S op's z, and both ops' W, U, K^, Q~).
+// saved: what the backward reads; scratch: the forward-only panels (the packed h
+// and both ops' W, U, K^, Q~).
 WideFwd carve_wide_fwd(void* saved, void* scratch, const WideDims& d, size_t* saved_bytes,
                        size_t* scratch_bytes) {
   WCarver c{(char*)saved};
   const size_t tok = (size_t)d.n * d.Tp, pk = tok * d.KP, pv = tok * d.VP;
   const size_t mat = (size_t)d.n * d.NT * WBT * WBT;
   WideFwd w;
-  w.G = c.take(pk); w.uh = c.take(pk); w.kh = c.take(pk); w.qh = c.take(pk);
-  w.xC = c.take(pk); w.gam = c.take(tok); w.rs = c.take(tok * 3);
+  w.G = c.take(pk);
+  w.ub = c.take<__bf16>(pk); w.kb = c.take<__bf16>(pk); w.qb = c.take<__bf16>(pk);
+  w.tok = c.take<Tok>(tok);
   w.delta = c.take(pk); w.oC = c.take(pk); w.d = c.take(pk); w.e = c.take(pk);
   w.chi = c.take(pk); w.wS = c.take(pv);
   w.AC = c.take(mat); w.AS = c.take(mat); w.PS = c.take(mat);
@@ -2163,14 +2297,14 @@ WideFwd carve_wide_fwd(void* saved, void* scratch, const WideDims& d, size_t* sa
   if (saved_bytes) *saved_bytes = c.off + 256;
   WCarver t{(char*)scratch};
   const size_t pm = d.KP > d.VP ? pk : pv;
-  w.vC = t.take(pk); w.z = t.take(pv);
+  w.hb = t.take<__bf16>(pk);
   w.Wneg = t.take<_Float16>(pk); w.U = t.take(pm); w.Kt = t.take<_Float16>(pk); w.Qt = t.take(pk);
   if (scratch_bytes) *scratch_bytes = t.off + 256;
   return w;
 }
 
 struct WideBwd {
-  float* dO;
+  __bf16* dO;
   ls_t *LC, *LS;
   float *dU, *Pp;
   __bf16 *Wneg, *Kt, *At;
@@ -2183,7 +2317,7 @@ WideBwd carve_wide_bwd(void* base, const WideDims& d, size_t* total) {
   const size_t tok = (size_t)d.n * d.Tp, pk = tok * d.KP, pv = tok * d.VP;
   const size_t pm = d.KP > d.VP ? pk : pv;
   WideBwd w;
-  w.dO = c.take(pv);
+  w.dO = c.take<__bf16>(pv);
   w.LC = c.take<ls_t>((size_t)d.n * (d.NT + 1) * d.KP * d.KP);
   w.LS = c.take<ls_t>((size_t)d.n * (d.NT + 1) * d.KP * d.VP);
   w.dU = c.take(pm); w.Wneg = c.take<__bf16>(pk); w.Kt = c.take<__bf16>(pk); w.At = c.take<__bf16>(pk);
@@ -2238,14 +2372,13 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
 
   TokParams tp{};
   tp.in = *in; tp.NT = d.NT; tp.Tp = d.Tp; tp.KP = d.KP;
-  tp.G = w.G; tp.uh = w.uh; tp.kh = w.kh; tp.qh = w.qh; tp.xC = w.xC; tp.vC = w.vC;
-  tp.gam = w.gam; tp.rs = w.rs;
+  tp.G = w.G; tp.ub = w.ub; tp.kb = w.kb; tp.qb = w.qb; tp.hb = w.hb; tp.tok = w.tok;
   SD_LAUNCH("k_w_tokens", k_w_tokens, dim3(d.NT, d.n), dim3(WT), 0, st, tp);
 
   // predictor C: X = C^T, k = u^, x = gamma u^, v = gamma h, q = k^, row output
   OpParams oc{};
-  oc.NT = d.NT; oc.Tp = d.Tp; oc.kw = d.KP; oc.vw = d.KP; oc.excl = 1; oc.colout = 0;
-  oc.k = w.uh; oc.x = w.xC; oc.v = w.vC; oc.q = w.kh; oc.G = w.G;
+  oc.NT = d.NT; oc.Tp = d.Tp; oc.kw = d.KP; oc.vw = d.KP; oc.colout = 0;
+  oc.ub = w.ub; oc.hb = w.hb; oc.tok = w.tok; oc.G = w.G;
   oc.A = w.AC; oc.P = w.PS; oc.Wneg = w.Wneg; oc.U = w.U; oc.Kt = w.Kt; oc.Qt = w.Qt; oc.Gam = w.Gam;
   launch_wprep(oc, d.n, st);
   WStateParams sc{};
@@ -2256,21 +2389,21 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
   launch_wstate("w_state_c_fwd", sc, d.n, st);
   OutParams orow{};
   orow.NT = d.NT; orow.Tp = d.Tp; orow.kw = d.KP; orow.vw = d.KP; orow.colout = 0;
-  orow.slots = w.XC; orow.w = w.delta; orow.q = w.kh; orow.k = w.uh; orow.G = w.G;
-  orow.base = w.kh; orow.o = w.oC; orow.d = w.d;
+  orow.slots = w.XC; orow.w = w.delta; orow.ub = w.ub; orow.kb = w.kb; orow.tok = w.tok;
+  orow.G = w.G; orow.o = w.oC; orow.d = w.d;
   SD_SMEM_ONCE(k_w_out, (int)(out_smem(WMAX, WMAX, 0) > out_smem(WMAX, WMAX, 1) ? out_smem(WMAX, WMAX, 0) : out_smem(WMAX, WMAX, 1)));
   SD_LAUNCH("k_w_out_c", k_w_out, dim3(d.NT, d.n), dim3(WT), out_smem(d.KP, d.KP, 0), st, orow);
 
   SrcParams sp{};
   sp.in = *in; sp.Tp = d.Tp; sp.KP = d.KP; sp.VP = d.VP;
-  sp.uh = w.uh; sp.delta = w.delta; sp.kh = w.kh; sp.qh = w.qh;
-  sp.e = w.e; sp.chi = w.chi; sp.z = w.z;
+  sp.ub = w.ub; sp.kb = w.kb; sp.qb = w.qb; sp.tok = w.tok; sp.delta = w.delta;
+  sp.e = w.e; sp.chi = w.chi;
   SD_LAUNCH("k_w_sources", k_w_sources, dim3(d.Tp / (WT / 64), d.n), dim3(WT), 0, st, sp);
 
   // memory S: k = d, x = e, v = z, q = chi, column output
   OpParams os{};
-  os.NT = d.NT; os.Tp = d.Tp; os.kw = d.KP; os.vw = d.VP; os.excl = 0; os.colout = 1;
-  os.k = w.d; os.x = w.e; os.v = w.z; os.q = w.chi; os.G = w.G;
+  os.NT = d.NT; os.Tp = d.Tp; os.kw = d.KP; os.vw = d.VP; os.colout = 1;
+  os.k = w.d; os.x = w.e; os.q = w.chi; os.G = w.G; os.in = *in;
   os.A = w.AS; os.P = w.PS; os.Wneg = w.Wneg; os.U = w.U; os.Kt = w.Kt; os.Qt = w.Qt; os.Gam = w.Gam;
   launch_wprep(os, d.n, st);
   WStateParams ss{};
@@ -2304,9 +2437,9 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
 
   // ---- memory S op ----
   BprepParams bs{};
-  bs.NT = d.NT; bs.Tp = d.Tp; bs.kw = d.KP; bs.vw = d.VP; bs.excl = 0; bs.colout = 1;
+  bs.NT = d.NT; bs.Tp = d.Tp; bs.kw = d.KP; bs.vw = d.VP;
   bs.k = f.d; bs.x = f.e; bs.q = f.chi; bs.G = f.G; bs.A = f.AS; bs.P = f.PS;
-  bs.dO = w.dO; bs.dW = nullptr;
+  bs.dOb = w.dO;
   bs.dU = w.dU; bs.Wneg = w.Wneg; bs.Kt = w.Kt; bs.At = w.At; bs.Pp = w.Pp;
   SD_SMEM_ONCE(k_w_bprep<true>, (int)bprep_smem());
   SD_LAUNCH("k_w_bprep_s", k_w_bprep<true>, dim3(d.NT, d.n), dim3(PT), bprep_smem(), st, bs);
@@ -2318,7 +2451,7 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   launch_wstate("w_state_s_bwd", rs, d.n, st);
   GradParams gs{};
   gs.NT = d.NT; gs.Tp = d.Tp; gs.kw = d.KP; gs.vw = d.VP;
-  gs.k = f.d; gs.x = f.e; gs.q = f.chi; gs.G = f.G; gs.dO = w.dO; gs.o = nullptr;
+  gs.k = f.d; gs.x = f.e; gs.q = f.chi; gs.G = f.G; gs.dOb = w.dO;
   gs.w = f.wS; gs.dw = w.dwS; gs.Xslots = f.XS; gs.Lslots = w.LS; gs.Pp = nullptr;
   gs.dk = w.dd; gs.dx = w.de; gs.dq = w.dchi; gs.dg = w.dgS;
   SD_SMEM_ONCE(k_w_grad<true>, (int)grad_smem());
@@ -2326,32 +2459,31 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
 
   SrcBwdParams sb{};
   sb.in = *in; sb.Tp = d.Tp; sb.KP = d.KP; sb.VP = d.VP;
-  sb.uh = f.uh; sb.delta = f.delta; sb.kh = f.kh; sb.qh = f.qh;
+  sb.ub = f.ub; sb.kb = f.kb; sb.qb = f.qb; sb.tok = f.tok; sb.delta = f.delta;
   sb.de = w.de; sb.dchi = w.dchi; sb.dz = w.dwS;
-  sb.rs = f.rs;
   sb.duh = w.duh; sb.ddelta = w.ddelta; sb.dkh = w.dkh; sb.dq = (__bf16*)dq;
   sb.derase = (__bf16*)derase; sb.dwrite = (__bf16*)dwrite; sb.dv = (__bf16*)dv;
   SD_LAUNCH("k_w_src_bwd", k_w_src_bwd, dim3(d.Tp / (WT / 64), d.n), dim3(WT), 0, st, sb);
 
   // ---- predictor C op: output cotangent dd (d = k^ + o_C), dW = ddelta ----
   BprepParams bc{};
-  bc.NT = d.NT; bc.Tp = d.Tp; bc.kw = d.KP; bc.vw = d.KP; bc.excl = 1; bc.colout = 0;
-  bc.k = f.uh; bc.x = f.xC; bc.q = f.kh; bc.G = f.G; bc.A = f.AC; bc.P = nullptr;
+  bc.NT = d.NT; bc.Tp = d.Tp; bc.kw = d.KP; bc.vw = d.KP;
+  bc.ub = f.ub; bc.kb = f.kb; bc.tok = f.tok; bc.G = f.G; bc.A = f.AC;
   bc.dO = w.dd; bc.dW = w.ddelta;
   bc.dU = w.dU; bc.Wneg = w.Wneg; bc.Kt = w.Kt; bc.At = w.At; bc.Pp = w.Pp;
   SD_SMEM_ONCE(k_w_bprep<false>, (int)bprep_smem());
   SD_LAUNCH("k_w_bprep_c", k_w_bprep<false>, dim3(d.NT, d.n), dim3(PT), bprep_smem(), st, bc);
   WStateParams rc{};
   rc.NT = d.NT; rc.Tp = d.Tp; rc.kw = d.KP; rc.vw = d.KP; rc.rows = in->r; rc.cols = in->r; rc.rev = 1;
-  rc.Wneg = w.Wneg; rc.U = w.dU; rc.Kt = w.Kt; rc.Gam = f.Gam; rc.At = w.At; rc.Ib = f.kh;
+  rc.Wneg = w.Wneg; rc.U = w.dU; rc.Kt = w.Kt; rc.Gam = f.Gam; rc.At = w.At; rc.Ib = f.kb;
   rc.slots = w.LC; rc.wout = w.dwC;
   rc.init = dC_T; rc.init_t = 1; rc.fin = dC0; rc.fin_t = 1;
   launch_wstate("w_state_c_bwd", rc, d.n, st);
   GradParams gc{};
   gc.NT = d.NT; gc.Tp = d.Tp; gc.kw = d.KP; gc.vw = d.KP;
-  gc.k = f.uh; gc.x = f.xC; gc.q = f.kh; gc.G = f.G; gc.dO = w.dd; gc.o = f.oC;
+  gc.ub = f.ub; gc.kb = f.kb; gc.tok = f.tok; gc.G = f.G; gc.dO = w.dd; gc.o = f.oC;
   gc.w = f.delta; gc.dw = w.dwC; gc.Xslots = f.XC; gc.Lslots = w.LC; gc.Pp = w.Pp;
-  gc.in = *in; gc.gam = f.gam; gc.rs = f.rs; gc.duh = w.duh; gc.dkh = w.dkh; gc.dgS = w.dgS;
+  gc.in = *in; gc.duh = w.duh; gc.dkh = w.dkh; gc.dgS = w.dgS;
   gc.du = (__bf16*)du; gc.dh = (__bf16*)dh; gc.dkey = (__bf16*)dk;
   gc.dlog_decay = dlog_decay; gc.dgamma = dgamma;
   gc.vec = in->r % 4 == 0 && (((uintptr_t)du | (uintptr_t)dh | (uintptr_t)dk) & 7) == 0 &&
