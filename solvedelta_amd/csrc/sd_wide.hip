@@ -202,7 +202,7 @@ struct OpParams {
   const Tok* tok;
   sd_inputs in;                // column output: v = sigmoid(write_raw) v from the raw inputs
   float *A, *P;                    // [NT][32][32]
-  _Float16 *Wneg, *Kt;             // state-pass panels: -W [Tp][kw] (fragment order), K^ transposed per chunk [NT][kw][32]
+  _Float16 *Wneg, *Kt;             // state-pass panels: -W (w_off order), K^ transposed per chunk [NT][kw][32]
   float *U, *Qt, *Gam;             // Qt [Tp][kw]; U [Tp][vw] (accumulator order); Gam [NT][kw]
 };
 
@@ -217,6 +217,21 @@ struct OpParams {
 // holding tokens 16 tb + 4 g .. + 3 of column 16 cb + m, as an MFMA writes it.
 __device__ __forceinline__ unsigned acc_off(int tb, int cb, int lane, int C) {
   return (unsigned)(((tb * (C >> 4) + cb) * 64 + lane) * 4);
+}
+
+// Position of W's element (token t, state row) in its panel: the two token
+// blocks' operands of a 16-row block side by side, 16 bytes per lane.
+__device__ __forceinline__ unsigned w_off(int rb, int lane, int tb) {
+  return (unsigned)(((rb * 64 + lane) * 2 + tb) * 4);
+}
+
+// A state slot [kw][vw] is kept in 32-column tiles, [vw / 32][kw][32]: a state
+// workgroup writes whole lines of its own tile, and a 16-row operand fragment
+// of 32 columns is 1 KiB contiguous.  Row-major slots held the state passes to
+// the rate of their half-line stores: SLOT_US
+constexpr int STILE = 32;  // state columns per workgroup
+__device__ __forceinline__ unsigned slot_off(int row, int col, int kw) {
+  return (unsigned)(((col / STILE) * kw + row) * STILE + col % STILE);
 }
 
 constexpr float WILD = 60.f;
@@ -540,8 +555,8 @@ __global__ __launch_bounds__(PT, 4) void k_w_prep(OpParams p) {
     *reinterpret_cast<Quad*>(p.A + cbase * WBT * WBT + i * WBT + j) = *reinterpret_cast<const Quad*>(Ls + i * AS + j);
   }
   // W = A x~ and U = A v on FP32 matrix cores over A's lower blocks.  W is
-  // formed transposed (a lane holds four neighbouring columns of one token: one
-  // 8-byte store), -W fp16 for the state pass; U in accumulator order.
+  // formed transposed (a lane holds four neighbouring columns of a token, the
+  // state pass's operand order), -W fp16; U in accumulator order.
 #pragma unroll
   for (int j = 0; j < PNB; ++j) {
     const int nb = w + PW * j;
@@ -560,16 +575,15 @@ __global__ __launch_bounds__(PT, 4) void k_w_prep(OpParams p) {
           au[t2] = mfma4(av, vb[j][kb][e], au[t2]);
         }
       }
+    if (nb < nkb) {
+      f16x8 h;
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      if (nb < nkb) {
-        f16x4 h;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = (_Float16)(-aw[t2][e]);
-        *reinterpret_cast<f16x4*>(p.Wneg + tb * kw + frag_off(t2 * 16 + m, nb * 16 + 4 * g, kw)) = h;
-      }
-      if (nb < nvb) *reinterpret_cast<f4*>(p.U + tb * vw + acc_off(t2, nb, l, vw)) = au[t2];
+      for (int e = 0; e < 8; ++e) h[e] = (_Float16)(-aw[e >> 2][e & 3]);
+      *reinterpret_cast<f16x8*>(p.Wneg + tb * kw + w_off(nb, l, 0)) = h;
     }
+    if (nb < nvb)
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) *reinterpret_cast<f4*>(p.U + tb * vw + acc_off(t2, nb, l, vw)) = au[t2];
   }
   store_transposed(p.Kt + cbase * kw * WBT, kh, kw);
 }
@@ -585,7 +599,7 @@ constexpr size_t prep_smem() {
 // ---------------------------------------------------------------------------
 struct WStateParams {
   int NT, Tp, kw, vw, rows, cols, rev;
-  const void* Wneg;  // -W [Tp][kw] in fragment order (frag_off; fp16 forward, bf16 reverse)
+  const void* Wneg;  // -W per chunk in w_off order (fp16 forward, bf16 reverse)
   const void* Kt;    // K^T per chunk [NT][kw][32] (fp16 forward, bf16 reverse)
   const __bf16* At;  // injection A^T per chunk [NT][kw][32] (reverse only; nullable)
   const float *U, *Gam;  // U [Tp][vw] (accumulator order); Gam [NT][kw]
@@ -596,39 +610,40 @@ struct WStateParams {
   float* fin; int fin_t;
 };
 
-// Matrix-core form on 16-bit MFMAs (v_mfma_f32_16x16x32_{f16,bf16}), as the
-// main kernels' state pass: a workgroup of 8 waves owns a 32-column tile of the
-// state, wave w holding the 16-row blocks w and w + 8 of both 16-column halves
-// in FP32 accumulators.  Per chunk step:
-//   the state X0 is staged into LDS split into high and low 16-bit halves,
-//   transposed ([column][row]), as the B operand of w = U + Wneg X0, which
-//   waves 0-3 form (one 16-token x 16-column tile each, over all kw rows);
-//   w is staged split the same way ([column][token]) as the B operand of
+// Matrix-core form on 16-bit MFMAs: a workgroup of 8 waves owns a 32-column
+// tile of the state, wave w holding the 16-row blocks w and w + 8 of both
+// 16-column halves in FP32 accumulators.  Per chunk step:
+//   w = U + Wneg X0: an accumulator (lane (g, m): rows 4 g .. + 3 of column m)
+//   is the B operand of v_mfma_f32_16x16x16 as it stands, so each wave
+//   multiplies its own rows, split into high and low 16-bit halves, into a
+//   partial w of all 32 tokens; the partials meet in LDS, where every thread
+//   sums two elements over the eight waves, adds U and stores w, and w again
+//   split and transposed ([column][token]) as the B operand of
 //   X = Gamma X + K^T w (+ At^T Ib, reverse), which every wave forms for its
 //   own rows.
+// The state itself never passes through LDS (the form that staged it there for
+// four waves to read moved 170 KB of LDS and 64 KB of Wneg per step against 90
+// and 16): STATE_US
 // The panels Wneg, K^T and At are stored 16-bit by the prep kernels in the
 // order the MFMA operands read them, so each lane's fragment is one 16-byte
 // load; they, U, Gamma and Ib are fetched SPF - 1 chunks ahead into a ring of
-// registers (Ib as two bf16 elements per thread, staged through LDS).  Forward: panels fp16 (W and K are bounded by construction), X
+// registers (Ib as two bf16 elements per thread, staged through LDS).
+// Forward: panels fp16 (W and K are bounded by construction), X
 // and w split into fp16 halves (~22 bits).  Reverse: bf16 throughout (its
 // exponent range keeps any scale of the cotangent), lambda and dw split
-// into bf16 halves (Ib, a bf16 input, enters as it is).  Two barriers per step: the next step writes the X0
-// staging only after this step's second barrier (its readers, the w tiles,
-// are done), and the w staging only after its own first barrier.
+// into bf16 halves (Ib, a bf16 input, enters as it is).  Two barriers per step:
+// the partials are read between them and written again only before the next
+// step's first; the split w is written between them and read before that.
 constexpr int WRB = WMAX / 16 / 4;   // row blocks per wave (four-wave kernels)
 constexpr int SW = 8;                // state-pass waves: two per SIMD
 constexpr int ST = SW * 64;
 constexpr int SRB = WMAX / 16 / SW;  // state-pass row blocks per wave
-constexpr int STILE = 32;            // state columns per workgroup
 constexpr int NSUB = STILE / 16;
-constexpr int WKS = WMAX / 32;       // K = 32 steps of the w product
-constexpr int SPF = 2;               // prefetch ring depth (chunks)
-constexpr int XLD = WMAX + 8;        // row stride (16-bit) of the staged X0
+constexpr int SPF = 3;               // prefetch ring depth (chunks)
 constexpr int WLD = WBT + 8;         // row stride (16-bit) of the staged w
-constexpr int XRS = STILE + 8;       // row stride (16-bit) of the row-major slot copy
-constexpr int WFS = WBT + 4;         // row stride (FP32) of the w tile
+constexpr int NTILE = WBT / 16 * NSUB;  // 16 x 16 tiles of w: tile = token block * NSUB + half
 constexpr size_t state_smem() {
-  return (size_t)(2 * STILE * XLD + 3 * STILE * WLD + WMAX * XRS) * 2 + (size_t)STILE * WFS * 4;
+  return (size_t)SW * NTILE * 256 * 4 + (size_t)3 * STILE * WLD * 2;
 }
 
 template <bool REV> struct WStateT;
@@ -639,6 +654,9 @@ template <> struct WStateT<false> {
   static __device__ __forceinline__ f4 mma(V8 a, V8 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f4 mma16(V4 a, V4 b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
+  }
 };
 template <> struct WStateT<true> {
   using E = __bf16;
@@ -647,27 +665,31 @@ template <> struct WStateT<true> {
   static __device__ __forceinline__ f4 mma(V8 a, V8 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f4 mma16(V4 a, V4 b, f4 c) {
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s4, a), __builtin_bit_cast(s4, b), c,
+                                                     0, 0, 0);
+  }
 };
 
 template <bool REV>
 struct WFrags {
   using V8 = typename WStateT<REV>::V8;
-  V8 W[WKS];                      // Wneg rows of token block w & 1
+  V8 W[SRB];                      // Wneg's two token blocks against this wave's row blocks
   V8 K[SRB];                      // K^T rows of this wave's row blocks, the chunk's 32 tokens
   bf16x8 A[REV ? SRB : 1];        // At rows (reverse)
   unsigned ib;                    // reverse: this thread's two elements of the Ib tile
-  f4 U;                           // U tile (C-operand layout)
+  float2 U;                       // this thread's two elements of the U tile
   float4 G[SRB];                  // Gamma of this wave's rows 16 rb + 4 g .. + 3
 };
 
 // Chunk-uniform bases with 32-bit lane offsets throughout: 64-bit per-lane
-// addresses for the ~20 fragment loads of a chunk would not fit in registers
-// beside the prefetch ring.  Every load is unconditional (indices clamped into
+// addresses for a chunk's fragment loads would not fit in registers beside the
+// prefetch ring.  Every load is unconditional (indices clamped into
 // the panel; a null At replaced by a panel of the same shape): a memory
 // operation under a branch gives the two paths different counts of
 // operations in flight, and the compiler then waits for all of them (the
-// ring's prefetches included) wherever the paths meet.  Waves 4-7 fetch the
-// W and U fragments waves 0-3 use, for the same reason.
+// ring's prefetches included) wherever the paths meet.
 template <bool REV>
 __device__ __forceinline__ void wstate_load(const WStateParams& p, int s, int ch, int c0,
                                             WFrags<REV>& f) {
@@ -677,15 +699,12 @@ __device__ __forceinline__ void wstate_load(const WStateParams& p, int s, int ch
   const int kw = p.kw, vw = p.vw, nrb = kw / 16;
   const long long tb = (long long)s * p.Tp + (long long)ch * WBT;
   const long long cb = ((long long)s * p.NT + ch) * kw;  // chunk base of [kw][32] and [kw] panels
-  {
-    const int tbk = w & 1, hh = (w >> 1) & 1, nks = kw >> 5;
-    const E* Wc = static_cast<const E*>(p.Wneg) + tb * kw;
-    // fragment order: a K = 32 step of a 16-token block is 1 KiB, lane-contiguous
-    const unsigned wo = (unsigned)(tbk * nks * 512 + l * 8);
-#pragma unroll
-    for (int ks = 0; ks < WKS; ++ks)
-      f.W[ks] = *reinterpret_cast<const V8*>(Wc + wo + min(ks, nks - 1) * 512);
-    f.U = *reinterpret_cast<const f4*>(p.U + tb * vw + acc_off(tbk, (c0 >> 4) + hh, l, vw));
+  const E* Wc = static_cast<const E*>(p.Wneg) + tb * kw;
+  {  // thread t: elements 2 t, 2 t + 1 of the tiles in accumulator order
+    const int tile = threadIdx.x >> 7;
+    f.U = *reinterpret_cast<const float2*>(
+        p.U + tb * vw + acc_off(tile / NSUB, (c0 >> 4) + tile % NSUB, (threadIdx.x & 127) >> 1, vw) +
+        (threadIdx.x & 1) * 2);
   }
   const E* Kc = static_cast<const E*>(p.Kt) + cb * WBT;
   const float* Gc = p.Gam + cb;
@@ -693,6 +712,7 @@ __device__ __forceinline__ void wstate_load(const WStateParams& p, int s, int ch
   for (int q = 0; q < SRB; ++q) {
     const int rb = min(w + SW * q, nrb - 1);
     const unsigned ko = (unsigned)((rb * 16 + m) * WBT + kq);
+    f.W[q] = *reinterpret_cast<const V8*>(Wc + w_off(rb, l, 0));
     f.K[q] = *reinterpret_cast<const V8*>(Kc + ko);
     f.G[q] = *reinterpret_cast<const float4*>(Gc + (unsigned)(rb * 16 + 4 * g));
     if constexpr (REV) {
@@ -708,19 +728,20 @@ __device__ __forceinline__ void wstate_load(const WStateParams& p, int s, int ch
   }
 }
 
-// Four 16-bit values split from an FP32 accumulator fragment, stored as two
-// 8-byte pieces (high and low halves).
-template <class E, class V4>
-__device__ __forceinline__ void wsplit4(E* hi, E* lo, f4 v) {
-  V4 h, o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const E a = (E)v[e];
-    h[e] = a;
-    o[e] = (E)(v[e] - (float)a);
-  }
-  *reinterpret_cast<V4*>(hi) = h;
-  *reinterpret_cast<V4*>(lo) = o;
+// An accumulator fragment in 16 bits (lane (g, m): rows 4 g .. + 3 of column m)
+// turned into four neighbouring columns of one row: a 4 x 4 transpose within
+// each quad of lanes.  Lane m ends with row 4 g + quad_row(m), columns m & 12 .. + 3.
+__device__ __forceinline__ int quad_row(int m) { return ((m & 1) << 1) | ((m >> 1) & 1); }
+template <class V4>
+__device__ __forceinline__ uint2 quad_transpose(V4 v) {
+  const uint2 in = __builtin_bit_cast(uint2, v);  // rows 0, 1 and rows 2, 3 of this lane's column
+  const bool odd = threadIdx.x & 1, up = threadIdx.x & 2;
+  const unsigned got = __builtin_amdgcn_update_dpp(0, odd ? in.x : in.y, 0xB1, 0xF, 0xF, false);
+  const unsigned own = odd ? in.y : in.x;
+  const unsigned lo = odd ? got : own, hi = odd ? own : got;  // rows (0,1) or (2,3) of two columns
+  const unsigned ra = (lo & 0xffffu) | (hi << 16), rb = (lo >> 16) | (hi & 0xffff0000u);
+  const unsigned got2 = __builtin_amdgcn_update_dpp(0, up ? ra : rb, 0x4E, 0xF, 0xF, false);
+  return up ? make_uint2(got2, rb) : make_uint2(ra, got2);
 }
 
 template <bool REV>
@@ -734,27 +755,41 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15, kq = g * 8;
   const int kw = p.kw, vw = p.vw, nrb = kw / 16;
   const long long tb = (long long)s * p.Tp + (long long)ch * WBT;
-  E* Xh = reinterpret_cast<E*>(sm);  // X0 [32 columns][XLD], high and low halves
-  E* Xl = Xh + STILE * XLD;
-  E* wh = Xl + STILE * XLD;          // w [32 columns][WLD]
+  float* part = reinterpret_cast<float*>(sm);  // partial w [wave][tile][lane][4]
+  E* wh = reinterpret_cast<E*>(part + SW * NTILE * 256);  // w [32 columns][WLD], high and low halves
   E* wl = wh + STILE * WLD;
   E* ih = wl + STILE * WLD;          // reverse: the injection's Ib tile [32 columns][WLD]
-  E* Xr = ih + STILE * WLD;          // X0 row-major [rows][XRS]: the slot, written back below
-  float* wf = reinterpret_cast<float*>(Xr + WMAX * XRS);  // w FP32 [32 columns][WFS]
-  static_assert(std::is_same<S, E>::value, "the slot holds the staged high half");
-  // X0 staged split and transposed for the w product, and row-major for the slot
+  static_assert(std::is_same<S, E>::value, "the slot holds the high half");
+  // this wave's partial w and its rows of slot[ch]
+  f4 pw[NTILE];
+#pragma unroll
+  for (int t = 0; t < NTILE; ++t) pw[t] = zero4();
+  S* slot = static_cast<S*>(p.slots) + ((long long)s * (p.NT + 1) + ch) * kw * vw + c0 * kw;
 #pragma unroll
   for (int q = 0; q < SRB; ++q) {
     const int rb = w + SW * q;
     if (rb >= nrb) continue;
+    const V4 w0 = __builtin_shufflevector(f.W[q], f.W[q], 0, 1, 2, 3);
+    const V4 w1 = __builtin_shufflevector(f.W[q], f.W[q], 4, 5, 6, 7);
 #pragma unroll
     for (int h = 0; h < NSUB; ++h) {
-      const int col = h * 16 + m, row = rb * 16 + 4 * g;
-      wsplit4<E, V4>(Xh + col * XLD + row, Xl + col * XLD + row, X[q][h]);
+      V4 xh, xl;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) Xr[(row + e) * XRS + col] = (E)X[q][h][e];
+      for (int e = 0; e < 4; ++e) {
+        const E a = (E)X[q][h][e];
+        xh[e] = a;
+        xl[e] = (E)(X[q][h][e] - (float)a);
+      }
+      pw[h] = T::mma16(w0, xl, pw[h]);
+      pw[NSUB + h] = T::mma16(w1, xl, pw[NSUB + h]);
+      pw[h] = T::mma16(w0, xh, pw[h]);
+      pw[NSUB + h] = T::mma16(w1, xh, pw[NSUB + h]);
+      *reinterpret_cast<uint2*>(slot + (unsigned)((rb * 16 + 4 * g + quad_row(m)) * STILE + h * 16 + (m & 12))) =
+          quad_transpose(xh);
     }
   }
+#pragma unroll
+  for (int t = 0; t < NTILE; ++t) *reinterpret_cast<f4*>(part + ((w * NTILE + t) * 64 + l) * 4) = pw[t];
   if constexpr (REV) {
     if (p.At) {  // the Ib tile (exact in bf16) staged transposed ([column][token])
       const int tok = threadIdx.x / (STILE / 2), col = (threadIdx.x % (STILE / 2)) * 2;
@@ -763,39 +798,31 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
     }
   }
   __syncthreads();
-  {  // slot[ch] = X0: 16 columns of one row per thread, two 16-byte pieces
-    static_assert(WMAX * 2 == ST && STILE == 32, "one half row of the slot tile per thread");
-    // (rows past kw repeat row kw - 1: same values, and no store under a branch)
-    const int row = min(threadIdx.x >> 1, kw - 1), c = (threadIdx.x & 1) * 16;
-    typedef E E8 __attribute__((ext_vector_type(8)));
-    const E8 v0 = *reinterpret_cast<const E8*>(Xr + row * XRS + c);
-    const E8 v1 = *reinterpret_cast<const E8*>(Xr + row * XRS + c + 8);
-    S* dst = static_cast<S*>(p.slots) + ((long long)s * (p.NT + 1) + ch) * kw * vw + c0 +
-             (unsigned)(row * vw + c);
-    *reinterpret_cast<E8*>(dst) = v0;
-    *reinterpret_cast<E8*>(dst + 8) = v1;
-  }
-  // w = U + Wneg X0 (waves 0-3, one 16 x 16 tile each; high and low halves of
-  // X0 in two accumulators so the two dependent chains interleave)
-  if (w < 4) {
-    const int tbk = w & 1, hh = w >> 1;
-    f4 a0 = f.U, a1 = zero4();
-    const E* bh = Xh + (hh * 16 + m) * XLD + kq;
-    const E* bl = Xl + (hh * 16 + m) * XLD + kq;
+  {  // w: two elements (neighbouring tokens of one column) per thread
+    static_assert(NTILE * 256 == 2 * ST, "two w elements per thread");
+    float2 v = f.U;
 #pragma unroll
-    for (int ks = 0; ks < WKS; ++ks)
-      if (ks * 32 < kw) {
-        a1 = T::mma(f.W[ks], *reinterpret_cast<const V8*>(bl + ks * 32), a1);
-        a0 = T::mma(f.W[ks], *reinterpret_cast<const V8*>(bh + ks * 32), a0);
-      }
-    f4 wv;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) wv[e] = a0[e] + a1[e];
-    const int col = hh * 16 + m, tok = tbk * 16 + 4 * g;
-    wsplit4<E, V4>(wh + col * WLD + tok, wl + col * WLD + tok, wv);
-    *reinterpret_cast<f4*>(wf + col * WFS + tok) = wv;
+    for (int k = 0; k < SW; ++k) {
+      const float2 a = *reinterpret_cast<const float2*>(part + k * NTILE * 256 + threadIdx.x * 2);
+      v.x += a.x;
+      v.y += a.y;
+    }
+    const int tile = threadIdx.x >> 7, wl_ = (threadIdx.x & 127) >> 1;
+    const int col = (tile % NSUB) * 16 + (wl_ & 15);
+    const int tok = (tile / NSUB) * 16 + (wl_ >> 4) * 4 + (threadIdx.x & 1) * 2;
+    typedef E E2 __attribute__((ext_vector_type(2)));
+    E2 hi, lo;
+    hi[0] = (E)v.x;
+    hi[1] = (E)v.y;
+    lo[0] = (E)(v.x - (float)hi[0]);
+    lo[1] = (E)(v.y - (float)hi[1]);
+    *reinterpret_cast<E2*>(wh + col * WLD + tok) = hi;
+    *reinterpret_cast<E2*>(wl + col * WLD + tok) = lo;
+    float* wo = p.wout + tb * vw + c0;
+    wo[(unsigned)(tok * vw + col)] = v.x;
+    wo[(unsigned)((tok + 1) * vw + col)] = v.y;
   }
-  // X = Gamma X (+ At^T Ib): independent of w, so it overlaps the w tiles
+  // X = Gamma X (+ At^T Ib): independent of w
 #pragma unroll
   for (int q = 0; q < SRB; ++q) {
     const int rb = w + SW * q;
@@ -814,12 +841,6 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
     }
   }
   __syncthreads();
-  {  // w to global memory, two elements per thread
-    static_assert(WBT * STILE == 2 * ST, "two w elements per thread");
-    const int tok = threadIdx.x / (STILE / 2), col = (threadIdx.x % (STILE / 2)) * 2;
-    const float2 v = make_float2(wf[col * WFS + tok], wf[(col + 1) * WFS + tok]);
-    *reinterpret_cast<float2*>(p.wout + tb * vw + c0 + (unsigned)(tok * vw + col)) = v;
-  }
   // X += K^T w
 #pragma unroll
   for (int h = 0; h < NSUB; ++h) {
@@ -890,7 +911,7 @@ __global__ __launch_bounds__(ST) void k_w_state(WStateParams p) {
       for (int e = 0; e < 4; ++e) {
         const int row = rb * 16 + 4 * g + e, col = c0 + h * 16 + m;
         if (!REV)
-          static_cast<S*>(p.slots)[((long long)s * (p.NT + 1) + p.NT) * kw * p.vw + (long long)row * p.vw + col] =
+          static_cast<S*>(p.slots)[((long long)s * (p.NT + 1) + p.NT) * kw * p.vw + slot_off(row, col, kw)] =
               (S)X[q][h][e];
         if (p.fin && row < p.rows && col < p.cols) {
           if (p.fin_t) p.fin[((long long)s * p.cols + col) * p.rows + row] = X[q][h][e];
@@ -951,7 +972,7 @@ __global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
         const int task = threadIdx.x + WT * q, c = task % vw, rg = task / vw;
         if (task < vw * 4)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) xr[q][j] = X0[(long long)(rb + rg * 8 + j) * vw + c];
+          for (int j = 0; j < 8; ++j) xr[q][j] = X0[slot_off(rb + rg * 8 + j, c, kw)];
       }
     };
     fetch(0);
@@ -1111,7 +1132,7 @@ __global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
     f4 acc[2] = {zero4(), zero4()};
 #pragma unroll 4
     for (int cb = 0; cb < vw; cb += 32) {
-      const f16x8 bx = *reinterpret_cast<const f16x8*>(X0 + (long long)rr * vw + cb + kq);
+      const f16x8 bx = *reinterpret_cast<const f16x8*>(X0 + slot_off(rr, cb + kq, kw));
 #pragma unroll
       for (int t2 = 0; t2 < 2; ++t2) {
         const f16x8 ah = *reinterpret_cast<const f16x8*>(Qh + (t2 * 16 + m) * QLD + cb + kq);
@@ -1258,7 +1279,7 @@ struct BprepParams {
   const __bf16 *dOb, *ub, *kb;  // column output: dO; row output: u, k (k = u^, x = gx u^, q = k^)
   const Tok* tok;
   float *dU, *Pp;  // dU [Tp][vw] in accumulator order (acc_off)
-  __bf16 *Wneg, *Kt, *At;  // reverse-pass panels: -Wn [Tp][kw] (fragment order); Kn, Ia transposed per chunk [NT][kw][32]
+  __bf16 *Wneg, *Kt, *At;  // reverse-pass panels: -Wn (w_off order); Kn, Ia transposed per chunk [NT][kw][32]
 };
 
 // Same organisation as k_w_prep: a lane's four coordinates of a token are loaded
@@ -1446,14 +1467,12 @@ __global__ __launch_bounds__(PT, 4) void k_w_bprep(BprepParams p) {
 #pragma unroll
         for (int t2 = 0; t2 <= kb; ++t2) aw[t2] = mfma4(kv, Al[k * AS + t2 * 16 + m], aw[t2]);
       }
-    if (nb < nkb)
+    if (nb < nkb) {
+      bf16x8 h;
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
-        bf16x4 h;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = (__bf16)aw[t2][e];
-        *reinterpret_cast<bf16x4*>(p.Wneg + tb * kw + frag_off(t2 * 16 + m, nb * 16 + 4 * g, kw)) = h;
-      }
+      for (int e = 0; e < 8; ++e) h[e] = (__bf16)aw[e >> 2][e & 3];
+      *reinterpret_cast<bf16x8*>(p.Wneg + tb * kw + w_off(nb, l, 0)) = h;
+    }
   }
   store_transposed(p.Kt + cbase * kw * WBT, kn, kw);
   store_transposed(p.At + cbase * kw * WBT, ia, kw);
@@ -1642,15 +1661,15 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   {
     unsigned ro[GRB];  // row offsets of this wave's blocks (clamped: loads stay unconditional)
 #pragma unroll
-    for (int q = 0; q < GRB; ++q) ro[q] = (unsigned)((min(w + GW * q, nrb - 1) * 16 + m) * vw + kq);
+    for (int q = 0; q < GRB; ++q) ro[q] = slot_off(min(w + GW * q, nrb - 1) * 16 + m, kq, kw);
     f16x8 x8[2][GRB], c8[2][GRB];
     bf16x8 l8[2][GRB];
     auto fetch = [&](int cb, int f) {
 #pragma unroll
       for (int q = 0; q < GRB; ++q) {
-        x8[f][q] = *reinterpret_cast<const f16x8*>(X0 + cb + ro[q]);
-        l8[f][q] = *reinterpret_cast<const bf16x8*>(Lm + cb + ro[q]);
-        c8[f][q] = *reinterpret_cast<const f16x8*>(XC + cb + ro[q]);
+        x8[f][q] = *reinterpret_cast<const f16x8*>(X0 + cb * kw + ro[q]);
+        l8[f][q] = *reinterpret_cast<const bf16x8*>(Lm + cb * kw + ro[q]);
+        c8[f][q] = *reinterpret_cast<const f16x8*>(XC + cb * kw + ro[q]);
       }
     };
     auto step = [&](int cb, int f) {
@@ -1757,14 +1776,15 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
 #pragma unroll
       for (int q = 0; q < XQ; ++q) {
         const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 8 - 1);
-        xb[q] = *reinterpret_cast<const f16x8*>(X0 + (long long)rb * vw + idx * 8);
+        // piece idx: column tile idx / 128, row (idx / 4) % 32, columns 8 (idx % 4) .. + 7
+        xb[q] = *reinterpret_cast<const f16x8*>(X0 + slot_off(rb + (idx >> 2) % 32, (idx >> 7) * STILE + (idx & 3) * 8, kw));
       }
     };
     auto put = [&](int f) {
 #pragma unroll
       for (int q = 0; q < XQ; ++q) {
         const int idx = min((int)(threadIdx.x + GT * q), WBT * vw / 8 - 1);
-        *reinterpret_cast<f16x8*>(Xt + f * RP + (idx * 8) / vw * KHS + (idx * 8) % vw) = xb[q];
+        *reinterpret_cast<f16x8*>(Xt + f * RP + (idx >> 2) % 32 * KHS + (idx >> 7) * STILE + (idx & 3) * 8) = xb[q];
       }
     };
     fetch(0);
