@@ -15,7 +15,7 @@
 //     k_w_prep    decayed Gram L, (I+L)^-1, WY panels W, U, decayed keys,
 //                 readout pair P (column output);
 //     k_w_state   sequential chunk pass over one 32-column state tile;
-//     k_w_out     chunk readout (row output also forms d = k^ + C^T k^);
+//     k_w_out_c, k_w_out_s  chunk readouts (the predictor's forms d = k^ + C^T k^);
 //   k_w_sources (per token)  dual sources e, chi and gated values z;
 // and backward, per op in reverse order:
 //     k_w_bprep   dU = A^T (dW + pair^T dO), W' = -A^T K^, K' = -x~, injection;
@@ -38,23 +38,12 @@ namespace wide {
 constexpr int WBT = 32;    // chunk length
 constexpr int WMAX = 256;  // widest padded width
 constexpr int WT = 256;    // threads per workgroup
-constexpr int MS = WBT + 1;  // row stride of 32 x 32 LDS matrices
 
 // Chunk-boundary state slots in a 2-byte type, as in the main kernels: the
 // forward states X (C^T and S) in fp16, the reverse passes' cotangent states
 // lambda in bf16.  The final states handed to the caller stay FP32.
 using xs_t = xslot_t;
 using ls_t = lslot_t;
-__device__ __forceinline__ float4 ld4s(const _Float16* p) {
-  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  const h4 v = *reinterpret_cast<const h4*>(p);
-  return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
-}
-__device__ __forceinline__ float4 ld4s(const __bf16* p) {
-  typedef __bf16 b4 __attribute__((ext_vector_type(4)));
-  const b4 v = *reinterpret_cast<const b4*>(p);
-  return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
-}
 
 // Workgroup ids are dealt round-robin over the 8 XCDs (each with its own L2).
 // Maps a linear id over (inner, outer) = (L % inner, L / inner) so that, when the
@@ -228,7 +217,7 @@ __device__ __forceinline__ unsigned w_off(int rb, int lane, int tb) {
 // A state slot [kw][vw] is kept in 32-column tiles, [vw / 32][kw][32]: a state
 // workgroup writes whole lines of its own tile, and a 16-row operand fragment
 // of 32 columns is 1 KiB contiguous.  Row-major slots held the state passes to
-// the rate of their half-line stores: SLOT_US
+// the rate of their half-line stores (forward 187 us, in tiles 165).
 constexpr int STILE = 32;  // state columns per workgroup
 __device__ __forceinline__ unsigned slot_off(int row, int col, int kw) {
   return (unsigned)(((col / STILE) * kw + row) * STILE + col % STILE);
@@ -623,7 +612,9 @@ struct WStateParams {
 //   own rows.
 // The state itself never passes through LDS (the form that staged it there for
 // four waves to read moved 170 KB of LDS and 64 KB of Wneg per step against 90
-// and 16): STATE_US
+// and 16): forward passes 159 us, reverse 190 at B4 T2048 H8 r = V = 256 (196 and
+// 227 before), 59 us forward at 12 sequences of 1333 tokens, r = 192 (80 before).
+// What is left is the slot store: a build without it runs the forward pass in 94 us.
 // The panels Wneg, K^T and At are stored 16-bit by the prep kernels in the
 // order the MFMA operands read them, so each lane's fragment is one 16-byte
 // load; they, U, Gamma and Ib are fetched SPF - 1 chunks ahead into a ring of
@@ -634,7 +625,6 @@ struct WStateParams {
 // into bf16 halves (Ib, a bf16 input, enters as it is).  Two barriers per step:
 // the partials are read between them and written again only before the next
 // step's first; the split w is written between them and read before that.
-constexpr int WRB = WMAX / 16 / 4;   // row blocks per wave (four-wave kernels)
 constexpr int SW = 8;                // state-pass waves: two per SIMD
 constexpr int ST = SW * 64;
 constexpr int SRB = WMAX / 16 / SW;  // state-pass row blocks per wave
@@ -744,7 +734,9 @@ __device__ __forceinline__ uint2 quad_transpose(V4 v) {
   return up ? make_uint2(got2, rb) : make_uint2(ra, got2);
 }
 
-template <bool REV>
+// FULL: kw = WMAX, every wave has all of its row blocks (a memory operation
+// under a branch would make the compiler wait for more than it needs).
+template <bool REV, bool FULL>
 __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch, int c0,
                                             const WFrags<REV>& f, f4 (&X)[SRB][NSUB], unsigned char* sm) {
   using T = WStateT<REV>;
@@ -768,7 +760,7 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
 #pragma unroll
   for (int q = 0; q < SRB; ++q) {
     const int rb = w + SW * q;
-    if (rb >= nrb) continue;
+    if (!FULL && rb >= nrb) continue;
     const V4 w0 = __builtin_shufflevector(f.W[q], f.W[q], 0, 1, 2, 3);
     const V4 w1 = __builtin_shufflevector(f.W[q], f.W[q], 4, 5, 6, 7);
 #pragma unroll
@@ -826,7 +818,7 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
 #pragma unroll
   for (int q = 0; q < SRB; ++q) {
     const int rb = w + SW * q;
-    if (rb >= nrb) continue;
+    if (!FULL && rb >= nrb) continue;
     const float gv[4] = {f.G[q].x, f.G[q].y, f.G[q].z, f.G[q].w};
 #pragma unroll
     for (int h = 0; h < NSUB; ++h) {
@@ -849,14 +841,14 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
 #pragma unroll
     for (int q = 0; q < SRB; ++q) {
       const int rb = w + SW * q;
-      if (rb >= nrb) continue;
+      if (!FULL && rb >= nrb) continue;
       X[q][h] = T::mma(f.K[q], wlv, X[q][h]);
       X[q][h] = T::mma(f.K[q], whv, X[q][h]);
     }
   }
 }
 
-template <bool REV>
+template <bool REV, bool FULL>
 __global__ __launch_bounds__(ST) void k_w_state(WStateParams p) {
   extern __shared__ __align__(16) unsigned char wsm[];
   int tile, s;
@@ -893,18 +885,19 @@ __global__ __launch_bounds__(ST) void k_w_state(WStateParams p) {
 #pragma unroll
     for (int j = 0; j < SPF; ++j) {
       wstate_load<REV>(p, s, clampc(it + j + SPF - 1), c0, f[(j + SPF - 1) % SPF]);
-      wstate_step<REV>(p, s, chunk_of(it + j), c0, f[j], X, wsm);
+      __builtin_amdgcn_sched_barrier(0);
+      wstate_step<REV, FULL>(p, s, chunk_of(it + j), c0, f[j], X, wsm);
     }
   }
 #pragma unroll
   for (int j = 0; j < SPF - 1; ++j)
-    if (it + j < NT) wstate_step<REV>(p, s, chunk_of(it + j), c0, f[j], X, wsm);
+    if (it + j < NT) wstate_step<REV, FULL>(p, s, chunk_of(it + j), c0, f[j], X, wsm);
   // final state (forward: also slot NT for the backward)
   using S = typename std::conditional<REV, ls_t, xs_t>::type;
 #pragma unroll
   for (int q = 0; q < SRB; ++q) {
     const int rb = w + SW * q;
-    if (rb >= nrb) continue;
+    if (!FULL && rb >= nrb) continue;
 #pragma unroll
     for (int h = 0; h < NSUB; ++h)
 #pragma unroll
@@ -921,277 +914,311 @@ __global__ __launch_bounds__(ST) void k_w_state(WStateParams p) {
   }
 }
 
+// Four elements of an output row at column c of r (a padded column is dropped).
+__device__ __forceinline__ void store_row4(__bf16* row, int c, int r, int vec, bf16x4 h) {
+  if (vec) {
+    if (c < r) *reinterpret_cast<bf16x4*>(row + c) = h;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < r) row[c + e] = h[e];
+  }
+}
+__device__ __forceinline__ void store_row4(__bf16* row, int c, int r, int vec, const Quad& q) {
+  bf16x4 h;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) h[e] = f2bf(q.v[e]);
+  store_row4(row, c, r, vec, h);
+}
+__device__ __forceinline__ void store_row4(float* row, int c, int r, int vec, const Quad& q) {
+  if (vec) {
+    if (c < r) *reinterpret_cast<Quad*>(row + c) = q;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < r) row[c + e] = q.v[e];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Chunk readouts, transposed like the other chunk kernels' products (a lane
+// holds four neighbouring coordinates of one token), two workgroups per CU.
+// What bounds them: the state slot (128 KiB of a chunk's 208 (S) / 256 (C) KiB
+// at r = V = 256).
+// ---------------------------------------------------------------------------
 struct OutParams {
-  int NT, Tp, kw, vw, colout, H, T, V;
+  int NT, Tp, kw, vw;
   const xs_t* slots;
-  const float *w, *Qt, *P, *G;
-  const __bf16 *ub, *kb;  // row output: q = base = k^, k = u^
+  const float *w, *G;           // w [Tp][vw]
+  const float *Qt, *P;          // column output
+  int H, T, V, vec;
+  __bf16* out;
+  const __bf16 *ub, *kb;        // row output: q = base = k^, k = u^
   const Tok* tok;
   float *o, *d;
-  __bf16* out;
 };
 
-__global__ __launch_bounds__(WT) void k_w_out(OutParams p) {
+constexpr int GS16 = 20;  // row stride (FP32) of a wave's staged [32 tokens][16 coordinates] panel
+
+// Four values split into fp16 halves.
+__device__ __forceinline__ void split4_h(_Float16* hi, _Float16* lo, const Quad& q) {
+  f16x4 h, o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    h[e] = (_Float16)q.v[e];
+    o[e] = (_Float16)(q.v[e] - (float)h[e]);
+  }
+  *reinterpret_cast<f16x4*>(hi) = h;
+  *reinterpret_cast<f16x4*>(lo) = o;
+}
+__device__ __forceinline__ f4 mma_h(f16x8 a, f16x8 b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// Column output o = Q~ X0 + P w.  Q~ X0 on fp16 matrix cores (Q~ split into high
+// and low halves in LDS, X0 exact in its slot): the contraction runs along the
+// slot's rows, so 32-row blocks pass through LDS (double buffered, one barrier
+// each) and are read down their columns.  P w in FP32.  Wave w owns the
+// 16-column blocks w, w + 8.  91 us (4.8 TB/s) at B4 T2048 H8
+// r = V = 256, where four waves with one workgroup per CU took 155 us.
+__global__ __launch_bounds__(PT, 4) void k_w_out_s(OutParams p) {
   extern __shared__ __align__(16) float sm[];
-  const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, vw = p.vw;
+  const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, vw = p.vw, nvb = vw / 16;
   const long long tb = (long long)s * p.Tp + ch * WBT;
   const xs_t* X0 = p.slots + ((long long)s * (p.NT + 1) + ch) * kw * vw;
-  if (p.colout) {
-    // Column output on matrix cores: o = Q~ X0 + P w.
-    //   Q~ X0 on v_mfma_f32_16x16x32_f16: Q~ (|Q~| <= 1) split into fp16 high and
-    //   low halves, X0 exact in its fp16 slot; the slot is row-major, so each
-    //   32-row block is staged transposed ([column][row]) through LDS, the
-    //   next block's loads in flight while the current one is used;
-    //   P w (32 tokens) on v_mfma_f32_16x16x4f32 from FP32 P and w.
-    // Wave w owns output tiles (token block t2, column block w + 4 j).
-    using h8 = f16x8;
-    constexpr int QLD = WMAX + 8, XTL = WBT + 8, PLD = WBT + 4, NJ = WMAX / 16 / 4;
-    _Float16* Qh = reinterpret_cast<_Float16*>(sm);  // Q~ high / low [32][QLD]
-    _Float16* Qo = Qh + WBT * QLD;
-    _Float16* Xt = Qo + WBT * QLD;                   // X0 row block, transposed [vw][XTL]
-    float* Pl = reinterpret_cast<float*>(Xt + WMAX * XTL);  // P [32][PLD]
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15, kq = g * 8;
-    const int nvb = vw / 16;
-    // this lane's w values for the P w product: B[k = 4 g + e][n = m] of token block kb
-    float wb[NJ][2][4];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int nb = w + 4 * j;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          wb[j][kb][e] = nb < nvb ? p.w[(tb + kb * 16 + 4 * g + e) * vw + nb * 16 + m] : 0.f;
-    }
-    // X0 row-block staging: task (column c, 8-row group rg), 8 rows of one column
-    constexpr int XQ = WMAX * 4 / WT;  // tasks per thread at vw = 256
-    h8 xr[XQ];
-    auto fetch = [&](int rb) {
-#pragma unroll
-      for (int q = 0; q < XQ; ++q) {
-        const int task = threadIdx.x + WT * q, c = task % vw, rg = task / vw;
-        if (task < vw * 4)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) xr[q][j] = X0[slot_off(rb + rg * 8 + j, c, kw)];
-      }
-    };
-    fetch(0);
-    // Q~ split into LDS; P into LDS
-    {
-      const long long mb = ((long long)s * p.NT + ch) * WBT * WBT;
-      for (int idx = threadIdx.x; idx < WBT * WBT; idx += WT) Pl[(idx >> 5) * PLD + (idx & 31)] = p.P[mb + idx];
-      constexpr int PQ = WBT * WMAX / 4 / WT;
-      float4 qv[PQ];
-#pragma unroll
-      for (int q = 0; q < PQ; ++q) {
-        const int idx = threadIdx.x + WT * q, i = (idx * 4) / kw, c = (idx * 4) % kw;
-        if (idx < WBT * kw / 4) qv[q] = *reinterpret_cast<const float4*>(p.Qt + (tb + i) * kw + c);
-      }
-#pragma unroll
-      for (int q = 0; q < PQ; ++q) {
-        const int idx = threadIdx.x + WT * q, i = (idx * 4) / kw, c = (idx * 4) % kw;
-        if (idx < WBT * kw / 4) {
-          f4 v = {qv[q].x, qv[q].y, qv[q].z, qv[q].w};
-          f16x4 hi, lo;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            hi[e] = (_Float16)v[e];
-            lo[e] = (_Float16)(v[e] - (float)hi[e]);
-          }
-          *reinterpret_cast<f16x4*>(Qh + i * QLD + c) = hi;
-          *reinterpret_cast<f16x4*>(Qo + i * QLD + c) = lo;
-        }
-      }
-    }
-    f4 acc[2][NJ];
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[t2][j] = zero4();
-    for (int rb = 0; rb < kw; rb += 32) {
-      __syncthreads();  // the previous block's readers are done
-#pragma unroll
-      for (int q = 0; q < XQ; ++q) {
-        const int task = threadIdx.x + WT * q, c = task % vw, rg = task / vw;
-        if (task < vw * 4) *reinterpret_cast<h8*>(Xt + c * XTL + rg * 8) = xr[q];
-      }
-      __syncthreads();
-      if (rb + 32 < kw) fetch(rb + 32);
-      h8 ah[2], al[2];
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
-        ah[t2] = *reinterpret_cast<const h8*>(Qh + (t2 * 16 + m) * QLD + rb + kq);
-        al[t2] = *reinterpret_cast<const h8*>(Qo + (t2 * 16 + m) * QLD + rb + kq);
-      }
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int nb = w + 4 * j;
-        if (nb >= nvb) continue;
-        const h8 bx = *reinterpret_cast<const h8*>(Xt + (nb * 16 + m) * XTL + kq);
-#pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
-          acc[t2][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t2], bx, acc[t2][j], 0, 0, 0);
-          acc[t2][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t2], bx, acc[t2][j], 0, 0, 0);
-        }
-      }
-    }
-    // + P w, then the bf16 output
-    const int b = s / p.H, h = s % p.H;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int nb = w + 4 * j;
-      if (nb >= nvb) continue;
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-          const float4 a4 = *reinterpret_cast<const float4*>(Pl + (t2 * 16 + m) * PLD + kb * 16 + 4 * g);
-          acc[t2][j] = mfma4(a4.x, wb[j][kb][0], acc[t2][j]);
-          acc[t2][j] = mfma4(a4.y, wb[j][kb][1], acc[t2][j]);
-          acc[t2][j] = mfma4(a4.z, wb[j][kb][2], acc[t2][j]);
-          acc[t2][j] = mfma4(a4.w, wb[j][kb][3], acc[t2][j]);
-        }
-        const int c = nb * 16 + m;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int t = ch * WBT + t2 * 16 + 4 * g + e;
-          if (t < p.T && c < p.V) p.out[(((long long)b * p.T + t) * p.H + h) * p.V + c] = f2bf(acc[t2][j][e]);
-        }
-      }
-    }
-    return;
-  }
-  // row output on matrix cores: M = q w^T (j <= i), then
-  //   o_ir = e^{G_ir} ((q X0^T)_ir + (M k~)_ir),  k~_jr = k_jr e^{-G_jr}
-  // with the decay factored per state row r (wild rows: exact per-term sum).
-  // q X0^T runs on v_mfma_f32_16x16x32_f16: q (unit rows) split into fp16 high
-  // and low halves in LDS, X0 exact in its fp16 slot (the contraction runs
-  // along the slot's rows, so each lane's fragment is one 16-byte load).
-  constexpr int QLD = WMAX + 8;
-  float* Ml = sm;  // [32][33]
-  _Float16* Qh = reinterpret_cast<_Float16*>(Ml + WBT * MS);  // q high / low [32][QLD]
-  _Float16* Qo = Qh + WBT * QLD;
+  const float *Qc = p.Qt + tb * kw, *wc = p.w + tb * vw;
+  constexpr int RP = WBT * KHS;
+  _Float16* Qh = reinterpret_cast<_Float16*>(sm);  // Q~ high / low [32][KHS]
+  _Float16 *Ql = Qh + RP, *Xt = Ql + RP;           // X0 row blocks [2][32][KHS]
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15, kq = g * 8;
-  {
-    constexpr int PQ = WBT * WMAX / 4 / WT;
-    Quad qv[PQ];
+  constexpr int XQ = WBT * WMAX / 8 / PT, QQ = WBT * WMAX / 4 / PT;
+  f16x8 xb[XQ];
+  auto fetch = [&](int rb) {
 #pragma unroll
-    for (int q = 0; q < PQ; ++q) {
-      const int idx = threadIdx.x + WT * q, i = (idx * 4) / vw, c = (idx * 4) % vw;
-      if (idx < WBT * vw / 4) qv[q] = scaled(ldq(p.kb + (tb + i) * vw + c), p.tok[tb + i].rk);
+    for (int q = 0; q < XQ; ++q) {
+      // piece idx: column tile idx / 128, row (idx / 4) % 32, columns 8 (idx % 4) .. + 7
+      const int idx = min((int)(threadIdx.x + PT * q), WBT * vw / 8 - 1);
+      xb[q] = *reinterpret_cast<const f16x8*>(X0 + slot_off(rb + (idx >> 2) % 32, (idx >> 7) * STILE + (idx & 3) * 8, kw));
     }
+  };
+  auto put = [&](int f) {
 #pragma unroll
-    for (int q = 0; q < PQ; ++q) {
-      const int idx = threadIdx.x + WT * q, i = (idx * 4) / vw, c = (idx * 4) % vw;
-      if (idx < WBT * vw / 4) {
-        f4 v = {qv[q].v[0], qv[q].v[1], qv[q].v[2], qv[q].v[3]};
-        f16x4 hi, lo;
+    for (int q = 0; q < XQ; ++q) {
+      const int idx = min((int)(threadIdx.x + PT * q), WBT * vw / 8 - 1);
+      *reinterpret_cast<f16x8*>(Xt + f * RP + (idx >> 2) % 32 * KHS + (idx >> 7) * STILE + (idx & 3) * 8) = xb[q];
+    }
+  };
+  fetch(0);
+  {
+    Quad qv[QQ];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          hi[e] = (_Float16)v[e];
-          lo[e] = (_Float16)(v[e] - (float)hi[e]);
-        }
-        *reinterpret_cast<f16x4*>(Qh + i * QLD + c) = hi;
-        *reinterpret_cast<f16x4*>(Qo + i * QLD + c) = lo;
-      }
+    for (int q = 0; q < QQ; ++q) qv[q] = ldq(Qc + (unsigned)(min((int)(threadIdx.x + PT * q), WBT * kw / 4 - 1) * 4));
+#pragma unroll
+    for (int q = 0; q < QQ; ++q) {
+      const int idx = min((int)(threadIdx.x + PT * q), WBT * kw / 4 - 1) * 4, o = idx / kw * KHS + idx % kw;
+      split4_h(Qh + o, Ql + o, qv[q]);
     }
   }
-  {
-    const int bi = w >> 1, bj = w & 1;
-    f4 acc = zero4();
-    const float rk = p.tok[tb + bi * 16 + m].rk;
-    for (int cb = 0; cb < vw; cb += 16) {
-      const Quad a4 = scaled(ldq(p.kb + (tb + bi * 16 + m) * vw + cb + 4 * g), rk);
-      const Quad b4 = ldq(p.w + (tb + bj * 16 + m) * vw + cb + 4 * g);
+  // P's rows and this lane's w values for P w, whose loads overlap the products
+  float wv[PNB][2][4];
+  int nb[PNB];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = mfma4(a4.v[e], b4.v[e], acc);
-    }
+  for (int q = 0; q < PNB; ++q) {
+    nb[q] = min(w + PW * q, nvb - 1) * 16;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int i = bi * 16 + 4 * g + e, j = bj * 16 + m;
-      Ml[i * MS + j] = j <= i ? acc[e] : 0.f;
-    }
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wv[q][kb][e] = wc[(unsigned)((kb * 16 + 4 * g + e) * vw + nb[q] + m)];
   }
+  Quad pp[2][2];
+#pragma unroll
+  for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+    for (int kb = 0; kb <= t2; ++kb)
+      pp[t2][kb] = ldq(p.P + ((long long)s * p.NT + ch) * WBT * WBT + (t2 * 16 + m) * WBT + kb * 16 + 4 * g);
+  put(0);
   __syncthreads();
-  const int nrb = kw / 16;
-  float ro[WRB][2][4], rbase[WRB][2][4];
-  float tru[2][4], trk[2][4];
+  f4 acc[PNB][2];
 #pragma unroll
-  for (int jb = 0; jb < 2; ++jb)
+  for (int q = 0; q < PNB; ++q) acc[q][0] = acc[q][1] = zero4();
+  for (int rb = 0; rb < kw; rb += 32) {
+    const int f = (rb >> 5) & 1;
+    if (rb + 32 < kw) fetch(rb + 32);
+    f16x8 qh[2], ql[2];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      tru[jb][e] = p.tok[tb + jb * 16 + 4 * g + e].ru;
-      trk[jb][e] = p.tok[tb + jb * 16 + 4 * g + e].rk;
+    for (int t2 = 0; t2 < 2; ++t2) {
+      qh[t2] = *reinterpret_cast<const f16x8*>(Qh + (t2 * 16 + m) * KHS + rb + kq);
+      ql[t2] = *reinterpret_cast<const f16x8*>(Ql + (t2 * 16 + m) * KHS + rb + kq);
     }
 #pragma unroll
-  for (int q = 0; q < WRB; ++q) {
-    const int rb = w + 4 * q;
-    if (rb >= nrb) continue;
-    const int rr = rb * 16 + m;
-    const bool wild = -p.G[(tb + WBT - 1) * kw + rr] > WILD;
-    f4 acc[2] = {zero4(), zero4()};
-#pragma unroll 4
-    for (int cb = 0; cb < vw; cb += 32) {
-      const f16x8 bx = *reinterpret_cast<const f16x8*>(X0 + slot_off(rr, cb + kq, kw));
+    for (int q = 0; q < PNB; ++q) {
+      f16x8 xc;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) xc[j] = Xt[f * RP + (kq + j) * KHS + nb[q] + m];
 #pragma unroll
       for (int t2 = 0; t2 < 2; ++t2) {
-        const f16x8 ah = *reinterpret_cast<const f16x8*>(Qh + (t2 * 16 + m) * QLD + cb + kq);
-        const f16x8 al = *reinterpret_cast<const f16x8*>(Qo + (t2 * 16 + m) * QLD + cb + kq);
-        acc[t2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bx, acc[t2], 0, 0, 0);
-        acc[t2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bx, acc[t2], 0, 0, 0);
+        acc[q][t2] = mma_h(xc, ql[t2], acc[q][t2]);
+        acc[q][t2] = mma_h(xc, qh[t2], acc[q][t2]);
       }
     }
-    float kt[2][4];
+    if (rb + 32 < kw) put(f ^ 1);
+    __syncthreads();
+  }
+  const int b = s / p.H, h = s % p.H;
+#pragma unroll
+  for (int q = 0; q < PNB; ++q)
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+#pragma unroll
+      for (int kb = 0; kb <= t2; ++kb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[q][t2] = mfma4(wv[q][kb][e], pp[t2][kb].v[e], acc[q][t2]);
+      const int t = ch * WBT + t2 * 16 + m;
+      if (t < p.T && w + PW * q < nvb)
+        store_row4(p.out + (((long long)b * p.T + t) * p.H + h) * p.V, nb[q] + 4 * g, p.V, p.vec,
+                   Quad{{acc[q][t2][0], acc[q][t2][1], acc[q][t2][2], acc[q][t2][3]}});
+    }
+}
+
+// Row output: M = q w^T (j <= i), then
+//   o_ir = e^{G_ir} ((q X0^T)_ir + (M k~)_ir),  k~_jr = k_jr e^{-G_jr},  d = q + o
+// with the decay factored per state row r (wild rows: exact per-term sum).  M as
+// the prep's Grams, in FP32 over the waves; q X0^T on fp16 matrix cores (q, unit
+// rows, split into high and low halves in LDS; X0 exact in its slot).  Wave w
+// owns the 16-row blocks w, w + 8.  131 us (4.6 TB/s) at B4 T2048 H8 r = V = 256, where
+// four waves with 4-byte panel accesses took 208 us.
+__global__ __launch_bounds__(PT, 4) void k_w_out_c(OutParams p) {
+  extern __shared__ __align__(16) float sm[];
+  const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, nkb = kw / 16;
+  const long long tb = (long long)s * p.Tp + ch * WBT;
+  const xs_t* X0 = p.slots + ((long long)s * (p.NT + 1) + ch) * kw * kw;
+  const __bf16 *ubc = p.ub + tb * kw, *kbc = p.kb + tb * kw;
+  const float *Gc = p.G + tb * kw, *wc = p.w + tb * kw;
+  const Tok* tokc = p.tok + tb;
+  _Float16* Qh = reinterpret_cast<_Float16*>(sm);  // q high / low [32][KHS]
+  _Float16* Ql = Qh + WBT * KHS;
+  float* Ml = reinterpret_cast<float*>(Ql + WBT * KHS);  // M [32][AS]
+  float* part = Ml + WBT * AS;  // partial Ms; then per wave k~ [32][GS16]
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, m = l & 15, kq = g * 8;
+  float tru[2], trk[2];
+#pragma unroll
+  for (int t2 = 0; t2 < 2; ++t2) {
+    tru[t2] = tokc[t2 * 16 + m].ru;
+    trk[t2] = tokc[t2 * 16 + m].rk;
+  }
+  Quad kn[PNB][2], u[PNB][2], G[PNB][2], gl[PNB];
+  int c0[PNB];
+  f4 am[3] = {zero4(), zero4(), zero4()};
+#pragma unroll
+  for (int q = 0; q < PNB; ++q) {
+    c0[q] = min(w + PW * q, nkb - 1) * 16 + 4 * g;
+    Quad wv[2];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const unsigned o = (t2 * 16 + m) * kw + c0[q];
+      kn[q][t2] = scaled(ldq(kbc + o), trk[t2]);
+      wv[t2] = ldq(wc + o);
+      u[q][t2] = scaled(ldq(ubc + o), tru[t2]);
+      G[q][t2] = ldq(Gc + o);
+    }
+    gl[q] = ldq(Gc + (unsigned)((WBT - 1) * kw + c0[q]));
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const int o = (t2 * 16 + m) * KHS + c0[q];
+      split4_h(Qh + o, Ql + o, kn[q][t2]);
+    }
+    if (w + PW * q < nkb) gram3(kn[q], wv, am);
+  }
+  gram3_put(part, w, am);
+  __syncthreads();
+  if (threadIdx.x < 192) {
+    const int q = threadIdx.x >> 6;
+    const f4 v = gram3_sum<PW>(part, 0, q, l);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = (q > 0 ? 16 : 0) + 4 * g + e, j = (q > 1 ? 16 : 0) + m;
+      Ml[i * AS + j] = j <= i ? v[e] : 0.f;
+    }
+  }
+  f4 acc[PNB][2];
+#pragma unroll
+  for (int q = 0; q < PNB; ++q) acc[q][0] = acc[q][1] = zero4();
+  unsigned ro[PNB];
+#pragma unroll
+  for (int q = 0; q < PNB; ++q) ro[q] = slot_off(min(w + PW * q, nkb - 1) * 16 + m, kq, kw);
+#pragma unroll 4
+  for (int cb = 0; cb < kw; cb += 32) {
+    f16x8 x[PNB];
+#pragma unroll
+    for (int q = 0; q < PNB; ++q) x[q] = *reinterpret_cast<const f16x8*>(X0 + cb * kw + ro[q]);
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const f16x8 qh = *reinterpret_cast<const f16x8*>(Qh + (t2 * 16 + m) * KHS + cb + kq);
+      const f16x8 ql = *reinterpret_cast<const f16x8*>(Ql + (t2 * 16 + m) * KHS + cb + kq);
+#pragma unroll
+      for (int q = 0; q < PNB; ++q) {
+        acc[q][t2] = mma_h(x[q], ql, acc[q][t2]);
+        acc[q][t2] = mma_h(x[q], qh, acc[q][t2]);
+      }
+    }
+  }
+  __syncthreads();  // M complete, its partials dead
+  float* kt = part + w * WBT * GS16;
+#pragma unroll
+  for (int q = 0; q < PNB; ++q) {
+    if (w + PW * q >= nkb) continue;
+    bool wild[4], any = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      wild[e] = -gl[q].v[e] > WILD;
+      any |= wild[e];
+    }
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      Quad a;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a.v[e] = keep_exp(!wild[e], u[q][t2].v[e], -G[q][t2].v[e]);
+      *reinterpret_cast<Quad*>(kt + (t2 * 16 + m) * GS16 + 4 * g) = a;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own panel
 #pragma unroll
     for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const long long o = (tb + jb * 16 + 4 * g + e) * kw + rr;
-        kt[jb][e] = keep_exp(!wild, bf2f(p.ub[o]) * tru[jb][e], -p.G[o]);
+        const float kv = kt[(jb * 16 + 4 * g + e) * GS16 + m];
+#pragma unroll
+        for (int t2 = jb; t2 < 2; ++t2)
+          acc[q][t2] = mfma4(kv, Ml[(t2 * 16 + m) * AS + jb * 16 + 4 * g + e], acc[q][t2]);
       }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block overwrites it
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      f4 a = acc[t2];
+      Quad o, d;
 #pragma unroll
-      for (int jb = 0; jb < 2; ++jb)
+      for (int e = 0; e < 4; ++e) o.v[e] = __expf(G[q][t2].v[e]) * acc[q][t2][e];
+      if (__any(any)) {  // exact sums of the wild rows' in-chunk terms
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a = mfma4(Ml[(t2 * 16 + m) * MS + jb * 16 + 4 * g + e], kt[jb][e], a);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = t2 * 16 + 4 * g + e;
-        const long long o = (tb + i) * kw + rr;
-        const float gi = p.G[o];
-        float v = __expf(gi) * a[e];
-        if (wild)
+        for (int e = 0; e < 4; ++e) {
+          if (!wild[e]) continue;
+          const int i = t2 * 16 + m, c = c0[q] + e;
           for (int j = 0; j <= i; ++j)
-            v += Ml[i * MS + j] * (bf2f(p.ub[(tb + j) * kw + rr]) * p.tok[tb + j].ru) *
-                 __expf(gi - p.G[(tb + j) * kw + rr]);
-        ro[q][t2][e] = v;
-        rbase[q][t2][e] = bf2f(p.kb[o]) * trk[t2][e];
+            o.v[e] += Ml[i * AS + j] * (bf2f(ubc[j * kw + c]) * tokc[j].ru) * __expf(G[q][t2].v[e] - Gc[j * kw + c]);
+        }
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d.v[e] = kn[q][t2].v[e] + o.v[e];
+      const unsigned off = (t2 * 16 + m) * kw + c0[q];
+      *reinterpret_cast<Quad*>(p.o + tb * kw + off) = o;
+      *reinterpret_cast<Quad*>(p.d + tb * kw + off) = d;
     }
-  }
-  // stores after every row block's loads (a load issued after a store waits for it)
-#pragma unroll
-  for (int q = 0; q < WRB; ++q) {
-    const int rb = w + 4 * q;
-    if (rb >= nrb) continue;
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const long long o = (tb + t2 * 16 + 4 * g + e) * kw + rb * 16 + m;
-        p.o[o] = ro[q][t2][e];
-        p.d[o] = rbase[q][t2][e] + ro[q][t2][e];
-      }
   }
 }
 
-constexpr size_t out_smem(int kw, int vw, int colout) {
-  // column output: Q~ high / low [32][WMAX+8] and X0 block [WMAX][40] fp16, P [32][36]
-  if (colout) return (size_t)(2 * WBT * (WMAX + 8) + WMAX * (WBT + 8)) * 2 + WBT * (WBT + 4) * sizeof(float);
-  return (size_t)(WBT * MS) * sizeof(float) + (size_t)2 * WBT * (WMAX + 8) * 2;  // M; q high / low
+constexpr size_t out_s_smem() { return (size_t)4 * WBT * KHS * 2; }
+constexpr size_t out_c_smem() {
+  return (size_t)2 * WBT * KHS * 2 + (size_t)(WBT * AS + PW * 3 * 256) * sizeof(float);
 }
+static_assert(PW * 3 * 256 >= PW * WBT * GS16, "the waves' k~ panels fit the partial Ms' storage");
 
 // ---------------------------------------------------------------------------
 // Dual sources (per token): phi, den, e, chi.
@@ -1511,39 +1538,12 @@ struct GradParams {
   int vec;  // the gradients' rows take 4-element stores
 };
 
-// Four elements of a gradient row at column c of r (a padded column is dropped).
-__device__ __forceinline__ void store_row4(__bf16* row, int c, int r, int vec, bf16x4 h) {
-  if (vec) {
-    if (c < r) *reinterpret_cast<bf16x4*>(row + c) = h;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (c + e < r) row[c + e] = h[e];
-  }
-}
-__device__ __forceinline__ void store_row4(__bf16* row, int c, int r, int vec, const Quad& q) {
-  bf16x4 h;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) h[e] = f2bf(q.v[e]);
-  store_row4(row, c, r, vec, h);
-}
-__device__ __forceinline__ void store_row4(float* row, int c, int r, int vec, const Quad& q) {
-  if (vec) {
-    if (c < r) *reinterpret_cast<Quad*>(row + c) = q;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (c + e < r) row[c + e] = q.v[e];
-  }
-}
 
 // Eight waves (two per SIMD, so one wave's loads overlap another's matrix
 // work), each owning the 16-row blocks rb = wave + 8 q of the state.
 constexpr int GW = 8;
 constexpr int GT = GW * 64;
 constexpr int GRB = WMAX / 16 / GW;
-constexpr int GS16 = 20;  // row stride (FP32) of a wave's staged [32 tokens][16 coordinates] panel
-
 // Lane i of a 16-lane row takes lane i + N's value, 0 past the row's end.
 template <int N>
 __device__ __forceinline__ float row_next(float v) {
@@ -2350,8 +2350,8 @@ WideBwd carve_wide_bwd(void* base, const WideDims& d, size_t* total) {
 }
 
 constexpr size_t kMaxLds = 160 * 1024;  // LDS of one gfx950 CU
-static_assert(prep_smem() <= kMaxLds / 2 && state_smem() <= kMaxLds && out_smem(WMAX, WMAX, 0) <= kMaxLds &&
-                  out_smem(WMAX, WMAX, 1) <= kMaxLds && bprep_smem() <= kMaxLds / 2 &&
+static_assert(prep_smem() <= kMaxLds / 2 && state_smem() <= kMaxLds && out_s_smem() <= kMaxLds / 2 &&
+                  out_c_smem() <= kMaxLds / 2 && bprep_smem() <= kMaxLds / 2 &&
                   grad_smem() <= kMaxLds,
               "a wide kernel's LDS exceeds the CU");
 
@@ -2367,10 +2367,15 @@ void launch_wprep(const OpParams& op, int n, hipStream_t st) {
 
 void launch_wstate(const char* name, const WStateParams& sp, int n, hipStream_t st) {
   const dim3 grid(sp.vw / STILE * n), blk(ST);
-  if (sp.rev)
-    SD_LAUNCH(name, k_w_state<true>, grid, blk, state_smem(), st, sp);
+  const bool full = sp.kw == WMAX;
+  if (sp.rev && full)
+    SD_LAUNCH(name, (k_w_state<true, true>), grid, blk, state_smem(), st, sp);
+  else if (sp.rev)
+    SD_LAUNCH(name, (k_w_state<true, false>), grid, blk, state_smem(), st, sp);
+  else if (full)
+    SD_LAUNCH(name, (k_w_state<false, true>), grid, blk, state_smem(), st, sp);
   else
-    SD_LAUNCH(name, k_w_state<false>, grid, blk, state_smem(), st, sp);
+    SD_LAUNCH(name, (k_w_state<false, false>), grid, blk, state_smem(), st, sp);
 }
 
 }  // namespace
@@ -2408,11 +2413,11 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
   sc.init = in->C0; sc.init_t = 1; sc.fin = C_T; sc.fin_t = 1;
   launch_wstate("w_state_c_fwd", sc, d.n, st);
   OutParams orow{};
-  orow.NT = d.NT; orow.Tp = d.Tp; orow.kw = d.KP; orow.vw = d.KP; orow.colout = 0;
+  orow.NT = d.NT; orow.Tp = d.Tp; orow.kw = d.KP; orow.vw = d.KP;
   orow.slots = w.XC; orow.w = w.delta; orow.ub = w.ub; orow.kb = w.kb; orow.tok = w.tok;
   orow.G = w.G; orow.o = w.oC; orow.d = w.d;
-  SD_SMEM_ONCE(k_w_out, (int)(out_smem(WMAX, WMAX, 0) > out_smem(WMAX, WMAX, 1) ? out_smem(WMAX, WMAX, 0) : out_smem(WMAX, WMAX, 1)));
-  SD_LAUNCH("k_w_out_c", k_w_out, dim3(d.NT, d.n), dim3(WT), out_smem(d.KP, d.KP, 0), st, orow);
+  SD_SMEM_ONCE(k_w_out_c, (int)out_c_smem());
+  SD_LAUNCH("k_w_out_c", k_w_out_c, dim3(d.NT, d.n), dim3(PT), out_c_smem(), st, orow);
 
   SrcParams sp{};
   sp.in = *in; sp.Tp = d.Tp; sp.KP = d.KP; sp.VP = d.VP;
@@ -2433,10 +2438,12 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
   ss.init = in->S0; ss.init_t = 0; ss.fin = S_T; ss.fin_t = 0;
   launch_wstate("w_state_s_fwd", ss, d.n, st);
   OutParams ocol{};
-  ocol.NT = d.NT; ocol.Tp = d.Tp; ocol.kw = d.KP; ocol.vw = d.VP; ocol.colout = 1;
+  ocol.NT = d.NT; ocol.Tp = d.Tp; ocol.kw = d.KP; ocol.vw = d.VP;
   ocol.H = in->H; ocol.T = in->T; ocol.V = in->V;
   ocol.slots = w.XS; ocol.w = w.wS; ocol.Qt = w.Qt; ocol.P = w.PS; ocol.out = (__bf16*)out;
-  SD_LAUNCH("k_w_out_s", k_w_out, dim3(d.NT, d.n), dim3(WT), out_smem(d.KP, d.VP, 1), st, ocol);
+  ocol.vec = in->V % 4 == 0 && ((uintptr_t)out & 7) == 0;
+  SD_SMEM_ONCE(k_w_out_s, (int)out_s_smem());
+  SD_LAUNCH("k_w_out_s", k_w_out_s, dim3(d.NT, d.n), dim3(PT), out_s_smem(), st, ocol);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 
