@@ -955,7 +955,7 @@ struct OutParams {
   __bf16* out;
   const __bf16 *ub, *kb;        // row output: q = base = k^, k = u^
   const Tok* tok;
-  float *o, *d;
+  float* d;
 };
 
 constexpr int GS16 = 20;  // row stride (FP32) of a wave's staged [32 tokens][16 coordinates] panel
@@ -1085,7 +1085,7 @@ __global__ __launch_bounds__(PT, 4) void k_w_out_s(OutParams p) {
 // with the decay factored per state row r (wild rows: exact per-term sum).  M as
 // the prep's Grams, in FP32 over the waves; q X0^T on fp16 matrix cores (q, unit
 // rows, split into high and low halves in LDS; X0 exact in its slot).  Wave w
-// owns the 16-row blocks w, w + 8.  131 us (4.6 TB/s) at B4 T2048 H8 r = V = 256, where
+// owns the 16-row blocks w, w + 8.  117 us (4.6 TB/s) at B4 T2048 H8 r = V = 256, where
 // four waves with 4-byte panel accesses took 208 us.
 __global__ __launch_bounds__(PT, 4) void k_w_out_c(OutParams p) {
   extern __shared__ __align__(16) float sm[];
@@ -1193,7 +1193,7 @@ __global__ __launch_bounds__(PT, 4) void k_w_out_c(OutParams p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block overwrites it
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      Quad o, d;
+      Quad o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o.v[e] = __expf(G[q][t2].v[e]) * acc[q][t2][e];
       if (__any(any)) {  // exact sums of the wild rows' in-chunk terms
@@ -1206,10 +1206,8 @@ __global__ __launch_bounds__(PT, 4) void k_w_out_c(OutParams p) {
         }
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) d.v[e] = kn[q][t2].v[e] + o.v[e];
-      const unsigned off = (t2 * 16 + m) * kw + c0[q];
-      *reinterpret_cast<Quad*>(p.o + tb * kw + off) = o;
-      *reinterpret_cast<Quad*>(p.d + tb * kw + off) = d;
+      for (int e = 0; e < 4; ++e) o.v[e] += kn[q][t2].v[e];
+      *reinterpret_cast<Quad*>(p.d + tb * kw + (unsigned)((t2 * 16 + m) * kw + c0[q])) = o;
     }
   }
 }
@@ -1523,7 +1521,7 @@ constexpr size_t bprep_smem() {
 // ---------------------------------------------------------------------------
 struct GradParams {
   int NT, Tp, kw, vw;
-  const float *k, *x, *q, *G, *dO, *o, *w, *dw, *Pp;  // k, x, q: column output; dO, o, Pp: row output
+  const float *k, *x, *q, *G, *dO, *d, *w, *dw, *Pp;  // k, x, q: column output; dO, d (= q + o), Pp: row output
   const __bf16 *dOb, *ub, *kb;  // column output: dO; row output: u, k (k = u^, x = gx u^, q = k^)
   const Tok* tok;
   const xs_t* Xslots;
@@ -1617,7 +1615,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   const float *Yk = (COL ? p.q : p.dO) + tb * kw, *Gc = p.G + tb * kw;  // [32][kw]
   const float *dwc = p.dw + tb * vw, *wc = p.w + tb * vw;
   const float *kpc = COL ? p.k + tb * kw : nullptr, *xpc = COL ? p.x + tb * kw : nullptr,
-              *opc = COL ? nullptr : p.o + tb * kw;
+              *dpc = COL ? nullptr : p.d + tb * kw;
   const __bf16 *ubc = COL ? nullptr : p.ub + tb * kw, *kbc = COL ? nullptr : p.kb + tb * kw;
   const Tok* tokc = COL ? nullptr : p.tok + tb;
   {
@@ -1752,7 +1750,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
       }
       yr[q][t2] = ldq(Yk + o);
       G[q][t2] = ldq(Gc + o);
-      if constexpr (!COL) orw[q][t2] = ldq(opc + o);
+      if constexpr (!COL) orw[q][t2] = ldq(dpc + o);
     }
   }
   // rowsum(X_C (.) lam): the four lane groups' partials of each state row
@@ -1892,6 +1890,8 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
         gu[q][t2] = ldq(p.duh + tb * kw + o);
         gk[q][t2] = ldq(p.dkh + tb * kw + o);
         kn[t2] = scaled(ldq(kbc + o), tk[t2].rk);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) orw[q][t2].v[e] -= kn[t2].v[e];  // the readout o = d - q
         dv[t2] = ldq(dwc + o);
         dgo[q][t2] = ldq(p.dgS + tb * kw + o);
         const __bf16* hr = wrow(p.in.h, hb, min(ch * WBT + t2 * 16 + m, T - 1), hh);
@@ -2235,18 +2235,29 @@ __global__ __launch_bounds__(WT) void k_w_src_bwd(SrcBwdParams p) {
 
 // Output cotangent as a padded bf16 panel (zero when absent and on padded entries).
 struct DoutParams {
-  int H, T, V, Tp, VP;
+  int H, T, V, Tp, VP, vec;  // vec: rows take 4-element loads
   const __bf16* dout;
   __bf16* dO;
 };
 __global__ __launch_bounds__(WT) void k_w_dout(DoutParams p) {
-  const int s = blockIdx.y, b = s / p.H, h = s % p.H;
-  const long long n = (long long)p.Tp * p.VP;
-  for (long long idx = (long long)blockIdx.x * WT + threadIdx.x; idx < n; idx += (long long)gridDim.x * WT) {
-    const int t = (int)(idx / p.VP), c = (int)(idx % p.VP);
-    __bf16 v = f2bf(0.f);
-    if (p.dout && t < p.T && c < p.V) v = p.dout[(((long long)b * p.T + t) * p.H + h) * p.V + c];
-    p.dO[(long long)s * n + idx] = v;
+  // four neighbouring elements per thread (64-bit divisions per element held
+  // the copy to 2 TB/s: 34 us at B4 T2048 H8 V = 256, now 15)
+  const int s = blockIdx.y, b = s / p.H, h = s % p.H, q4 = p.VP / 4;
+  const long long ib = ((long long)b * p.T * p.H + h) * p.V;
+  for (int idx = blockIdx.x * WT + threadIdx.x; idx < p.Tp * q4; idx += gridDim.x * WT) {
+    const int t = idx / q4, c = (idx - t * q4) * 4;
+    bf16x4 v = {};
+    if (p.dout && t < p.T) {
+      const __bf16* row = p.dout + ib + (long long)t * p.H * p.V;
+      if (p.vec) {
+        if (c < p.V) v = *reinterpret_cast<const bf16x4*>(row + c);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < p.V) v[e] = row[c + e];
+      }
+    }
+    *reinterpret_cast<bf16x4*>(p.dO + ((long long)s * p.Tp + t) * p.VP + c) = v;
   }
 }
 
@@ -2290,7 +2301,7 @@ struct WideFwd {
   float* G;
   __bf16 *ub, *kb, *qb, *hb;
   Tok* tok;
-  float *delta, *oC, *d, *e, *chi, *wS;
+  float *delta, *d, *e, *chi, *wS;
   float *AC, *AS, *PS;
   xs_t *XC, *XS;
   _Float16 *Wneg, *Kt;
@@ -2308,7 +2319,7 @@ WideFwd carve_wide_fwd(void* saved, void* scratch, const WideDims& d, size_t* sa
   w.G = c.take(pk);
   w.ub = c.take<__bf16>(pk); w.kb = c.take<__bf16>(pk); w.qb = c.take<__bf16>(pk);
   w.tok = c.take<Tok>(tok);
-  w.delta = c.take(pk); w.oC = c.take(pk); w.d = c.take(pk); w.e = c.take(pk);
+  w.delta = c.take(pk); w.d = c.take(pk); w.e = c.take(pk);
   w.chi = c.take(pk); w.wS = c.take(pv);
   w.AC = c.take(mat); w.AS = c.take(mat); w.PS = c.take(mat);
   w.XC = c.take<xs_t>((size_t)d.n * (d.NT + 1) * d.KP * d.KP);
@@ -2415,7 +2426,7 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
   OutParams orow{};
   orow.NT = d.NT; orow.Tp = d.Tp; orow.kw = d.KP; orow.vw = d.KP;
   orow.slots = w.XC; orow.w = w.delta; orow.ub = w.ub; orow.kb = w.kb; orow.tok = w.tok;
-  orow.G = w.G; orow.o = w.oC; orow.d = w.d;
+  orow.G = w.G; orow.d = w.d;
   SD_SMEM_ONCE(k_w_out_c, (int)out_c_smem());
   SD_LAUNCH("k_w_out_c", k_w_out_c, dim3(d.NT, d.n), dim3(PT), out_c_smem(), st, orow);
 
@@ -2460,6 +2471,7 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   DoutParams dp{};
   dp.H = in->H; dp.T = in->T; dp.V = in->V; dp.Tp = d.Tp; dp.VP = d.VP;
   dp.dout = (const __bf16*)dout; dp.dO = w.dO;
+  dp.vec = in->V % 4 == 0 && ((uintptr_t)dout & 7) == 0;
   SD_LAUNCH("k_w_dout", k_w_dout, dim3(64, d.n), dim3(WT), 0, st, dp);
 
   // ---- memory S op ----
@@ -2508,7 +2520,7 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   launch_wstate("w_state_c_bwd", rc, d.n, st);
   GradParams gc{};
   gc.NT = d.NT; gc.Tp = d.Tp; gc.kw = d.KP; gc.vw = d.KP;
-  gc.ub = f.ub; gc.kb = f.kb; gc.tok = f.tok; gc.G = f.G; gc.dO = w.dd; gc.o = f.oC;
+  gc.ub = f.ub; gc.kb = f.kb; gc.tok = f.tok; gc.G = f.G; gc.dO = w.dd; gc.d = f.d;
   gc.w = f.delta; gc.dw = w.dwC; gc.Xslots = f.XC; gc.Lslots = w.LC; gc.Pp = w.Pp;
   gc.in = *in; gc.duh = w.duh; gc.dkh = w.dkh; gc.dgS = w.dgS;
   gc.du = (__bf16*)du; gc.dh = (__bf16*)dh; gc.dkey = (__bf16*)dk;
