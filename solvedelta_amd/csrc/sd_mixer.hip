@@ -16,15 +16,39 @@
 
 namespace sd {
 
-__device__ __forceinline__ float silu(float a) { return a / (1.f + __expf(-a)); }
-__device__ __forceinline__ float sigm(float a) { return 1.f / (1.f + __expf(-a)); }
-// torch.nn.functional.softplus with its default threshold 20
-__device__ __forceinline__ float softplus20(float x) {
-  return x > 20.f ? x : log1pf(__expf(x));
+// These kernels' element work is transcendental: an IEEE division costs ten vector
+// instructions and log1pf thirty, which, not HBM, bounded the decay gate and the
+// convolution.  The quotients here have denominators in [1, 3], so they take the
+// hardware's reciprocal and one residual (Newton) step instead.
+// sigmoid(a) from t = e^{-|a|}: 1 / (1 + t) or t / (1 + t)
+__device__ __forceinline__ float sigm_t(float a, float t) {
+  const float n = a < 0.f ? t : 1.f, s = 1.f + t, r = __builtin_amdgcn_rcpf(s), q = n * r;
+  return __builtin_fmaf(__builtin_fmaf(-s, q, n), r, q);
+}
+__device__ __forceinline__ float sigm(float a) { return sigm_t(a, __expf(-fabsf(a))); }
+__device__ __forceinline__ float silu(float a) { return a * sigm(a); }
+// softplus(x) = max(x, 0) + log(1 + t), t = e^{-|x|}: log(1 + t) = 2 atanh(z) with
+// z = t / (2 + t) <= 1/3, by its series through z^17 (the next term is below
+// 2e-10 of the sum).  z's residual, with what the sum 2 + t rounded off, is added
+// to the small terms, so the result is rounded once.  Above torch's threshold of
+// 20 it rounds to x as torch's does.
+__device__ __forceinline__ float softplus_t(float x, float t) {
+  const float s = 2.f + t, r = __builtin_amdgcn_rcpf(s), z = t * r, y = z * z, zz = z + z;
+  const float e = __builtin_fmaf(-z, t - (s - 2.f), __builtin_fmaf(-s, z, t));  // t - (2 + t) z
+  float p = 1.f / 17.f;
+  p = __builtin_fmaf(p, y, 1.f / 15.f);
+  p = __builtin_fmaf(p, y, 1.f / 13.f);
+  p = __builtin_fmaf(p, y, 1.f / 11.f);
+  p = __builtin_fmaf(p, y, 1.f / 9.f);
+  p = __builtin_fmaf(p, y, 1.f / 7.f);
+  p = __builtin_fmaf(p, y, 1.f / 5.f);
+  p = __builtin_fmaf(p, y, 1.f / 3.f);
+  const float l = zz + __builtin_fmaf(zz * y, p, (r + r) * e);
+  return x > 0.f ? x + l : l;
 }
 
-// VEC (1 or 2) neighbouring bf16 channels of one token, kept packed until used:
-// two channels are one 4-byte access.
+// VEC (1, 2, 4 or 8) neighbouring bf16 channels of one token, kept packed until used:
+// one access of 2 VEC bytes.
 template <int VEC> struct BfV;
 template <> struct BfV<1> {
   __bf16 v;
@@ -35,6 +59,26 @@ template <> struct BfV<2> {
   __device__ __forceinline__ void get(float (&x)[2]) const {
     x[0] = __uint_as_float(v << 16);
     x[1] = __uint_as_float(v & 0xffff0000u);
+  }
+};
+template <> struct BfV<4> {
+  uint2 v;
+  __device__ __forceinline__ void get(float (&x)[4]) const {
+    x[0] = __uint_as_float(v.x << 16);
+    x[1] = __uint_as_float(v.x & 0xffff0000u);
+    x[2] = __uint_as_float(v.y << 16);
+    x[3] = __uint_as_float(v.y & 0xffff0000u);
+  }
+};
+template <> struct BfV<8> {
+  uint4 v;
+  __device__ __forceinline__ void get(float (&x)[8]) const {
+    const unsigned u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[2 * i] = __uint_as_float(u[i] << 16);
+      x[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
+    }
   }
 };
 template <int VEC>
@@ -178,69 +222,131 @@ __global__ __launch_bounds__(NTHREADS) void k_conv_bwd(ConvArgs a, const __bf16*
   p[0] = g0; p[1] = g1; p[2] = g2; p[3] = g3;
 }
 
-// out[i] = sum_p part[p][i]: 32 columns x 8 partial rows per workgroup, the
-// eight row sums combined through LDS.
+// out[i] = sum_p part[p][i]: COLS columns x 256 / COLS partial rows per workgroup,
+// the row sums combined through LDS.  32 columns (whole lines) for wide sums; 8
+// where the width alone would leave the chip idle and each thread a long chain
+// of loads (1024 rows of 128: 11 us with 32 columns, 4 workgroups).
+template <int COLS>
 __global__ __launch_bounds__(NTHREADS) void k_sum_parts(const float* __restrict__ part, int nparts,
                                                         int width, float* __restrict__ out) {
-  __shared__ float red[8][33];
-  const int cx = threadIdx.x & 31, ry = threadIdx.x >> 5;
-  const int i = blockIdx.x * 32 + cx;
+  constexpr int ROWS = NTHREADS / COLS;
+  __shared__ float red[ROWS][COLS + 1];
+  const int cx = threadIdx.x % COLS, ry = threadIdx.x / COLS;
+  const int i = blockIdx.x * COLS + cx;
   float s = 0.f;
   if (i < width) {
-#pragma unroll 4
-    for (int p = ry; p < nparts; p += 8) s += part[(long long)p * width + i];
+#pragma unroll 8
+    for (int p = ry; p < nparts; p += ROWS) s += part[(long long)p * width + i];
   }
   red[ry][cx] = s;
   __syncthreads();
   if (ry == 0 && i < width) {
     float t = 0.f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) t += red[k][cx];
+    for (int k = 0; k < ROWS; ++k) t += red[k][cx];
     out[i] = t;
   }
+}
+
+static void launch_sum_parts(const float* part, int nparts, int width, float* out, hipStream_t st) {
+  if (width <= 1024)
+    SD_LAUNCH("k_sum_parts", k_sum_parts<8>, dim3((width + 7) / 8), dim3(NTHREADS), 0, st, part, nparts, width, out);
+  else
+    SD_LAUNCH("k_sum_parts", k_sum_parts<32>, dim3((width + 31) / 32), dim3(NTHREADS), 0, st, part, nparts, width,
+              out);
 }
 
 // ---------------------------------------------------------------------------
 // KDA decay gate.  raw [N][H*r] bf16 (row stride), bias [H*r], log_rate [H].
 // ---------------------------------------------------------------------------
-constexpr int GATE_TR = 16;  // rows per backward workgroup
+constexpr int GATE_TR = 16;  // rows per thread (and per partial row) in the backward
+constexpr int GATE_FR = 8;   // rows per thread in the forward
 
-__global__ __launch_bounds__(NTHREADS) void k_gate_fwd(int N, int H, int r, const __bf16* raw,
-                                                       long long rs, const float* log_rate,
-                                                       const float* bias, float* out) {
-  const int HR = H * r;
-  const long long i = (long long)blockIdx.x * NTHREADS + threadIdx.x;
-  if (i >= (long long)N * HR) return;
-  const int c = (int)(i % HR);
-  const long long n = i / HR;
-  const float x = bf2f(raw[n * rs + c]) + bias[c];
-  out[i] = -__expf(log_rate[c / r]) * softplus20(x);
+// Thread (row group, VEC neighbouring columns): the columns' rate and bias are
+// loaded once, the rows' loads are all in flight before the first use.  VEC = 4
+// where rows start on 8-byte (raw) and 16-byte (FP32) boundaries; one column
+// per element otherwise.  15 us forward (3.4 TB/s) and 22 us backward (3.0 TB/s) at
+// 8192 rows of 1024, bound about equally by HBM and the transcendentals, where
+// a thread per element (a 64-bit division each, log1pf) took 37 and 37 us.
+struct GateArgs {
+  int N, H, r, HR;
+  const __bf16* __restrict__ raw;
+  long long rs;
+  const float* __restrict__ log_rate;
+  const float* __restrict__ bias;
+};
+template <int VEC>
+__device__ __forceinline__ void gate_cols(const GateArgs& a, int c, float (&rate)[VEC], float (&b)[VEC]) {
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    rate[k] = __expf(a.log_rate[(c + k) / a.r]);
+    b[k] = a.bias[c + k];
+  }
+}
+template <int VEC> struct FV { float v[VEC]; };
+
+template <int VEC>
+__global__ __launch_bounds__(NTHREADS) void k_gate_fwd(GateArgs a, float* __restrict__ out) {
+  const int Q = a.HR / VEC, idx = blockIdx.x * NTHREADS + threadIdx.x;
+  const int rg = idx / Q, c = (idx - rg * Q) * VEC, n0 = rg * GATE_FR;
+  if (n0 >= a.N) return;
+  BfV<VEC> x[GATE_FR];
+#pragma unroll
+  for (int j = 0; j < GATE_FR; ++j) x[j] = ldv<VEC>(a.raw + (long long)min(n0 + j, a.N - 1) * a.rs + c);
+  float rate[VEC], b[VEC];
+  gate_cols<VEC>(a, c, rate, b);
+#pragma unroll
+  for (int j = 0; j < GATE_FR; ++j) {
+    float v[VEC];
+    x[j].get(v);
+    FV<VEC> o;
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      const float t = v[k] + b[k];
+      o.v[k] = -rate[k] * softplus_t(t, __expf(-fabsf(t)));
+    }
+    if (n0 + j < a.N) *reinterpret_cast<FV<VEC>*>(out + (long long)(n0 + j) * a.HR + c) = o;
+  }
 }
 
 // draw = dout * (-exp(lr)) * sigmoid(raw + bias) (softplus' is 1 above the
 // threshold); partials: dbias_c = sum draw, dlr_c = sum dout * out.
-__global__ __launch_bounds__(NTHREADS) void k_gate_bwd(int N, int H, int r, const __bf16* raw,
-                                                       long long rs, const float* log_rate,
-                                                       const float* bias, const float* dout,
-                                                       __bf16* draw, float* part) {
-  const int HR = H * r;
-  const int c = blockIdx.x * NTHREADS + threadIdx.x;
-  if (c >= HR) return;
-  const int n0 = blockIdx.y * GATE_TR, n1 = min(N, n0 + GATE_TR);
-  const float rate = __expf(log_rate[c / r]), bc = bias[c];
-  float db = 0.f, dl = 0.f;
-#pragma unroll 4
-  for (int n = n0; n < n1; ++n) {
-    const float x = bf2f(raw[(long long)n * rs + c]) + bc;
-    const float g = dout[(long long)n * HR + c];
-    const float sp = softplus20(x);
-    const float dx = -rate * g * (x > 20.f ? 1.f : sigm(x));
-    draw[(long long)n * HR + c] = f2bf(dx);
-    db += dx;
-    dl += -rate * sp * g;
+template <int VEC>
+__global__ __launch_bounds__(NTHREADS) void k_gate_bwd(GateArgs a, const float* __restrict__ dout,
+                                                       __bf16* __restrict__ draw,
+                                                       float* __restrict__ part) {
+  const int Q = a.HR / VEC, idx = blockIdx.x * NTHREADS + threadIdx.x;
+  const int rg = idx / Q, c = (idx - rg * Q) * VEC, n0 = rg * GATE_TR;
+  if (n0 >= a.N) return;
+  BfV<VEC> x[GATE_TR];
+  FV<VEC> g[GATE_TR];
+#pragma unroll
+  for (int j = 0; j < GATE_TR; ++j) {
+    const long long n = min(n0 + j, a.N - 1);
+    x[j] = ldv<VEC>(a.raw + n * a.rs + c);
+    g[j] = *reinterpret_cast<const FV<VEC>*>(dout + n * a.HR + c);
   }
-  part[(long long)blockIdx.y * 2 * HR + c] = db;
-  part[(long long)blockIdx.y * 2 * HR + HR + c] = dl;
+  float rate[VEC], b[VEC];
+  gate_cols<VEC>(a, c, rate, b);
+  FV<VEC> db = {}, dl = {};
+#pragma unroll
+  for (int j = 0; j < GATE_TR; ++j) {
+    if (n0 + j >= a.N) break;
+    float v[VEC], dx[VEC];
+    x[j].get(v);
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      const float t = v[k] + b[k];
+      const float et = __expf(-fabsf(t));
+      dx[k] = -rate[k] * g[j].v[k] * sigm_t(t, et);
+      db.v[k] += dx[k];
+      dl.v[k] += -rate[k] * softplus_t(t, et) * g[j].v[k];
+    }
+    stv<VEC>(draw + (long long)(n0 + j) * a.HR + c, dx);
+  }
+  float* p = part + (long long)rg * 2 * a.HR + c;
+  *reinterpret_cast<FV<VEC>*>(p) = db;
+  *reinterpret_cast<FV<VEC>*>(p + a.HR) = dl;
 }
 
 // One workgroup per head: dbias[c] for the head's columns, dlog_rate[h], from
@@ -388,6 +494,129 @@ __global__ __launch_bounds__(RMS_ROWS * 64) void k_rms_bwd(int N, int D, float e
 #pragma unroll
     for (int k = 0; k < RMS_ROWS; ++k) s += pw[k][c];
     part[(long long)blockIdx.x * D + c] = s;
+  }
+}
+
+// The same with LPR (8, 16, 32) lanes per row, eight neighbouring columns each:
+// D <= 8 LPR a multiple of 8 and 16-byte aligned rows, so a row is one 16-byte
+// load per lane and a wave covers 64 / LPR rows.  HBM bound: 14 us forward,
+// 17 us backward (3.6 and 4.9 TB/s) at 65536 rows of 128, where a wave per row with 2-byte loads
+// (half its lanes idle at D = 128) took 19 and 30 us.
+template <int LPR>
+__device__ __forceinline__ float lanes_sum(float v) {
+  v = dpp_add(v, 0);
+  v = dpp_add(v, 1);
+  v = dpp_add(v, 2);
+  if constexpr (LPR >= 16) v = dpp_add(v, 3);
+  if constexpr (LPR >= 32) v += __shfl_xor(v, 16);
+  return v;
+}
+constexpr int RMSV_U = 4;  // rows per lane group and batch, all loads in flight
+
+template <int LPR>
+__global__ __launch_bounds__(NTHREADS) void k_rmsv_fwd(int N, int D, float eps, const __bf16* __restrict__ x,
+                                                       const __bf16* __restrict__ g, const float* __restrict__ w,
+                                                       __bf16* __restrict__ y, float* __restrict__ rstd_out) {
+  constexpr int G = NTHREADS / LPR;
+  const int c = (threadIdx.x % LPR) * 8, cc = c < D ? c : 0, n0 = blockIdx.x * G * RMSV_U + threadIdx.x / LPR;
+  BfV<8> xr[RMSV_U], gr[RMSV_U];
+#pragma unroll
+  for (int u = 0; u < RMSV_U; ++u) {
+    const long long o = (long long)min(n0 + u * G, N - 1) * D + cc;
+    xr[u] = ldv<8>(x + o);
+    gr[u] = ldv<8>(g + o);
+  }
+  float wv[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) wv[e] = w[cc + e];
+#pragma unroll
+  for (int u = 0; u < RMSV_U; ++u) {
+    const int n = n0 + u * G;
+    float xv[8], gv[8], o[8], ss = 0.f;
+    xr[u].get(xv);
+    gr[u].get(gv);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += xv[e] * xv[e];
+    const float rs = rsqrtf(lanes_sum<LPR>(c < D ? ss : 0.f) / D + eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = xv[e] * rs * wv[e] * sigm(gv[e]);
+    if (n < N && c < D) stv<8>(y + (long long)n * D + c, o);
+    if (rstd_out && n < N && c == 0) rstd_out[n] = rs;
+  }
+}
+
+// rows: per workgroup, a multiple of NTHREADS / LPR * RMSV_U
+template <int LPR>
+__global__ __launch_bounds__(NTHREADS) void k_rmsv_bwd(int N, int D, float eps, int rows,
+                                                       const __bf16* __restrict__ x,
+                                                       const __bf16* __restrict__ g,
+                                                       const float* __restrict__ w,
+                                                       const __bf16* __restrict__ dy,
+                                                       __bf16* __restrict__ dx, __bf16* __restrict__ dg,
+                                                       __bf16* __restrict__ y, float* __restrict__ part) {
+  constexpr int G = NTHREADS / LPR;
+  __shared__ float pw[G][LPR * 8 + 4];
+  const int c = (threadIdx.x % LPR) * 8, cc = c < D ? c : 0, gr_ = threadIdx.x / LPR;
+  const bool in = c < D;
+  float wv[8], acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    wv[e] = w[cc + e];
+    acc[e] = 0.f;
+  }
+  const int base = blockIdx.x * rows;
+  for (int r0 = gr_; r0 < rows; r0 += G * RMSV_U) {
+    BfV<8> xr[RMSV_U], gr[RMSV_U], dr[RMSV_U];
+#pragma unroll
+    for (int u = 0; u < RMSV_U; ++u) {
+      const long long o = (long long)min(base + r0 + u * G, N - 1) * D + cc;
+      xr[u] = ldv<8>(x + o);
+      gr[u] = ldv<8>(g + o);
+      dr[u] = ldv<8>(dy + o);
+    }
+#pragma unroll
+    for (int u = 0; u < RMSV_U; ++u) {
+      const int n = base + r0 + u * G;
+      const bool ok = in && n < N;
+      float xh[8], gv[8], dv[8], sg[8], gy[8], ss = 0.f, dot = 0.f;
+      xr[u].get(xh);
+      gr[u].get(gv);
+      dr[u].get(dv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += xh[e] * xh[e];
+      const float rs = rsqrtf(lanes_sum<LPR>(in ? ss : 0.f) / D + eps);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        sg[e] = sigm(gv[e]);
+        xh[e] *= rs;
+        gy[e] = dv[e] * wv[e] * sg[e];
+        dot += gy[e] * xh[e];
+      }
+      dot = lanes_sum<LPR>(in ? dot : 0.f) / D;
+      float ox[8], og[8], oy[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        acc[e] += ok ? dv[e] * xh[e] * sg[e] : 0.f;
+        ox[e] = rs * (gy[e] - xh[e] * dot);
+        og[e] = dv[e] * xh[e] * wv[e] * sg[e] * (1.f - sg[e]);
+        oy[e] = xh[e] * wv[e] * sg[e];
+      }
+      if (ok) {
+        const long long o = (long long)n * D + c;
+        stv<8>(dx + o, ox);
+        stv<8>(dg + o, og);
+        if (y) stv<8>(y + o, oy);
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) pw[gr_][c + e] = acc[e];
+  __syncthreads();
+  for (int k = threadIdx.x; k < D; k += NTHREADS) {
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < G; ++q) t += pw[q][k];
+    part[(long long)blockIdx.x * D + k] = t;
   }
 }
 
@@ -714,6 +943,16 @@ static bool conv_pairs(const ConvArgs& a, const void* p, const void* q) {
   return a.D % 2 == 0 && a.sb % 2 == 0 && a.st % 2 == 0 && bits % 4 == 0;
 }
 
+// Four columns per thread where every row of the bf16 operands starts on an
+// 8-byte and of the FP32 operand on a 16-byte boundary.
+static bool gate_quads(const GateArgs& a, const void* bf, const void* f32) {
+  return a.HR % 4 == 0 && a.rs % 4 == 0 && (((uintptr_t)a.raw | (uintptr_t)bf) & 7) == 0 &&
+         ((uintptr_t)f32 & 15) == 0;
+}
+
+// Eight columns per lane where rows are multiples of 8 wide and 16-byte aligned.
+static bool rms_vec(int D, uintptr_t bits) { return D % 8 == 0 && (bits & 15) == 0; }
+
 extern "C" {
 
 size_t sd_conv4_workspace_bytes(int B, int T, int D) {
@@ -744,8 +983,7 @@ int sd_conv4_silu_bwd(int B, int T, int D, const void* x, int64_t x_sb, int64_t 
   hipStream_t st = (hipStream_t)stream;
   SD_LAUNCH("k_conv_bwd", k_conv_bwd, dim3(cdiv(D, NTHREADS), nch, B), dim3(NTHREADS), 0, st, a,
             (const __bf16*)dy, (const __bf16*)dfinal, (__bf16*)dx, dinit, (float*)workspace);
-  SD_LAUNCH("k_sum_parts", k_sum_parts, dim3(cdiv(4LL * D, 32)), dim3(NTHREADS), 0, st,
-            (const float*)workspace, B * nch, 4 * D, dw);
+  launch_sum_parts((const float*)workspace, B * nch, 4 * D, dw, st);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 
@@ -794,8 +1032,7 @@ int sd_conv4_silu_masked_bwd(int B, int T, int D, const void* x, int64_t x_sb, i
   else
     SD_LAUNCH("k_conv_masked_bwd", k_conv_masked_bwd<1>, grid, dim3(NTHREADS), 0, st, a, m,
               (const __bf16*)dy, (const __bf16*)dfinal, (__bf16*)dx, dinit, (float*)workspace);
-  SD_LAUNCH("k_sum_parts", k_sum_parts, dim3(cdiv(4LL * D, 32)), dim3(NTHREADS), 0, st,
-            (const float*)workspace, B * parts, 4 * D, dw);
+  launch_sum_parts((const float*)workspace, B * parts, 4 * D, dw, st);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 
@@ -809,9 +1046,14 @@ int sd_kda_gate_fwd(int N, int H, int r, const void* raw, int64_t raw_row_stride
                     const float* log_rate, const float* bias, float* out, void* stream) {
   if (N <= 0 || H <= 0 || r <= 0) return SD_ERR_SHAPE;
   if (!raw || !log_rate || !bias || !out) return SD_ERR_ARG;
-  SD_LAUNCH("k_gate_fwd", k_gate_fwd, dim3(cdiv((long long)N * H * r, NTHREADS)), dim3(NTHREADS),
-            0, (hipStream_t)stream, N, H, r, (const __bf16*)raw, raw_row_stride, log_rate, bias,
-            out);
+  const GateArgs a{N, H, r, H * r, (const __bf16*)raw, raw_row_stride, log_rate, bias};
+  const int groups = cdiv(N, GATE_FR);
+  if (gate_quads(a, nullptr, out))
+    SD_LAUNCH("k_gate_fwd", k_gate_fwd<4>, dim3(cdiv((long long)groups * (H * r / 4), NTHREADS)), dim3(NTHREADS),
+              0, (hipStream_t)stream, a, out);
+  else
+    SD_LAUNCH("k_gate_fwd", k_gate_fwd<1>, dim3(cdiv((long long)groups * H * r, NTHREADS)), dim3(NTHREADS),
+              0, (hipStream_t)stream, a, out);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 
@@ -825,14 +1067,17 @@ int sd_kda_gate_bwd(int N, int H, int r, const void* raw, int64_t raw_row_stride
   if (workspace_bytes < sd_kda_gate_workspace_bytes(N, H, r)) return SD_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   const int np = cdiv(N, GATE_TR);
-  SD_LAUNCH("k_gate_bwd", k_gate_bwd, dim3(cdiv(H * r, NTHREADS), np), dim3(NTHREADS), 0, st, N,
-            H, r, (const __bf16*)raw, raw_row_stride, log_rate, bias, dout, (__bf16*)draw,
-            (float*)workspace);
+  const GateArgs a{N, H, r, H * r, (const __bf16*)raw, raw_row_stride, log_rate, bias};
+  if (gate_quads(a, draw, dout) && ((uintptr_t)workspace & 15) == 0)
+    SD_LAUNCH("k_gate_bwd", k_gate_bwd<4>, dim3(cdiv((long long)np * (H * r / 4), NTHREADS)), dim3(NTHREADS), 0,
+              st, a, dout, (__bf16*)draw, (float*)workspace);
+  else
+    SD_LAUNCH("k_gate_bwd", k_gate_bwd<1>, dim3(cdiv((long long)np * H * r, NTHREADS)), dim3(NTHREADS), 0, st, a,
+              dout, (__bf16*)draw, (float*)workspace);
   // column sums over the partial rows spread over many workgroups (a per-head
   // walk over every partial row kept only H workgroups busy), then per head
   float* colsum = (float*)workspace + (size_t)np * 2 * H * r;
-  SD_LAUNCH("k_sum_parts", k_sum_parts, dim3(cdiv(2 * H * r, 32)), dim3(NTHREADS), 0, st,
-            (const float*)workspace, np, 2 * H * r, colsum);
+  launch_sum_parts((const float*)workspace, np, 2 * H * r, colsum, st);
   SD_LAUNCH("k_gate_reduce", k_gate_reduce, dim3(H), dim3(NTHREADS), 0, st, H, r, 1,
             (const float*)colsum, dbias, dlog_rate);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
@@ -847,9 +1092,21 @@ int sd_rmsnorm_gated_fwd(int N, int D, float eps, const void* x, const void* gat
                          const float* weight, void* y, float* rstd, void* stream) {
   if (N <= 0 || D <= 0 || D > 256) return SD_ERR_SHAPE;
   if (!x || !gate || !weight || !y) return SD_ERR_ARG;
-  SD_LAUNCH("k_rms_fwd", k_rms_fwd, dim3(cdiv(N, RMS_ROWS)), dim3(RMS_ROWS * 64), 0,
-            (hipStream_t)stream, N, D, eps, (const __bf16*)x, (const __bf16*)gate, weight,
-            (__bf16*)y, rstd);
+  const __bf16 *xb = (const __bf16*)x, *gb = (const __bf16*)gate;
+  __bf16* yb = (__bf16*)y;
+  hipStream_t st = (hipStream_t)stream;
+  if (!rms_vec(D, (uintptr_t)x | (uintptr_t)gate | (uintptr_t)y))
+    SD_LAUNCH("k_rms_fwd", k_rms_fwd, dim3(cdiv(N, RMS_ROWS)), dim3(RMS_ROWS * 64), 0, st, N, D, eps, xb, gb,
+              weight, yb, rstd);
+  else if (D <= 64)
+    SD_LAUNCH("k_rms_fwd", k_rmsv_fwd<8>, dim3(cdiv(N, NTHREADS / 8 * RMSV_U)), dim3(NTHREADS), 0, st, N, D, eps,
+              xb, gb, weight, yb, rstd);
+  else if (D <= 128)
+    SD_LAUNCH("k_rms_fwd", k_rmsv_fwd<16>, dim3(cdiv(N, NTHREADS / 16 * RMSV_U)), dim3(NTHREADS), 0, st, N, D, eps,
+              xb, gb, weight, yb, rstd);
+  else
+    SD_LAUNCH("k_rms_fwd", k_rmsv_fwd<32>, dim3(cdiv(N, NTHREADS / 32 * RMSV_U)), dim3(NTHREADS), 0, st, N, D, eps,
+              xb, gb, weight, yb, rstd);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 
@@ -861,12 +1118,28 @@ int sd_rmsnorm_gated_bwd(int N, int D, float eps, const void* x, const void* gat
   if (!x || !gate || !weight || !dy || !dx || !dgate || !dweight || !workspace) return SD_ERR_ARG;
   if (workspace_bytes < sd_rmsnorm_gated_workspace_bytes(N, D)) return SD_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
-  const int np = cdiv(N, RMS_PART);
-  SD_LAUNCH("k_rms_bwd", k_rms_bwd, dim3(np), dim3(RMS_ROWS * 64), 0, st, N, D, eps,
-            (const __bf16*)x, (const __bf16*)gate, weight, (const __bf16*)dy, (__bf16*)dx,
-            (__bf16*)dgate, (__bf16*)y, (float*)workspace);
-  SD_LAUNCH("k_sum_parts", k_sum_parts, dim3(cdiv(D, 32)), dim3(NTHREADS), 0, st,
-            (const float*)workspace, np, D, dweight);
+  const __bf16 *xb = (const __bf16*)x, *gb = (const __bf16*)gate, *db = (const __bf16*)dy;
+  __bf16 *dxb = (__bf16*)dx, *dgb = (__bf16*)dgate, *yb = (__bf16*)y;
+  float* part = (float*)workspace;
+  int np = cdiv(N, RMS_PART);
+  if (!rms_vec(D, (uintptr_t)x | (uintptr_t)gate | (uintptr_t)dy | (uintptr_t)dx | (uintptr_t)dgate | (uintptr_t)y)) {
+    SD_LAUNCH("k_rms_bwd", k_rms_bwd, dim3(np), dim3(RMS_ROWS * 64), 0, st, N, D, eps, xb, gb, weight, db, dxb, dgb,
+              yb, part);
+  } else {
+    // at most ~512 partial rows (two workgroups per CU), 128 rows a batch at most
+    const int rows = cdiv(cdiv(N, 512), 128) * 128 > 128 ? cdiv(cdiv(N, 512), 128) * 128 : (D <= 64 ? 128 : RMS_PART);
+    np = cdiv(N, rows);
+    if (D <= 64)
+      SD_LAUNCH("k_rms_bwd", k_rmsv_bwd<8>, dim3(np), dim3(NTHREADS), 0, st, N, D, eps, rows, xb, gb, weight, db,
+                dxb, dgb, yb, part);
+    else if (D <= 128)
+      SD_LAUNCH("k_rms_bwd", k_rmsv_bwd<16>, dim3(np), dim3(NTHREADS), 0, st, N, D, eps, rows, xb, gb, weight, db,
+                dxb, dgb, yb, part);
+    else
+      SD_LAUNCH("k_rms_bwd", k_rmsv_bwd<32>, dim3(np), dim3(NTHREADS), 0, st, N, D, eps, rows, xb, gb, weight, db,
+                dxb, dgb, yb, part);
+  }
+  launch_sum_parts((const float*)workspace, np, D, dweight, st);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 

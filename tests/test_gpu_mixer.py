@@ -81,6 +81,58 @@ def test_kda_gate_forward_backward():
         assert e < tol, name
 
 
+@pytest.mark.parametrize("B,T,H,r", [(1, 7, 3, 5), (2, 9, 2, 2), (1, 17, 5, 64), (1, 40, 4, 129)])
+def test_kda_gate_widths_and_tails(B, T, H, r):
+    """Four columns per thread or one, row groups with a remainder; the whole
+    range of softplus, and non-finite inputs as torch gives them."""
+    mx = _mx()
+    g = torch.Generator().manual_seed(B * 100 + T + r)
+    raw = (12 * torch.randn(B, T, H, r, generator=g)).to(torch.bfloat16)
+    raw.view(-1)[:5] = torch.tensor([float("inf"), float("-inf"), 88.0, -88.0, 1e-3])
+    lr, bias = torch.randn(H, generator=g), torch.randn(H, r, generator=g)
+    rc, lc, bc = (t.cuda().requires_grad_() for t in (raw, lr, bias))
+    out = mx.kda_decay_gate(rc, lc, bc)
+    ro, lo, bo = (_d(t).requires_grad_() for t in (raw, lr, bias))
+    oo = kda_decay(ro, lo, bo)
+    assert torch.isinf(out.view(-1)[0]) and out.view(-1)[1] == 0
+    # x = raw + bias and x log2(e) are each rounded to 24 bits, which e^{-|x|} (the
+    # value itself for x far below zero) turns into 2 |x| 2^-24 relative; a few
+    # units of 2^-24 more for the rest; values below 1e-30 compared absolutely
+    fin = torch.isfinite(ro)
+    tol = (16 + 2 * (ro + bo).abs()) * 2.0 ** -24 * oo.abs() + 1e-30
+    assert torch.all(((out.double().cpu() - oo).abs() <= tol)[fin])
+    dout = torch.randn(B, T, H, r, generator=g)
+    dout.view(-1)[:2] = 0.0
+    raw2 = raw.clone()
+    raw2.view(-1)[:2] = 0.0
+    rc, ro = raw2.cuda().requires_grad_(), _d(raw2).requires_grad_()
+    ga = torch.autograd.grad(mx.kda_decay_gate(rc, lc, bc), (rc, lc, bc), dout.cuda())
+    gb = torch.autograd.grad(kda_decay(ro, lo, bo), (ro, lo, bo), _d(dout))
+    for name, a, b, tol in zip(("draw", "dlog_rate", "dbias"), ga, gb, (4e-3, 1e-5, 1e-5)):
+        assert rel(a.float(), b) < tol, name
+
+
+@pytest.mark.parametrize("N,D,off", [(1, 8, 0), (131, 64, 0), (300, 72, 0), (65, 128, 0), (70000, 128, 0),
+                                     (33, 136, 0), (129, 256, 0), (77, 100, 0), (40, 64, 1)])
+def test_rmsnorm_gated_row_layouts(N, D, off):
+    """8, 16 and 32 lanes per row, the general path (widths off 8 and rows off
+    16 bytes), batches with a remainder, and more rows than dweight partials."""
+    from solvedelta_amd.mixer import _rms_bwd, _rms_fwd
+    g = torch.Generator(device="cuda").manual_seed(N + D)
+    mk = lambda: torch.randn(N * D + off, generator=g, device="cuda").to(torch.bfloat16)[off:].view(N, D)
+    x, gate, dy = mk(), mk(), mk()
+    w = torch.rand(D, generator=g, device="cuda") + 0.5
+    y = _rms_fwd(x, gate, w, 1e-6)
+    dx, dg, dw, y2 = _rms_bwd(x, gate, w, dy, 1e-6, True)
+    xo, go, wo = (t.double().requires_grad_() for t in (x, gate, w))
+    yo = rms_norm_gated(xo, go, wo, 1e-6)
+    gr = torch.autograd.grad(yo, (xo, go, wo), dy.double())
+    assert torch.equal(y, y2)
+    for name, a, b, tol in zip(("y", "dx", "dgate", "dweight"), (y, dx, dg, dw), (yo, *gr),
+                               (4e-3, 4e-3, 4e-3, 1e-5)):
+        assert rel(a.float(), b) < tol, name
+
+
 def test_rmsnorm_gated_and_linear_owner():
     mx = _mx()
     g = torch.Generator().manual_seed(11)
