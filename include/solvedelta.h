@@ -92,6 +92,12 @@ int sd_fwd(const sd_inputs *in, void *out, float *C_T, float *S_T, void *workspa
 int sd_fwd_split(const sd_inputs *in, void *out, float *C_T, float *S_T, void *saved,
                  size_t saved_bytes, void *scratch, size_t scratch_bytes, void *stream);
 
+/* A forward that no sd_bwd follows: the same results, without the panels only the
+ * backward reads (widths above 128 run as sd_fwd). */
+size_t sd_fwd_infer_bytes(int B, int T, int H, int r, int V);
+int sd_fwd_infer(const sd_inputs *in, void *out, float *C_T, float *S_T, void *workspace,
+                 size_t workspace_bytes, void *stream);
+
 /* Backward of sd_fwd with the same inputs and the forward's workspace.
  * dout: bf16 [B,T,H,V] contiguous (nullable = zero); dC_T, dS_T fp32 (nullable).
  * Gradient outputs, all contiguous: du,dh,dq,dk,dv,derase,dwrite bf16 in the

@@ -45,6 +45,10 @@ EXPORTS = {
                                     ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "sd_fwd": (ctypes.c_int, [ctypes.POINTER(SdInputs), ctypes.c_void_p, ctypes.c_void_p,
                               ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "sd_fwd_infer_bytes": (ctypes.c_size_t, [ctypes.c_int] * 5),
+    "sd_fwd_infer": (ctypes.c_int, [ctypes.POINTER(SdInputs), ctypes.c_void_p, ctypes.c_void_p,
+                                    ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
+                                    ctypes.c_void_p]),
     "sd_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 5),
     "sd_bwd": (ctypes.c_int, [ctypes.POINTER(SdInputs), ctypes.c_void_p, ctypes.c_void_p,
                               ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_void_p] * 11

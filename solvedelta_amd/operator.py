@@ -63,7 +63,7 @@ def _ptr(t: Optional[torch.Tensor]):
 class _SolveDeltaFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma, C0, S0,
-                want_state: bool, fresh=None):
+                want_state: bool, fresh=None, infer=False):
         lib = _lib.load()
         B, T, H, r = u.shape
         V = values.shape[-1]
@@ -72,6 +72,14 @@ class _SolveDeltaFn(torch.autograd.Function):
         out = torch.empty(B, T, H, V, dtype=torch.bfloat16, device=dev)
         C_T = torch.empty(B, H, r, r, dtype=torch.float32, device=dev) if want_state else None
         S_T = torch.empty(B, H, r, V, dtype=torch.float32, device=dev) if want_state else None
+        ctx.set_materialize_grads(False)
+        if infer:  # no backward will follow: its panels are neither kept nor written
+            nws = lib.sd_fwd_infer_bytes(B, T, H, r, V)
+            ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+            rc = lib.sd_fwd_infer(ctypes.byref(ins), out.data_ptr(), _ptr(C_T), _ptr(S_T),
+                                  ws.data_ptr(), nws, _stream(dev))
+            _lib.check(rc, "sd_fwd_infer")
+            return out, C_T, S_T
         # the saved region is held for the backward; the scratch region (panels
         # only the forward's state passes read) returns to the allocator here
         nsaved = lib.sd_fwd_saved_bytes(B, T, H, r, V)
@@ -82,7 +90,6 @@ class _SolveDeltaFn(torch.autograd.Function):
                               ws.data_ptr(), nsaved, scratch.data_ptr(), nscratch, _stream(dev))
         _lib.check(rc, "sd_fwd_split")
         del scratch
-        ctx.set_materialize_grads(False)
         ctx.has_C0, ctx.has_S0 = C0 is not None, S0 is not None
         ctx.has_fresh = fresh is not None
         empty = u.new_empty(0)
@@ -127,7 +134,7 @@ class _SolveDeltaFn(torch.autograd.Function):
             dgam = dgam.sum(dim=(0, 1)).reshape(gamma.shape)
         return (du.to(u.dtype), dh.to(h.dtype), dq.to(q.dtype), dk.to(keys.dtype),
                 dv.to(values.dtype), dg.to(log_decay.dtype), der.to(erase_raw.dtype),
-                dwr.to(write_raw.dtype), dgam.to(gamma.dtype), dC0, dS0, None, None)
+                dwr.to(write_raw.dtype), dgam.to(gamma.dtype), dC0, dS0, None, None, None)
 
 
 def _decode(u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma, initial_state,
@@ -240,12 +247,16 @@ def _dispatch(u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma, ini
     if initial_state is not None:
         C0, S0 = (s.contiguous() for s in initial_state)
     group = _WIDE_MAX if value_route(r, V) == "wide" else _MAX_WIDTH
+    infer = not (torch.is_grad_enabled() and any(
+        x.requires_grad for x in (u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma)
+        + (() if C0 is None else (C0, S0))))
     if V <= group:
         out, C_T, S_T = _SolveDeltaFn.apply(u, h, q, keys, values, log_decay, erase_raw,
-                                            write_raw, gamma, C0, S0, return_final_state, fresh)
+                                            write_raw, gamma, C0, S0, return_final_state, fresh,
+                                            infer)
     else:
         out, C_T, S_T = _value_groups(u, h, q, keys, values, log_decay, erase_raw, write_raw,
-                                      gamma, C0, S0, return_final_state, group, fresh)
+                                      gamma, C0, S0, return_final_state, group, fresh, infer)
     if not return_final_state:
         return out, None
     return out, SolveDeltaState(C_T, S_T)
@@ -264,7 +275,7 @@ def value_route(r: int, V: int) -> str:
 
 
 def _value_groups(u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma, C0, S0,
-                  want_state, group, fresh=None):
+                  want_state, group, fresh=None, infer=False):
     """V above the kernels' value width (128, or 256 on the wide kernels): the
     columns of S (and of the output) evolve independently given the shared predictor C and the sources d, e, chi, so the value axis is cut
     into groups of at most `group` columns, each run by the HIP path with the same
@@ -277,7 +288,8 @@ def _value_groups(u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma,
         g1 = min(V, g0 + group)
         S0g = None if S0 is None else S0[..., g0:g1].contiguous()
         o, C, S = _SolveDeltaFn.apply(u, h, q, keys, values[..., g0:g1], log_decay, erase_raw,
-                                      write_raw[..., g0:g1], gamma, C0, S0g, want_state, fresh)
+                                      write_raw[..., g0:g1], gamma, C0, S0g, want_state, fresh,
+                                      infer)
         outs.append(o)
         S_parts.append(S)
         if g0 == 0:

@@ -57,6 +57,9 @@ def test_workspace_queries_and_argument_rejection():
     # key widths 129..256 take the wide-width kernels' own (larger) layout
     wide = lib.sd_fwd_workspace_bytes(1, 64, 1, 200, 16)
     assert wide > small and lib.sd_bwd_workspace_bytes(1, 64, 1, 200, 256) > 0
+    # the forward without a backward leaves out the panels only the backward reads
+    assert 0 < lib.sd_fwd_infer_bytes(4, 2048, 8, 128, 128) < big
+    assert lib.sd_fwd_infer_bytes(1, 64, 1, 200, 16) == wide
     ins = _lib.SdInputs()
     ins.B, ins.T, ins.H, ins.r, ins.V = 1, 4, 1, 264, 16  # r > 256
     assert lib.sd_fwd(ctypes.byref(ins), None, None, None, None, 0, None) == _lib.SD_ERR_SHAPE

@@ -146,3 +146,29 @@ def test_decode_multi_step_matches_oracle():
     out = torch.cat(outs, 1)
     print(f"[decode x{steps}] rel out {rel(out.float(), eo):.2e} S {rel(st.S, es.S):.2e}", flush=True)
     assert rel(out.float(), eo) < 1e-2 and rel(st.S, es.S) < 1e-2 and rel(st.predictor, es.predictor) < 1e-2
+
+
+@pytest.mark.parametrize("B,T,H,r,V,decay,masked", [
+    (2, 130, 2, 128, 128, "softplus", False),  # a ragged last chunk
+    (1, 64, 1, 40, 100, "mixed", False),       # narrow widths; wild coordinates (d read back)
+    (2, 65, 3, 64, 128, "softplus", True),     # token flags
+    (1, 17, 2, 160, 144, "softplus", False),   # wide kernels
+])
+def test_forward_without_gradients_equals_forward_with(B, T, H, r, V, decay, masked):
+    """The forward that keeps nothing for a backward gives the training
+    forward's output and final states bitwise."""
+    from solvedelta_amd import solvedelta_masked_native, solvedelta_native
+    args = make_inputs(B, T, H, r, V, seed=T + r, decay=decay, requires_grad=True)
+    state = make_state(B, H, r, V, seed=T)
+    masks = ()
+    if masked:
+        g = torch.Generator().manual_seed(T)
+        masks = ((torch.rand(B, T, generator=g) > 0.1).cuda(), (torch.rand(B, T, generator=g) < 0.05).cuda())
+    fn = solvedelta_masked_native if masked else solvedelta_native
+    out, st = fn(*args, *masks, initial_state=state, return_final_state=True)
+    assert out.requires_grad
+    with torch.no_grad():
+        out2, st2 = fn(*args, *masks, initial_state=state, return_final_state=True)
+    out3, _ = fn(*[a.detach() for a in args], *masks, initial_state=state)
+    assert torch.equal(out, out2) and torch.equal(out, out3)
+    assert torch.equal(st.predictor, st2.predictor) and torch.equal(st.S, st2.S)
