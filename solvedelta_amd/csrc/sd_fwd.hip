@@ -53,18 +53,29 @@ constexpr int PS = KD + 8;  // bf16 panel row stride
 struct PrepCSmem {
   ChunkDecay cd;
   float M[BT * LS];
-  float tmp[BT * LS];
-  float Uh[BT][GS];   // normalised u
-  __bf16 Hh[BT][PS];  // h (raw bf16, exact)
+  __bf16 Ub[BT][PS];  // u, later h (raw bf16, exact)
+  float ru[BT];       // inverse norms of u
   float gam[BT];
   float xm[BT];       // 1, or 0 on fresh tokens (no erase read)
-  LPanel Yt;          // the L Gram's Y side (u), transformed and split once
 };
 
 // FL: the call has token flags (sd_inputs.fresh).  KEEP: a backward will read
 // what the forward alone does not (sd_fwd_infer runs without)
+//
+// One chunk is a chain of short phases (loads, decay table, Gram, inverse,
+// products), each waiting for the one before, so what bounds the kernel is how
+// many chunks a CU has in flight.  71 KB of LDS and 128 registers let two run
+// side by side: u stays packed bf16 with a norm per token, the Gram's factors
+// are formed from it and the decay table in registers by the wave that uses
+// them (a staged, split Y side took 34 KB), h follows u into its panel, and the
+// inverse's scratch blocks lie in M's unused corner.
+// Against one 153 KB workgroup per CU: 70 -> 57 us at 4 x 2048 tokens, 8 heads,
+// r = V = 128 (151 MB moved, 32 us at a large copy's rate), 97 -> 78 us at
+// 1 x 16384 without (I+L)^-1.  The opening loads come in bursts (9 us of a
+// workgroup's 20); h gathered in operand layout from memory instead cost 7 us
+// of latency before the inverse (67 / 90 us).
 template <bool FL, bool KEEP>
-__global__ __launch_bounds__(CT) void k_prep_c(FwdParams p) {
+__global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   PrepCSmem& s = *reinterpret_cast<PrepCSmem*>(smem_raw);
   // chunk-major dispatch, last chunk first (chunk 0, where the C state pass
@@ -76,14 +87,15 @@ __global__ __launch_bounds__(CT) void k_prep_c(FwdParams p) {
   const float* g = (const float*)in.log_decay.data + (long long)b * in.log_decay.sb +
                    (long long)hh * in.log_decay.sh;
   const int w = wave_id(), l = lane_id();
-{
+  float hx[2][RQ];  // rows of h, until u's panel is free for them
+  {
     // every load of the opening phase first (the decay column, then every row's
     // u and h): a row's reduction would otherwise hold the next row's loads
     // behind it, and the decay table's build would wait for its own
     const int cl = l & 15;
     float xdec[BS];
     decay_load(g, in.log_decay.st, t0, T, r, xdec, FL ? tok_flag_row(in, b) : nullptr, tok_flag_st(in));
-    float ux[2][RQ], hx[2][RQ];
+    float ux[2][RQ];
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       const int t = t0 + row16(w, g);
@@ -101,43 +113,99 @@ __global__ __launch_bounds__(CT) void k_prep_c(FwdParams p) {
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       const int i = row16(w, g);
-      l2norm16(ux[g]);
 #pragma unroll
-      for (int q = 0; q < RQ; ++q) {
-        s.Uh[i][cl + 16 * q] = ux[g][q];
-        s.Hh[i][cl + 16 * q] = f2bf(hx[g][q]);
-      }
+      for (int q = 0; q < RQ; ++q) s.Ub[i][cl + 16 * q] = f2bf(ux[g][q]);  // exact
+      const float rn = l2norm16(ux[g]);
+      if (cl == 0) s.ru[i] = rn;
     }
   }
   __syncthreads();
   const ChunkDecay& cd = s.cd;
-  // L_ij = gamma_i sum_c u_ic u_jc exp(G_{i-1,c} - G_jc), j < i
-  stage_ytilde(s.Yt, cd, [&](int j, int c) { return s.Uh[j][c]; });
-  decayed_gram_yt<true>(
-      cd, [&](int i, int c) { return s.gam[i] * s.xm[i] * s.Uh[i][c]; }, s.Yt,
-      [&](int j, int c) { return s.Uh[j][c]; }, true, s.M);
-  unit_lower_inverse(s.M, s.tmp);
+  const int m = l & 15, kq = (l >> 4) * 8;
+  auto U = [&](int i, int c) { return bf2f(s.Ub[i][c]) * s.ru[i]; };
+  // L_ij = gamma_i sum_c u_ic u_jc exp(G_{i-1,c} - G_jc), j < i: block pair (I, J)
+  // from x = gamma u exp(G_excl - R_J) and y = u exp(R_J - G), 32 columns at a time
+  for (int pr = w; pr < 10; pr += CW) {
+    int I = 0, J = pr;
+    while (J > I) { J -= I + 1; ++I; }  // pr -> (I, J) with J <= I
+    const int i = I * BS + m, j = J * BS + m;
+    const float xs = s.gam[i] * s.xm[i], ui = s.ru[i], uj = s.ru[j];
+    const float* Gi = cd.G[i > 0 ? i - 1 : 0];
+    const float* Gj = cd.G[j];
+    f4 acc = zero4();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int c0 = ks * 32 + kq;
+      const bf16x8 xu = *reinterpret_cast<const bf16x8*>(&s.Ub[i][c0]);
+      const bf16x8 yu = *reinterpret_cast<const bf16x8*>(&s.Ub[j][c0]);
+      Frag x, y;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float R = cd.R[J][c0 + e];
+        __bf16 hi, lo;
+        split_bf(xs * (bf2f(xu[e]) * ui) * __expf(keep_if(i > 0, Gi[c0 + e]) - R), hi, lo);
+        x.h[e] = hi;
+        x.l[e] = lo;
+        split_bf(bf2f(yu[e]) * uj * exp_unless_wild(cd.wild[J][c0 + e] != 0, R - Gj[c0 + e]), hi, lo);
+        y.h[e] = hi;
+        y.l[e] = lo;
+      }
+      acc = mma3f(x, y, acc);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int ii = I * BS + out_row(e), jj = J * BS + out_col();
+      s.M[ii * LS + jj] = jj < ii ? acc[e] : 0.f;
+    }
+  }
+  {  // blocks (0, 1) and (2, 3), which the products below read as zeros
+    const int half = threadIdx.x >> 8, i = (threadIdx.x >> 4) & 15;
+    s.M[(half * 32 + i) * LS + half * 32 + BS + m] = 0.f;
+  }
+  __syncthreads();
+  gram_wild_fixup<true>(
+      cd, [&](int i, int c) { return s.gam[i] * s.xm[i] * U(i, c); }, U, true, s.M);
+  // everything else that reads u: the decayed keys (transposed per chunk), the
+  // chunk decay and, in operand layout, the right side of W's product
+  const long long cbase = ((long long)n * p.NT + ch);
+  store_frag_panel1<KD, BT>(p.Kc, cbase * KD * BT, [&](int c, int i) {
+    return U(i, c) * __expf(cd.G[BT - 1][c] - cd.G[i][c]);
+  });
+  if (threadIdx.x < KD) p.Gam[cbase * KD + threadIdx.x] = __expf(cd.G[BT - 1][threadIdx.x]);
+  const int c = w * 16 + m;
+  bf16x8 bh[2], bl[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int k = ks * 32 + kq + e;
+      __bf16 hi, lo;
+      split_bf(s.xm[k] * U(k, c) * __expf(gx_excl(cd, k, c)), hi, lo);
+      bh[ks][e] = hi;
+      bl[ks][e] = lo;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) s.Ub[row16(w, g)][m + 16 * q] = f2bf(hx[g][q]);  // exact
+  // scratch blocks (2..3, 0..1) of the inverse lie at M's blocks (0..1, 2..3)
+  unit_lower_inverse(s.M, s.M - 32 * LS + 32);
   if constexpr (KEEP)
-    for (int idx = threadIdx.x; idx < BT * BT; idx += CT)
-      p.Ac[((long long)n * p.NT + ch) * BT * BT + idx] = s.M[(idx / BT) * LS + idx % BT];
-  // W = A diag(gamma) (u e^{Gexcl} masked on fresh tokens),  U = A diag(gamma) h
+    for (int idx = threadIdx.x; idx < BT * BT; idx += CT) {
+      const int i = idx / BT, j = idx % BT;
+      p.Ac[((long long)n * p.NT + ch) * BT * BT + idx] = j > i ? 0.f : s.M[i * LS + j];
+    }
+  // W = A diag(gamma) (u e^{Gexcl} masked on fresh tokens),  U = A diag(gamma) h:
+  // wave w holds columns 16w..16w+15 of both right sides, and the product is
+  // taken transposed, so that a lane's four results are one token's neighbours
   const long long rowbase = (long long)n * p.Tp + t0;
   {
-    const int cb = w;
-    // B operands, the same for every row block I: formed and split once
-    const int m = l & 15, kq = (l >> 4) * 8;
-    bf16x8 bh[2], bl[2], hb[2];
+    bf16x8 hb[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = ks * 32 + kq + e, c = cb * 16 + m;
-        __bf16 h, lo;
-        split_bf(s.xm[k] * s.Uh[k][c] * __expf(gx_excl(cd, k, c)), h, lo);
-        bh[ks][e] = h;
-        bl[ks][e] = lo;
-        hb[ks][e] = s.Hh[k][c];  // h is the raw bf16 input: exact
-      }
+      for (int e = 0; e < 8; ++e) hb[ks][e] = s.Ub[ks * 32 + kq + e][c];
 #pragma unroll
     for (int I = 0; I < NB; ++I) {
       const int K = I < 2 ? 32 : 64;
@@ -149,32 +217,26 @@ __global__ __launch_bounds__(CT) void k_prep_c(FwdParams p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int k = ks * 32 + kq + e;
-          __bf16 h, lo;
-          split_bf(s.M[(I * BS + m) * LS + k] * s.gam[k], h, lo);
-          ah[e] = h;
+          __bf16 hi, lo;
+          split_bf(s.M[(I * BS + m) * LS + k] * s.gam[k], hi, lo);
+          ah[e] = hi;
           al[e] = lo;
         }
-        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[ks], aw, 0, 0, 0);
-        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, hb[ks], au, 0, 0, 0);
-        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[ks], aw, 0, 0, 0);
-        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[ks], aw, 0, 0, 0);
-        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, hb[ks], au, 0, 0, 0);
+        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[ks], al, aw, 0, 0, 0);
+        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hb[ks], al, au, 0, 0, 0);
+        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[ks], ah, aw, 0, 0, 0);
+        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[ks], ah, aw, 0, 0, 0);
+        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hb[ks], ah, au, 0, 0, 0);
       }
+      typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+      const int row = I * BS + m, oc = w * 16 + (l >> 4) * 4;
+      h4 wv;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const long long row = rowbase + I * BS + out_row(e);
-        const int c = cb * 16 + out_col();
-        p.Wc[rowbase * KD + frag_off(I * BS + out_row(e), c, KD)] = (_Float16)(-aw[e]);
-        p.Uc[row * KD + c] = au[e];
-      }
+      for (int e = 0; e < 4; ++e) wv[e] = (_Float16)(-aw[e]);
+      *reinterpret_cast<h4*>(&p.Wc[rowbase * KD + frag_off(row, oc, KD)]) = wv;
+      *reinterpret_cast<f4*>(&p.Uc[(rowbase + row) * KD + oc]) = au;
     }
   }
-  // decayed keys (transposed per chunk) and chunk decay
-  const long long cbase = ((long long)n * p.NT + ch);
-  store_frag_panel1<KD, BT>(p.Kc, cbase * KD * BT, [&](int c, int i) {
-    return s.Uh[i][c] * __expf(cd.G[BT - 1][c] - cd.G[i][c]);
-  });
-  if (threadIdx.x < KD) p.Gam[cbase * KD + threadIdx.x] = __expf(cd.G[BT - 1][threadIdx.x]);
 }
 
 // ---------------------------------------------------------------------------

@@ -247,9 +247,12 @@ def _dispatch(u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma, ini
     if initial_state is not None:
         C0, S0 = (s.contiguous() for s in initial_state)
     group = _WIDE_MAX if value_route(r, V) == "wide" else _MAX_WIDTH
-    infer = not (torch.is_grad_enabled() and any(
-        x.requires_grad for x in (u, h, q, keys, values, log_decay, erase_raw, write_raw, gamma)
-        + (() if C0 is None else (C0, S0))))
+    # no backward can follow (written out: a generator costs a training call 2 us)
+    infer = not (torch.is_grad_enabled() and (
+        u.requires_grad or h.requires_grad or q.requires_grad or keys.requires_grad
+        or values.requires_grad or log_decay.requires_grad or erase_raw.requires_grad
+        or write_raw.requires_grad or gamma.requires_grad
+        or (C0 is not None and (C0.requires_grad or S0.requires_grad))))
     if V <= group:
         out, C_T, S_T = _SolveDeltaFn.apply(u, h, q, keys, values, log_decay, erase_raw,
                                             write_raw, gamma, C0, S0, return_final_state, fresh,
