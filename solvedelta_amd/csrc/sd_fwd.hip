@@ -57,6 +57,7 @@ struct PrepCSmem {
   float ru[BT];       // inverse norms of u
   float gam[BT];
   float xm[BT];       // 1, or 0 on fresh tokens (no erase read)
+  float cap[NB][KD];  // largest exponent of y: TAU, or -inf (y = 0) on a wild coordinate
 };
 
 // FL: the call has token flags (sd_inputs.fresh).  KEEP: a backward will read
@@ -69,11 +70,13 @@ struct PrepCSmem {
 // are formed from it and the decay table in registers by the wave that uses
 // them (a staged, split Y side took 34 KB), h follows u into its panel, and the
 // inverse's scratch blocks lie in M's unused corner.
-// Against one 153 KB workgroup per CU: 70 -> 57 us at 4 x 2048 tokens, 8 heads,
-// r = V = 128 (151 MB moved, 32 us at a large copy's rate), 97 -> 78 us at
+// Against one 153 KB workgroup per CU: 70 -> 56 us at 4 x 2048 tokens, 8 heads,
+// r = V = 128 (151 MB moved, 32 us at a large copy's rate), 97 -> 76 us at
 // 1 x 16384 without (I+L)^-1.  The opening loads come in bursts (9 us of a
 // workgroup's 20); h gathered in operand layout from memory instead cost 7 us
-// of latency before the inverse (67 / 90 us).
+// of latency before the inverse (67 / 90 us).  With 128 chunks, one for every
+// second CU, the chain itself is the time: 18.7 us, 20.3 with the ten Gram pairs
+// in two turns of the eight waves.
 template <bool FL, bool KEEP>
 __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -110,6 +113,10 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
       s.xm[threadIdx.x] = erase_keep_f(f);
     }
     decay_build(s.cd, xdec);
+    {
+      const int J = threadIdx.x / KD, cc = threadIdx.x & (KD - 1);
+      s.cap[J][cc] = s.cd.wild[J][cc] ? -INFINITY : TAU;
+    }
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       const int i = row16(w, g);
@@ -124,45 +131,67 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
   const int m = l & 15, kq = (l >> 4) * 8;
   auto U = [&](int i, int c) { return bf2f(s.Ub[i][c]) * s.ru[i]; };
   // L_ij = gamma_i sum_c u_ic u_jc exp(G_{i-1,c} - G_jc), j < i: block pair (I, J)
-  // from x = gamma u exp(G_excl - R_J) and y = u exp(R_J - G), 32 columns at a time
-  for (int pr = w; pr < 10; pr += CW) {
-    int I = 0, J = pr;
-    while (J > I) { J -= I + 1; ++I; }  // pr -> (I, J) with J <= I
-    const int i = I * BS + m, j = J * BS + m;
-    const float xs = s.gam[i] * s.xm[i], ui = s.ru[i], uj = s.ru[j];
-    const float* Gi = cd.G[i > 0 ? i - 1 : 0];
+  // from x = u exp(G_excl - R_J) and y = u^ exp(R_J - G), 32 columns at a time.
+  // Ten pairs on eight waves: a wave takes one whole pair and a quarter of pair 8
+  // or 9, whose partial sums meet in M's blocks above the diagonal.
+  auto pair_step = [&](int I, int J, int ks, f4 acc) {
+    const int i = I * BS + m, j = J * BS + m, c0 = ks * 32 + kq;
+    const float uj = s.ru[j];
+    const float* Gi = i > 0 ? cd.G[i - 1] : cd.R[0];  // R[0] is zero
     const float* Gj = cd.G[j];
-    f4 acc = zero4();
+    const bf16x8 xu = *reinterpret_cast<const bf16x8*>(&s.Ub[i][c0]);
+    const bf16x8 yu = *reinterpret_cast<const bf16x8*>(&s.Ub[j][c0]);
+    Frag x, y;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int c0 = ks * 32 + kq;
-      const bf16x8 xu = *reinterpret_cast<const bf16x8*>(&s.Ub[i][c0]);
-      const bf16x8 yu = *reinterpret_cast<const bf16x8*>(&s.Ub[j][c0]);
-      Frag x, y;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float R = cd.R[J][c0 + e];
-        __bf16 hi, lo;
-        split_bf(xs * (bf2f(xu[e]) * ui) * __expf(keep_if(i > 0, Gi[c0 + e]) - R), hi, lo);
-        x.h[e] = hi;
-        x.l[e] = lo;
-        split_bf(bf2f(yu[e]) * uj * exp_unless_wild(cd.wild[J][c0 + e] != 0, R - Gj[c0 + e]), hi, lo);
-        y.h[e] = hi;
-        y.l[e] = lo;
-      }
-      acc = mma3f(x, y, acc);
+    for (int e = 0; e < 8; ++e) {
+      const float R = cd.R[J][c0 + e];
+      __bf16 hi, lo;
+      split_bf(bf2f(xu[e]) * __expf(Gi[c0 + e] - R), hi, lo);
+      x.h[e] = hi;
+      x.l[e] = lo;
+      split_bf(bf2f(yu[e]) * uj * __expf(fminf(R - Gj[c0 + e], s.cap[J][c0 + e])), hi, lo);
+      y.h[e] = hi;
+      y.l[e] = lo;
     }
+    return mma3f(x, y, acc);
+  };
+  auto put_pair = [&](int I, int J, f4 acc) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int ii = I * BS + out_row(e), jj = J * BS + out_col();
-      s.M[ii * LS + jj] = jj < ii ? acc[e] : 0.f;
+      s.M[ii * LS + jj] = jj < ii ? s.gam[ii] * s.xm[ii] * s.ru[ii] * acc[e] : 0.f;
     }
+  };
+  {
+    int I = 0, J = w;
+    while (J > I) { J -= I + 1; ++I; }  // w -> (I, J) with J <= I
+    const int half = w >> 2, part = w & 3;
+    f4 acc = zero4();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) acc = pair_step(I, J, ks, acc);
+    f4 acc2 = pair_step(3, 2 + half, part, zero4());
+    put_pair(I, J, acc);
+    auto slot = [&](int q, int e) -> float& {  // q-th partial block of this half
+      const int r0 = q == 1 ? 2 * half : half, c0 = q == 1 ? 2 * half + 1 : q;
+      return s.M[(r0 * BS + out_row(e)) * LS + c0 * BS + out_col()];
+    };
+    if (part != 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) slot(part, e) = acc2[e];
+    }
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+      for (int q = 1; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc2[e] += slot(q, e);
+      put_pair(3, 2 + half, acc2);
+      // blocks (0, 1) and (2, 3), which the products below read as zeros
+#pragma unroll
+      for (int e = 0; e < 4; ++e) slot(1, e) = 0.f;
+    }
+    __syncthreads();
   }
-  {  // blocks (0, 1) and (2, 3), which the products below read as zeros
-    const int half = threadIdx.x >> 8, i = (threadIdx.x >> 4) & 15;
-    s.M[(half * 32 + i) * LS + half * 32 + BS + m] = 0.f;
-  }
-  __syncthreads();
   gram_wild_fixup<true>(
       cd, [&](int i, int c) { return s.gam[i] * s.xm[i] * U(i, c); }, U, true, s.M);
   // everything else that reads u: the decayed keys (transposed per chunk), the
