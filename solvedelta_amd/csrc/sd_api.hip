@@ -58,10 +58,10 @@ FwdWs carve_fwd(void* saved, void* scratch, int B, int T, int H, size_t* saved_b
 // Workspace of a forward that no backward follows: one region, without the
 // buffers only a backward reads (both ops' inverses, e, chi, the S op's slots
 // and w; null pointers leave their stores out).  The forward is bound by its
-// serial chunk phases, and these stores sat in them: at one sequence of 16384
-// tokens, 8 heads, r = V = 128, a pass went 429 -> 396 us (the S state pass
+// serial chunk phases, and these stores sat in them: at 2 x 3001 tokens,
+// 16 heads, r = V = 128, a pass went 429 -> 396 us (the S state pass
 // 87 -> 68, k_prep_s 206 -> 200, k_prep_c 101 -> 97) and the workspace from
-// 20.5 to 13.5 16-bit panels (689 to 454 MB).
+// 508 to 334 MB.
 FwdWs carve_infer(void* base, int B, int T, int H, size_t* bytes) {
   const size_t n = (size_t)B * H, NT = (T + kBT - 1) / kBT, Tp = NT * kBT;
   const size_t panel = n * Tp * kKD;

@@ -65,14 +65,14 @@ struct PrepCSmem {
 //
 // One chunk is a chain of short phases (loads, decay table, Gram, inverse,
 // products), each waiting for the one before, so what bounds the kernel is how
-// many chunks a CU has in flight.  71 KB of LDS and 128 registers let two run
+// many chunks a CU has in flight.  73 KB of LDS and 128 registers let two run
 // side by side: u stays packed bf16 with a norm per token, the Gram's factors
 // are formed from it and the decay table in registers by the wave that uses
 // them (a staged, split Y side took 34 KB), h follows u into its panel, and the
 // inverse's scratch blocks lie in M's unused corner.
 // Against one 153 KB workgroup per CU: 70 -> 56 us at 4 x 2048 tokens, 8 heads,
 // r = V = 128 (151 MB moved, 32 us at a large copy's rate), 97 -> 76 us at
-// 1 x 16384 without (I+L)^-1.  The opening loads come in bursts (9 us of a
+// 2 x 3001, 16 heads, without (I+L)^-1.  The opening loads come in bursts (9 us of a
 // workgroup's 20); h gathered in operand layout from memory instead cost 7 us
 // of latency before the inverse (67 / 90 us).  With 128 chunks, one for every
 // second CU, the chain itself is the time: 18.7 us, 20.3 with the ten Gram pairs
@@ -484,8 +484,8 @@ __device__ __forceinline__ void store_readout(const StateParams& p, const StateS
 // o = Q~ X0 + P w for its 16 columns: wave w's token block, from the X0 and w
 // fragments the recurrence loads anyway; o is off the recurrence's critical path.
 // Without KEEP (the S pass of a forward that no backward follows) the slots and
-// w, which only the backward reads, are not stored: 87 -> 68 us over 256 chunks
-// of 8 sequences.
+// w, which only the backward reads, are not stored: 87 -> 68 us over 47 chunks
+// of 32 sequences.
 template <bool REV, bool OUT, bool KEEP, class Prefetch>
 __device__ __forceinline__ void state_step(const StateParams& p, StateSmem<REV>& s, int n, int ch,
                                            int tile, const StateFrags<REV, OUT>& cur,

@@ -269,9 +269,9 @@ def value_route(r: int, V: int) -> str:
     """How a call of key width r and value width V runs: "main" (r, V <= 128:
     the 64-token kernels) or "wide" (the wide-width kernels, which take r, V <=
     256; V above 256 in groups of 256 columns).  For r <= 128 < V <= 256 one
-    wide call (F+B 1.95 ms at B4 T2048 H8 r=128 V=256 on MI355X) beat two
+    wide call (F+B 1.44 ms at B4 T2048 H8 r=128 V=256 on MI355X) beat two
     128-column groups on the main kernels, each recomputing the predictor
-    (2.13 ms)."""
+    (1.96 ms)."""
     if r <= _MAX_WIDTH and V <= _MAX_WIDTH:
         return "main"
     return "wide"
