@@ -93,7 +93,7 @@ int sd_fwd_split(const sd_inputs *in, void *out, float *C_T, float *S_T, void *s
                  size_t saved_bytes, void *scratch, size_t scratch_bytes, void *stream);
 
 /* A forward that no sd_bwd follows: the same results, without the panels only the
- * backward reads (widths above 128 run as sd_fwd). */
+ * backward reads (widths above 128: in a workspace of sd_fwd's size). */
 size_t sd_fwd_infer_bytes(int B, int T, int H, int r, int V);
 int sd_fwd_infer(const sd_inputs *in, void *out, float *C_T, float *S_T, void *workspace,
                  size_t workspace_bytes, void *stream);

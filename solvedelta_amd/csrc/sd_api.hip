@@ -99,7 +99,7 @@ int check_chunk_grid(const sd_inputs* in);
 int fwd_launch(const sd_inputs* in, void* out, float* C_T, float* S_T, void* saved,
                void* scratch, hipStream_t st) {
   if (int rc = check_chunk_grid(in)) return rc;
-  if (is_wide(in->r, in->V)) return launch_wide_fwd(in, out, C_T, S_T, saved, scratch, st);
+  if (is_wide(in->r, in->V)) return launch_wide_fwd(in, out, C_T, S_T, saved, scratch, true, st);
   FwdWs w = carve_fwd(saved, scratch, in->B, in->T, in->H, nullptr, nullptr);
   return launch_fwd(in, out, C_T, S_T, w, st);
 }
@@ -218,9 +218,12 @@ int sd_fwd_infer(const sd_inputs* in, void* out, float* C_T, float* S_T, void* w
   int rc = check_inputs(in);
   if (rc) return rc;
   if (!out || !workspace) return SD_ERR_ARG;
-  if (is_wide(in->r, in->V)) return sd_fwd(in, out, C_T, S_T, workspace, workspace_bytes, stream);
   if (workspace_bytes < sd_fwd_infer_bytes(in->B, in->T, in->H, in->r, in->V)) return SD_ERR_WORKSPACE;
   if ((rc = check_chunk_grid(in))) return rc;
+  if (is_wide(in->r, in->V)) {  // the training layout
+    const size_t saved = align256(sd_fwd_saved_bytes(in->B, in->T, in->H, in->r, in->V));
+    return launch_wide_fwd(in, out, C_T, S_T, workspace, (char*)workspace + saved, false, (hipStream_t)stream);
+  }
   const FwdWs w = carve_infer(workspace, in->B, in->T, in->H, nullptr);
   return launch_fwd(in, out, C_T, S_T, w, (hipStream_t)stream);
 }

@@ -955,7 +955,7 @@ struct OutParams {
   __bf16* out;
   const __bf16 *ub, *kb;        // row output: q = base = k^, k = u^
   const Tok* tok;
-  float* d;
+  float *o, *d;                 // o: null where no backward follows
 };
 
 constexpr int GS16 = 20;  // row stride (FP32) of a wave's staged [32 tokens][16 coordinates] panel
@@ -1082,7 +1082,9 @@ __global__ __launch_bounds__(PT, 4) void k_w_out_s(OutParams p) {
 
 // Row output: M = q w^T (j <= i), then
 //   o_ir = e^{G_ir} ((q X0^T)_ir + (M k~)_ir),  k~_jr = k_jr e^{-G_jr},  d = q + o
-// with the decay factored per state row r (wild rows: exact per-term sum).  M as
+// with the decay factored per state row r (wild rows: exact per-term sum).  o is
+// kept beside d for the backward's o dO: taken back from the rounded sum it would
+// hold only the bits above k^'s last (20 us of a training step at B4 T2048 H8 r = V = 256).  M as
 // the prep's Grams, in FP32 over the waves; q X0^T on fp16 matrix cores (q, unit
 // rows, split into high and low halves in LDS; X0 exact in its slot).  Wave w
 // owns the 16-row blocks w, w + 8.  117 us (4.6 TB/s) at B4 T2048 H8 r = V = 256, where
@@ -1193,7 +1195,7 @@ __global__ __launch_bounds__(PT, 4) void k_w_out_c(OutParams p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block overwrites it
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2) {
-      Quad o;
+      Quad o, d;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o.v[e] = __expf(G[q][t2].v[e]) * acc[q][t2][e];
       if (__any(any)) {  // exact sums of the wild rows' in-chunk terms
@@ -1206,8 +1208,10 @@ __global__ __launch_bounds__(PT, 4) void k_w_out_c(OutParams p) {
         }
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o.v[e] += kn[q][t2].v[e];
-      *reinterpret_cast<Quad*>(p.d + tb * kw + (unsigned)((t2 * 16 + m) * kw + c0[q])) = o;
+      for (int e = 0; e < 4; ++e) d.v[e] = kn[q][t2].v[e] + o.v[e];
+      const unsigned off = (t2 * 16 + m) * kw + c0[q];
+      if (p.o) *reinterpret_cast<Quad*>(p.o + tb * kw + off) = o;
+      *reinterpret_cast<Quad*>(p.d + tb * kw + off) = d;
     }
   }
 }
@@ -1521,7 +1525,7 @@ constexpr size_t bprep_smem() {
 // ---------------------------------------------------------------------------
 struct GradParams {
   int NT, Tp, kw, vw;
-  const float *k, *x, *q, *G, *dO, *d, *w, *dw, *Pp;  // k, x, q: column output; dO, d (= q + o), Pp: row output
+  const float *k, *x, *q, *G, *dO, *o, *w, *dw, *Pp;  // k, x, q: column output; dO, o, Pp: row output
   const __bf16 *dOb, *ub, *kb;  // column output: dO; row output: u, k (k = u^, x = gx u^, q = k^)
   const Tok* tok;
   const xs_t* Xslots;
@@ -1615,7 +1619,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
   const float *Yk = (COL ? p.q : p.dO) + tb * kw, *Gc = p.G + tb * kw;  // [32][kw]
   const float *dwc = p.dw + tb * vw, *wc = p.w + tb * vw;
   const float *kpc = COL ? p.k + tb * kw : nullptr, *xpc = COL ? p.x + tb * kw : nullptr,
-              *dpc = COL ? nullptr : p.d + tb * kw;
+              *opc = COL ? nullptr : p.o + tb * kw;
   const __bf16 *ubc = COL ? nullptr : p.ub + tb * kw, *kbc = COL ? nullptr : p.kb + tb * kw;
   const Tok* tokc = COL ? nullptr : p.tok + tb;
   {
@@ -1750,7 +1754,7 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
       }
       yr[q][t2] = ldq(Yk + o);
       G[q][t2] = ldq(Gc + o);
-      if constexpr (!COL) orw[q][t2] = ldq(dpc + o);
+      if constexpr (!COL) orw[q][t2] = ldq(opc + o);
     }
   }
   // rowsum(X_C (.) lam): the four lane groups' partials of each state row
@@ -1890,8 +1894,6 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
         gu[q][t2] = ldq(p.duh + tb * kw + o);
         gk[q][t2] = ldq(p.dkh + tb * kw + o);
         kn[t2] = scaled(ldq(kbc + o), tk[t2].rk);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) orw[q][t2].v[e] -= kn[t2].v[e];  // the readout o = d - q
         dv[t2] = ldq(dwc + o);
         dgo[q][t2] = ldq(p.dgS + tb * kw + o);
         const __bf16* hr = wrow(p.in.h, hb, min(ch * WBT + t2 * 16 + m, T - 1), hh);
@@ -2301,7 +2303,7 @@ struct WideFwd {
   float* G;
   __bf16 *ub, *kb, *qb, *hb;
   Tok* tok;
-  float *delta, *d, *e, *chi, *wS;
+  float *delta, *oC, *d, *e, *chi, *wS;
   float *AC, *AS, *PS;
   xs_t *XC, *XS;
   _Float16 *Wneg, *Kt;
@@ -2319,7 +2321,7 @@ WideFwd carve_wide_fwd(void* saved, void* scratch, const WideDims& d, size_t* sa
   w.G = c.take(pk);
   w.ub = c.take<__bf16>(pk); w.kb = c.take<__bf16>(pk); w.qb = c.take<__bf16>(pk);
   w.tok = c.take<Tok>(tok);
-  w.delta = c.take(pk); w.d = c.take(pk); w.e = c.take(pk);
+  w.delta = c.take(pk); w.oC = c.take(pk); w.d = c.take(pk); w.e = c.take(pk);
   w.chi = c.take(pk); w.wS = c.take(pv);
   w.AC = c.take(mat); w.AS = c.take(mat); w.PS = c.take(mat);
   w.XC = c.take<xs_t>((size_t)d.n * (d.NT + 1) * d.KP * d.KP);
@@ -2402,7 +2404,7 @@ size_t wide_bwd_workspace_bytes(int B, int T, int H, int r, int V) {
 }
 
 int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void* saved,
-                    void* scratch, hipStream_t st) {
+                    void* scratch, bool keep, hipStream_t st) {
   const WideDims d = wide_dims(in->B, in->T, in->H, in->r, in->V);
   const WideFwd w = carve_wide_fwd(saved, scratch, d, nullptr, nullptr);
 
@@ -2426,7 +2428,7 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
   OutParams orow{};
   orow.NT = d.NT; orow.Tp = d.Tp; orow.kw = d.KP; orow.vw = d.KP;
   orow.slots = w.XC; orow.w = w.delta; orow.ub = w.ub; orow.kb = w.kb; orow.tok = w.tok;
-  orow.G = w.G; orow.d = w.d;
+  orow.G = w.G; orow.o = keep ? w.oC : nullptr; orow.d = w.d;
   SD_SMEM_ONCE(k_w_out_c, (int)out_c_smem());
   SD_LAUNCH("k_w_out_c", k_w_out_c, dim3(d.NT, d.n), dim3(PT), out_c_smem(), st, orow);
 
@@ -2520,7 +2522,7 @@ int launch_wide_bwd(const sd_inputs* in, const void* fws, void* bws, const void*
   launch_wstate("w_state_c_bwd", rc, d.n, st);
   GradParams gc{};
   gc.NT = d.NT; gc.Tp = d.Tp; gc.kw = d.KP; gc.vw = d.KP;
-  gc.ub = f.ub; gc.kb = f.kb; gc.tok = f.tok; gc.G = f.G; gc.dO = w.dd; gc.d = f.d;
+  gc.ub = f.ub; gc.kb = f.kb; gc.tok = f.tok; gc.G = f.G; gc.dO = w.dd; gc.o = f.oC;
   gc.w = f.delta; gc.dw = w.dwC; gc.Xslots = f.XC; gc.Lslots = w.LC; gc.Pp = w.Pp;
   gc.in = *in; gc.duh = w.duh; gc.dkh = w.dkh; gc.dgS = w.dgS;
   gc.du = (__bf16*)du; gc.dh = (__bf16*)dh; gc.dkey = (__bf16*)dk;

@@ -162,3 +162,31 @@ def test_wide_larger_forward_matches_fp64_token_loop():
     errs = [rel(out.float(), eo), rel(st.predictor, eC), rel(st.S, eS)]
     print("[wide B2 T1024 H4 r256] " + " ".join(f"{e:.1e}" for e in errs), flush=True)
     assert errs[0] < 5e-3 and errs[1] < 1e-3 and errs[2] < 1e-3
+
+
+def test_wide_decay_gradient_of_a_readout_far_below_the_key():
+    """The predictor's readout o enters d log_decay by itself, not as what is left
+    of d = k^ + o: with one-hot operands every FP32 operation is exact, o = 2^-30
+    beside k^ = 1, and the log-decay's only nonzero gradient is o (FP64 oracle).
+    A readout taken back from the rounded sum would be 0."""
+    r, V, a, c, tiny = 160, 32, 3, 7, 2.0 ** -30
+    zeros = lambda *s: torch.zeros(*s)
+    u, h, q = (zeros(1, 2, 1, r) for _ in range(3))
+    k, er, v, wr = (zeros(1, 2, 1, 1, w) for w in (r, r, V, V))
+    u[0, 0, 0, a] = u[0, 1, 0, c] = h[0, 0, 0, a] = 1
+    q[..., a] = k[..., a] = 1
+    v[0, 1, 0, 0, 0] = 2
+    args = [x.to(torch.bfloat16).cuda().requires_grad_() for x in (u, h, q, k, v)]
+    args += [zeros(1, 2, 1, r).cuda().requires_grad_()]
+    args += [x.to(torch.bfloat16).cuda().requires_grad_() for x in (er, wr)]
+    args += [torch.full((1, 2, 1), tiny, device="cuda", requires_grad=True)]
+    out, _ = _native()(*args)
+    dout = torch.zeros_like(out)
+    dout[0, 1, 0, 0] = 1
+    grad = torch.autograd.grad(out, args, dout)[5]
+    ref = [x.detach().double().cpu().requires_grad_() for x in args]
+    eo, _ = solvedelta_oracle_raw(*ref)
+    eg = torch.autograd.grad(eo, ref, dout.double().cpu())[5]
+    assert eg[0, 1, 0, a] == tiny and eg.count_nonzero() == 1
+    # exact products and sums; a few ulp for the rsqrt and exp of exact arguments
+    assert (grad.double().cpu() - eg).abs().max().item() <= 2.0 ** -20 * tiny
