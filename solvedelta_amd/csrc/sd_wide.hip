@@ -1726,7 +1726,10 @@ __global__ __launch_bounds__(GT, 2) void k_w_grad(GradParams p) {
     for (int e = 0; e < 4; ++e) {
       const int i = bi * 16 + 4 * g + e, j = bj * 16 + m;
       float v = am[e];
-      if (!COL && w >= 3) v *= tokc[i].rk;
+      if (!COL && w >= 3) {  // (a zero inverse norm: the raw row's products may have overflowed)
+        const float rk = tokc[i].rk;
+        v = rk != 0.f ? v * rk : 0.f;
+      }
       M[i * AS + j] = (w < 3 ? j < i : j <= i) ? v : 0.f;
     }
   }

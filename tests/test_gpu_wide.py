@@ -190,3 +190,20 @@ def test_wide_decay_gradient_of_a_readout_far_below_the_key():
     assert eg[0, 1, 0, a] == tiny and eg.count_nonzero() == 1
     # exact products and sums; a few ulp for the rsqrt and exp of exact arguments
     assert (grad.double().cpu() - eg).abs().max().item() <= 2.0 ** -20 * tiny
+
+
+def test_wide_rows_whose_norm_overflows_read_as_zero():
+    """Keys of 1e38: the FP32 sum of squares overflows, the inverse norm is 0 and
+    the row acts as a zero row; no gradient turns NaN through raw k times 0."""
+    def run(fill):
+        args = make_inputs(1, 70, 2, 160, 64, seed=81)
+        args[3][:, 40] = fill
+        for x in args:
+            x.requires_grad_()
+        out, st = _native()(*args, return_final_state=True)
+        return [out, st.predictor, st.S, *torch.autograd.grad(out, args, torch.ones_like(out))]
+    for i, (a, b) in enumerate(zip(run(1e38), run(0.0))):
+        a, b = a.detach(), b.detach()
+        if i == 3 + 3:  # the row's own key gradient goes by the inverse norm
+            a, b = (torch.cat([x[:, :40], x[:, 41:]], dim=1) for x in (a, b))
+        assert torch.isfinite(a).all() and torch.equal(a, b), i
