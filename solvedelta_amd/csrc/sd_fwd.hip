@@ -159,7 +159,9 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int ii = I * BS + out_row(e), jj = J * BS + out_col();
-      s.M[ii * LS + jj] = jj < ii ? s.gam[ii] * s.xm[ii] * s.ru[ii] * acc[e] : 0.f;
+      // (a zero inverse norm: the raw row's products may have overflowed)
+      const float ru = s.ru[ii];
+      s.M[ii * LS + jj] = jj < ii && ru != 0.f ? s.gam[ii] * s.xm[ii] * ru * acc[e] : 0.f;
     }
   };
   {

@@ -172,3 +172,20 @@ def test_forward_without_gradients_equals_forward_with(B, T, H, r, V, decay, mas
     out3, _ = fn(*[a.detach() for a in args], *masks, initial_state=state)
     assert torch.equal(out, out2) and torch.equal(out, out3)
     assert torch.equal(st.predictor, st2.predictor) and torch.equal(st.S, st2.S)
+
+
+@pytest.mark.parametrize("T,token", [(16, 3), (70, 40), (70, 69)])
+def test_predictor_rows_whose_norm_overflows_read_as_zero(T, token):
+    """u of 3.3e38 along the other tokens' signs: the FP32 sum of squares overflows,
+    the inverse norm is 0 and the token's u acts as a zero row, wherever it lies in
+    the chunk's Gram blocks; no product of the raw values turns it into NaN."""
+    outs = []
+    for fill in (3.3e38, 0.0):
+        args = make_inputs(1, T, 2, 128, 64, seed=83, decay="small")
+        args[0].copy_(args[0].abs())
+        args[0][:, token] = fill
+        with torch.no_grad():
+            out, st = _native()(*args, return_final_state=True)
+        outs.append((out, st.predictor, st.S))
+    for a, b in zip(*outs):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
