@@ -287,12 +287,13 @@ template <int VEC> struct FV { float v[VEC]; };
 
 template <int VEC>
 __global__ __launch_bounds__(NTHREADS) void k_gate_fwd(GateArgs a, float* __restrict__ out) {
-  const int Q = a.HR / VEC, idx = blockIdx.x * NTHREADS + threadIdx.x;
-  const int rg = idx / Q, c = (idx - rg * Q) * VEC, n0 = rg * GATE_FR;
-  if (n0 >= a.N) return;
+  const unsigned Q = a.HR / VEC, idx = blockIdx.x * NTHREADS + threadIdx.x, rg = idx / Q;
+  const unsigned N = a.N, n0 = rg * GATE_FR;
+  const int c = (idx - rg * Q) * VEC;
+  if (n0 >= N) return;
   BfV<VEC> x[GATE_FR];
 #pragma unroll
-  for (int j = 0; j < GATE_FR; ++j) x[j] = ldv<VEC>(a.raw + (long long)min(n0 + j, a.N - 1) * a.rs + c);
+  for (int j = 0; j < GATE_FR; ++j) x[j] = ldv<VEC>(a.raw + (long long)min(n0 + j, N - 1) * a.rs + c);
   float rate[VEC], b[VEC];
   gate_cols<VEC>(a, c, rate, b);
 #pragma unroll
@@ -305,7 +306,7 @@ __global__ __launch_bounds__(NTHREADS) void k_gate_fwd(GateArgs a, float* __rest
       const float t = v[k] + b[k];
       o.v[k] = -rate[k] * softplus_t(t, __expf(-fabsf(t)));
     }
-    if (n0 + j < a.N) *reinterpret_cast<FV<VEC>*>(out + (long long)(n0 + j) * a.HR + c) = o;
+    if (n0 + j < N) *reinterpret_cast<FV<VEC>*>(out + (long long)(n0 + j) * a.HR + c) = o;
   }
 }
 
@@ -315,14 +316,15 @@ template <int VEC>
 __global__ __launch_bounds__(NTHREADS) void k_gate_bwd(GateArgs a, const float* __restrict__ dout,
                                                        __bf16* __restrict__ draw,
                                                        float* __restrict__ part) {
-  const int Q = a.HR / VEC, idx = blockIdx.x * NTHREADS + threadIdx.x;
-  const int rg = idx / Q, c = (idx - rg * Q) * VEC, n0 = rg * GATE_TR;
-  if (n0 >= a.N) return;
+  const unsigned Q = a.HR / VEC, idx = blockIdx.x * NTHREADS + threadIdx.x, rg = idx / Q;
+  const unsigned N = a.N, n0 = rg * GATE_TR;
+  const int c = (idx - rg * Q) * VEC;
+  if (n0 >= N) return;
   BfV<VEC> x[GATE_TR];
   FV<VEC> g[GATE_TR];
 #pragma unroll
   for (int j = 0; j < GATE_TR; ++j) {
-    const long long n = min(n0 + j, a.N - 1);
+    const long long n = min(n0 + j, N - 1);
     x[j] = ldv<VEC>(a.raw + n * a.rs + c);
     g[j] = *reinterpret_cast<const FV<VEC>*>(dout + n * a.HR + c);
   }
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(NTHREADS) void k_gate_bwd(GateArgs a, const float* 
   FV<VEC> db = {}, dl = {};
 #pragma unroll
   for (int j = 0; j < GATE_TR; ++j) {
-    if (n0 + j >= a.N) break;
+    if (n0 + j >= N) break;
     float v[VEC], dx[VEC];
     x[j].get(v);
 #pragma unroll
@@ -518,11 +520,12 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsv_fwd(int N, int D, float eps, 
                                                        const __bf16* __restrict__ g, const float* __restrict__ w,
                                                        __bf16* __restrict__ y, float* __restrict__ rstd_out) {
   constexpr int G = NTHREADS / LPR;
-  const int c = (threadIdx.x % LPR) * 8, cc = c < D ? c : 0, n0 = blockIdx.x * G * RMSV_U + threadIdx.x / LPR;
+  const int c = (threadIdx.x % LPR) * 8, cc = c < D ? c : 0;
+  const unsigned n0 = blockIdx.x * G * RMSV_U + threadIdx.x / LPR;  // (rows past N may pass 2^31)
   BfV<8> xr[RMSV_U], gr[RMSV_U];
 #pragma unroll
   for (int u = 0; u < RMSV_U; ++u) {
-    const long long o = (long long)min(n0 + u * G, N - 1) * D + cc;
+    const long long o = (long long)min(n0 + u * G, (unsigned)N - 1) * D + cc;
     xr[u] = ldv<8>(x + o);
     gr[u] = ldv<8>(g + o);
   }
@@ -531,7 +534,7 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsv_fwd(int N, int D, float eps, 
   for (int e = 0; e < 8; ++e) wv[e] = w[cc + e];
 #pragma unroll
   for (int u = 0; u < RMSV_U; ++u) {
-    const int n = n0 + u * G;
+    const unsigned n = n0 + u * G;
     float xv[8], gv[8], o[8], ss = 0.f;
     xr[u].get(xv);
     gr[u].get(gv);
@@ -540,8 +543,8 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsv_fwd(int N, int D, float eps, 
     const float rs = rsqrtf(lanes_sum<LPR>(c < D ? ss : 0.f) / D + eps);
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = xv[e] * rs * wv[e] * sigm(gv[e]);
-    if (n < N && c < D) stv<8>(y + (long long)n * D + c, o);
-    if (rstd_out && n < N && c == 0) rstd_out[n] = rs;
+    if (n < (unsigned)N && c < D) stv<8>(y + (long long)n * D + c, o);
+    if (rstd_out && n < (unsigned)N && c == 0) rstd_out[n] = rs;
   }
 }
 
@@ -564,20 +567,20 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsv_bwd(int N, int D, float eps, 
     wv[e] = w[cc + e];
     acc[e] = 0.f;
   }
-  const int base = blockIdx.x * rows;
+  const unsigned base = blockIdx.x * rows;
   for (int r0 = gr_; r0 < rows; r0 += G * RMSV_U) {
     BfV<8> xr[RMSV_U], gr[RMSV_U], dr[RMSV_U];
 #pragma unroll
     for (int u = 0; u < RMSV_U; ++u) {
-      const long long o = (long long)min(base + r0 + u * G, N - 1) * D + cc;
+      const long long o = (long long)min(base + r0 + u * G, (unsigned)N - 1) * D + cc;
       xr[u] = ldv<8>(x + o);
       gr[u] = ldv<8>(g + o);
       dr[u] = ldv<8>(dy + o);
     }
 #pragma unroll
     for (int u = 0; u < RMSV_U; ++u) {
-      const int n = base + r0 + u * G;
-      const bool ok = in && n < N;
+      const unsigned n = base + r0 + u * G;
+      const bool ok = in && n < (unsigned)N;
       float xh[8], gv[8], dv[8], sg[8], gy[8], ss = 0.f, dot = 0.f;
       xr[u].get(xh);
       gr[u].get(gv);
@@ -943,6 +946,13 @@ static bool conv_pairs(const ConvArgs& a, const void* p, const void* q) {
   return a.D % 2 == 0 && a.sb % 2 == 0 && a.st % 2 == 0 && bits % 4 == 0;
 }
 
+// Workgroups of a launch of one thread per (group of rows, column), whose index the
+// kernels hold in 32 unsigned bits; 0 where it would not fit.
+static int gate_blocks(int N, int rows, int cols) {
+  const long long t = (long long)cdiv(N, rows) * cols;
+  return t > 0xffffffffLL - NTHREADS ? 0 : cdiv(t, NTHREADS);
+}
+
 // Four columns per thread where every row of the bf16 operands starts on an
 // 8-byte and of the FP32 operand on a 16-byte boundary.
 static bool gate_quads(const GateArgs& a, const void* bf, const void* f32) {
@@ -1044,16 +1054,16 @@ size_t sd_kda_gate_workspace_bytes(int N, int H, int r) {
 
 int sd_kda_gate_fwd(int N, int H, int r, const void* raw, int64_t raw_row_stride,
                     const float* log_rate, const float* bias, float* out, void* stream) {
-  if (N <= 0 || H <= 0 || r <= 0) return SD_ERR_SHAPE;
+  if (N <= 0 || H <= 0 || r <= 0 || (long long)H * r > 0x7fffffff) return SD_ERR_SHAPE;
   if (!raw || !log_rate || !bias || !out) return SD_ERR_ARG;
   const GateArgs a{N, H, r, H * r, (const __bf16*)raw, raw_row_stride, log_rate, bias};
-  const int groups = cdiv(N, GATE_FR);
-  if (gate_quads(a, nullptr, out))
-    SD_LAUNCH("k_gate_fwd", k_gate_fwd<4>, dim3(cdiv((long long)groups * (H * r / 4), NTHREADS)), dim3(NTHREADS),
-              0, (hipStream_t)stream, a, out);
+  const bool v4 = gate_quads(a, nullptr, out);
+  const int blocks = gate_blocks(N, GATE_FR, v4 ? a.HR / 4 : a.HR);
+  if (!blocks) return SD_ERR_SHAPE;
+  if (v4)
+    SD_LAUNCH("k_gate_fwd", k_gate_fwd<4>, dim3(blocks), dim3(NTHREADS), 0, (hipStream_t)stream, a, out);
   else
-    SD_LAUNCH("k_gate_fwd", k_gate_fwd<1>, dim3(cdiv((long long)groups * H * r, NTHREADS)), dim3(NTHREADS),
-              0, (hipStream_t)stream, a, out);
+    SD_LAUNCH("k_gate_fwd", k_gate_fwd<1>, dim3(blocks), dim3(NTHREADS), 0, (hipStream_t)stream, a, out);
   return hipGetLastError() == hipSuccess ? SD_OK : SD_ERR_LAUNCH;
 }
 
@@ -1061,19 +1071,22 @@ int sd_kda_gate_bwd(int N, int H, int r, const void* raw, int64_t raw_row_stride
                     const float* log_rate, const float* bias, const float* dout, void* draw,
                     float* dlog_rate, float* dbias, void* workspace, size_t workspace_bytes,
                     void* stream) {
-  if (N <= 0 || H <= 0 || r <= 0) return SD_ERR_SHAPE;
+  if (N <= 0 || H <= 0 || r <= 0 || (long long)H * r > 0x3fffffff) return SD_ERR_SHAPE;  // (2 H r columns of sums)
   if (!raw || !log_rate || !bias || !dout || !draw || !dlog_rate || !dbias || !workspace)
     return SD_ERR_ARG;
   if (workspace_bytes < sd_kda_gate_workspace_bytes(N, H, r)) return SD_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   const int np = cdiv(N, GATE_TR);
   const GateArgs a{N, H, r, H * r, (const __bf16*)raw, raw_row_stride, log_rate, bias};
-  if (gate_quads(a, draw, dout) && ((uintptr_t)workspace & 15) == 0)
-    SD_LAUNCH("k_gate_bwd", k_gate_bwd<4>, dim3(cdiv((long long)np * (H * r / 4), NTHREADS)), dim3(NTHREADS), 0,
-              st, a, dout, (__bf16*)draw, (float*)workspace);
+  const bool v4 = gate_quads(a, draw, dout) && ((uintptr_t)workspace & 15) == 0;
+  const int blocks = gate_blocks(N, GATE_TR, v4 ? a.HR / 4 : a.HR);
+  if (!blocks) return SD_ERR_SHAPE;
+  if (v4)
+    SD_LAUNCH("k_gate_bwd", k_gate_bwd<4>, dim3(blocks), dim3(NTHREADS), 0, st, a, dout, (__bf16*)draw,
+              (float*)workspace);
   else
-    SD_LAUNCH("k_gate_bwd", k_gate_bwd<1>, dim3(cdiv((long long)np * H * r, NTHREADS)), dim3(NTHREADS), 0, st, a,
-              dout, (__bf16*)draw, (float*)workspace);
+    SD_LAUNCH("k_gate_bwd", k_gate_bwd<1>, dim3(blocks), dim3(NTHREADS), 0, st, a, dout, (__bf16*)draw,
+              (float*)workspace);
   // column sums over the partial rows spread over many workgroups (a per-head
   // walk over every partial row kept only H workgroups busy), then per head
   float* colsum = (float*)workspace + (size_t)np * 2 * H * r;

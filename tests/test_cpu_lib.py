@@ -72,6 +72,22 @@ def test_workspace_queries_and_argument_rejection():
     assert lib.sd_fwd(ctypes.byref(ins), None, None, None, None, 0, None) == _lib.SD_ERR_ARG
 
 
+@pytest.mark.parametrize("N,H,r", [
+    (2**31 - 1, 64, 33),  # 2^28 groups of 8 rows, 528 threads each
+    (2**31 - 1, 1, 129),  # one column per thread
+    (1, 2**16, 2**16),    # H r past 32 bits
+])
+def test_decay_gate_refuses_calls_past_its_index(N, H, r):
+    """The gate's kernels index (row group, columns) with 32 unsigned bits: a call
+    with more threads is refused on the host (the addresses are never read)."""
+    from solvedelta_amd import _lib
+    lib = _lib.load()
+    p = [ctypes.c_void_p(64 * (i + 1)) for i in range(8)]
+    assert lib.sd_kda_gate_fwd(N, H, r, p[0], H * r, p[1], p[2], p[3], None) == _lib.SD_ERR_SHAPE
+    assert lib.sd_kda_gate_bwd(N, H, r, p[0], H * r, p[1], p[2], p[3], p[4], p[5], p[6], p[7],
+                               2**62, None) == _lib.SD_ERR_SHAPE
+
+
 def test_operator_rejects_like_the_reference():
     from solvedelta_amd import solvedelta_native
     x = torch.zeros(1, 4, 1, 8, dtype=torch.bfloat16)
