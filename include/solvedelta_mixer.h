@@ -53,6 +53,9 @@ int sd_conv4_silu_masked_fwd(int B, int T, int D, const void *x, int64_t x_sb, i
                              const float *w, const void *init, const uint8_t *valid,
                              const uint8_t *reset, int64_t m_sb, int64_t m_st, void *y,
                              void *final_state, void *stream);
+/* The backward's workspace: sd_conv4_masked_bwd_workspace_bytes for rows of T
+ * tokens; sd_conv4_masked_workspace_bytes is its bound over every T. */
+size_t sd_conv4_masked_bwd_workspace_bytes(int B, int T, int D);
 size_t sd_conv4_masked_workspace_bytes(int B, int D);
 int sd_conv4_silu_masked_bwd(int B, int T, int D, const void *x, int64_t x_sb, int64_t x_st,
                              const float *w, const void *init, const uint8_t *valid,

@@ -946,6 +946,12 @@ static bool conv_pairs(const ConvArgs& a, const void* p, const void* q) {
   return a.D % 2 == 0 && a.sb % 2 == 0 && a.st % 2 == 0 && bits % 4 == 0;
 }
 
+// Backward workgroups per batch row (and dw partial rows) of a row of T tokens.
+static int mconv_parts(int T) {
+  const int nch = cdiv(T, MCONV_TC);
+  return nch < MCONV_PARTS ? nch : MCONV_PARTS;
+}
+
 // Workgroups of a launch of one thread per (group of rows, column), whose index the
 // kernels hold in 32 unsigned bits; 0 where it would not fit.
 static int gate_blocks(int N, int rows, int cols) {
@@ -1002,6 +1008,11 @@ size_t sd_conv4_masked_workspace_bytes(int B, int D) {
   return (size_t)B * MCONV_PARTS * D * 4 * sizeof(float);
 }
 
+size_t sd_conv4_masked_bwd_workspace_bytes(int B, int T, int D) {
+  if (B <= 0 || T <= 0 || D <= 0) return 0;
+  return (size_t)B * mconv_parts(T) * D * 4 * sizeof(float);
+}
+
 int sd_conv4_silu_masked_fwd(int B, int T, int D, const void* x, int64_t x_sb, int64_t x_st,
                              const float* w, const void* init, const uint8_t* valid,
                              const uint8_t* reset, int64_t m_sb, int64_t m_st, void* y,
@@ -1029,12 +1040,12 @@ int sd_conv4_silu_masked_bwd(int B, int T, int D, const void* x, int64_t x_sb, i
                              void* workspace, size_t workspace_bytes, void* stream) {
   if (B <= 0 || T <= 0 || D <= 0) return SD_ERR_SHAPE;
   if (!x || !w || !dy || !dx || !dw || !workspace) return SD_ERR_ARG;
-  if (workspace_bytes < sd_conv4_masked_workspace_bytes(B, D)) return SD_ERR_WORKSPACE;
+  if (workspace_bytes < sd_conv4_masked_bwd_workspace_bytes(B, T, D)) return SD_ERR_WORKSPACE;
   ConvArgs a{B, T, D, (const __bf16*)x, x_sb, x_st, w, (const __bf16*)init};
   ConvMask m{valid, reset, m_sb, m_st};
   hipStream_t st = (hipStream_t)stream;
   const bool v2 = conv_pairs(a, dy, dx);
-  const int nch = cdiv(T, MCONV_TC), parts = nch < MCONV_PARTS ? nch : MCONV_PARTS;
+  const int parts = mconv_parts(T);
   const dim3 grid(cdiv(D, NTHREADS * (v2 ? 2 : 1)), parts, B);
   if (v2)
     SD_LAUNCH("k_conv_masked_bwd", k_conv_masked_bwd<2>, grid, dim3(NTHREADS), 0, st, a, m,

@@ -191,7 +191,7 @@ class _Conv4SiluMaskedFn(torch.autograd.Function):
         dx = torch.empty(B, T, D, dtype=torch.bfloat16, device=x.device)
         dw = torch.empty(D, 4, dtype=torch.float32, device=x.device)
         dinit = torch.empty(B, D, 3, dtype=torch.float32, device=x.device) if init is not None else None
-        nb = lib.sd_conv4_masked_workspace_bytes(B, D)
+        nb = lib.sd_conv4_masked_bwd_workspace_bytes(B, T, D)
         ws = torch.empty(nb, dtype=torch.uint8, device=x.device)
         rc = lib.sd_conv4_silu_masked_bwd(B, T, D, x.data_ptr(), x.stride(0), x.stride(1),
                                           w32.data_ptr(), _ptr(init), valid.data_ptr(),

@@ -88,6 +88,20 @@ def test_decay_gate_refuses_calls_past_its_index(N, H, r):
                                2**62, None) == _lib.SD_ERR_SHAPE
 
 
+@pytest.mark.parametrize("T,parts", [(1, 1), (32, 1), (33, 2), (2016, 63), (2048, 64), (100000, 64)])
+def test_masked_conv_workspace_goes_by_the_row_length(T, parts):
+    """One partial row of [D][4] sums per 32-token chunk, at most 64 per batch row."""
+    from solvedelta_amd import _lib
+    lib = _lib.load()
+    B, D = 3, 40
+    need = lib.sd_conv4_masked_bwd_workspace_bytes(B, T, D)
+    assert need == B * parts * D * 16 <= lib.sd_conv4_masked_workspace_bytes(B, D)
+    p = [ctypes.c_void_p(64 * (i + 1)) for i in range(8)]
+    rc = lib.sd_conv4_silu_masked_bwd(B, T, D, p[0], T * D, D, p[1], None, None, None, T, 1, p[2],
+                                      None, p[3], p[4], None, p[5], need - 1, None)
+    assert rc == _lib.SD_ERR_WORKSPACE
+
+
 def test_operator_rejects_like_the_reference():
     from solvedelta_amd import solvedelta_native
     x = torch.zeros(1, 4, 1, 8, dtype=torch.bfloat16)
