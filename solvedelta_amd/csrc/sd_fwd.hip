@@ -60,6 +60,46 @@ struct PrepCSmem {
   float cap[NB][KD];  // largest exponent of y: TAU, or -inf (y = 0) on a wild coordinate
 };
 
+// W = A diag(gamma) (u e^{Gexcl} masked on fresh tokens) and U = A diag(gamma) h
+// from A in M: wave w's columns 16 w .. 16 w + 15 of both right sides come as B
+// operands (W's split, h exact in bf16).  The products are taken transposed, so
+// that a lane's four results are one token's neighbours.
+__device__ __forceinline__ void prep_c_products(const FwdParams& p, const float* M, const float* gam,
+                                                const bf16x8 (&bh)[2], const bf16x8 (&bl)[2],
+                                                const bf16x8 (&hb)[2], long long rowbase) {
+  const int w = wave_id(), l = lane_id(), m = l & 15, kq = (l >> 4) * 8;
+#pragma unroll
+  for (int I = 0; I < NB; ++I) {
+    const int K = I < 2 ? 32 : 64;
+    f4 aw = zero4(), au = zero4();
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      if (ks * 32 >= K) break;
+      bf16x8 ah, al;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = ks * 32 + kq + e;
+        __bf16 hi, lo;
+        split_bf(M[(I * BS + m) * LS + k] * gam[k], hi, lo);
+        ah[e] = hi;
+        al[e] = lo;
+      }
+      aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[ks], al, aw, 0, 0, 0);
+      au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hb[ks], al, au, 0, 0, 0);
+      aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[ks], ah, aw, 0, 0, 0);
+      aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[ks], ah, aw, 0, 0, 0);
+      au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hb[ks], ah, au, 0, 0, 0);
+    }
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    const int row = I * BS + m, oc = w * 16 + (l >> 4) * 4;
+    h4 wv;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wv[e] = (_Float16)(-aw[e]);
+    *reinterpret_cast<h4*>(&p.Wc[rowbase * KD + frag_off(row, oc, KD)]) = wv;
+    *reinterpret_cast<f4*>(&p.Uc[(rowbase + row) * KD + oc]) = au;
+  }
+}
+
 // FL: the call has token flags (sd_inputs.fresh).  KEEP: a backward will read
 // what the forward alone does not (sd_fwd_infer runs without)
 //
@@ -74,9 +114,7 @@ struct PrepCSmem {
 // r = V = 128 (151 MB moved, 32 us at a large copy's rate), 97 -> 76 us at
 // 2 x 3001, 16 heads, without (I+L)^-1.  The opening loads come in bursts (9 us of a
 // workgroup's 20); h gathered in operand layout from memory instead cost 7 us
-// of latency before the inverse (67 / 90 us).  With 128 chunks, one for every
-// second CU, the chain itself is the time: 18.7 us, 20.3 with the ten Gram pairs
-// in two turns of the eight waves.
+// of latency before the inverse (67 / 90 us).
 template <bool FL, bool KEEP>
 __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -227,47 +265,109 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
       const int i = idx / BT, j = idx % BT;
       p.Ac[((long long)n * p.NT + ch) * BT * BT + idx] = j > i ? 0.f : s.M[i * LS + j];
     }
-  // W = A diag(gamma) (u e^{Gexcl} masked on fresh tokens),  U = A diag(gamma) h:
-  // wave w holds columns 16w..16w+15 of both right sides, and the product is
-  // taken transposed, so that a lane's four results are one token's neighbours
-  const long long rowbase = (long long)n * p.Tp + t0;
   {
     bf16x8 hb[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
       for (int e = 0; e < 8; ++e) hb[ks][e] = s.Ub[ks * 32 + kq + e][c];
+    prep_c_products(p, s.M, s.gam, bh, bl, hb, (long long)n * p.Tp + t0);
+  }
+}
+
+// The same where every chunk has a CU to itself (at most kFewChunks of them): two
+// workgroups never share a CU, so LDS is not short and the chain of phases is the
+// time.  The Gram's Y side is transformed and split once into LDS instead of by
+// each block pair's wave, u and h lie side by side, and the inverse has its own
+// scratch (153 KB).  r = V = 128, k_prep_c / this kernel, us: 15.4 / 13.7 at one
+// chunk, 17.8-18.3 / 16.3-16.7 at 64, 20.7-21.2 / 17.4-17.8 at 128, 21.3 / 19.7-20.2
+// at 256; from one more chunk than CUs on the other way round, 26.1 / 29.2-29.7 at 288.
+struct PrepCFewSmem {
+  ChunkDecay cd;
+  float M[BT * LS];
+  float tmp[BT * LS];
+  float Uh[BT][GS];   // normalised u
+  __bf16 Hh[BT][PS];  // h (raw bf16, exact)
+  float gam[BT];
+  float xm[BT];       // 1, or 0 on fresh tokens (no erase read)
+  LPanel Yt;          // the L Gram's Y side (u), transformed and split once
+};
+constexpr int kFewChunks = 256;  // one per CU
+
+template <bool FL, bool KEEP>
+__global__ __launch_bounds__(CT) void k_prep_c_few(FwdParams p) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  PrepCFewSmem& s = *reinterpret_cast<PrepCFewSmem*>(smem_raw);
+  const int n = blockIdx.x, ch = gridDim.y - 1 - blockIdx.y;  // as k_prep_c
+  const int b = n / p.H, hh = n % p.H, t0 = ch * BT;
+  const int T = p.T, r = p.r;
+  const sd_inputs& in = p.in;
+  const float* g = (const float*)in.log_decay.data + (long long)b * in.log_decay.sb +
+                   (long long)hh * in.log_decay.sh;
+  const int w = wave_id(), l = lane_id(), m = l & 15, kq = (l >> 4) * 8;
+  {
+    // every load of the opening phase first, as in k_prep_c
+    float xdec[BS];
+    decay_load(g, in.log_decay.st, t0, T, r, xdec, FL ? tok_flag_row(in, b) : nullptr, tok_flag_st(in));
+    float ux[2][RQ], hx[2][RQ];
 #pragma unroll
-    for (int I = 0; I < NB; ++I) {
-      const int K = I < 2 ? 32 : 64;
-      f4 aw = zero4(), au = zero4();
+    for (int g = 0; g < 2; ++g) {
+      const int t = t0 + row16(w, g);
+      load_row16(in.u, b, t, hh, T, r, ux[g]);
+      load_row16(in.h, b, t, hh, T, r, hx[g]);
+    }
+    if (threadIdx.x < BT) {  // branch-free: clamped token, then select
+      const int t = t0 + threadIdx.x;
+      const float gv = gamma_at(in.gamma, b, t < T ? t : T - 1, hh);
+      const unsigned f = tok_flags(in, b, t < T ? t : T - 1);
+      s.gam[threadIdx.x] = keep_if(t < T, gv) * operand_keep(f);  // 0 on invalid tokens
+      s.xm[threadIdx.x] = erase_keep_f(f);
+    }
+    decay_build(s.cd, xdec);
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        if (ks * 32 >= K) break;
-        bf16x8 ah, al;
+    for (int g = 0; g < 2; ++g) {
+      const int i = row16(w, g);
+      l2norm16(ux[g]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int k = ks * 32 + kq + e;
-          __bf16 hi, lo;
-          split_bf(s.M[(I * BS + m) * LS + k] * s.gam[k], hi, lo);
-          ah[e] = hi;
-          al[e] = lo;
-        }
-        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[ks], al, aw, 0, 0, 0);
-        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hb[ks], al, au, 0, 0, 0);
-        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[ks], ah, aw, 0, 0, 0);
-        aw = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[ks], ah, aw, 0, 0, 0);
-        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hb[ks], ah, au, 0, 0, 0);
+      for (int q = 0; q < RQ; ++q) {
+        s.Uh[i][m + 16 * q] = ux[g][q];
+        s.Hh[i][m + 16 * q] = f2bf(hx[g][q]);
       }
-      typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-      const int row = I * BS + m, oc = w * 16 + (l >> 4) * 4;
-      h4 wv;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) wv[e] = (_Float16)(-aw[e]);
-      *reinterpret_cast<h4*>(&p.Wc[rowbase * KD + frag_off(row, oc, KD)]) = wv;
-      *reinterpret_cast<f4*>(&p.Uc[(rowbase + row) * KD + oc]) = au;
     }
   }
+  __syncthreads();
+  const ChunkDecay& cd = s.cd;
+  // L_ij = gamma_i sum_c u_ic u_jc exp(G_{i-1,c} - G_jc), j < i
+  stage_ytilde(s.Yt, cd, [&](int j, int c) { return s.Uh[j][c]; });
+  decayed_gram_yt<true>(
+      cd, [&](int i, int c) { return s.gam[i] * s.xm[i] * s.Uh[i][c]; }, s.Yt,
+      [&](int j, int c) { return s.Uh[j][c]; }, true, s.M);
+  unit_lower_inverse(s.M, s.tmp);
+  const long long cbase = ((long long)n * p.NT + ch);
+  if constexpr (KEEP)
+    for (int idx = threadIdx.x; idx < BT * BT; idx += CT)
+      p.Ac[cbase * BT * BT + idx] = s.M[(idx / BT) * LS + idx % BT];
+  {
+    // B operands, the same for every row block: formed and split once
+    bf16x8 bh[2], bl[2], hb[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = ks * 32 + kq + e, c = w * 16 + m;
+        __bf16 hi, lo;
+        split_bf(s.xm[k] * s.Uh[k][c] * __expf(gx_excl(cd, k, c)), hi, lo);
+        bh[ks][e] = hi;
+        bl[ks][e] = lo;
+        hb[ks][e] = s.Hh[k][c];  // h is the raw bf16 input: exact
+      }
+    prep_c_products(p, s.M, s.gam, bh, bl, hb, (long long)n * p.Tp + t0);
+  }
+  // decayed keys (transposed per chunk) and chunk decay
+  store_frag_panel1<KD, BT>(p.Kc, cbase * KD * BT, [&](int c, int i) {
+    return s.Uh[i][c] * __expf(cd.G[BT - 1][c] - cd.G[i][c]);
+  });
+  if (threadIdx.x < KD) p.Gam[cbase * KD + threadIdx.x] = __expf(cd.G[BT - 1][threadIdx.x]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1149,6 +1249,11 @@ size_t prep_s_smem() { return sizeof(PrepSSmem); }
 
 template <bool FL, bool KEEP>
 static void run_prep_c(const FwdParams& fp, int n, hipStream_t st) {
+  if ((long long)n * fp.NT <= kFewChunks) {
+    SD_SMEM_ONCE((k_prep_c_few<FL, KEEP>), (int)sizeof(PrepCFewSmem));
+    SD_LAUNCH("k_prep_c", (k_prep_c_few<FL, KEEP>), dim3(n, fp.NT), dim3(CT), sizeof(PrepCFewSmem), st, fp);
+    return;
+  }
   SD_SMEM_ONCE((k_prep_c<FL, KEEP>), (int)prep_c_smem());
   SD_LAUNCH("k_prep_c", (k_prep_c<FL, KEEP>), dim3(n, fp.NT), dim3(CT), prep_c_smem(), st, fp);
 }

@@ -174,14 +174,15 @@ def test_forward_without_gradients_equals_forward_with(B, T, H, r, V, decay, mas
     assert torch.equal(st.predictor, st2.predictor) and torch.equal(st.S, st2.S)
 
 
+@pytest.mark.parametrize("H", [2, 140])  # k_prep_c's forms for few and for many chunks
 @pytest.mark.parametrize("T,token", [(16, 3), (70, 40), (70, 69)])
-def test_predictor_rows_whose_norm_overflows_read_as_zero(T, token):
+def test_predictor_rows_whose_norm_overflows_read_as_zero(T, token, H):
     """u of 3.3e38 along the other tokens' signs: the FP32 sum of squares overflows,
     the inverse norm is 0 and the token's u acts as a zero row, wherever it lies in
     the chunk's Gram blocks; no product of the raw values turns it into NaN."""
     outs = []
     for fill in (3.3e38, 0.0):
-        args = make_inputs(1, T, 2, 128, 64, seed=83, decay="small")
+        args = make_inputs(4 if T < 64 else 2, T, H, 128, 64, seed=83, decay="small")
         args[0].copy_(args[0].abs())
         args[0][:, token] = fill
         with torch.no_grad():
@@ -189,3 +190,25 @@ def test_predictor_rows_whose_norm_overflows_read_as_zero(T, token):
         outs.append((out, st.predictor, st.S))
     for a, b in zip(*outs):
         assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H", [64, 65])  # 256 chunks, one per CU; and the first count above
+@pytest.mark.parametrize("decay,masked", [("softplus", False), ("mixed", False), ("extreme", False),
+                                          ("mixed", True)])
+def test_forward_on_both_sides_of_one_chunk_per_cu(H, decay, masked):
+    """The two forms of the predictor's chunk preparation at their dividing line,
+    a ragged last chunk and wild coordinates among them."""
+    from solvedelta_amd import solvedelta_masked_native
+    B, T, r, V = 2, 81, 24, 16
+    args = make_inputs(B, T, H, r, V, seed=91, decay=decay)
+    state = make_state(B, H, r, V, seed=92)
+    masks, kw = (), {}
+    if masked:
+        g = torch.Generator().manual_seed(93)
+        masks = (torch.rand(B, T, generator=g) >= 0.2, torch.rand(B, T, generator=g) < 0.1)
+        kw = dict(valid_mask=masks[0], reset_mask=masks[1])
+    with torch.no_grad():
+        fn = solvedelta_masked_native if masked else _native()
+        out, st = fn(*args, *(m.cuda() for m in masks), initial_state=state, return_final_state=True)
+    eo, es = oracle_of(args, state, **kw)
+    _check(out, st, eo, es, f"H{H} {decay} masked={masked}")
