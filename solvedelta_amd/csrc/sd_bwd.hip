@@ -91,25 +91,6 @@ __device__ __forceinline__ void dout_panel_store(__bf16 (*dst)[LPS], const BwdPa
   }
 }
 
-// Branch-free row load: out-of-range tokens and coordinates read a valid element
-// and are selected to 0 (a guarded load would branch and wait).
-__device__ __forceinline__ void ldrow2(const sd_view& v, int b, int t, int h, int T, int w,
-                                       float& x0, float& x1) {
-  const int l = lane_id();
-  const bool tv = t < T;
-  const __bf16* q = brow(v, b, tv ? t : T - 1, h);
-  const float a0 = bf2f(q[l < w ? l : w - 1]), a1 = bf2f(q[l + 64 < w ? l + 64 : w - 1]);
-  x0 = keep_if(tv && l < w, a0);
-  x1 = keep_if(tv && l + 64 < w, a1);
-}
-
-__device__ __forceinline__ float norm2(float& x0, float& x1) {
-  const float rs = rsqrtf(wave_sum(x0 * x0 + x1 * x1) + 1e-24f);
-  x0 *= rs;
-  x1 *= rs;
-  return rs;
-}
-
 __device__ __forceinline__ const float* gptr(const sd_inputs& in, int b, int h) {
   return (const float*)in.log_decay.data + (long long)b * in.log_decay.sb +
          (long long)h * in.log_decay.sh;
@@ -210,20 +191,6 @@ __device__ __forceinline__ void stage_dout_rows(const BwdParams& p, int b, int t
   }
 }
 
-// A fragment of an fp16 panel, re-split into bf16 high + low halves (exact:
-// fp16's 11-bit significand fits the two bf16 halves) for the 3-term product.
-__device__ __forceinline__ Frag ldfrag_h(const _Float16* p, long long off) {
-  const f16x8 v = *reinterpret_cast<const f16x8*>(p + off);
-  Frag f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    __bf16 a, b;
-    split_bf((float)v[e], a, b);
-    f.h[e] = a;
-    f.l[e] = b;
-  }
-  return f;
-}
 static_assert(2 * BT * LS >= BT * KD, "P + N hold a 64 x 128 panel");
 
 template <bool VEC, bool FL>  // FL: the call has token flags (sd_inputs.fresh)

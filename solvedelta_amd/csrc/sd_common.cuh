@@ -170,49 +170,6 @@ __device__ __forceinline__ f4 mma_k32(FA fa, FB fb, int K, f4 acc, int K0 = 0) {
   return acc;
 }
 
-// Two products sharing the A operand (A B1 and A B2): A is gathered and split once.
-// B2_EXACT: fb2's values are exact in bf16 (no low half), so its product takes two
-// MFMAs per K slice.
-template <bool B2_EXACT = false, class FA, class FB1, class FB2>
-__device__ __forceinline__ void mma_k32x2(FA fa, FB1 fb1, FB2 fb2, int K, f4& acc1, f4& acc2) {
-  const int l = lane_id();
-  const int m = l & 15, kq = (l >> 4) * 8;
-  float av[4][8], b1[4][8], b2[4][8];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    if (ks * 32 < K) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        av[ks][e] = fa(m, ks * 32 + kq + e);
-        b1[ks][e] = fb1(ks * 32 + kq + e, m);
-        b2[ks][e] = fb2(ks * 32 + kq + e, m);
-      }
-    }
-  }
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    if (ks * 32 < K) {
-      bf16x8 ah, al, ch, cl, dh, dl;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        __bf16 h, lo;
-        split_bf(av[ks][e], h, lo);
-        ah[e] = h; al[e] = lo;
-        split_bf(b1[ks][e], h, lo);
-        ch[e] = h; cl[e] = lo;
-        split_bf(b2[ks][e], h, lo);
-        dh[e] = h; dl[e] = lo;
-      }
-      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, ch, acc1, 0, 0, 0);
-      acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, dh, acc2, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, cl, acc1, 0, 0, 0);
-      if constexpr (!B2_EXACT) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, dl, acc2, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, ch, acc1, 0, 0, 0);
-      acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, dh, acc2, 0, 0, 0);
-    }
-  }
-}
-
 // mma_k32 with the operand gathers split into a raw-load pass and a transform
 // pass: la(m, k) / lb(k, n) fetch the raw values (for global operands, every
 // load is issued before the first use), xa(m, k, x) / xb(k, n, x) turn them into
@@ -390,70 +347,11 @@ __device__ __forceinline__ float gx_excl(const ChunkDecay& cd, int i, int c) {
   return keep_if(i > 0, cd.G[i > 0 ? i - 1 : 0][c]);  // clamped read + mask: no branch
 }
 
-// Decayed Gram M_ij = sum_c X_ic Y_jc exp(Gx_ic - G_jc), j<i (strict) or j<=i,
-// written to M (64 x LS, fp32); entries above the diagonal set to 0.
-// X(i,c), Y(j,c) are lambdas returning fp32; EXCL selects Gx.
-template <bool EXCL, class FX, class FY>
-__device__ void decayed_gram(const ChunkDecay& cd, FX X, FY Y, bool strict, float* M,
-                             int ldm = LS) {
-  const int w = wave_id();
-  // 10 lower block pairs (I >= J), distributed over 4 waves.
-  for (int p = w; p < 10; p += CW) {
-    int I = 0, J = p;
-    while (J > I) { J -= I + 1; ++I; }  // p -> (I, J) with J <= I
-    const int I0 = I * BS, J0 = J * BS;
-    const float* RJ = cd.R[J];
-    f4 acc = mma_k32_lx(
-        [&](int m, int c) { return X(I0 + m, c); },
-        [&](int m, int c, float x) {
-          const int i = I0 + m;
-          const float gx = EXCL ? gx_excl(cd, i, c) : cd.G[i][c];
-          return x * __expf(gx - RJ[c]);
-        },
-        [&](int c, int n) { return Y(J0 + n, c); },
-        [&](int c, int n, float y) {
-          return y * exp_unless_wild(cd.wild[J][c] != 0, RJ[c] - cd.G[J0 + n][c]);
-        },
-        KD, zero4());
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int i = I0 + out_row(e), j = J0 + out_col();
-      const bool keep = strict ? (j < i) : (j <= i);
-      M[i * ldm + j] = keep ? acc[e] : 0.f;
-    }
-  }
-  // Zero the strictly-upper block pairs.
-  for (int idx = threadIdx.x; idx < BT * BT; idx += CT) {
-    const int i = idx / BT, j = idx % BT;
-    if ((j / BS) > (i / BS)) M[i * ldm + j] = 0.f;
-  }
-  __syncthreads();
-  // Exact fix-up for wild coordinates.
-  for (int J = 0; J < NB; ++J) {
-    const int nw = cd.nwild[J];
-    if (nw == 0) continue;
-    const int J0 = J * BS;
-    const int npairs = (BT - J0) * BS;
-    for (int idx = threadIdx.x; idx < npairs; idx += CT) {
-      const int i = J0 + idx / BS, j = J0 + idx % BS;
-      const bool keep = strict ? (j < i) : (j <= i);
-      if (!keep) continue;
-      float s = 0.f;
-      for (int q = 0; q < nw; ++q) {
-        const int c = cd.wlist[J][q];
-        const float gx = EXCL ? gx_excl(cd, i, c) : cd.G[i][c];
-        s += X(i, c) * Y(j, c) * __expf(fminf(gx - cd.G[j][c], 0.f));
-      }
-      M[i * ldm + j] += s;
-    }
-  }
-  __syncthreads();
-}
-
-// decayed_gram with the X side a 64 x 128 bf16 panel in global memory (row
-// stride KD): each lane's 8-column slice of its row is one 16-byte load, all
-// four issued before the first use (the per-element form makes 32 two-byte
-// loads per block pair).
+// Decayed Gram M_ij = sum_c X_ic Y_jc exp(Gx_ic - G_jc), j < i (strict) or j <= i,
+// written to M (64 x ldm, FP32), entries above the diagonal set to 0; EXCL selects
+// Gx.  The X side is a 64 x 128 bf16 panel in global memory (row stride KD): each
+// lane's 8-column slice of its row is one 16-byte load, all four issued before the
+// first use (the per-element form makes 32 two-byte loads per block pair).
 template <bool EXCL, class FY>
 __device__ void decayed_gram_gx(const ChunkDecay& cd, const __bf16* Xg, FY Y, bool strict, float* M,
                                 int ldm = LS) {
@@ -1032,15 +930,6 @@ __device__ __forceinline__ void stage_panel_bf(__bf16 (*dst)[LPS], const __bf16*
   }
 }
 
-template <class E>
-__device__ __forceinline__ void load_split_blk_g(const E* rows, BlkS& o) {
-  Blk raw;
-  load_blk(raw, rows, KD);
-  split_blk(raw, o);
-}
-
-
-
 // Pair matrix M = A Y^T over K = 128 (strict: j < i, else j <= i) from two LDS
 // panels, A exact in bf16 (staged from bf16 values: no low half).
 __device__ __forceinline__ void lds_pair_h(const LPanel& A, const LPanel& Y, float* M, bool strict) {
@@ -1163,9 +1052,10 @@ __device__ void gram_wild_fixup(const ChunkDecay& cd, FX X, FYR Yraw, bool stric
   __syncthreads();
 }
 
-// decayed_gram with its Y side staged by stage_ytilde: per pair only the X side
-// (X(i, c) exp(Gx_ic - R_J[c])) is transformed and split; Yraw(j, c) gives the
-// untransformed Y for the exact wild-coordinate fix-up.
+// Decayed Gram (as decayed_gram_gx forms it, X(i, c) a lambda) with its Y side
+// staged by stage_ytilde: per pair only the X side (X(i, c) exp(Gx_ic - R_J[c])) is
+// transformed and split; Yraw(j, c) gives the untransformed Y for the exact
+// wild-coordinate fix-up.
 template <bool EXCL, class FX, class FYR>
 __device__ void decayed_gram_yt(const ChunkDecay& cd, FX X, const LPanel& Yt, FYR Yraw, bool strict,
                                 float* M, int ldm = LS) {
