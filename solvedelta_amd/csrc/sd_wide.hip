@@ -190,9 +190,9 @@ struct OpParams {
   const __bf16 *ub, *hb;       // row output: k = u^, x = gx u^, v = gamma h
   const Tok* tok;
   sd_inputs in;                // column output: v = sigmoid(write_raw) v from the raw inputs
-  float *A, *P;                    // [NT][32][32]
+  float *A, *P;                    // [NT][32][32] (P: column output)
   _Float16 *Wneg, *Kt;             // state-pass panels: -W (w_off order), K^ transposed per chunk [NT][kw][32]
-  float *U, *Qt, *Gam;             // Qt [Tp][kw]; U [Tp][vw] (accumulator order); Gam [NT][kw]
+  float *U, *Qt, *Gam;             // Qt [Tp][kw] (column output); U [Tp][vw] (accumulator order); Gam [NT][kw]
 };
 
 // Decay factors of the matrix-core Grams and applies are factored per
@@ -590,7 +590,7 @@ struct WStateParams {
   int NT, Tp, kw, vw, rows, cols, rev;
   const void* Wneg;  // -W per chunk in w_off order (fp16 forward, bf16 reverse)
   const void* Kt;    // K^T per chunk [NT][kw][32] (fp16 forward, bf16 reverse)
-  const __bf16* At;  // injection A^T per chunk [NT][kw][32] (reverse only; nullable)
+  const __bf16* At;  // injection A^T per chunk [NT][kw][32] (reverse)
   const float *U, *Gam;  // U [Tp][vw] (accumulator order); Gam [NT][kw]
   const __bf16* Ib;      // [Tp][vw]
   void* slots;  // xs_t (forward) or ls_t (reverse)
@@ -675,10 +675,9 @@ struct WFrags {
 
 // Chunk-uniform bases with 32-bit lane offsets throughout: 64-bit per-lane
 // addresses for a chunk's fragment loads would not fit in registers beside the
-// prefetch ring.  Every load is unconditional (indices clamped into
-// the panel; a null At replaced by a panel of the same shape): a memory
-// operation under a branch gives the two paths different counts of
-// operations in flight, and the compiler then waits for all of them (the
+// prefetch ring.  Every load is unconditional (indices clamped into the
+// panel): a memory operation under a branch gives the two paths different counts
+// of operations in flight, and the compiler then waits for all of them (the
 // ring's prefetches included) wherever the paths meet.
 template <bool REV>
 __device__ __forceinline__ void wstate_load(const WStateParams& p, int s, int ch, int c0,
@@ -705,16 +704,12 @@ __device__ __forceinline__ void wstate_load(const WStateParams& p, int s, int ch
     f.W[q] = *reinterpret_cast<const V8*>(Wc + w_off(rb, l, 0));
     f.K[q] = *reinterpret_cast<const V8*>(Kc + ko);
     f.G[q] = *reinterpret_cast<const float4*>(Gc + (unsigned)(rb * 16 + 4 * g));
-    if constexpr (REV) {
-      const __bf16* Ap = p.At ? p.At : static_cast<const __bf16*>(p.Kt);
-      f.A[q] = *reinterpret_cast<const bf16x8*>(Ap + cb * WBT + ko);
-    }
+    if constexpr (REV) f.A[q] = *reinterpret_cast<const bf16x8*>(p.At + cb * WBT + ko);
   }
   if constexpr (REV) {
     static_assert(WBT * STILE == 2 * ST, "two Ib elements per thread");
-    const __bf16* Ip = p.At ? p.Ib : reinterpret_cast<const __bf16*>(p.U);  // (U is the larger)
     const int tok = threadIdx.x / (STILE / 2), col = (threadIdx.x % (STILE / 2)) * 2;
-    f.ib = *reinterpret_cast<const unsigned*>(Ip + tb * vw + c0 + (unsigned)(tok * vw + col));
+    f.ib = *reinterpret_cast<const unsigned*>(p.Ib + tb * vw + c0 + (unsigned)(tok * vw + col));
   }
 }
 
@@ -782,12 +777,10 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
   }
 #pragma unroll
   for (int t = 0; t < NTILE; ++t) *reinterpret_cast<f4*>(part + ((w * NTILE + t) * 64 + l) * 4) = pw[t];
-  if constexpr (REV) {
-    if (p.At) {  // the Ib tile (exact in bf16) staged transposed ([column][token])
-      const int tok = threadIdx.x / (STILE / 2), col = (threadIdx.x % (STILE / 2)) * 2;
-      ih[col * WLD + tok] = __builtin_bit_cast(E, (unsigned short)f.ib);
-      ih[(col + 1) * WLD + tok] = __builtin_bit_cast(E, (unsigned short)(f.ib >> 16));
-    }
+  if constexpr (REV) {  // the Ib tile (exact in bf16) staged transposed ([column][token])
+    const int tok = threadIdx.x / (STILE / 2), col = (threadIdx.x % (STILE / 2)) * 2;
+    ih[col * WLD + tok] = __builtin_bit_cast(E, (unsigned short)f.ib);
+    ih[(col + 1) * WLD + tok] = __builtin_bit_cast(E, (unsigned short)(f.ib >> 16));
   }
   __syncthreads();
   {  // w: two elements (neighbouring tokens of one column) per thread
@@ -825,10 +818,8 @@ __device__ __forceinline__ void wstate_step(const WStateParams& p, int s, int ch
 #pragma unroll
       for (int e = 0; e < 4; ++e) X[q][h][e] *= gv[e];
       if constexpr (REV) {
-        if (p.At) {
-          const bf16x8 bh = *reinterpret_cast<const bf16x8*>(ih + (h * 16 + m) * WLD + kq);
-          X[q][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.A[q], bh, X[q][h], 0, 0, 0);
-        }
+        const bf16x8 bh = *reinterpret_cast<const bf16x8*>(ih + (h * 16 + m) * WLD + kq);
+        X[q][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.A[q], bh, X[q][h], 0, 0, 0);
       }
     }
   }
@@ -1227,7 +1218,7 @@ static_assert(PW * 3 * 256 >= PW * WBT * GS16, "the waves' k~ panels fit the par
 // ---------------------------------------------------------------------------
 struct SrcParams {
   sd_inputs in;
-  int Tp, KP, VP;
+  int Tp, KP;
   const __bf16 *ub, *kb, *qb;
   const Tok* tok;
   const float* delta;
@@ -2420,7 +2411,7 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
   OpParams oc{};
   oc.NT = d.NT; oc.Tp = d.Tp; oc.kw = d.KP; oc.vw = d.KP; oc.colout = 0;
   oc.ub = w.ub; oc.hb = w.hb; oc.tok = w.tok; oc.G = w.G;
-  oc.A = w.AC; oc.P = w.PS; oc.Wneg = w.Wneg; oc.U = w.U; oc.Kt = w.Kt; oc.Qt = w.Qt; oc.Gam = w.Gam;
+  oc.A = w.AC; oc.Wneg = w.Wneg; oc.U = w.U; oc.Kt = w.Kt; oc.Gam = w.Gam;
   launch_wprep(oc, d.n, st);
   WStateParams sc{};
   sc.NT = d.NT; sc.Tp = d.Tp; sc.kw = d.KP; sc.vw = d.KP; sc.rows = in->r; sc.cols = in->r;
@@ -2436,7 +2427,7 @@ int launch_wide_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, void
   SD_LAUNCH("k_w_out_c", k_w_out_c, dim3(d.NT, d.n), dim3(PT), out_c_smem(), st, orow);
 
   SrcParams sp{};
-  sp.in = *in; sp.Tp = d.Tp; sp.KP = d.KP; sp.VP = d.VP;
+  sp.in = *in; sp.Tp = d.Tp; sp.KP = d.KP;
   sp.ub = w.ub; sp.kb = w.kb; sp.qb = w.qb; sp.tok = w.tok; sp.delta = w.delta;
   sp.e = w.e; sp.chi = w.chi;
   SD_LAUNCH("k_w_sources", k_w_sources, dim3(d.Tp / (WT / 64), d.n), dim3(WT), 0, st, sp);
