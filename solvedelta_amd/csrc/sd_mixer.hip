@@ -548,7 +548,7 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsv_fwd(int N, int D, float eps, 
   }
 }
 
-// rows: per workgroup, a multiple of NTHREADS / LPR * RMSV_U
+// rows: per workgroup (rmsv_rows), a multiple of NTHREADS / LPR * RMSV_U
 template <int LPR>
 __global__ __launch_bounds__(NTHREADS) void k_rmsv_bwd(int N, int D, float eps, int rows,
                                                        const __bf16* __restrict__ x,
@@ -966,6 +966,19 @@ static bool gate_quads(const GateArgs& a, const void* bf, const void* f32) {
          ((uintptr_t)f32 & 15) == 0;
 }
 
+// Rows per workgroup (and dweight partial) of the vector backward: one batch of its
+// lanes (128 rows for D <= 64, 64 for D <= 128; two of 32 above, whose partials then
+// fit the general path's workspace), and for D <= 128 two batches where that leaves
+// two workgroups per CU and more.  Longer workgroups gain nothing and lose the CUs'
+// balance; us with the sum of the partials, one / two / four batches, D = 128:
+// 32768 rows 13.1 / 14.1 / 18.8, 65537 20.9 / 20.7 / 22.1, 98304 28.4 / 27.1 / 31.0,
+// 262144 86.8 / 82.5 / 86.3.  D = 64: 32768 8.6 / 11.3 / 15.6, 262144 36.3 / 35.1 /
+// 35.4.  D = 256: 131072 rows 82.5 in 64s, 84.8 in 128s.
+static int rmsv_rows(int N, int D) {
+  const int rows = D <= 64 ? 128 : RMS_PART;
+  return D <= 128 && N > 2 * 512 * rows ? 2 * rows : rows;
+}
+
 // Eight columns per lane where rows are multiples of 8 wide and 16-byte aligned.
 static bool rms_vec(int D, uintptr_t bits) { return D % 8 == 0 && (bits & 15) == 0; }
 
@@ -1150,8 +1163,7 @@ int sd_rmsnorm_gated_bwd(int N, int D, float eps, const void* x, const void* gat
     SD_LAUNCH("k_rms_bwd", k_rms_bwd, dim3(np), dim3(RMS_ROWS * 64), 0, st, N, D, eps, xb, gb, weight, db, dxb, dgb,
               yb, part);
   } else {
-    // at most ~512 partial rows (two workgroups per CU), 128 rows a batch at most
-    const int rows = cdiv(cdiv(N, 512), 128) * 128 > 128 ? cdiv(cdiv(N, 512), 128) * 128 : (D <= 64 ? 128 : RMS_PART);
+    const int rows = rmsv_rows(N, D);
     np = cdiv(N, rows);
     if (D <= 64)
       SD_LAUNCH("k_rms_bwd", k_rmsv_bwd<8>, dim3(np), dim3(NTHREADS), 0, st, N, D, eps, rows, xb, gb, weight, db,

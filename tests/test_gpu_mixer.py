@@ -113,10 +113,12 @@ def test_kda_gate_widths_and_tails(B, T, H, r):
 
 
 @pytest.mark.parametrize("N,D,off", [(1, 8, 0), (131, 64, 0), (300, 72, 0), (65, 128, 0), (70000, 128, 0),
-                                     (33, 136, 0), (129, 256, 0), (77, 100, 0), (40, 64, 1)])
+                                     (33, 136, 0), (129, 256, 0), (77, 100, 0), (40, 64, 1),
+                                     (65535, 128, 0), (65537, 72, 0), (131073, 64, 0), (65537, 200, 0)])
 def test_rmsnorm_gated_row_layouts(N, D, off):
     """8, 16 and 32 lanes per row, the general path (widths off 8 and rows off
-    16 bytes), batches with a remainder, and more rows than dweight partials."""
+    16 bytes), batches with a remainder, and both sides of the row counts from
+    which a workgroup takes two batches."""
     from solvedelta_amd.mixer import _rms_bwd, _rms_fwd
     g = torch.Generator(device="cuda").manual_seed(N + D)
     mk = lambda: torch.randn(N * D + off, generator=g, device="cuda").to(torch.bfloat16)[off:].view(N, D)
