@@ -1052,60 +1052,6 @@ __device__ void gram_wild_fixup(const ChunkDecay& cd, FX X, FYR Yraw, bool stric
   __syncthreads();
 }
 
-// Decayed Gram (as decayed_gram_gx forms it, X(i, c) a lambda) with its Y side
-// staged by stage_ytilde: per pair only the X side (X(i, c) exp(Gx_ic - R_J[c])) is
-// transformed and split; Yraw(j, c) gives the untransformed Y for the exact
-// wild-coordinate fix-up.
-template <bool EXCL, class FX, class FYR>
-__device__ void decayed_gram_yt(const ChunkDecay& cd, FX X, const LPanel& Yt, FYR Yraw, bool strict,
-                                float* M, int ldm = LS) {
-  const int w = wave_id(), l = lane_id(), m = l & 15, kq = (l >> 4) * 8;
-  for (int p = w; p < 10; p += CW) {
-    int I = 0, J = p;
-    while (J > I) { J -= I + 1; ++I; }  // p -> (I, J) with J <= I
-    const int I0 = I * BS, J0 = J * BS, i = I0 + m;
-    const float* RJ = cd.R[J];
-    float xr[4][8];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) xr[ks][e] = X(i, ks * 32 + kq + e);
-    BlkS A, B;
-    lblk(Yt, J0, B);
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int c = ks * 32 + kq + e;
-        const float gx = EXCL ? gx_excl(cd, i, c) : cd.G[i][c];
-        v[e] = xr[ks][e] * __expf(gx - RJ[c]);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        __bf16 h, lo;
-        split_bf(v[e], h, lo);
-        A.f[ks].h[e] = h;
-        A.f[ks].l[e] = lo;
-      }
-    }
-    const f4 acc = mma_blks(A, B, zero4());
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int ii = I0 + out_row(e), j = J0 + out_col();
-      const bool keep = strict ? (j < ii) : (j <= ii);
-      M[ii * ldm + j] = keep ? acc[e] : 0.f;
-    }
-  }
-  // Zero the strictly-upper block pairs.
-  for (int idx = threadIdx.x; idx < BT * BT; idx += CT) {
-    const int ii = idx / BT, j = idx % BT;
-    if ((j / BS) > (ii / BS)) M[ii * ldm + j] = 0.f;
-  }
-  __syncthreads();
-  gram_wild_fixup<EXCL>(cd, X, Yraw, strict, M, ldm);
-}
-
 // Two decayed Grams against one staged Y side, in one pass over the block
 // pairs:  M1 = X1 Y~ (j <= i) into M, and M2 = X2 Y~ (j < i) returned in the
 // caller's registers (the pairs p = wave, wave + CW of the 10, in that order)

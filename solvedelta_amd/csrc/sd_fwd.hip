@@ -50,6 +50,7 @@ constexpr int PS = KD + 8;  // bf16 panel row stride
 // ---------------------------------------------------------------------------
 // k_prep_c
 // ---------------------------------------------------------------------------
+template <bool FEW>
 struct PrepCSmem {
   ChunkDecay cd;
   float M[BT * LS];
@@ -58,6 +59,8 @@ struct PrepCSmem {
   float gam[BT];
   float xm[BT];       // 1, or 0 on fresh tokens (no erase read)
   float cap[NB][KD];  // largest exponent of y: TAU, or -inf (y = 0) on a wild coordinate
+  __bf16 Hh[FEW ? BT : 1][PS];  // FEW: h (raw bf16, exact)
+  __bf16 Yh[FEW ? BT : 1][LPS], Yl[FEW ? BT : 1][LPS];  // FEW: y, split
 };
 
 // W = A diag(gamma) (u e^{Gexcl} masked on fresh tokens) and U = A diag(gamma) h
@@ -110,15 +113,24 @@ __device__ __forceinline__ void prep_c_products(const FwdParams& p, const float*
 // are formed from it and the decay table in registers by the wave that uses
 // them (a staged, split Y side took 34 KB), h follows u into its panel, and the
 // inverse's scratch blocks lie in M's unused corner.
-// Against one 153 KB workgroup per CU: 70 -> 56 us at 4 x 2048 tokens, 8 heads,
+// Against one 153 KB workgroup per CU: 70 -> 51-55 us at 4 x 2048 tokens, 8 heads,
 // r = V = 128 (151 MB moved, 32 us at a large copy's rate), 97 -> 76 us at
 // 2 x 3001, 16 heads, without (I+L)^-1.  The opening loads come in bursts (9 us of a
 // workgroup's 20); h gathered in operand layout from memory instead cost 7 us
 // of latency before the inverse (67 / 90 us).
-template <bool FL, bool KEEP>
-__global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
+//
+// FEW: every chunk has a CU to itself (at most kFewChunks of them), so LDS is not
+// short and the chain of phases is the time: y is transformed and split once into
+// LDS instead of by each block pair's wave, and h has a panel beside u's.  The
+// arithmetic is the same, operation by operation, so a sequence's results do not
+// depend on how many others are in the call.  r = V = 128, the shared / this form,
+// us: one chunk 15.2 / 14.2, 64 16.3 / 15.7, 128 17.7 / 16.4, 256 20.1 / 18.9; from
+// one more chunk than CUs on it would need a second round, 26.2 / 30.7 at 288.
+constexpr int kFewChunks = 256;  // one per CU
+template <bool FL, bool KEEP, bool FEW>
+__global__ __launch_bounds__(CT, FEW ? 2 : 4) void k_prep_c(FwdParams p) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  PrepCSmem& s = *reinterpret_cast<PrepCSmem*>(smem_raw);
+  PrepCSmem<FEW>& s = *reinterpret_cast<PrepCSmem<FEW>*>(smem_raw);
   // chunk-major dispatch, last chunk first (chunk 0, where the C state pass
   // starts, is written last)
   const int n = blockIdx.x, ch = gridDim.y - 1 - blockIdx.y;
@@ -128,7 +140,7 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
   const float* g = (const float*)in.log_decay.data + (long long)b * in.log_decay.sb +
                    (long long)hh * in.log_decay.sh;
   const int w = wave_id(), l = lane_id();
-  float hx[2][RQ];  // rows of h, until u's panel is free for them
+  float hx[2][RQ];  // rows of h, until a panel is free for them
   {
     // every load of the opening phase first (the decay column, then every row's
     // u and h): a row's reduction would otherwise hold the next row's loads
@@ -164,32 +176,63 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
       if (cl == 0) s.ru[i] = rn;
     }
   }
+  auto put_h = [&](__bf16 (*dst)[PS]) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) dst[row16(w, g)][(l & 15) + 16 * q] = f2bf(hx[g][q]);  // exact
+  };
+  if constexpr (FEW) put_h(s.Hh);
   __syncthreads();
   const ChunkDecay& cd = s.cd;
   const int m = l & 15, kq = (l >> 4) * 8;
   auto U = [&](int i, int c) { return bf2f(s.Ub[i][c]) * s.ru[i]; };
+  // eight columns of y from c0 on: token j as a column of block J
+  auto y_frag = [&](int J, int j, int c0) {
+    const float uj = s.ru[j];
+    const float* Gj = cd.G[j];
+    const bf16x8 yu = *reinterpret_cast<const bf16x8*>(&s.Ub[j][c0]);
+    Frag y;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      __bf16 hi, lo;
+      split_bf(bf2f(yu[e]) * uj * __expf(fminf(cd.R[J][c0 + e] - Gj[c0 + e], s.cap[J][c0 + e])), hi, lo);
+      y.h[e] = hi;
+      y.l[e] = lo;
+    }
+    return y;
+  };
+  if constexpr (FEW) {
+#pragma unroll
+    for (int q = 0; q < BT * KD / 8 / CT; ++q) {
+      const int idx = threadIdx.x + q * CT, j = idx / (KD / 8), c0 = idx % (KD / 8) * 8;
+      const Frag y = y_frag(j / BS, j, c0);
+      *reinterpret_cast<bf16x8*>(&s.Yh[j][c0]) = y.h;
+      *reinterpret_cast<bf16x8*>(&s.Yl[j][c0]) = y.l;
+    }
+    __syncthreads();
+  }
   // L_ij = gamma_i sum_c u_ic u_jc exp(G_{i-1,c} - G_jc), j < i: block pair (I, J)
   // from x = u exp(G_excl - R_J) and y = u^ exp(R_J - G), 32 columns at a time.
   // Ten pairs on eight waves: a wave takes one whole pair and a quarter of pair 8
   // or 9, whose partial sums meet in M's blocks above the diagonal.
   auto pair_step = [&](int I, int J, int ks, f4 acc) {
     const int i = I * BS + m, j = J * BS + m, c0 = ks * 32 + kq;
-    const float uj = s.ru[j];
     const float* Gi = i > 0 ? cd.G[i - 1] : cd.R[0];  // R[0] is zero
-    const float* Gj = cd.G[j];
     const bf16x8 xu = *reinterpret_cast<const bf16x8*>(&s.Ub[i][c0]);
-    const bf16x8 yu = *reinterpret_cast<const bf16x8*>(&s.Ub[j][c0]);
     Frag x, y;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float R = cd.R[J][c0 + e];
       __bf16 hi, lo;
-      split_bf(bf2f(xu[e]) * __expf(Gi[c0 + e] - R), hi, lo);
+      split_bf(bf2f(xu[e]) * __expf(Gi[c0 + e] - cd.R[J][c0 + e]), hi, lo);
       x.h[e] = hi;
       x.l[e] = lo;
-      split_bf(bf2f(yu[e]) * uj * __expf(fminf(R - Gj[c0 + e], s.cap[J][c0 + e])), hi, lo);
-      y.h[e] = hi;
-      y.l[e] = lo;
+    }
+    if constexpr (FEW) {
+      y.h = *reinterpret_cast<const bf16x8*>(&s.Yh[j][c0]);
+      y.l = *reinterpret_cast<const bf16x8*>(&s.Yl[j][c0]);
+    } else {
+      y = y_frag(J, j, c0);
     }
     return mma3f(x, y, acc);
   };
@@ -237,10 +280,13 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
   // everything else that reads u: the decayed keys (transposed per chunk), the
   // chunk decay and, in operand layout, the right side of W's product
   const long long cbase = ((long long)n * p.NT + ch);
-  store_frag_panel1<KD, BT>(p.Kc, cbase * KD * BT, [&](int c, int i) {
-    return U(i, c) * __expf(cd.G[BT - 1][c] - cd.G[i][c]);
-  });
-  if (threadIdx.x < KD) p.Gam[cbase * KD + threadIdx.x] = __expf(cd.G[BT - 1][threadIdx.x]);
+  auto put_keys = [&] {
+    store_frag_panel1<KD, BT>(p.Kc, cbase * KD * BT, [&](int c, int i) {
+      return U(i, c) * __expf(cd.G[BT - 1][c] - cd.G[i][c]);
+    });
+    if (threadIdx.x < KD) p.Gam[cbase * KD + threadIdx.x] = __expf(cd.G[BT - 1][threadIdx.x]);
+  };
+  if constexpr (!FEW) put_keys();
   const int c = w * 16 + m;
   bf16x8 bh[2], bl[2];
 #pragma unroll
@@ -253,11 +299,10 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
       bh[ks][e] = hi;
       bl[ks][e] = lo;
     }
-  __syncthreads();
-#pragma unroll
-  for (int g = 0; g < 2; ++g)
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) s.Ub[row16(w, g)][m + 16 * q] = f2bf(hx[g][q]);  // exact
+  if constexpr (!FEW) {
+    __syncthreads();
+    put_h(s.Ub);
+  }
   // scratch blocks (2..3, 0..1) of the inverse lie at M's blocks (0..1, 2..3)
   unit_lower_inverse(s.M, s.M - 32 * LS + 32);
   if constexpr (KEEP)
@@ -270,104 +315,10 @@ __global__ __launch_bounds__(CT, 4) void k_prep_c(FwdParams p) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) hb[ks][e] = s.Ub[ks * 32 + kq + e][c];
+      for (int e = 0; e < 8; ++e) hb[ks][e] = (FEW ? s.Hh : s.Ub)[ks * 32 + kq + e][c];
     prep_c_products(p, s.M, s.gam, bh, bl, hb, (long long)n * p.Tp + t0);
   }
-}
-
-// The same where every chunk has a CU to itself (at most kFewChunks of them): two
-// workgroups never share a CU, so LDS is not short and the chain of phases is the
-// time.  The Gram's Y side is transformed and split once into LDS instead of by
-// each block pair's wave, u and h lie side by side, and the inverse has its own
-// scratch (153 KB).  r = V = 128, k_prep_c / this kernel, us: 15.4 / 13.7 at one
-// chunk, 17.8-18.3 / 16.3-16.7 at 64, 20.7-21.2 / 17.4-17.8 at 128, 21.3 / 19.7-20.2
-// at 256; from one more chunk than CUs on the other way round, 26.1 / 29.2-29.7 at 288.
-struct PrepCFewSmem {
-  ChunkDecay cd;
-  float M[BT * LS];
-  float tmp[BT * LS];
-  float Uh[BT][GS];   // normalised u
-  __bf16 Hh[BT][PS];  // h (raw bf16, exact)
-  float gam[BT];
-  float xm[BT];       // 1, or 0 on fresh tokens (no erase read)
-  LPanel Yt;          // the L Gram's Y side (u), transformed and split once
-};
-constexpr int kFewChunks = 256;  // one per CU
-
-template <bool FL, bool KEEP>
-__global__ __launch_bounds__(CT) void k_prep_c_few(FwdParams p) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  PrepCFewSmem& s = *reinterpret_cast<PrepCFewSmem*>(smem_raw);
-  const int n = blockIdx.x, ch = gridDim.y - 1 - blockIdx.y;  // as k_prep_c
-  const int b = n / p.H, hh = n % p.H, t0 = ch * BT;
-  const int T = p.T, r = p.r;
-  const sd_inputs& in = p.in;
-  const float* g = (const float*)in.log_decay.data + (long long)b * in.log_decay.sb +
-                   (long long)hh * in.log_decay.sh;
-  const int w = wave_id(), l = lane_id(), m = l & 15, kq = (l >> 4) * 8;
-  {
-    // every load of the opening phase first, as in k_prep_c
-    float xdec[BS];
-    decay_load(g, in.log_decay.st, t0, T, r, xdec, FL ? tok_flag_row(in, b) : nullptr, tok_flag_st(in));
-    float ux[2][RQ], hx[2][RQ];
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const int t = t0 + row16(w, g);
-      load_row16(in.u, b, t, hh, T, r, ux[g]);
-      load_row16(in.h, b, t, hh, T, r, hx[g]);
-    }
-    if (threadIdx.x < BT) {  // branch-free: clamped token, then select
-      const int t = t0 + threadIdx.x;
-      const float gv = gamma_at(in.gamma, b, t < T ? t : T - 1, hh);
-      const unsigned f = tok_flags(in, b, t < T ? t : T - 1);
-      s.gam[threadIdx.x] = keep_if(t < T, gv) * operand_keep(f);  // 0 on invalid tokens
-      s.xm[threadIdx.x] = erase_keep_f(f);
-    }
-    decay_build(s.cd, xdec);
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const int i = row16(w, g);
-      l2norm16(ux[g]);
-#pragma unroll
-      for (int q = 0; q < RQ; ++q) {
-        s.Uh[i][m + 16 * q] = ux[g][q];
-        s.Hh[i][m + 16 * q] = f2bf(hx[g][q]);
-      }
-    }
-  }
-  __syncthreads();
-  const ChunkDecay& cd = s.cd;
-  // L_ij = gamma_i sum_c u_ic u_jc exp(G_{i-1,c} - G_jc), j < i
-  stage_ytilde(s.Yt, cd, [&](int j, int c) { return s.Uh[j][c]; });
-  decayed_gram_yt<true>(
-      cd, [&](int i, int c) { return s.gam[i] * s.xm[i] * s.Uh[i][c]; }, s.Yt,
-      [&](int j, int c) { return s.Uh[j][c]; }, true, s.M);
-  unit_lower_inverse(s.M, s.tmp);
-  const long long cbase = ((long long)n * p.NT + ch);
-  if constexpr (KEEP)
-    for (int idx = threadIdx.x; idx < BT * BT; idx += CT)
-      p.Ac[cbase * BT * BT + idx] = s.M[(idx / BT) * LS + idx % BT];
-  {
-    // B operands, the same for every row block: formed and split once
-    bf16x8 bh[2], bl[2], hb[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = ks * 32 + kq + e, c = w * 16 + m;
-        __bf16 hi, lo;
-        split_bf(s.xm[k] * s.Uh[k][c] * __expf(gx_excl(cd, k, c)), hi, lo);
-        bh[ks][e] = hi;
-        bl[ks][e] = lo;
-        hb[ks][e] = s.Hh[k][c];  // h is the raw bf16 input: exact
-      }
-    prep_c_products(p, s.M, s.gam, bh, bl, hb, (long long)n * p.Tp + t0);
-  }
-  // decayed keys (transposed per chunk) and chunk decay
-  store_frag_panel1<KD, BT>(p.Kc, cbase * KD * BT, [&](int c, int i) {
-    return s.Uh[i][c] * __expf(cd.G[BT - 1][c] - cd.G[i][c]);
-  });
-  if (threadIdx.x < KD) p.Gam[cbase * KD + threadIdx.x] = __expf(cd.G[BT - 1][threadIdx.x]);
+  if constexpr (FEW) put_keys();  // (with nothing waiting for u's panel, off the chain)
 }
 
 // ---------------------------------------------------------------------------
@@ -1244,18 +1195,18 @@ __global__ __launch_bounds__(CT) void k_prep_s(FwdParams p) {
   store_frag_panel1<BT, KD>(p.Ws, rowbase * KD, [&](int i, int c) { return s.Pc[i][c]; });
 }
 
-size_t prep_c_smem() { return sizeof(PrepCSmem); }
 size_t prep_s_smem() { return sizeof(PrepSSmem); }
 
+template <bool FL, bool KEEP, bool FEW>
+static void launch_prep_c(const FwdParams& fp, int n, hipStream_t st) {
+  constexpr int smem = sizeof(PrepCSmem<FEW>);
+  SD_SMEM_ONCE((k_prep_c<FL, KEEP, FEW>), smem);
+  SD_LAUNCH("k_prep_c", (k_prep_c<FL, KEEP, FEW>), dim3(n, fp.NT), dim3(CT), smem, st, fp);
+}
 template <bool FL, bool KEEP>
 static void run_prep_c(const FwdParams& fp, int n, hipStream_t st) {
-  if ((long long)n * fp.NT <= kFewChunks) {
-    SD_SMEM_ONCE((k_prep_c_few<FL, KEEP>), (int)sizeof(PrepCFewSmem));
-    SD_LAUNCH("k_prep_c", (k_prep_c_few<FL, KEEP>), dim3(n, fp.NT), dim3(CT), sizeof(PrepCFewSmem), st, fp);
-    return;
-  }
-  SD_SMEM_ONCE((k_prep_c<FL, KEEP>), (int)prep_c_smem());
-  SD_LAUNCH("k_prep_c", (k_prep_c<FL, KEEP>), dim3(n, fp.NT), dim3(CT), prep_c_smem(), st, fp);
+  if ((long long)n * fp.NT <= kFewChunks) launch_prep_c<FL, KEEP, true>(fp, n, st);
+  else launch_prep_c<FL, KEEP, false>(fp, n, st);
 }
 template <bool FL, bool KEEP>
 static void run_prep_s(const FwdParams& fp, int n, hipStream_t st) {

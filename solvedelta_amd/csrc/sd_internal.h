@@ -150,7 +150,6 @@ inline void set_smem_once(const void* fn, int bytes, unsigned char* done) {
   } while (0)
 
 void launch_state(const char* name, const StateParams& sp, int nseq, hipStream_t st);
-size_t prep_c_smem();
 size_t prep_s_smem();
 
 int launch_fwd(const sd_inputs* in, void* out, float* C_T, float* S_T, const FwdWs& w,

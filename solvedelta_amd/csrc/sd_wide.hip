@@ -6,17 +6,20 @@
 // hold a 64-token chunk's 128-wide panels in LDS; at 256 they would not fit, so
 // this path states the same chunked algebra (the generic pre-decay-read delta
 // op restated in tests/chunk_model.py) with 32-token chunks, runtime padded
-// widths KP, VP (multiples of 32, <= 256), FP32 token panels and a 16-bit
+// widths KP, VP (multiples of 32, <= 256), u, k, q, h as packed bf16 rows with
+// FP32 scalars per token, FP32 panels for what is computed, and a 16-bit
 // matrix-core state pass (its panels and the chunk states in fp16 / bf16):
 //
-//   k_w_tokens  (chunk-parallel)  in-chunk log-decay prefix G, L2 norms, gamma;
+//   k_w_tokens  (chunk-parallel)  in-chunk log-decay prefix G, packed rows, L2
+//               norms, gamma;
 //   per op (predictor C: X = C^T, erase read before the token's decay, row
 //   output; memory S: erase read after it, column output):
-//     k_w_prep    decayed Gram L, (I+L)^-1, WY panels W, U, decayed keys,
-//                 readout pair P (column output);
+//     k_w_prep    decayed Gram L, (I+L)^-1, WY panels W, U (the memory's from
+//                 z = sigmoid(write_raw) v, formed there), decayed keys, readout
+//                 pair P (column output);
 //     k_w_state   sequential chunk pass over one 32-column state tile;
 //     k_w_out_c, k_w_out_s  chunk readouts (the predictor's forms d = k^ + C^T k^);
-//   k_w_sources (per token)  dual sources e, chi and gated values z;
+//   k_w_sources (per token)  dual sources e, chi;
 // and backward, per op in reverse order:
 //     k_w_bprep   dU = A^T (dW + pair^T dO), W' = -A^T K^, K' = -x~, injection;
 //     k_w_state   reverse cotangent pass (lambda, dw);
@@ -70,7 +73,7 @@ __device__ __forceinline__ float wgamma(const sd_view& g, int b, int t, int h) {
 }
 
 // ---------------------------------------------------------------------------
-// Token preparation: G prefix, norms, gamma-scaled predictor operands.
+// Token preparation: G prefix, packed rows, norms and gamma.
 // ---------------------------------------------------------------------------
 // Per-token scalars: the inverse norms 1/|u|, 1/|k|, 1/|q| (u^ = ru u and so on
 // are formed from the packed bf16 rows where they are read: half the bytes of
@@ -115,8 +118,8 @@ __global__ __launch_bounds__(WT) void k_w_tokens(TokParams p) {
       p.G[(pb + t0 + i) * KP + c] = acc;
     }
   }
-  // per token: norms and the gamma-scaled predictor operands, two tokens per
-  // wave at a time with all their loads in flight together
+  // per token: packed rows, norms and gamma, two tokens per wave at a time with
+  // all their loads in flight together
   constexpr int NW = WT / 64, TU = 2;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   static_assert(WBT % (NW * TU) == 0, "tokens per wave");
@@ -382,12 +385,13 @@ __device__ __forceinline__ void store_transposed(E* dst, const E* src, int kw) {
   }
 }
 
-// What bounds it: at r = V = 256 a chunk moves 192 KiB (C) / 256 KiB (S) through
+// What bounds it: at r = V = 256 a chunk moves 133 KiB (C) / 265 KiB (S) through
 // one or two workgroups per CU, so the phases between its loads and stores must
-// be short: two workgroups fit a CU (79 KB of LDS, 128 VGPRs) and overlap.  110 us
-// (C, 3.7 TB/s) and 123 us (S, 4.4 TB/s) at B4 T2048 H8 r = V = 256; one
-// four-wave workgroup per CU with every operand panel staged in LDS (110-140 KB,
-// each Gram element formed once per 16 x 16 block) took 226 us per op.
+// be short: two workgroups fit a CU (79 KB of LDS, 128 VGPRs) and overlap.  76 us
+// (C, 3.7 TB/s) and 132 us (S, 4.2 TB/s) at B4 T2048 H8 r = V = 256; 110 and 123
+// when C read FP32 panels and S its z; one four-wave workgroup per CU with
+// every operand panel staged in LDS (110-140 KB, each Gram element formed once per
+// 16 x 16 block) took 226 us per op.
 template <bool COL>
 __global__ __launch_bounds__(PT, 4) void k_w_prep(OpParams p) {
   extern __shared__ __align__(16) float sm[];
@@ -1305,9 +1309,10 @@ struct BprepParams {
 // Same organisation as k_w_prep: a lane's four coordinates of a token are loaded
 // once and give the Pp Gram's operands, K^, Kn and Ia; the value side runs
 // straight from registers.  Two workgroups per CU (76 KB of LDS, 128 VGPRs):
-// 91 us (S, 4.6 TB/s) and 127 us (C, 4.2 TB/s) at B4 T2048 H8 r = V = 256, where
-// one four-wave workgroup per CU (LDS copies of every operand, 4-byte loads of
-// each panel's columns) took 174 us per op.
+// 92 us (S, 232 KiB a chunk, 5.3 TB/s with what the last-level cache still holds)
+// and 104 us (C, 216 KiB, 4.4 TB/s) at B4 T2048 H8 r = V = 256, where one four-wave
+// workgroup per CU (LDS copies of every operand, 4-byte loads of each panel's
+// columns) took 174 us per op.
 template <bool COL>
 __global__ __launch_bounds__(PT, 4) void k_w_bprep(BprepParams p) {
   extern __shared__ __align__(16) float sm[];
@@ -1578,12 +1583,13 @@ __device__ __forceinline__ void split4_to(__bf16* hi, __bf16* lo, const Quad& q)
   *reinterpret_cast<bf16x4*>(lo) = o;
 }
 
-// What bounds it: the state slots (X0 and lambda, 256 KiB of a chunk's 608 KiB
-// at r = V = 256) stream through phase 1; every product's output is formed
+// What bounds it: the state slots (X0 and lambda, 256 KiB of a chunk's 592 KiB
+// (S) or 644 KiB (C) at r = V = 256) stream through phase 1; every product's output is formed
 // transposed, so a lane holds four neighbouring coordinates of one token and
 // reads and writes the token panels 16 bytes at a time, and the rows shared by
-// all waves are split into bf16 halves once, in LDS.  301 us (S, 4.2 TB/s) and
-// 468 us (C, with the layer's closure) per launch at B4 T2048 H8 r = V = 256; with
+// all waves are split into bf16 halves once, in LDS.  290 us (S, 4.3 TB/s) and
+// 460 us (C, with the layer's closure: 2.9 TB/s, one workgroup per CU whose tail
+// reads more rows after its products) per launch at B4 T2048 H8 r = V = 256; with
 // 4-byte panel accesses in the MFMA layout, the rows split by every wave and
 // dO e^G X0 on FP32 MFMAs over 2-byte gathers of the slot, 360 us and, with the
 // closure as a kernel of its own, 500 + 217 us.

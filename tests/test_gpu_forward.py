@@ -212,3 +212,28 @@ def test_forward_on_both_sides_of_one_chunk_per_cu(H, decay, masked):
         out, st = fn(*args, *(m.cuda() for m in masks), initial_state=state, return_final_state=True)
     eo, es = oracle_of(args, state, **kw)
     _check(out, st, eo, es, f"H{H} {decay} masked={masked}")
+
+
+@pytest.mark.parametrize("T,r,V,decay,masked", [(81, 24, 16, "mixed", False), (130, 128, 128, "softplus", False),
+                                                (65, 65, 80, "extreme", False), (81, 128, 64, "mixed", True)])
+def test_a_sequence_is_the_same_alone_and_in_a_large_batch(T, r, V, decay, masked):
+    """Rows of a call with more chunks than CUs against calls of one row each with
+    fewer: bitwise, gradients and final states included."""
+    from solvedelta_amd import solvedelta_masked_native
+    B, H = 3, 80  # 160 or 240 chunks a row
+    args = make_inputs(B, T, H, r, V, seed=95, decay=decay)
+    state = make_state(B, H, r, V, seed=96)
+    g = torch.Generator().manual_seed(97)
+    masks = (torch.rand(B, T, generator=g) >= 0.2, torch.rand(B, T, generator=g) < 0.1) if masked else ()
+    masks = [m.cuda() for m in masks]
+    dout = torch.randn(B, T, H, V, generator=g).to(torch.bfloat16).cuda()
+    def run(rows):
+        a = [x[rows].contiguous().requires_grad_() for x in (*args, *state)]
+        fn = solvedelta_masked_native if masked else _native()
+        out, st = fn(*a[:9], *(m[rows] for m in masks), initial_state=tuple(a[9:]), return_final_state=True)
+        grads = torch.autograd.grad((out, st.S), a, (dout[rows], torch.ones_like(st.S)))
+        return [out, st.predictor, st.S, *grads]
+    whole = run(slice(0, B))
+    for b in range(B):
+        for i, (x, y) in enumerate(zip(whole, run(slice(b, b + 1)))):
+            assert torch.equal(x[b:b + 1], y), (b, i)
