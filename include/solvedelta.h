@@ -18,7 +18,7 @@
  *   Widths: 1 <= r, V <= 256, as the reference's state pass
  *   (residual_frame/common_left_h.py:139-140).  r, V <= 128 run on the main
  *   kernels (64-token chunks); a call with either width above 128 runs on the
- *   wide-width kernels (32-token chunks, FP32 panels) with their own workspace
+ *   wide-width kernels (32-token chunks) with their own workspace
  *   layout, which the *_workspace_bytes queries size from (r, V).  The Python
  *   operator cuts wider value axes into groups.  sd_decode takes r, V <= 128
  *   (wider T = 1 calls take the chunked path, as in the reference).

@@ -1079,11 +1079,11 @@ __global__ __launch_bounds__(PT, 4) void k_w_out_s(OutParams p) {
 //   o_ir = e^{G_ir} ((q X0^T)_ir + (M k~)_ir),  k~_jr = k_jr e^{-G_jr},  d = q + o
 // with the decay factored per state row r (wild rows: exact per-term sum).  o is
 // kept beside d for the backward's o dO: taken back from the rounded sum it would
-// hold only the bits above k^'s last (20 us of a training step at B4 T2048 H8 r = V = 256).  M as
-// the prep's Grams, in FP32 over the waves; q X0^T on fp16 matrix cores (q, unit
-// rows, split into high and low halves in LDS; X0 exact in its slot).  Wave w
-// owns the 16-row blocks w, w + 8.  117 us (4.6 TB/s) at B4 T2048 H8 r = V = 256, where
-// four waves with 4-byte panel accesses took 208 us.
+// hold only the bits above k^'s last.  M as the prep's Grams, in FP32 over the
+// waves; q X0^T on fp16 matrix cores (q, unit rows, split into high and low halves
+// in LDS; X0 exact in its slot).  Wave w owns the 16-row blocks w, w + 8.  134 us
+// (288 KiB a chunk, 4.5 TB/s) at B4 T2048 H8 r = V = 256, 117 without o; four waves
+// with 4-byte panel accesses took 208 us.
 __global__ __launch_bounds__(PT, 4) void k_w_out_c(OutParams p) {
   extern __shared__ __align__(16) float sm[];
   const int ch = blockIdx.x, s = blockIdx.y, kw = p.kw, nkb = kw / 16;
