@@ -225,7 +225,10 @@ __global__ __launch_bounds__(NTHREADS) void k_conv_bwd(ConvArgs a, const __bf16*
 // out[i] = sum_p part[p][i]: COLS columns x 256 / COLS partial rows per workgroup,
 // the row sums combined through LDS.  32 columns (whole lines) for wide sums; 8
 // where the width alone would leave the chip idle and each thread a long chain
-// of loads (1024 rows of 128: 11 us with 32 columns, 4 workgroups).
+// of loads (1024 rows of 128: 11 us with 32 columns, 4 workgroups).  The row sums are
+// added in chains of eight, the chains pairwise: one chain of 32 doubled the
+// rounding error (125 rows of sums of 16 terms in [1, 2]: 8.9e-8 relative; 5.3e-8
+// with the eight row sums of 32 columns, 4.3e-8 in chains).
 template <int COLS>
 __global__ __launch_bounds__(NTHREADS) void k_sum_parts(const float* __restrict__ part, int nparts,
                                                         int width, float* __restrict__ out) {
@@ -241,10 +244,15 @@ __global__ __launch_bounds__(NTHREADS) void k_sum_parts(const float* __restrict_
   red[ry][cx] = s;
   __syncthreads();
   if (ry == 0 && i < width) {
-    float t = 0.f;
+    constexpr int NC = ROWS / 8;
+    float t[NC] = {};
 #pragma unroll
-    for (int k = 0; k < ROWS; ++k) t += red[k][cx];
-    out[i] = t;
+    for (int k = 0; k < ROWS; ++k) t[k % NC] += red[k][cx];
+#pragma unroll
+    for (int n = NC / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int k = 0; k < n; ++k) t[k] += t[k + n];
+    out[i] = t[0];
   }
 }
 

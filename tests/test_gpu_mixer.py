@@ -112,6 +112,30 @@ def test_kda_gate_widths_and_tails(B, T, H, r):
         assert rel(a.float(), b) < tol, name
 
 
+def test_narrow_column_sums_lose_no_more_than_eight_chains():
+    """The gate's bias gradient with exact terms (sigmoid 1, rate 1), so that its
+    error is the summation's alone: no larger than with the partial rows taken in
+    eight chains and these added one by one (emulated in FP32)."""
+    from solvedelta_amd import mixer as mx
+    N, H, r = 2000, 4, 128
+    g = torch.rand(1, N, H, r, generator=torch.Generator().manual_seed(5)) + 1
+    raw = torch.full((1, N, H, r), 100.0, dtype=torch.bfloat16, device="cuda")
+    rate, bias = torch.zeros(H, device="cuda"), torch.zeros(H, r, device="cuda", requires_grad=True)
+    db, = torch.autograd.grad(mx.kda_decay_gate(raw, rate, bias), bias, g.cuda())
+    g = -g.view(N, H * r)
+    def chain(rows):
+        s = torch.zeros(H * r)
+        for x in rows:
+            s = s + x
+        return s
+    parts = [chain(g[i:i + 16]) for i in range(0, N, 16)]
+    eight = chain([chain(parts[k::8]) for k in range(8)])
+    ref = g.double().sum(0)
+    err = lambda x: (x.double().view(-1) / ref - 1).square().mean().sqrt().item()
+    print(f"[narrow sums] {err(db.cpu()):.2e}, eight chains {err(eight):.2e}", flush=True)
+    assert err(db.cpu()) <= err(eight)
+
+
 @pytest.mark.parametrize("N,D,off", [(1, 8, 0), (131, 64, 0), (300, 72, 0), (65, 128, 0), (70000, 128, 0),
                                      (33, 136, 0), (129, 256, 0), (77, 100, 0), (40, 64, 1),
                                      (65535, 128, 0), (65537, 72, 0), (131073, 64, 0), (65537, 200, 0)])
